@@ -76,7 +76,10 @@ struct Seg {
   long long P;
   const dev::Term* hx;         // [n var][hxT][n eq]
   const dev::Term* ht;         // [htT][n eq]
-  const int* hx_cnt;           // [n] real terms per Jacobian column (max over equations)
+  // real terms per Jacobian column (max over equations), 16 bits each; hx_cnt
+  // (device memory) replaces them when a count does not fit, else nullptr
+  unsigned int hxc[kMaxN / 2];
+  const int* hx_cnt;
   const double2* start;        // [K][start_stride]
   const double2* chx;          // [I][C+1][M+1]
   const double2* cht;          // [I][C+1][M]
@@ -142,6 +145,20 @@ __device__ __forceinline__ T* iteration_view(T* p, int iter) {
   return p;
 }
 
+// Real terms of Jacobian column j (j a compile-time constant after
+// unrolling).  The counts travel in the kernel arguments: read from device
+// memory, each column's count was a vector load and a full memory latency at
+// the head of the column's loop (the compiler cannot prove the memory
+// constant).  Size-specialised instances (their tables fit LDS) always have
+// 16-bit counts.
+template <bool PACKED, class SegT>
+__device__ __forceinline__ int column_terms(const SegT& S, int j) {
+  if constexpr (!PACKED) {
+    if (S.hx_cnt) return S.hx_cnt[j];
+  }
+  return (int)((S.hxc[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+}
+
 // ------------------------------------------------------------ evaluation
 // sum_k s_k * coef[c_k] * prod_{d < NV} x[var_kd] over the cnt terms of one
 // table row (records n apart from tp, full Term records in global memory or
@@ -187,7 +204,7 @@ __device__ __forceinline__ void eval_jac_row(const SegT& S, int n, int gle, cons
   for (int j = 0; j < NMAX; ++j) {
     cx<T> acc = cmk<T>(0, 0);
     if (j < n) {
-      const int cnt = S.hx_cnt[j];
+      const int cnt = column_terms<LT>(S, j);
       if constexpr (LT) {
         const CTerm<DEG>* tp = static_cast<const CTerm<DEG>*>(lt) + (size_t)j * S.hxT * n + gle;
 #pragma unroll kTermUnroll<T>

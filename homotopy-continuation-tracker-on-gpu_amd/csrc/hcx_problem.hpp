@@ -21,6 +21,8 @@ struct hcx_problem {
   hcx::dev::Term* d_hx = nullptr;
   hcx::dev::Term* d_ht = nullptr;
   int* d_hx_cnt = nullptr;
+  unsigned int hxc[hcx::kMaxN / 2] = {};  // the same counts, 16 bits each ...
+  bool hxc_fits = false;                  // ... when every count fits
   int* d_cslot = nullptr;              // [C+1] LDS slot of each coefficient
   int* d_cinv = nullptr;               // [C+1] coefficient of each slot
   uint32_t* d_ctab = nullptr;          // compact hx + ht tables (8-byte terms), or null

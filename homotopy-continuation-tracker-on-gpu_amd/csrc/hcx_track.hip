@@ -529,7 +529,7 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
     in_set = in_set && (n == 3 || n == 5 || n == 6 || n == 9 || n == 12) && Gs[s] == n;
     const void* ct = t4 ? (const void*)probs[s]->d_ctab4 : (const void*)probs[s]->d_ctab;
     const int cb = t4 ? probs[s]->ctab4_bytes : probs[s]->ctab_bytes;
-    tab_ok = tab_ok && ct && cb <= kMaxTabLds;
+    tab_ok = tab_ok && ct && cb <= kMaxTabLds && probs[s]->hxc_fits;
     tab = std::max(tab, cb);
   }
   if (specialize && !same && in_set && tab_ok && max_deg <= 2) {
@@ -586,7 +586,8 @@ void seg_from_problem(Seg& S, SegOut& O, const hcx_problem* p, int G, int mode, 
   S.lds_group = lds_group_bytes(nmax, p->C, p->M);
   S.hx = p->d_hx;
   S.ht = p->d_ht;
-  S.hx_cnt = p->d_hx_cnt;
+  std::memcpy(S.hxc, p->hxc, sizeof(S.hxc));
+  S.hx_cnt = p->hxc_fits ? nullptr : p->d_hx_cnt;
   S.cslot = p->d_cslot;
   S.cinv = p->d_cinv;
   S.ctab = tab4 ? p->d_ctab4 : p->d_ctab;
@@ -940,6 +941,11 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   p->hx_vars = hxv;
   p->ht_vars = htv;
   p->deg = std::max(deg, 2);
+  p->hxc_fits = true;
+  for (int j = 0; j < n; ++j) {
+    p->hxc_fits = p->hxc_fits && hx_cnt[j] <= 0xffff;
+    p->hxc[j >> 1] |= ((unsigned int)hx_cnt[j] & 0xffffu) << (16 * (j & 1));
+  }
   auto fail = [&](hipError_t e, const char* what) {
     set_error("hcx_problem_create: %s: %s", what, hipGetErrorString(e));
     hcx_problem_destroy(p);
