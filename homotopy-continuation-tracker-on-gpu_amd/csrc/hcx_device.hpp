@@ -87,18 +87,36 @@ __device__ __forceinline__ double frcp(double x) {
   r = fma(r, fma(-x, r, 1.0), r);
   return r;
 }
-// Complex reciprocal 1/b by Smith's scaling (as cdiv) with the fast real reciprocal.
+// Complex reciprocal 1/b, without branches (the lanes of a wave hold pivots
+// of either kind, so a branch runs both of its sides).
+// Smith's scaling (as cdiv), the roles of the components selected.
 template <class T>
-__device__ __forceinline__ cx<T> crecip(cx<T> b) {
-  if (fabs(b.re) >= fabs(b.im)) {
-    const T r = b.im * frcp(b.re);
-    const T inv = frcp(b.re + b.im * r);
-    return cmk<T>(inv, -r * inv);
-  } else {
-    const T r = b.re * frcp(b.im);
-    const T inv = frcp(b.re * r + b.im);
-    return cmk<T>(r * inv, -inv);
-  }
+__device__ __forceinline__ cx<T> crecip_smith(cx<T> b) {
+  const bool rbig = fabs(b.re) >= fabs(b.im);
+  const T big = rbig ? b.re : b.im, small = rbig ? b.im : b.re;
+  const T r = small * frcp(big);
+  const T inv = frcp(big + small * r);
+  const T ri = r * inv;
+  return cmk<T>(rbig ? inv : ri, rbig ? -ri : -inv);
+}
+// FP64: conj(b) / |b|^2 with b scaled by a power of two (exact) so that
+// |b|^2 neither overflows nor underflows: one reciprocal in the dependency
+// chain instead of Smith's two.
+__device__ __forceinline__ cx<double> crecip_scaled(cx<double> b) {
+  const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(b.re), fabs(b.im)));
+  const double re = __builtin_amdgcn_ldexp(b.re, e), im = __builtin_amdgcn_ldexp(b.im, e);
+  const double r = __builtin_amdgcn_ldexp(frcp(re * re + im * im), e);
+  return cmk<double>(re * r, -im * r);
+}
+// a * b with the roundings spelled out: products of a.im rounded, those of
+// a.re fused (the mixed loop's results do not depend on what the compiler
+// fuses).
+template <class T>
+__device__ __forceinline__ cx<T> cmul_fused(cx<T> a, cx<T> b) {
+  return cmk<T>(__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.re, b.im, a.im * b.re));
+}
+__device__ __forceinline__ cx<float> cmul_fused(cx<float> a, cx<float> b) {
+  return cmk<float>(__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.re, b.im, a.im * b.re));
 }
 
 template <class T, class U>

@@ -460,36 +460,44 @@ __device__ __forceinline__ T group_max(T v, const Group& g) {
   return v;
 }
 
-// Argmax step of the pivot search: keep the larger candidate, ties to the
-// smaller key (position label << 6 | lane).
-template <class T>
-__device__ __forceinline__ void piv_take(T& v, int& key, T ov, int ok) {
-  const bool take = (ov > v) | ((ov == v) & (ok < key));
-  v = take ? ov : v;
-  key = take ? ok : key;
+// Pivot key of a candidate row: its magnitude's bits above 31 - label, so the
+// largest key is the largest magnitude and, among equal ones, the first row in
+// current row order.  A row that is no candidate holds key 0; a key below 32
+// is a zero magnitude.  FP64 gives up the 5 lowest of its 52 mantissa bits to
+// the label (candidates within 2^-47 of each other count as equal); FP32
+// magnitudes stay whole.  NaN orders above every number.
+__device__ __forceinline__ unsigned long long pivot_key(double mag, int label) {
+  return ((unsigned long long)__double_as_longlong(mag) & ~31ull) | (unsigned int)(31 - label);
+}
+__device__ __forceinline__ unsigned long long pivot_key(float mag, int label) {
+  return ((unsigned long long)(__float_as_uint(mag) & 0x7fffffffu) << 32) | (unsigned int)(31 - label);
 }
 
-// Pivot argmax over the group: GC = compile-time lanes per path when that is
-// a power of two (aligned groups; DPP inside 16-lane rows, one lane exchange
-// per further doubling), else 0 (ring of ceil(log2 G) lane exchanges).
-template <int GC, class T>
-__device__ __forceinline__ void group_argmax(T& v, int& key, const Group& g) {
-  if constexpr (GC > 0) {
-    static_assert(is_pow2(GC) && GC <= 64, "aligned power-of-two groups");
-    if constexpr (GC >= 2) piv_take(v, key, dpp_read<kDppQuadXor1>(v), dpp_read<kDppQuadXor1>(key));
-    if constexpr (GC >= 4) piv_take(v, key, dpp_read<kDppQuadXor2>(v), dpp_read<kDppQuadXor2>(key));
-    if constexpr (GC >= 8) piv_take(v, key, dpp_read<kDppHalfMirror>(v), dpp_read<kDppHalfMirror>(key));
-    if constexpr (GC >= 16) piv_take(v, key, dpp_read<kDppRowMirror>(v), dpp_read<kDppRowMirror>(key));
-    const int lane = g.gbase + g.gl;
-    if constexpr (GC >= 32) piv_take(v, key, lane_read(v, lane ^ 16), lane_read(key, lane ^ 16));
-    if constexpr (GC >= 64) piv_take(v, key, lane_read(v, lane ^ 32), lane_read(key, lane ^ 32));
-  } else {
-    for (int s = 1; s < g.G; s <<= 1) {
-      int src = g.gl + s;
-      src = (src >= g.G ? src - g.G : src) + g.gbase;
-      piv_take(v, key, lane_read(v, src), lane_read(key, src));
-    }
+// Largest key over an aligned group of GC lanes (a power of two), to every
+// lane: DPP inside 16-lane rows, a row swap between the two rows of 32.
+template <int CTRL>
+__device__ __forceinline__ unsigned long long key_max_dpp(unsigned long long k) {
+  const unsigned int lo = (unsigned int)dpp_read<CTRL>((int)(unsigned int)k);
+  const unsigned int hi = (unsigned int)dpp_read<CTRL>((int)(unsigned int)(k >> 32));
+  const unsigned long long o = ((unsigned long long)hi << 32) | lo;
+  return o > k ? o : k;
+}
+template <int GC>
+__device__ __forceinline__ unsigned long long group_max_key(unsigned long long k) {
+  static_assert(is_pow2(GC) && GC <= 32, "aligned power-of-two groups");
+  if constexpr (GC >= 2) k = key_max_dpp<kDppQuadXor1>(k);
+  if constexpr (GC >= 4) k = key_max_dpp<kDppQuadXor2>(k);
+  if constexpr (GC >= 8) k = key_max_dpp<kDppHalfMirror>(k);
+  if constexpr (GC >= 16) k = key_max_dpp<kDppRowMirror>(k);
+  if constexpr (GC >= 32) {
+    // rows (0, 0, 2, 2) and (1, 1, 3, 3) of the wave
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned int)k, (unsigned int)k, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned int)(k >> 32), (unsigned int)(k >> 32), false, false);
+    const unsigned long long u = ((unsigned long long)hi[0] << 32) | lo[0];
+    const unsigned long long v = ((unsigned long long)hi[1] << 32) | lo[1];
+    k = u > v ? u : v;
   }
+  return k;
 }
 
 // Sums over the group's rows of two per-row values (the corrector's and the
@@ -540,73 +548,84 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 // makes every component NaN (the reference's division by a zero U_ii gives
 // NaN in that component and in the rows that depend on it; the tracker only
 // reacts to whether any component is not finite).
-template <int NMAX, int GC, class T>
+//
+// The solve is a chain of n steps, each bound by its latencies: find the
+// pivot, broadcast its row, update.  So
+//  * a candidate packs its magnitude and position into one 64-bit key; the
+//    largest comes from DPP row permutations (aligned power-of-two groups) or
+//    from an LDS maximum per group and step (one instruction and one read in
+//    place of a scan of every candidate's magnitude);
+//  * the next step's candidates enter their search as soon as their column is
+//    updated, and the remaining columns are updated while it is under way;
+//  * every candidate computes the reciprocal of its own entry during the
+//    search, and the pivot's goes out with its row.
+// keys: NMAX LDS slots of the group (unused with GC > 0).
+// SCALED: the FP64 reciprocal with one step less in its chain; the mixed loop
+// keeps Smith's, since the last bits of its FP64 corrector decide which FP32
+// point the next predictor starts from.
+template <int NMAX, int GC, bool SCALED, class T>
 __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const Group& g, int n, bool row,
-                                                cx<T>* sp, bool& singular) {
+                                                cx<T>* sp, unsigned long long* keys, bool& singular) {
   int label = g.gl;
   cx<T> own_rinv = cmk<T>(T(0), T(0));  // 1 / U_ii of the row this lane ends up holding
   singular = false;
+  if constexpr (GC == 0) {
+    // the replicas of a group hold the same rows: replica 0 searches
+    if (row && g.s == 0) keys[g.gl] = 0ull;
+  }
   // sp shares the group's LDS slots with x: the evaluation's reads of x come first
   HCX_WAVE_SYNC();
+  unsigned long long key = 0;
+  auto search = [&](int k) {
+    const bool cand = row && label >= k;
+    key = cand ? pivot_key(cabs1(A[k]), label) : 0ull;
+    if constexpr (GC > 0) {
+      key = group_max_key<GC>(key);
+    } else {
+      if (cand && g.s == 0)
+        __hip_atomic_fetch_max(&keys[k], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    }
+  };
+  search(0);
 #pragma unroll
   for (int k = 0; k < NMAX; ++k) {
     if (k < n) {
-      T v = (row && label >= k) ? cabs1(A[k]) : T(-1);
-      if (v != v) v = T(INFINITY);
-      int blabel;
-      bool piv, zero;
-      if constexpr (GC > 0) {
-        int key = (label << 6) | g.gl;
-        group_argmax<GC>(v, key, g);
-        blabel = key >> 6;
-        zero = !(v > T(0));
-        piv = g.gl == (key & 63);
-      } else {
-        // other group sizes: the candidates publish their magnitudes by
-        // position label and every lane scans them in current row order
-        // (one LDS round trip instead of a ring of lane exchanges)
-        T* mag = reinterpret_cast<T*>(sp);
-        if (row && label >= k) mag[label] = v;
+      cx<T> rinv;
+      if constexpr (SCALED) rinv = crecip_scaled(A[k]);
+      else rinv = crecip_smith(A[k]);
+      if constexpr (GC == 0) {
         HCX_WAVE_SYNC();
-        T best = mag[k];
-        blabel = k;
-#pragma unroll
-        for (int j = k + 1; j < NMAX; ++j) {
-          if (j < n) {
-            const T mj = mag[j];
-            if (mj > best) {
-              best = mj;
-              blabel = j;
-            }
-          }
-        }
-        HCX_WAVE_SYNC();
-        zero = !(best > T(0));
-        piv = row && label == blabel;
+        key = keys[k];
       }
+      const int blabel = 31 - (int)((unsigned int)key & 31u);
+      const bool zero = key < 32ull;
+      const bool piv = row && label == blabel;
       singular = singular || zero;
-      if (g.in_grp && piv) {
-#pragma unroll
-        for (int j = k; j < NMAX; ++j)
-          if (j < n) sp[j] = A[j];
-        sp[NMAX] = b;
-      }
-      HCX_WAVE_SYNC();
-      if (piv) label = k;
-      else if (label == k) label = blabel;
-      const cx<T> rinv = zero ? cmk<T>(T(1), T(0)) : crecip(sp[k]);
-      if (piv) own_rinv = rinv;
-      if (row && !piv && !zero) {
-        const cx<T> l = cmul(A[k], rinv);
+      if (piv) {
+        sp[k] = rinv;
 #pragma unroll
         for (int j = k + 1; j < NMAX; ++j)
-          if (j < n) A[j] = cfnms(A[j], l, sp[j]);
-        b = cfnms(b, l, sp[NMAX]);
+          if (j < n) sp[j] = A[j];
+        sp[NMAX] = b;
+        own_rinv = rinv;
       }
+      HCX_WAVE_SYNC();
+      label = piv ? k : (label == k ? blabel : label);
+      const bool upd = row && !piv && !zero;
+      cx<T> l = cmul_fused(A[k], sp[k]);
+      l = cmk<T>(upd ? l.re : T(0), upd ? l.im : T(0));
+      if (k + 1 < NMAX && k + 1 < n) {
+        A[k + 1] = cfnms(A[k + 1], l, sp[k + 1]);
+        search(k + 1);
+      }
+#pragma unroll
+      for (int j = k + 2; j < NMAX; ++j)
+        if (j < n) A[j] = cfnms(A[j], l, sp[j]);
+      b = cfnms(b, l, sp[NMAX]);
       HCX_WAVE_SYNC();
     }
   }
-  const cx<T> xi = cmul(b, own_rinv);
+  const cx<T> xi = cmul_fused(b, own_rinv);
   if (row) sp[label] = xi;
   HCX_WAVE_SYNC();
   cx<T> sol = row ? sp[g.gl] : cmk<T>(T(0), T(0));
@@ -644,16 +663,20 @@ __device__ __forceinline__ const void* stage_terms(const Seg& S, int n, unsigned
   return d;
 }
 
-// Per-group view of the LDS region.  x (read by the evaluation) and the
-// pivot-row buffer (written by the LU that follows it) are never live at the
-// same time, so they share the first NMAX + 1 slots; group_lu_solve starts
-// with a wave-scope fence that keeps the evaluation's reads before its writes.
-template <int NMAX>
+// Per-group view of the LDS region: x / pivot row, pivot keys, coefficients.
+// x (read by the evaluation) and the pivot-row buffer (written by the LU that
+// follows it) are never live at the same time, so they share the first
+// NMAX + 1 slots; group_lu_solve starts with a wave-scope fence that keeps
+// the evaluation's reads before its writes.  KEYS: the instance searches
+// pivots through LDS (no DPP groups).
+constexpr int key_bytes(int nmax, bool keys) { return keys ? (8 * nmax + 15) & ~15 : 0; }
+template <int NMAX, bool KEYS>
 struct Lds {
   unsigned char* base;
   __device__ cx<double>* x64() const { return reinterpret_cast<cx<double>*>(base); }
   __device__ cx<double>* piv64() const { return x64(); }
-  __device__ unsigned char* coef() const { return reinterpret_cast<unsigned char*>(x64() + (NMAX + 1)); }
+  __device__ unsigned long long* keys() const { return reinterpret_cast<unsigned long long*>(x64() + (NMAX + 1)); }
+  __device__ unsigned char* coef() const { return base + 16 * (NMAX + 1) + key_bytes(NMAX, KEYS); }
   template <class T>
   __device__ cx<T>* x() const { return reinterpret_cast<cx<T>*>(base); }
   template <class T>
@@ -665,7 +688,7 @@ struct Lds {
 // set of groups to correct; ok / inf return the reference's r_isSuccessful /
 // r_isInfFail.
 template <int NMAX, int GC, int DEG, class T, bool LT, class OT, class SegT>
-__device__ __forceinline__ void newton_pass(const SegT& S, int n, const OT& o, const Group& g, const Lds<NMAX>& L,
+__device__ __forceinline__ void newton_pass(const SegT& S, int n, const OT& o, const Group& g, const Lds<NMAX, GC == 0>& L,
                                             const void* lt, bool run, bool row, cx<double>& x, int& nnewt, bool& ok,
                                             bool& inf) {
   ok = false;
@@ -681,7 +704,7 @@ __device__ __forceinline__ void newton_pass(const SegT& S, int n, const OT& o, c
     eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
     const cx<T> h = eval_t_row<DEG, T, LT>(S, n, gle, sx, sc, lt);
     bool sing;
-    const cx<T> d = group_lu_solve<NMAX, GC, T>(A, h, g, n, row, L.template piv<T>(), sing);
+    const cx<T> d = group_lu_solve<NMAX, GC, false, T>(A, h, g, n, row, L.template piv<T>(), L.keys(), sing);
     if (run && row) x = csub(x, ccast<double>(d));
     double rs = row ? (double)cnorm2(d) : 0.0;
     double rc = row ? cnorm2(x) : 0.0;
@@ -706,7 +729,7 @@ using namespace dev;
 // sd_ext: dc/dt table of the group's instance in global memory (constant in t,
 // M = 1) or nullptr to stage dc/dt(t) in LDS next to c(t).
 template <int NMAX, int GC, int DEG, class T, bool LT, class SegT>
-__device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group& g, const Lds<NMAX>& L, const void* lt,
+__device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group& g, const Lds<NMAX, GC == 0>& L, const void* lt,
                                               bool act, bool row, int gle, int inst, double ts, double dt,
                                               cx<double> xl, const cx<T>* sd_ext) {
   const double h = 0.5 * dt;
@@ -725,7 +748,7 @@ __device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group&
     eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
     const cx<T> bt = eval_t_row<DEG, T, LT>(S, n, gle, sx, sd, lt, sd_ext ? S.cinv : nullptr);
     bool sing;
-    const cx<T> k = group_lu_solve<NMAX, GC, T>(A, cmk<T>(-bt.re, -bt.im), g, n, row, L.template piv<T>(), sing);
+    const cx<T> k = group_lu_solve<NMAX, GC, false, T>(A, cmk<T>(-bt.re, -bt.im), g, n, row, L.template piv<T>(), L.keys(), sing);
     kprev = ccast<double>(k);
     const double w = (st == 1 || st == 2) ? 2.0 : 1.0;
     acc = cmk<double>(acc.re + w * kprev.re, acc.im + w * kprev.im);
@@ -777,7 +800,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
   // lanes outside the full groups (64 % G of them) alias region 0: they
   // track nothing and store nothing to LDS
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
-  Lds<NMAX> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
+  Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
 
   // per-group path state, replicated over the group's lanes
   long long path = -1;
@@ -960,7 +983,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
           eval_jac_row<NMAX, DEG, double, LT>(Sk, n, gle, sx, sc, A, lt);
           const cx<double> hv = eval_t_row<DEG, double, LT>(Sk, n, gle, sx, sc, lt);
           bool sing;
-          const cx<double> d = group_lu_solve<NMAX, GC, double>(A, hv, g, n, row, L.template piv<double>(), sing);
+          const cx<double> d = group_lu_solve<NMAX, GC, false, double>(A, hv, g, n, row, L.template piv<double>(), L.keys(), sing);
           if (run && row) x = csub(x, d);
           double nd = row ? cnorm2(d) : 0.0, nx = row ? cnorm2(x) : 0.0;
           nd = group_sum(nd, g, lane);
@@ -1130,7 +1153,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
     }
   }
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
-  Lds<NMAX> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
+  Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
   cx<double>* sx = L.template x<double>();
   const cx<double>* sc = reinterpret_cast<const cx<double>*>(L.coef());
   // dc/dt of the RK4 stages: constant (M = 1) -> read from the instance's
@@ -1280,7 +1303,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       }
       bool sing;
       const cx<double> d =
-          group_lu_solve<NMAX, GC, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.template piv<double>(), sing);
+          group_lu_solve<NMAX, GC, true, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.template piv<double>(), L.keys(), sing);
 
       // RK4 stage: k_s = solution, accumulate k1 + 2 k2 + 2 k3 + k4
       if (stg) {

@@ -478,15 +478,15 @@ Opts to_opts(const hcx_track_opts* o) {
 // coefficient area: with M = 1 (dc/dt constant, read by the FP64 stages from
 // the instance's table in global memory) FP32 c + dc/dt overlaid by FP64 c,
 // else (or dot_lds: FP64 stages with dc/dt in LDS) FP64 c + dc/dt.
-// The region stride is padded to 16 mod 256 bytes: the groups of a wave read
+// An instance without DPP groups (keys) has its pivot keys there too.
+// The region stride is an odd multiple of 16 bytes: the groups of a wave read
 // the same offsets of their regions together (pivot-row broadcasts, x and
-// coefficient gathers), and this stride spreads them over distinct LDS banks
+// coefficient gathers), and such a stride spreads them over distinct LDS banks
 // (64 banks x 4 bytes) for 8- and 16-byte accesses.
-int lds_group_bytes(int nmax, int C, int M, bool dot_lds = false) {
+int lds_group_bytes(int nmax, bool keys, int C, int M, bool dot_lds = false) {
   const int per = (M > 1 || dot_lds) ? 32 : 16;
-  int b = 16 * (nmax + 1) + (C + 1) * per;
-  b = (b + 15) & ~15;
-  return ((b - 16 + 255) / 256) * 256 + 16;
+  const int b = 16 * (nmax + 1) + dev::key_bytes(nmax, keys) + (C + 1) * per;
+  return (((b + 15) / 16) | 1) * 16;
 }
 
 struct Plan {
@@ -497,6 +497,7 @@ struct Plan {
   int tab_lds = 0;   // LDS bytes of the compact tables (instances that hold them there)
   size_t lds = 0;
   KernelFn fn = nullptr;
+  bool keys() const { return !(exact && is_pow2(exact_lanes(nmax))); }  // pivot keys in LDS
 };
 
 // Largest compact table the size-specialised instances (up to n = 16; n = 30
@@ -571,7 +572,7 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
 }
 
 // Fills the segment-independent part of a Seg from a problem.
-void seg_from_problem(Seg& S, SegOut& O, const hcx_problem* p, int G, int mode, int nmax, bool tab4) {
+void seg_from_problem(Seg& S, SegOut& O, const hcx_problem* p, int G, const Plan& pl) {
   std::memset(&S, 0, sizeof(S));
   std::memset(&O, 0, sizeof(O));
   O.roots_stride = p->n;
@@ -583,14 +584,14 @@ void seg_from_problem(Seg& S, SegOut& O, const hcx_problem* p, int G, int mode, 
   S.htT = p->htT;
   S.G = G;
   S.R = 1;
-  S.lds_group = lds_group_bytes(nmax, p->C, p->M);
+  S.lds_group = lds_group_bytes(pl.nmax, pl.keys(), p->C, p->M);
   S.hx = p->d_hx;
   S.ht = p->d_ht;
   std::memcpy(S.hxc, p->hxc, sizeof(S.hxc));
   S.hx_cnt = p->hxc_fits ? nullptr : p->d_hx_cnt;
   S.cslot = p->d_cslot;
   S.cinv = p->d_cinv;
-  S.ctab = tab4 ? p->d_ctab4 : p->d_ctab;
+  S.ctab = pl.tab4 ? p->d_ctab4 : p->d_ctab;
   S.start = p->d_start;
   S.start_stride = p->n;
 }
@@ -658,7 +659,7 @@ hcx_status choose_waves_per_block(Launch& LN, Plan& pl, int& best_wpb, int& best
 // tables), so that at least two waves share a CU.
 int default_lanes(int n, int C, int M) {
   const int ni = round_up_idx(kNmaxList, 3, n);
-  const int lg = lds_group_bytes(ni < 0 ? n : kNmaxList[ni], C, M);
+  const int lg = 16 * ((ni < 0 ? n : kNmaxList[ni]) + 1) + (C + 1) * (M > 1 ? 32 : 16) + 256;
   int G = exact_lanes(n);
   while (G < 64 && (size_t)(64 / G) * (size_t)lg > 65536) ++G;
   return G;
@@ -1156,7 +1157,6 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   Plan pl;
   st = choose_kernel(nseg, probs, Gs, max_deg, o->precision, specialize, pl);
   if (st != HCX_OK) return st;
-  const int nmax = pl.nmax;
   long long total_groups_needed = 0;
   std::vector<long long> seg_groups(nseg);
   for (int s = 0; s < nseg; ++s) {
@@ -1172,7 +1172,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     const int G = Gs[s];
     Seg& S = LN.seg[s];
     SegOut& O = OP.out[s];
-    seg_from_problem(S, O, p, G, o->precision, nmax, pl.tab4);
+    seg_from_problem(S, O, p, G, pl);
     S.I = b.num_instances;
     S.P = (long long)b.num_instances * p->K;
     if (empty) {
@@ -1244,7 +1244,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   if (o->precision == HCX_PREC_FP64 && nseg == 1 && (total_groups_needed <= 4LL * g_cu || o->replicas > 1)) {
     Seg& S = LN.seg[0];
     const hcx_problem* p = probs[0];
-    const int lg = lds_group_bytes(nmax, p->C, p->M, true);
+    const int lg = lds_group_bytes(pl.nmax, pl.keys(), p->C, p->M, true);
     const size_t terms =
         pl.exact ? 0 : ((size_t)p->n * p->n * p->hxT + (size_t)p->n * p->htT) * sizeof(dev::Term);
     auto waves = [&](int R) {
@@ -1388,10 +1388,10 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     size_t need = 0;
     for (int s = 0; s < nseg; ++s)
       need = std::max(need, (size_t)(64 / L2.seg[s].G) *
-                                (size_t)lds_group_bytes(p2.nmax, probs[s]->C, probs[s]->M, true));
+                                (size_t)lds_group_bytes(p2.nmax, p2.keys(), probs[s]->C, probs[s]->M, true));
     L2.dot_lds = need + (size_t)p2.tab_lds <= 65536 ? 1 : 0;
     for (int s = 0; s < nseg; ++s)
-      L2.seg[s].lds_group = lds_group_bytes(p2.nmax, probs[s]->C, probs[s]->M, L2.dot_lds != 0);
+      L2.seg[s].lds_group = lds_group_bytes(p2.nmax, p2.keys(), probs[s]->C, probs[s]->M, L2.dot_lds != 0);
     st = finish_plan(L2, p2);
     if (st != HCX_OK) return st;
     // a small persistent grid: the list holds few paths; idle waves exit at once
@@ -1471,7 +1471,7 @@ double hcx_kernel_HC_Solver(void* stream, const hcx_problem* pc, int max_steps, 
   if (choose_kernel(1, &p, &G, p->deg, HCX_PREC_FP64, 1, pl) != HCX_OK) return -1.0;
   Seg& S = LN.seg[0];
   SegOut& O = OP.out[0];
-  seg_from_problem(S, O, p, G, HCX_PREC_FP64, pl.nmax, pl.tab4);
+  seg_from_problem(S, O, p, G, pl);
   S.start = reinterpret_cast<const double2*>(d_start_sols);
   S.start_stride = p->n + 1;
   O.roots = reinterpret_cast<double2*>(d_track);
@@ -1636,7 +1636,7 @@ hcx_status hcx_autotune(hcx_problem* p, const hcx_batch_desc* sample, const hcx_
       std::memset(&LN, 0, sizeof(LN));
       SegOut O;
       LN.nseg = 1;
-      seg_from_problem(LN.seg[0], O, p, G, o->precision, pl.nmax, pl.tab4);
+      seg_from_problem(LN.seg[0], O, p, G, pl);
       if (finish_plan(LN, pl) == HCX_OK)
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(pl.fn), 64, pl.lds);
     }
