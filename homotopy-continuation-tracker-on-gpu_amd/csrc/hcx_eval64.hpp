@@ -1,0 +1,437 @@
+// Evaluation of the FP64 micro-step loop: term streams, coefficient staging.
+//
+// A row's terms are a STREAM per lane: position p of equation i at
+// [p][i], all positions of Jacobian column 0, then of column 1, and so on
+// (dH/dx), or all terms of the row (dH/dt, H), in the order of the problem's
+// tables.  The number of positions is the maximum over the equations; an
+// equation with fewer terms holds zero terms at its end (a variable index
+// that reads the constant 0).  A column begins with the positions up to the
+// last one at which some equation has a scalar other than 1 ("scaled"), the
+// rest needs no scaling.  Every instance adds the terms of a row in stream
+// order as acc = fma(coefficient, product of the variables, acc), the scalar
+// applied to the first variable, so instances that differ only in where the
+// streams live give the same bits.
+//
+// What bounds it: per term two or three 16-byte LDS gathers and four FP64
+// FMAs; everything else is overhead, so the records in LDS hold byte offsets
+// (no decoding beyond a mask and an add), unscaled positions skip the scaling,
+// and the counts come from the kernel arguments.
+#pragma once
+
+namespace hcx {
+namespace dev {
+
+__device__ __forceinline__ cx<double> lds_at(const unsigned char* base, uint32_t off) {
+  return *reinterpret_cast<const cx<double>*>(base + off);
+}
+
+// Compact records of the size-specialised instances, in LDS: byte offsets of
+// the coefficient slot (16 bits, from the group's coefficient area) and of
+// the variables (10 bits, from its x area), the scalar in the spare bits.
+//   word 0: c | v0 << 16 | low 6 bits of s << 26
+//   word 1: degree <= 2 (H only): v1 | j << 16
+//           degree 3, 4:          v1 | v2 << 16 | high 6 bits of s << 26
+//   word 2: degree 3, 4 (H only): v3 | j << 16   (word 3 unused)
+// with j the coefficient's number (index of dc/dt in global memory) and s 6
+// bits (degree <= 2) or 12, two's complement.
+template <int DEG>
+struct StreamRec {
+  static constexpr int kJ = DEG <= 2 ? 4 : 8;
+  static constexpr int kH = DEG <= 2 ? 8 : 16;
+};
+template <int DEG>
+__device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
+  if constexpr (DEG <= 2) return (double)((int)r0 >> 26);
+  return (double)((((int)r1 >> 26) << 6) | (int)(r0 >> 26));
+}
+
+// acc + one Jacobian term (xb, cb: the group's x and coefficient areas); SC: a
+// scaled position.
+template <int DEG, bool SC>
+__device__ __forceinline__ cx<double> jac_term(const unsigned char* rp, const unsigned char* xb,
+                                               const unsigned char* cb, cx<double> acc) {
+  uint32_t r0, r1 = 0;
+  if constexpr (DEG <= 2) {
+    r0 = *reinterpret_cast<const uint32_t*>(rp);
+  } else {
+    const uint2 q = *reinterpret_cast<const uint2*>(rp);
+    r0 = q.x;
+    r1 = q.y;
+  }
+  cx<double> p = lds_at(xb, (r0 >> 16) & 0x3ffu);
+  const cx<double> c = lds_at(cb, r0 & 0xffffu);
+  if constexpr (SC) p = cscale(p, rec_scalar<DEG>(r0, r1));
+  if constexpr (DEG > 2) p = cmul(p, lds_at(xb, r1 & 0xffffu));
+  if constexpr (DEG > 3) p = cmul(p, lds_at(xb, (r1 >> 16) & 0x3ffu));
+  return cfma(acc, c, p);
+}
+
+// Row gl of dH/dx from the compact streams at lt
+// (dev-eval-indxing-generalized_3views_4pts.cuh:70-86).  Positions k0, k0 +
+// ks, ... of each column only (a replica's share).
+template <int NMAX, int DEG, int UNR, class SegT>
+__device__ __forceinline__ void eval_jac_stream(const SegT& S, int gle, const unsigned char* xb,
+                                                const unsigned char* cb, cx<double> (&A)[NMAX],
+                                                const unsigned char* lt, int k0, int ks) {
+  constexpr int RS = StreamRec<DEG>::kJ;
+  const unsigned char* rp = lt + gle * RS;
+#pragma unroll
+  for (int j = 0; j < NMAX; ++j) {
+    const unsigned int cc = S.colc[j];
+    const int cnt = (int)(cc & 0xffffu), ns = (int)(cc >> 16);
+    cx<double> acc = cmk<double>(0, 0);
+    int k = k0;
+    for (; k < ns; k += ks) acc = jac_term<DEG, true>(rp + k * (NMAX * RS), xb, cb, acc);
+#pragma unroll UNR
+    for (; k < cnt; k += ks) acc = jac_term<DEG, false>(rp + k * (NMAX * RS), xb, cb, acc);
+    rp += cnt * (NMAX * RS);
+    A[j] = acc;
+  }
+}
+
+// Jacobian records of the latency instances: the scalar as the high word of
+// its double (the low word is 0), and one row of zero terms after each
+// column's positions.
+//   degree <= 2:  {c | v0 << 16, s}     degree 3, 4:  {c | v0 << 16, v1 | v2 << 16, s, 0}
+template <int DEG>
+struct LatencyRec {
+  static constexpr int kJ = DEG <= 2 ? 8 : 16;
+};
+
+// Row gl of dH/dx on the latency instances (one wave per SIMD: every LDS
+// round trip is exposed).  Round by round, one term of every column at once:
+// all records of up to eight columns are requested together, then all their
+// gathers, so a round costs two LDS latencies instead of two per column.
+// Replica s of R takes positions s, s + R, ...; past a column's last position
+// it reads the column's zero terms.
+template <int NMAX, int DEG, class SegT>
+__device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const unsigned char* xb,
+                                                const unsigned char* cb, cx<double> (&A)[NMAX],
+                                                const unsigned char* lt, int k0, int ks) {
+  constexpr int RS = LatencyRec<DEG>::kJ;
+  constexpr int NB = NMAX <= 8 ? NMAX : (NMAX + 1) / 2;  // columns at a time
+  const int rounds_end = S.max_terms;
+#pragma unroll
+  for (int j = 0; j < NMAX; ++j) A[j] = cmk<double>(0, 0);
+#pragma unroll 1
+  for (int r = 0; r < rounds_end; r += ks) {
+    const int k = r + k0;
+    const unsigned char* rp = lt + gle * RS;
+#pragma unroll
+    for (int jb = 0; jb < NMAX; jb += NB) {
+      uint32_t r0[NB], r1[NB], rs[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (jb + u < NMAX) {
+          const int cnt = (int)(S.colc[jb + u] & 0xffffu);
+          const unsigned char* a = rp + min(k, cnt) * (NMAX * RS);
+          if constexpr (DEG <= 2) {
+            const uint2 q = *reinterpret_cast<const uint2*>(a);
+            r0[u] = q.x;
+            rs[u] = q.y;
+          } else {
+            const uint4 q = *reinterpret_cast<const uint4*>(a);
+            r0[u] = q.x;
+            r1[u] = q.y;
+            rs[u] = q.z;
+          }
+          rp += (cnt + 1) * (NMAX * RS);
+        }
+      }
+      cx<double> c[NB], p[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (jb + u < NMAX) {
+          c[u] = lds_at(cb, r0[u] & 0xffffu);
+          p[u] = lds_at(xb, r0[u] >> 16);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (jb + u < NMAX) {
+          cx<double> v = cscale(p[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
+          if constexpr (DEG > 2) v = cmul(v, lds_at(xb, r1[u] & 0xffffu));
+          if constexpr (DEG > 3) v = cmul(v, lds_at(xb, r1[u] >> 16));
+          A[jb + u] = cfma(A[jb + u], c[u], v);
+        }
+      }
+    }
+  }
+}
+
+// One chunk of Q terms of a row of dH/dt or H, positions k, k + ks, ...
+// (positions past the last read the zero terms that end the stream).  dot:
+// this lane's group sums dc/dt (an RK4 stage) instead of c(t): from its LDS
+// area at db, or (GDOT) from global memory, requested for the whole chunk
+// before the first product.
+template <int NMAX, int DEG, bool SC, bool GDOT, int Q>
+__device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, int ks, int cnt,
+                                                const unsigned char* xb, const unsigned char* cb,
+                                                const double2* dg, bool dot, cx<double> acc) {
+  constexpr int RS = StreamRec<DEG>::kH;
+  uint32_t r[Q][3];
+  cx<double> c[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const unsigned char* a = rp + min(k + q * ks, cnt) * (NMAX * RS);
+    if constexpr (DEG <= 2) {
+      const uint2 v = *reinterpret_cast<const uint2*>(a);
+      r[q][0] = v.x;
+      r[q][1] = v.y;
+    } else {
+      const uint4 v = *reinterpret_cast<const uint4*>(a);
+      r[q][0] = v.x;
+      r[q][1] = v.y;
+      r[q][2] = v.z;
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) c[q] = lds_at(cb, r[q][0] & 0xffffu);
+  if constexpr (GDOT) {
+    if (dot) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const double2 d = dg[r[q][DEG <= 2 ? 1 : 2] >> 16];
+        c[q] = cmk<double>(d.x, d.y);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    cx<double> p = lds_at(xb, (r[q][0] >> 16) & 0x3ffu);
+    if constexpr (SC) p = cscale(p, rec_scalar<DEG>(r[q][0], r[q][1]));
+    p = cmul(p, lds_at(xb, r[q][1] & 0xffffu));
+    if constexpr (DEG > 2) p = cmul(p, lds_at(xb, (r[q][1] >> 16) & 0x3ffu));
+    if constexpr (DEG > 3) p = cmul(p, lds_at(xb, r[q][2] & 0xffffu));
+    acc = cfma(acc, c[q], p);
+  }
+  return acc;
+}
+
+// Row gl of sum_k s * coef * prod x over the dH/dt streams (…cuh:89-120):
+// H with c(t), dH/dt with dc/dt.
+template <int NMAX, int DEG, bool GDOT, int Q, class SegT>
+__device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int gle, const unsigned char* xb,
+                                                      const unsigned char* cb, const unsigned char* db,
+                                                      const double2* dg, bool dot, const unsigned char* lt, int k0,
+                                                      int ks) {
+  const unsigned char* base = (!GDOT && dot) ? db : cb;
+  const unsigned char* rp = lt + S.tab_h + gle * StreamRec<DEG>::kH;
+  const int cnt = S.htT;
+  cx<double> acc = cmk<double>(0, 0);
+  int k = 0;
+#pragma unroll 1
+  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<NMAX, DEG, true, GDOT, Q>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
+#pragma unroll 1
+  for (; k < cnt; k += Q * ks) acc = rhs_chunk<NMAX, DEG, false, GDOT, Q>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  return acc;
+}
+
+// sum over positions k0, k0 + ks, ... < cnt of a stream of full Term records
+// (n apart from tp; global memory or an LDS copy).  The records of a chunk
+// are requested before the first is used.  GDOT: lanes with dot take dc/dt
+// from global memory (dg, indexed by the coefficient numbers ci).
+template <int NV, bool GDOT>
+__device__ __forceinline__ cx<double> term_stream_sum(const Term* tp, int cnt, int n, const cx<double>* sx,
+                                                      const cx<double>* coef, const double2* dg, const int* ci,
+                                                      bool dot, int k0, int ks) {
+  cx<double> acc = cmk<double>(0, 0);
+  for (int kb = k0; kb < cnt; kb += kTermChunk * ks) {
+    Term tm[kTermChunk];
+    int cj[kTermChunk];
+    cx<double> c[kTermChunk];
+#pragma unroll
+    for (int q = 0; q < kTermChunk; ++q)
+      if (kb + q * ks < cnt) {
+        tm[q] = tp[(size_t)(kb + q * ks) * n];
+        if constexpr (GDOT) cj[q] = ci[(size_t)(kb + q * ks) * n];
+      }
+#pragma unroll
+    for (int q = 0; q < kTermChunk; ++q)
+      if (kb + q * ks < cnt) {
+        c[q] = coef[tm[q].c];
+        if constexpr (GDOT) {
+          if (dot) {
+            const double2 d = dg[cj[q]];
+            c[q] = cmk<double>(d.x, d.y);
+          }
+        }
+      }
+#pragma unroll
+    for (int q = 0; q < kTermChunk; ++q) {
+      if (kb + q * ks < cnt) {
+        cx<double> p = cscale(sx[term_var(tm[q], 0)], (double)tm[q].s);
+#pragma unroll
+        for (int d = 1; d < NV; ++d) p = cmul(p, sx[term_var(tm[q], d)]);
+        acc = cfma(acc, c[q], p);
+      }
+    }
+  }
+  return acc;
+}
+
+// Row gl of dH/dx from the full records: those of the LDS copy at tl, or in
+// global memory (tl null).
+template <int NMAX, int DEG, class SegT>
+__device__ __forceinline__ void eval_jac_terms(const SegT& S, int n, int gle, const cx<double>* sx,
+                                               const cx<double>* sc, cx<double> (&A)[NMAX], const Term* tl, int k0,
+                                               int ks) {
+  size_t off = gle;
+#pragma unroll
+  for (int j = 0; j < NMAX; ++j) {
+    cx<double> acc = cmk<double>(0, 0);
+    if (j < n) {
+      int cnt;
+      if (S.hx_cnt) {
+        cnt = S.hx_cnt[j];
+      } else {
+        cnt = (int)(S.colc[j] & 0xffffu);
+      }
+      if (tl)
+        acc = term_stream_sum<DEG - 1, false>(tl + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
+      else
+        acc = term_stream_sum<DEG - 1, false>(S.hx + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
+      off += (size_t)cnt * n;
+    }
+    A[j] = acc;
+  }
+}
+
+// Row gl of dH/dt or H from the full records (base: c(t) or dc/dt in LDS).
+template <int DEG, bool GDOT, class SegT>
+__device__ __forceinline__ cx<double> eval_rhs_terms(const SegT& S, int n, int gle, const cx<double>* sx,
+                                                     const cx<double>* base, const double2* dg, bool dot,
+                                                     const Term* tl, int k0, int ks) {
+  const int* ci = S.ht_ci + gle;
+  if (tl) return term_stream_sum<DEG, GDOT>(tl + (size_t)S.hx_recs + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
+  return term_stream_sum<DEG, GDOT>(S.ht + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
+}
+
+// ------------------------------------------------------------ staging
+// LDS byte offset of coefficient j's slot from the coefficient area;
+// kNoSlot: no term uses it.
+constexpr uint32_t kNoSlot = 0xffffffffu;
+// SL: the list is in LDS with the compact tables.
+template <bool SL, class SegT>
+__device__ __forceinline__ uint32_t slot_offset(const SegT& S, const unsigned char* lt, int j) {
+  if constexpr (SL) {
+    const uint32_t o = reinterpret_cast<const unsigned short*>(lt + S.tab_slot)[j];
+    return o == 0xffffu ? kNoSlot : o;
+  } else {
+    const int q = S.cslot[j];
+    return q < S.nslot ? (uint32_t)q * 16u : kNoSlot;
+  }
+}
+
+// c_j(t) and (with_dot) dc_j/dt(t) of order MC in t into the group's LDS
+// slots, Q of the lane's coefficients at a time: all of a chunk's loads are
+// requested before the first is used, so the staging costs one memory latency
+// per Q coefficients.  hx, ht: the instance's tables.  Surplus entries of the
+// last chunk repeat the last coefficient.
+template <int MC, int Q, bool SL, class SegT>
+__device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, const double2* hx, const double2* ht,
+                                             double t, unsigned char* cb, unsigned char* db, bool with_dot,
+                                             const unsigned char* lt) {
+  const int C1 = S.C + 1, st = g.G * g.R;
+#pragma unroll 1
+  for (int jb = g.gl + g.s * g.G; jb < C1; jb += Q * st) {
+    double2 a[Q][MC + 1], b[Q][MC];
+    uint32_t o[Q];
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+      const int j = min(jb + u * st, C1 - 1);
+      o[u] = slot_offset<SL>(S, lt, j);
+#pragma unroll
+      for (int m = 0; m <= MC; ++m) a[u][m] = hx[(size_t)((unsigned int)j * (MC + 1) + m)];
+      if (with_dot) {
+#pragma unroll
+        for (int m = 0; m < MC; ++m) b[u][m] = ht[(size_t)((unsigned int)j * MC + m)];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+      double cr = a[u][MC].x, ci = a[u][MC].y;
+#pragma unroll
+      for (int m = MC - 1; m >= 0; --m) {
+        cr = cr * t + a[u][m].x;
+        ci = ci * t + a[u][m].y;
+      }
+      if (o[u] != kNoSlot) *reinterpret_cast<cx<double>*>(cb + o[u]) = cmk<double>(cr, ci);
+      if (with_dot) {
+        double dr = b[u][MC - 1].x, di = b[u][MC - 1].y;
+#pragma unroll
+        for (int m = MC - 2; m >= 0; --m) {
+          dr = dr * t + b[u][m].x;
+          di = di * t + b[u][m].y;
+        }
+        if (o[u] != kNoSlot) *reinterpret_cast<cx<double>*>(db + o[u]) = cmk<double>(dr, di);
+      }
+    }
+  }
+}
+
+// Coefficient polynomials in t of the group's instance into LDS
+// (eval_parameter_homotopy, …cuh:34-67).  Coefficient j goes to slot
+// cslot[j]: slots follow the order in which the rows of a group read them
+// (term by term), so the lanes of a group that read term k of their rows
+// together hit consecutive LDS words instead of words one equation apart; a
+// coefficient that no term uses has no slot.  The replicas of a group share
+// its LDS region and stage every R-th coefficient each.  Q: coefficients in
+// flight per lane at order 1 (fewer at higher orders, by their registers).
+template <bool SL, int Q, class SegT>
+__device__ __forceinline__ void stage_coeffs64(const SegT& S, const Group& g, const double2* hx, const double2* ht,
+                                               double t, unsigned char* cb, unsigned char* db, bool with_dot,
+                                               const unsigned char* lt) {
+  if constexpr (Q >= 8) {
+    // the latency instances: a chunk that fits the lane's share
+    const int st = g.G * g.R;
+    const bool few = S.C + 1 <= 2 * st, some = S.C + 1 <= 4 * st;
+    if (S.M == 1) {
+      if (few) return stage_chunks<1, 2, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+      if (some) return stage_chunks<1, 4, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    } else if (S.M == 2 && few) {
+      return stage_chunks<2, 2, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    }
+  }
+  constexpr int Q2 = Q > 2 ? Q / 2 : 1, Q3 = Q > 3 ? Q / 3 : 1;
+  switch (S.M) {
+    case 1: return stage_chunks<1, Q, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    case 2: return stage_chunks<2, Q2, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    case 3: return stage_chunks<3, Q3, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    case 4: return stage_chunks<4, Q3, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    default: break;
+  }
+  const int C1 = S.C + 1, M = S.M;
+  for (int j = g.gl + g.s * g.G; j < C1; j += g.G * g.R) {
+    const uint32_t o = slot_offset<SL>(S, lt, j);
+    if (o == kNoSlot) continue;
+    const double2* ha = hx + (size_t)j * (M + 1);
+    double cr = ha[M].x, ci = ha[M].y;
+    for (int m = M - 1; m >= 0; --m) {
+      cr = cr * t + ha[m].x;
+      ci = ci * t + ha[m].y;
+    }
+    *reinterpret_cast<cx<double>*>(cb + o) = cmk<double>(cr, ci);
+    if (with_dot) {
+      const double2* hb = ht + (size_t)j * M;
+      double dr = hb[M - 1].x, di = hb[M - 1].y;
+      for (int m = M - 2; m >= 0; --m) {
+        dr = dr * t + hb[m].x;
+        di = di * t + hb[m].y;
+      }
+      *reinterpret_cast<cx<double>*>(db + o) = cmk<double>(dr, di);
+    }
+  }
+}
+
+// x and the constants 1 and 0 (variable indices n and n + 1).
+__device__ __forceinline__ void publish_x64(cx<double>* sx, cx<double> x, const Group& g, int n, bool act, bool row) {
+  if (act && row) sx[g.gl] = x;
+  if (act && g.gl == 0) {
+    sx[n] = cmk<double>(1.0, 0.0);
+    sx[n + 1] = cmk<double>(0.0, 0.0);
+  }
+}
+
+}  // namespace dev
+}  // namespace hcx

@@ -74,19 +74,26 @@ struct Seg {
   int start_stride;
   int I;
   long long P;
-  const dev::Term* hx;         // [n var][hxT][n eq]
+  const dev::Term* hx;         // mixed: [n var][hxT][n eq]; FP64: streams (hcx_eval64.hpp)
   const dev::Term* ht;         // [htT][n eq]
-  // real terms per Jacobian column (max over equations), 16 bits each; hx_cnt
-  // (device memory) replaces them when a count does not fit, else nullptr
-  unsigned int hxc[kMaxN / 2];
+  // terms per Jacobian column (max over equations); FP64 loop: positions of the
+  // column's stream | scaled ones << 16, and where a number does not fit,
+  // hx_cnt (device memory) holds the positions instead (else nullptr)
+  unsigned int colc[kMaxN];
   const int* hx_cnt;
+  const int* ht_ci;            // FP64 loop: coefficient numbers of the ht records
+  // FP64 loop: scaled positions of ht (htT: all); Term
+  // records of hx; coefficients with an LDS slot
+  int htS, hx_recs, nslot;
+  int max_terms;               // positions of the longest column
+  int tab_words;               // 4-byte words of the compact tables
+  int tab_h, tab_slot;         // byte offsets of their H streams and slot list
   const double2* start;        // [K][start_stride]
   const double2* chx;          // [I][C+1][M+1]
   const double2* cht;          // [I][C+1][M]
   const int* cslot;            // [C+1] LDS slot of coefficient j (the tables hold slots)
-  const int* cinv;             // [C+1] coefficient of LDS slot q
-  const uint32_t* ctab;        // compact hx then ht tables (LDS-table instances; 4-byte terms
-                               // for DEG <= 2, else 8-byte)
+  const uint32_t* ctab;        // compact tables (LDS-table instances): mixed: hx then ht, 4-byte
+                               // terms for DEG <= 2, else 8-byte; FP64: streams
   unsigned int* counter;
   const SegOut* out;           // device copy written by init_kernel
   const int* plist;            // optional: track only these paths (count in *plist_count)
@@ -119,6 +126,11 @@ struct Launch {
 typedef const __attribute__((address_space(4))) Opts KOpts;
 typedef const __attribute__((address_space(4))) Seg KSeg;
 
+}  // namespace hcx
+
+#include "hcx_eval64.hpp"
+
+namespace hcx {
 namespace dev {
 
 // The launch's options where the kernel argument holds them (the
@@ -145,44 +157,23 @@ __device__ __forceinline__ T* iteration_view(T* p, int iter) {
   return p;
 }
 
-// Real terms of Jacobian column j (j a compile-time constant after
-// unrolling).  The counts travel in the kernel arguments: read from device
-// memory, each column's count was a vector load and a full memory latency at
-// the head of the column's loop (the compiler cannot prove the memory
-// constant).  Size-specialised instances (their tables fit LDS) always have
-// 16-bit counts.
-template <bool PACKED, class SegT>
-__device__ __forceinline__ int column_terms(const SegT& S, int j) {
-  if constexpr (!PACKED) {
-    if (S.hx_cnt) return S.hx_cnt[j];
-  }
-  return (int)((S.hxc[j >> 1] >> (16 * (j & 1))) & 0xffffu);
-}
-
 // ------------------------------------------------------------ evaluation
 // sum_k s_k * coef[c_k] * prod_{d < NV} x[var_kd] over the cnt terms of one
-// table row (records n apart from tp, full Term records in global memory or
-// in an LDS copy).  The records of a chunk of terms are all requested before
-// the first is used, so their latencies overlap; remap (when not null) maps
-// a record's coefficient number to its index in coef.  Terms k0, k0 + ks,
-// k0 + 2 ks, ... only (the replica's share of the row).
+// table row (full Term records n apart from tp in global memory).  The
+// records of a chunk of terms are all requested before the first is used, so
+// their latencies overlap.
 template <int NV, class T>
-__device__ __forceinline__ cx<T> term_row_sum(const Term* tp, int cnt, int n, const cx<T>* sx, const cx<T>* coef,
-                                              const int* remap, int k0 = 0, int ks = 1) {
+__device__ __forceinline__ cx<T> term_row_sum(const Term* tp, int cnt, int n, const cx<T>* sx, const cx<T>* coef) {
   cx<T> acc = cmk<T>(0, 0);
-  for (int kb = k0; kb < cnt; kb += kTermChunk * ks) {
+  for (int kb = 0; kb < cnt; kb += kTermChunk) {
     Term tm[kTermChunk];
-    int ci[kTermChunk];
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q)
-      if (kb + q * ks < cnt) tm[q] = tp[(size_t)(kb + q * ks) * n];
-#pragma unroll
-    for (int q = 0; q < kTermChunk; ++q)
-      if (kb + q * ks < cnt) ci[q] = remap ? remap[tm[q].c] : tm[q].c;
+      if (kb + q < cnt) tm[q] = tp[(size_t)(kb + q) * n];
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q) {
-      if (kb + q * ks < cnt) {
-        cx<T> v = cscale(coef[ci[q]], (T)tm[q].s);
+      if (kb + q < cnt) {
+        cx<T> v = cscale(coef[tm[q].c], (T)tm[q].s);
 #pragma unroll
         for (int d = 0; d < NV; ++d) v = cmul(v, sx[term_var(tm[q], d)]);
         acc = cadd(acc, v);
@@ -192,23 +183,25 @@ __device__ __forceinline__ cx<T> term_row_sum(const Term* tp, int cnt, int n, co
   return acc;
 }
 
-// Row gl of dH/dx (dev-eval-indxing-generalized_3views_4pts.cuh:70-86).
+// Evaluation of the mixed loop: row gl of dH/dx
+// (dev-eval-indxing-generalized_3views_4pts.cuh:70-86).
 // LT: the tables are the compact copy in LDS at lt (hx part first); else
-// full Term records, from the LDS copy at lt when tl, else global memory.
-// Terms k0, k0 + ks, ... of each entry only (a replica's share).
+// full Term records in global memory.
 template <int NMAX, int DEG, class T, bool LT, class SegT>
 __device__ __forceinline__ void eval_jac_row(const SegT& S, int n, int gle, const cx<T>* sx, const cx<T>* sc,
-                                             cx<T> (&A)[NMAX], const void* lt, bool tl = false, int k0 = 0,
-                                             int ks = 1) {
+                                             cx<T> (&A)[NMAX], const void* lt) {
 #pragma unroll
   for (int j = 0; j < NMAX; ++j) {
     cx<T> acc = cmk<T>(0, 0);
     if (j < n) {
-      const int cnt = column_terms<LT>(S, j);
+      // the counts travel in the kernel arguments: read from device memory,
+      // each was a vector load and a full memory latency at the head of its
+      // column's loop
+      const int cnt = (int)S.colc[j];
       if constexpr (LT) {
         const CTerm<DEG>* tp = static_cast<const CTerm<DEG>*>(lt) + (size_t)j * S.hxT * n + gle;
 #pragma unroll kTermUnroll<T>
-        for (int k = k0; k < cnt; k += ks) {
+        for (int k = 0; k < cnt; ++k) {
           const CTerm<DEG> tm = tp[(size_t)k * n];
           cx<T> v = cscale(sc[cterm_c(tm)], (T)cterm_s(tm));
 #pragma unroll
@@ -216,11 +209,7 @@ __device__ __forceinline__ void eval_jac_row(const SegT& S, int n, int gle, cons
           acc = cadd(acc, v);
         }
       } else {
-        const size_t off = (size_t)j * S.hxT * n + gle;
-        if (tl)
-          acc = term_row_sum<DEG - 1, T>(static_cast<const Term*>(lt) + off, cnt, n, sx, sc, nullptr, k0, ks);
-        else
-          acc = term_row_sum<DEG - 1, T>(S.hx + off, cnt, n, sx, sc, nullptr, k0, ks);
+        acc = term_row_sum<DEG - 1, T>(S.hx + (size_t)j * S.hxT * n + gle, cnt, n, sx, sc);
       }
     }
     A[j] = acc;
@@ -229,155 +218,30 @@ __device__ __forceinline__ void eval_jac_row(const SegT& S, int n, int gle, cons
 
 // Row gl of sum_k s * coef[c] * prod x over the dHdt table: H when coef = c(t),
 // dH/dt when coef = dc/dt (…cuh:89-120).
-// coef is an LDS table indexed by slot, or (remap != nullptr) a global table
-// indexed by coefficient.
 template <int DEG, class T, bool LT, class SegT>
 __device__ __forceinline__ cx<T> eval_t_row(const SegT& S, int n, int gle, const cx<T>* sx, const cx<T>* coef,
-                                            const void* lt, const int* remap = nullptr) {
-  cx<T> acc = cmk<T>(0, 0);
+                                            const void* lt) {
   if constexpr (LT) {
+    cx<T> acc = cmk<T>(0, 0);
     const CTerm<DEG>* tp = static_cast<const CTerm<DEG>*>(lt) + (size_t)n * S.hxT * n + gle;
 #pragma unroll kTermUnroll<T>
     for (int k = 0; k < S.htT; ++k) {
       const CTerm<DEG> tm = tp[(size_t)k * n];
-      const int c = cterm_c(tm);
-      cx<T> v = cscale(coef[remap ? remap[c] : c], (T)cterm_s(tm));
+      cx<T> v = cscale(coef[cterm_c(tm)], (T)cterm_s(tm));
 #pragma unroll
       for (int q = 0; q < DEG; ++q) v = cmul(v, sx[cterm_var(tm, q)]);
       acc = cadd(acc, v);
     }
+    return acc;
   } else {
-    // records (and, with remap, the coefficient numbers) of a chunk of terms
-    // are requested together, as in eval_jac_row
-    const Term* tp = S.ht + gle;
-    for (int k0 = 0; k0 < S.htT; k0 += kTermChunk) {
-      Term tm[kTermChunk];
-      int ci[kTermChunk];
-#pragma unroll
-      for (int q = 0; q < kTermChunk; ++q)
-        if (k0 + q < S.htT) tm[q] = tp[(size_t)(k0 + q) * n];
-#pragma unroll
-      for (int q = 0; q < kTermChunk; ++q)
-        if (k0 + q < S.htT) ci[q] = remap ? remap[tm[q].c] : tm[q].c;
-#pragma unroll
-      for (int q = 0; q < kTermChunk; ++q) {
-        if (k0 + q < S.htT) {
-          cx<T> v = cscale(coef[ci[q]], (T)tm[q].s);
-#pragma unroll
-          for (int d = 0; d < DEG; ++d) v = cmul(v, sx[term_var(tm[q], d)]);
-          acc = cadd(acc, v);
-        }
-      }
-    }
-  }
-  return acc;
-}
-
-// c_j(t) and dc_j/dt(t) of order MC in t into LDS slot cslot[j] (Horner
-// from the highest term, as the general loop of stage_coeffs): the terms of
-// c_j are requested before the first Horner step uses one, then those of
-// dc_j/dt, so two memory latencies per coefficient instead of one per term.
-template <int MC, class T, class SegT>
-__device__ __forceinline__ void stage_coeffs_m(const SegT& S, const Group& g, const double2* hx, const double2* ht,
-                                               double t, cx<T>* sc, cx<T>* sd, bool with_dot) {
-  const int C1 = S.C + 1;
-#pragma unroll 1
-  for (int j = g.gl + g.s * g.G; j < C1; j += g.G * g.R) {
-    const int q = S.cslot[j];
-    {
-      const double2* ha = hx + (size_t)j * (MC + 1);
-      double2 a[MC + 1];
-#pragma unroll
-      for (int m = 0; m <= MC; ++m) a[m] = ha[m];
-      double cr = a[MC].x, ci = a[MC].y;
-#pragma unroll
-      for (int m = MC - 1; m >= 0; --m) {
-        const double nr = cr * t + a[m].x, ni = ci * t + a[m].y;
-        cr = nr;
-        ci = ni;
-      }
-      sc[q] = cmk<T>((T)cr, (T)ci);
-    }
-    if (with_dot) {
-      const double2* hb = ht + (size_t)j * MC;
-      double2 b[MC];
-#pragma unroll
-      for (int m = 0; m < MC; ++m) b[m] = hb[m];
-      double dr = b[MC - 1].x, di = b[MC - 1].y;
-#pragma unroll
-      for (int m = MC - 2; m >= 0; --m) {
-        const double nr = dr * t + b[m].x, ni = di * t + b[m].y;
-        dr = nr;
-        di = ni;
-      }
-      sd[q] = cmk<T>((T)dr, (T)di);
-    }
+    return term_row_sum<DEG, T>(S.ht + gle, S.htT, n, sx, coef);
   }
 }
 
-// c_j(t) and dc_j/dt(t) of order MC in t (MC >= 1) into LDS slot cslot[j]
-// for Q of the lane's coefficients at a time: every term of the Q
-// coefficients (both tables) is requested before the first Horner step, so
-// one memory latency per Q coefficients (the latency instances, whose
-// register budget is a whole SIMD's).  Surplus entries of the last chunk
-// reload coefficient C and store nothing.
-template <int MC, int Q, class T, class SegT>
-__device__ __forceinline__ void stage_coeffs_q(const SegT& S, const Group& g, const double2* hx, const double2* ht,
-                                               double t, cx<T>* sc, cx<T>* sd, bool with_dot) {
-  const int C1 = S.C + 1, st = g.G * g.R;
-#pragma unroll 1
-  for (int jb = g.gl + g.s * g.G; jb < C1; jb += Q * st) {
-    double2 a[Q][MC + 1], b[Q][MC];
-    int q[Q];
-#pragma unroll
-    for (int u = 0; u < Q; ++u) {
-      const int j = min(jb + u * st, C1 - 1);
-      q[u] = S.cslot[j];
-#pragma unroll
-      for (int m = 0; m <= MC; ++m) a[u][m] = hx[(size_t)j * (MC + 1) + m];
-      if (with_dot) {
-#pragma unroll
-        for (int m = 0; m < MC; ++m) b[u][m] = ht[(size_t)j * MC + m];
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < Q; ++u) {
-      if (jb + u * st < C1) {
-        double cr = a[u][MC].x, ci = a[u][MC].y;
-#pragma unroll
-        for (int m = MC - 1; m >= 0; --m) {
-          const double nr = cr * t + a[u][m].x, ni = ci * t + a[u][m].y;
-          cr = nr;
-          ci = ni;
-        }
-        sc[q[u]] = cmk<T>((T)cr, (T)ci);
-        if (with_dot) {
-          double dr = b[u][MC - 1].x, di = b[u][MC - 1].y;
-#pragma unroll
-          for (int m = MC - 2; m >= 0; --m) {
-            const double nr = dr * t + b[u][m].x, ni = di * t + b[u][m].y;
-            dr = nr;
-            di = ni;
-          }
-          sd[q[u]] = cmk<T>((T)dr, (T)di);
-        }
-      }
-    }
-  }
-}
-
-// Coefficient polynomials in t of the group's instance into LDS
-// (eval_parameter_homotopy, …cuh:34-67), computed in FP64 and stored as T.
-// Coefficient j goes to slot cslot[j]: slots follow the order in which the
-// rows of a group read them (term by term), so the lanes of a group that read
-// term k of their rows together hit consecutive LDS words instead of words one
-// equation apart (a bank conflict per lane pair when equations have many terms).
-// The replicas of a group share its LDS region and stage every R-th
-// coefficient each.  HOIST: orders M <= 4 request all terms of a coefficient
-// before its Horner steps (stage_coeffs_m; the FP64 loop, whose register
-// budget has room for them).  CH > 0: orders M <= 4 stage CH coefficients
-// per lane at a time (stage_coeffs_q; the latency instances).
-template <class T, bool HOIST = false, int CH = 0, class SegT>
+// Staging of the mixed loop: coefficient polynomials in t of the group's
+// instance into LDS (eval_parameter_homotopy, …cuh:34-67), computed in FP64
+// and stored as T, coefficient j in slot cslot[j].
+template <class T, class SegT>
 __device__ __forceinline__ void stage_coeffs(const SegT& S, const Group& g, bool act, int inst, double t,
                                              unsigned char* scb, bool with_dot) {
   if (!act) return;
@@ -386,20 +250,10 @@ __device__ __forceinline__ void stage_coeffs(const SegT& S, const Group& g, bool
   const int C1 = S.C + 1, M = S.M;
   const double2* hx = S.chx + (size_t)inst * C1 * (M + 1);
   const double2* ht = S.cht + (size_t)inst * C1 * M;
-  if constexpr (CH > 0) {
-    // chunks of CH coefficients up to order 2, CH / 2 above (registers)
-    switch (M) {
-      case 1: return stage_coeffs_q<1, CH, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      case 2: return stage_coeffs_q<2, CH, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      case 3: return stage_coeffs_q<3, (CH + 1) / 2, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      case 4: return stage_coeffs_q<4, (CH + 1) / 2, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      default: break;
-    }
-  }
   if (M == 1) {
     // c(t) = c0 + t c1, dc/dt = Ht[j][0]
 #pragma unroll kTermUnroll<T>
-    for (int j = g.gl + g.s * g.G; j < C1; j += g.G * g.R) {
+    for (int j = g.gl; j < C1; j += g.G) {
       const int q = S.cslot[j];
       const double2 a = hx[2 * (size_t)j], b = hx[2 * (size_t)j + 1];
       sc[q] = cmk<T>((T)(a.x + t * b.x), (T)(a.y + t * b.y));
@@ -410,15 +264,7 @@ __device__ __forceinline__ void stage_coeffs(const SegT& S, const Group& g, bool
     }
     return;
   }
-  if constexpr (HOIST) {
-    switch (M) {
-      case 2: return stage_coeffs_m<2, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      case 3: return stage_coeffs_m<3, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      case 4: return stage_coeffs_m<4, T>(S, g, hx, ht, t, sc, sd, with_dot);
-      default: break;
-    }
-  }
-  for (int j = g.gl + g.s * g.G; j < C1; j += g.G * g.R) {
+  for (int j = g.gl; j < C1; j += g.G) {
     double2 a = hx[(size_t)j * (M + 1) + M];
     double cr = a.x, ci = a.y;
     for (int m = M - 1; m >= 0; --m) {
@@ -638,36 +484,34 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
 // Every wave of the block takes part (one copy per block) and the block
 // barrier orders every wave's table reads after the copy; blocks of several
 // waves run one segment only, so each wave reaches the barrier once.
-template <int DEG>
-__device__ __forceinline__ const void* stage_tables(const Seg& S, int n, unsigned char* smem) {
+__device__ __forceinline__ const void* stage_tables(const Seg& S, unsigned char* smem) {
   uint32_t* d = reinterpret_cast<uint32_t*>(smem);
-  const int words = (S.hxT * n + S.htT) * n * (int)(sizeof(CTerm<DEG>) / 4);
-  for (int i = (int)threadIdx.x; i < words; i += (int)blockDim.x) d[i] = S.ctab[i];
+  for (int i = (int)threadIdx.x; i < S.tab_words; i += (int)blockDim.x) d[i] = S.ctab[i];
   __syncthreads();
   return d;
 }
 
-// The full Term records of the generic instances (dH/dx part, then dH/dt
-// part, in their global layout) copied into LDS by the block's waves; for
-// launches of few paths (latency bound: no other waves hide the global
-// latency of the evaluation's record loads).  Same barrier rule as
-// stage_tables.
-__device__ __forceinline__ const void* stage_terms(const Seg& S, int n, unsigned char* smem) {
+// The full Term records of the generic instances (dH/dx streams, then dH/dt)
+// copied into LDS by the block's waves; for launches of few paths (latency
+// bound: no other waves hide the global latency of the evaluation's record
+// loads).  Same barrier rule as stage_tables.
+__device__ __forceinline__ const Term* stage_terms(const Seg& S, int n, unsigned char* smem) {
   uint4* d = reinterpret_cast<uint4*>(smem);
-  const int nhx = S.hxT * n * n, nht = S.htT * n;
+  const int nhx = S.hx_recs, nht = S.htT * n;
   const uint4* hx = reinterpret_cast<const uint4*>(S.hx);
   const uint4* ht = reinterpret_cast<const uint4*>(S.ht);
   for (int i = (int)threadIdx.x; i < nhx; i += (int)blockDim.x) d[i] = hx[i];
   for (int i = (int)threadIdx.x; i < nht; i += (int)blockDim.x) d[nhx + i] = ht[i];
   __syncthreads();
-  return d;
+  return reinterpret_cast<const Term*>(d);
 }
 
 // Per-group view of the LDS region: x / pivot row, pivot keys, coefficients.
 // x (read by the evaluation) and the pivot-row buffer (written by the LU that
 // follows it) are never live at the same time, so they share the first
-// NMAX + 1 slots; group_lu_solve starts with a wave-scope fence that keeps
-// the evaluation's reads before its writes.  KEYS: the instance searches
+// NMAX + 1 slots (one more holds the evaluation's constant 0); group_lu_solve
+// starts with a wave-scope fence that keeps the evaluation's reads before its
+// writes.  KEYS: the instance searches
 // pivots through LDS (no DPP groups).
 constexpr int key_bytes(int nmax, bool keys) { return keys ? (8 * nmax + 15) & ~15 : 0; }
 template <int NMAX, bool KEYS>
@@ -675,8 +519,8 @@ struct Lds {
   unsigned char* base;
   __device__ cx<double>* x64() const { return reinterpret_cast<cx<double>*>(base); }
   __device__ cx<double>* piv64() const { return x64(); }
-  __device__ unsigned long long* keys() const { return reinterpret_cast<unsigned long long*>(x64() + (NMAX + 1)); }
-  __device__ unsigned char* coef() const { return base + 16 * (NMAX + 1) + key_bytes(NMAX, KEYS); }
+  __device__ unsigned long long* keys() const { return reinterpret_cast<unsigned long long*>(x64() + (NMAX + 2)); }
+  __device__ unsigned char* coef() const { return base + 16 * (NMAX + 2) + key_bytes(NMAX, KEYS); }
   template <class T>
   __device__ cx<T>* x() const { return reinterpret_cast<cx<T>*>(base); }
   template <class T>
@@ -726,27 +570,25 @@ using namespace dev;
 // One RK4 predictor step in precision T for the groups in `act`
 // (…4pts.cu:139-183): stages at (x0, t), (x0 + h k1, t + h), (x0 + h k2, t + h),
 // (x0 + dt k3, t + dt); returns k1 + 2 k2 + 2 k3 + k4 (component gl).
-// sd_ext: dc/dt table of the group's instance in global memory (constant in t,
-// M = 1) or nullptr to stage dc/dt(t) in LDS next to c(t).
 template <int NMAX, int GC, int DEG, class T, bool LT, class SegT>
 __device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group& g, const Lds<NMAX, GC == 0>& L, const void* lt,
                                               bool act, bool row, int gle, int inst, double ts, double dt,
-                                              cx<double> xl, const cx<T>* sd_ext) {
+                                              cx<double> xl) {
   const double h = 0.5 * dt;
   cx<double> acc = cmk<double>(0, 0), kprev = cmk<double>(0, 0);
   cx<T>* sx = L.template x<T>();
   const cx<T>* sc = reinterpret_cast<const cx<T>*>(L.coef());
-  const cx<T>* sd = sd_ext ? sd_ext : sc + (S.C + 1);
+  const cx<T>* sd = sc + (S.C + 1);
 #pragma unroll 1
   for (int st = 0; st < 4; ++st) {
     const double a = st == 0 ? 0.0 : (st == 3 ? dt : h);
-    if (st != 2) stage_coeffs<T>(S, g, act, inst, ts + a, L.coef(), sd_ext == nullptr);
+    if (st != 2) stage_coeffs<T>(S, g, act, inst, ts + a, L.coef(), true);
     const cx<double> xs = cmk<double>(xl.re + a * kprev.re, xl.im + a * kprev.im);
     publish_x<T>(sx, xs, g, n, act, row);
     HCX_WAVE_SYNC();
     cx<T> A[NMAX];
     eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
-    const cx<T> bt = eval_t_row<DEG, T, LT>(S, n, gle, sx, sd, lt, sd_ext ? S.cinv : nullptr);
+    const cx<T> bt = eval_t_row<DEG, T, LT>(S, n, gle, sx, sd, lt);
     bool sing;
     const cx<T> k = group_lu_solve<NMAX, GC, false, T>(A, cmk<T>(-bt.re, -bt.im), g, n, row, L.template piv<T>(), L.keys(), sing);
     kprev = ccast<double>(k);
@@ -761,11 +603,8 @@ __device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group&
 // predictor (Jacobian, dH/dt and LU of the four stages), FP64 Newton
 // corrector (FP32 before the end zone when o.newton32), FP64 refinement; a
 // path that ends without a refined root is re-tracked from t = 0 entirely in
-// FP64 (escalation): by the same group (KESC: the generic instances and
-// n = 30), or, for the size-specialised instances up to n = 16, by the FP64
-// pass after the launch, which keeps the FP64 predictor out of the kernel and
-// with it the registers of a second predictor.  The pass skips paths already
-// escalated, so either way each failed path is re-tracked once.
+// FP64 (escalation) by the FP64 pass after the launch, which keeps the FP64
+// predictor out of the kernel and with it the registers of a second predictor.
 template <int NMAX, int DEG, int MODE, bool EXACT>
 __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned char* smem, int lane) {
   static_assert(MODE == 1, "the FP64 mode runs run_segment_fp64");
@@ -773,7 +612,6 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
   // kernarg loads) instead of being re-read through a generic pointer
   Seg S = LN.seg[si];
   constexpr int GE = exact_lanes(NMAX);
-  constexpr bool KESC = !(EXACT && NMAX <= 16);
   if (EXACT) {
     // size-specialised instance: n = NMAX and G are compile-time constants,
     // so every loop bound and the lane-group geometry fold away
@@ -796,7 +634,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
   // several times sooner.
   constexpr bool LT = EXACT && (NMAX <= 16 || DEG <= 2);
   const void* lt = nullptr;
-  if constexpr (LT) lt = stage_tables<DEG>(S, n, smem);
+  if constexpr (LT) lt = stage_tables(S, smem);
   // lanes outside the full groups (64 % G of them) alias region 0: they
   // track nothing and store nothing to LDS
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
@@ -807,7 +645,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
   int inst = 0, root = 0;
   double t = 0.0, dt = 0.0;
   int cnt = 0, nsteps = 0, asteps = 0, nnewt = 0, nref = 0;
-  bool ez = false, esc = false;  // this path runs in FP64
+  bool ez = false;
   int status = 0;  // 0 idle, 1 tracking, 2 finishing
   uint32_t fl = 0;
   bool exhausted = !g.in_grp;
@@ -815,13 +653,12 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
   // lane-distributed state: component gl of x and of the last accepted x
   cx<double> x = cmk<double>(0, 0), xl = x;
 
-  auto start_path = [&](const KSeg& Sv, bool fp64) {
+  auto start_path = [&](const KSeg& Sv) {
     t = 0.0;
     dt = opts_arg->dt0;
     cnt = 0;
     asteps = 0;
     ez = false;
-    esc = fp64;
     status = 1;
     if (row) {
       const double2 v = Sv.start[(size_t)root * Sv.start_stride + g.gl];
@@ -863,7 +700,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
           nnewt = 0;
           nref = 0;
           fl = Sk.plist ? HCX_FLAG_ESCALATED : 0u;
-          start_path(Sk, false);
+          start_path(Sk);
           if (!LN.persistent) exhausted = true;
         }
       }
@@ -895,21 +732,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
         }
       }
       const double ts = t;
-      cx<double> acc;
-      if constexpr (!KESC) {
-        acc = predict<NMAX, GC, DEG, float, LT>(Sk, n, g, L, lt, stepping, row, gle, inst, ts, dt, xl, nullptr);
-      } else {
-        const bool p32 = stepping && !esc, p64 = stepping && esc;
-        cx<double> a32 = cmk<double>(0, 0), a64 = a32;
-        if (__any(p32)) a32 = predict<NMAX, GC, DEG, float, LT>(Sk, n, g, L, lt, p32, row, gle, inst, ts, dt, xl, nullptr);
-        if (__any(p64)) {
-          HCX_WAVE_SYNC();
-          const cx<double>* sd_ext =
-              Sk.M == 1 ? reinterpret_cast<const cx<double>*>(Sk.cht + (size_t)inst * (Sk.C + 1)) : nullptr;
-          a64 = predict<NMAX, GC, DEG, double, LT>(Sk, n, g, L, lt, p64, row, gle, inst, ts, dt, xl, sd_ext);
-        }
-        acc = esc ? a64 : a32;
-      }
+      const cx<double> acc = predict<NMAX, GC, DEG, float, LT>(Sk, n, g, L, lt, stepping, row, gle, inst, ts, dt, xl);
       if (stepping) {
         const double f = dt * (1.0 / 6.0);
         x = cmk<double>(xl.re + f * acc.re, xl.im + f * acc.im);
@@ -918,7 +741,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
       // Newton corrector at the new t (:189-223)
       bool ok = false, inf = false;
       {
-        const bool run32 = stepping && !ez && !esc && o.newton32, run64 = stepping && !run32;
+        const bool run32 = stepping && !ez && o.newton32, run64 = stepping && !run32;
         bool ok32 = false, inf32 = false, ok64 = false, inf64 = false;
         if (__any(run32)) newton_pass<NMAX, GC, DEG, float, LT>(Sk, n, o, g, L, lt, run32, row, x, nnewt, ok32, inf32);
         if (__any(run64)) {
@@ -1016,16 +839,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
         }
         HCX_WAVE_SYNC();
       }
-      if (KESC && fin && !esc && !(fl & HCX_FLAG_REFINED)) {
-        // precision escalation: the mixed attempt did not reach a refined
-        // root; track the same path again from t = 0 in FP64 (the counters
-        // then describe the FP64 attempt, as after the re-track pass)
-        fl = HCX_FLAG_ESCALATED;
-        nsteps = 0;
-        nnewt = 0;
-        nref = 0;
-        start_path(Sk, true);
-      } else if (fin) {
+      if (fin) {
         const SegOut* O = Sk.out;
         double2* roots = O->roots;
         const int rstride = O->roots_stride;
@@ -1054,40 +868,6 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
       }
     }
   }
-}
-
-// Right-hand side row of the FP64 micro-step loop: sum_k s * coef * prod x
-// over the dHdt table (…cuh:89-120), with coef = c(t) from the group's LDS
-// slots (H) or, for the lanes of groups in an RK4 stage (dot), dc/dt from
-// `dtab`: LDS slots next to c(t), or (GDOT) the instance's table in global
-// memory indexed by coefficient number (cinv maps slots to coefficients).
-template <int DEG, bool LT, bool GDOT, class SegT>
-__device__ __forceinline__ cx<double> eval_rhs_sel(const SegT& S, int n, int gle, const cx<double>* sx,
-                                                   const cx<double>* sc, const cx<double>* dtab, bool dot,
-                                                   const void* lt, bool tl = false, int k0 = 0, int ks = 1) {
-  const cx<double>* base = dot ? dtab : sc;
-  cx<double> acc = cmk<double>(0, 0);
-  if constexpr (LT) {
-    const CTerm<DEG>* tp = static_cast<const CTerm<DEG>*>(lt) + (size_t)n * S.hxT * n + gle;
-#pragma unroll kTermUnroll<double>
-    for (int k = k0; k < S.htT; k += ks) {
-      const CTerm<DEG> tm = tp[(size_t)k * n];
-      int c = cterm_c(tm);
-      if (GDOT && dot) c = S.cinv[c];
-      cx<double> v = cscale(base[c], (double)cterm_s(tm));
-#pragma unroll
-      for (int q = 0; q < DEG; ++q) v = cmul(v, sx[cterm_var(tm, q)]);
-      acc = cadd(acc, v);
-    }
-  } else {
-    const int* remap = (GDOT && dot) ? S.cinv : nullptr;
-    if (tl)
-      acc = term_row_sum<DEG, double>(static_cast<const Term*>(lt) + (size_t)n * S.hxT * n + gle, S.htT, n, sx, base,
-                                      remap, k0, ks);
-    else
-      acc = term_row_sum<DEG, double>(S.ht + gle, S.htT, n, sx, base, remap, k0, ks);
-  }
-  return acc;
 }
 
 // Phases of a lane group in the FP64 micro-step loop.
@@ -1119,10 +899,7 @@ enum : int {
 // REP: the latency instance (launches of few paths, one wave per SIMD at
 // most): R >= 1 replicas per path (Seg::R) and chunked coefficient staging,
 // compiled apart so that the throughput loop carries none of it.
-// HOIST: stage_coeffs requests all terms of a coefficient at once (orders
-// M <= 4; size-specialised instances up to n = 16 outside the multi-size
-// kernel: the others would lose occupancy to the registers).
-template <int NMAX, int DEG, bool EXACT, bool REP, bool HOIST = (EXACT && NMAX <= 16)>
+template <int NMAX, int DEG, bool EXACT, bool REP>
 __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsigned char* smem, int lane) {
   Seg S = LN.seg[si];
   constexpr int GE = exact_lanes(NMAX);
@@ -1140,22 +917,25 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   const bool row = g.in_grp && g.gl < n;
   const int gle = row ? g.gl : 0;
   constexpr bool LT = EXACT && (NMAX <= 16 || DEG <= 2);
-  const void* lt = nullptr;
-  // tl: the generic latency instance's full Term records are in LDS
-  // (tab_lds then holds their bytes)
-  bool tl = false;
+  const unsigned char* lt = nullptr;
+  // the generic latency instance's full Term records in LDS (tab_lds then
+  // holds their bytes)
+  const Term* tl = nullptr;
   if constexpr (LT) {
-    lt = stage_tables<DEG>(S, n, smem);
+    lt = static_cast<const unsigned char*>(stage_tables(S, smem));
   } else if constexpr (!EXACT && REP) {
-    if (LN.tab_lds > 0) {
-      lt = stage_terms(S, n, smem);
-      tl = true;
-    }
+    if (LN.tab_lds > 0) tl = stage_terms(S, n, smem);
   }
+  // coefficients in flight per lane while staging (order 1)
+  constexpr int SQ = REP ? 8 : (EXACT && NMAX <= 16 ? 4 : 2);
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
   Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
-  cx<double>* sx = L.template x<double>();
-  const cx<double>* sc = reinterpret_cast<const cx<double>*>(L.coef());
+  cx<double>* sx = L.x64();
+  unsigned char* const xb = L.base;
+  unsigned char* const cb = L.coef();
+  unsigned char* const db = cb + S.nslot * 16;  // dc/dt, when in LDS
+  // the path's instance tables
+  const double2 *hxi = S.chx, *hti = S.cht;
   // dc/dt of the RK4 stages: constant (M = 1) -> read from the instance's
   // table in global memory (half the group's LDS), unless the launch stages
   // it in LDS (dot_lds: launches of few paths, latency bound); M > 1 -> LDS
@@ -1198,6 +978,8 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
           path = p;
           inst = (int)(p / Sk.K);
           root = (int)(p - (long long)inst * Sk.K);
+          hxi = Sk.chx + (size_t)inst * (Sk.C + 1) * (Sk.M + 1);
+          hti = Sk.cht + (size_t)inst * (Sk.C + 1) * Sk.M;
           nsteps = asteps = nnewt = nref = cnt = 0;
           fl = Sk.plist ? HCX_FLAG_ESCALATED : 0u;
           t = 0.0;
@@ -1270,18 +1052,36 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       const double te = stg ? ts + a : (pe == kPhNewton ? t : 1.0);
       const cx<double> xe = stg ? cmk<double>(xl.re + a * kp.re, xl.im + a * kp.im) : x;
       const bool restage = act && te != tst;
-      if (__any(restage)) stage_coeffs<double, HOIST, REP ? 4 : 0>(Sk, g, restage, inst, te, L.coef(), !gdot);
-      if (restage) tst = te;
-      publish_x<double>(sx, xe, g, n, act, row);
+      if (restage) {
+        stage_coeffs64<LT && NMAX <= 16, SQ>(Sk, g, hxi, hti, te, cb, db, !gdot, lt);
+        tst = te;
+      }
+      publish_x64(sx, xe, g, n, act, row);
       HCX_WAVE_SYNC();
       cx<double> A[NMAX];
-      eval_jac_row<NMAX, DEG, double, LT>(Sk, n, gle, sx, sc, A, lt, tl, k0, ks);
       cx<double> r;
-      if (gdot) {
-        const cx<double>* dg = reinterpret_cast<const cx<double>*>(Sk.cht + (size_t)inst * (Sk.C + 1));
-        r = eval_rhs_sel<DEG, LT, true>(Sk, n, gle, sx, sc, dg, stg, lt, tl, k0, ks);
+      if constexpr (LT) {
+        if constexpr (REP) {
+          eval_jac_rounds<NMAX, DEG>(Sk, gle, xb, cb, A, lt, k0, ks);
+          if (Sk.htT <= 2 * ks)
+            r = eval_rhs_stream<NMAX, DEG, false, 2>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+          else
+            r = eval_rhs_stream<NMAX, DEG, false, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+        } else {
+          eval_jac_stream<NMAX, DEG, 2>(Sk, gle, xb, cb, A, lt, k0, ks);
+          if (gdot)
+            r = eval_rhs_stream<NMAX, DEG, true, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+          else
+            r = eval_rhs_stream<NMAX, DEG, false, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+        }
       } else {
-        r = eval_rhs_sel<DEG, LT, false>(Sk, n, gle, sx, sc, sc + (Sk.C + 1), stg, lt, tl, k0, ks);
+        const cx<double>* sc = reinterpret_cast<const cx<double>*>(cb);
+        eval_jac_terms<NMAX, DEG>(Sk, n, gle, sx, sc, A, tl, k0, ks);
+        if (gdot)
+          r = eval_rhs_terms<DEG, true>(Sk, n, gle, sx, sc, hti, stg, tl, k0, ks);
+        else
+          r = eval_rhs_terms<DEG, false>(Sk, n, gle, sx, reinterpret_cast<const cx<double>*>(stg ? db : cb), hti, stg,
+                                         tl, k0, ks);
       }
       if constexpr (REP) {
         // each replica summed every R-th term of the row's sums: a butterfly
@@ -1462,14 +1262,14 @@ void track_kernel_rep(const Launch LN) {
 template <int N, int DEG, int MODE>
 __device__ __forceinline__ void run_exact(const Launch& LN, int si, unsigned char* smem, int lane) {
   if constexpr (MODE == 0) {
-    run_segment_fp64<N, DEG, true, false, false>(LN, si, smem, lane);
+    run_segment_fp64<N, DEG, true, false>(LN, si, smem, lane);
   } else {
     run_segment<N, DEG, MODE, true>(LN, si, smem, lane);
   }
 }
 
 template <int DEG, int MODE>
-__global__ __launch_bounds__(256) void track_kernel_set(const Launch LN) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void track_kernel_set(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = (int)threadIdx.x & 63;
   int s = 0;

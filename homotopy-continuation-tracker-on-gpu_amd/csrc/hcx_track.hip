@@ -475,17 +475,17 @@ Opts to_opts(const hcx_track_opts* o) {
 }
 
 // Per-group LDS: the x / pivot-row slots (shared, FP64 capacity) and the
-// coefficient area: with M = 1 (dc/dt constant, read by the FP64 stages from
-// the instance's table in global memory) FP32 c + dc/dt overlaid by FP64 c,
-// else (or dot_lds: FP64 stages with dc/dt in LDS) FP64 c + dc/dt.
-// An instance without DPP groups (keys) has its pivot keys there too.
+// constants 1 and 0, the pivot keys (instances without DPP groups) and the
+// coefficient area of `slots` slots.  FP64: c(t), and dc/dt with M > 1 or
+// dot_lds (with M = 1 dc/dt is constant and read from the instance's table in
+// global memory); mixed: with M = 1 FP32 c + dc/dt overlaid by FP64 c.
 // The region stride is an odd multiple of 16 bytes: the groups of a wave read
 // the same offsets of their regions together (pivot-row broadcasts, x and
 // coefficient gathers), and such a stride spreads them over distinct LDS banks
 // (64 banks x 4 bytes) for 8- and 16-byte accesses.
-int lds_group_bytes(int nmax, bool keys, int C, int M, bool dot_lds = false) {
+int lds_group_bytes(int nmax, bool keys, int slots, int M, bool dot_lds = false) {
   const int per = (M > 1 || dot_lds) ? 32 : 16;
-  const int b = 16 * (nmax + 1) + dev::key_bytes(nmax, keys) + (C + 1) * per;
+  const int b = 16 * (nmax + 2) + dev::key_bytes(nmax, keys) + slots * per;
   return (((b + 15) / 16) | 1) * 16;
 }
 
@@ -493,11 +493,15 @@ struct Plan {
   int nmax = 0, mode = 0;
   int deg = 2;       // term degree of the instance (generic: rounded up to its instance's)
   bool exact = false;
-  bool tab4 = false; // the kernel reads 4-byte compact terms (DEG <= 2), else 8-byte
+  bool latency = false;  // the latency instance, with its own compact tables
+  bool tab4 = false; // the compact tables are those of DEG <= 2
   int tab_lds = 0;   // LDS bytes of the compact tables (instances that hold them there)
   size_t lds = 0;
   KernelFn fn = nullptr;
   bool keys() const { return !(exact && is_pow2(exact_lanes(nmax))); }  // pivot keys in LDS
+  int group_bytes(const hcx_problem* p, bool dot_lds = false) const {
+    return lds_group_bytes(nmax, keys(), mode == 0 ? p->nslot : p->C + 1, p->M, dot_lds);
+  }
 };
 
 // Largest compact table the size-specialised instances (up to n = 16; n = 30
@@ -530,8 +534,9 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
     in_set = in_set && (n == 3 || n == 5 || n == 6 || n == 9 || n == 12) && Gs[s] == n;
     const void* ct = t4 ? (const void*)probs[s]->d_ctab4 : (const void*)probs[s]->d_ctab;
     const int cb = t4 ? probs[s]->ctab4_bytes : probs[s]->ctab_bytes;
-    tab_ok = tab_ok && ct && cb <= kMaxTabLds && probs[s]->hxc_fits;
-    tab = std::max(tab, cb);
+    const auto& c64 = probs[s]->ctab64[t4 ? 0 : 1];
+    tab_ok = tab_ok && ct && cb <= kMaxTabLds && (mode != 0 || c64.d);
+    tab = std::max(tab, mode == 0 ? c64.words * 4 : cb);
   }
   if (specialize && !same && in_set && tab_ok && max_deg <= 2) {
     pl.fn = mode == 0 ? kernel_set_m0() : kernel_set_m1();
@@ -551,7 +556,11 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
       pl.deg = max_deg;
       pl.exact = true;
       pl.tab_lds = (n0 <= 16 || t4) ? tab : 0;
-      return HCX_OK;
+      size_t lds = 0;
+      for (int s = 0; s < nseg; ++s)
+        lds = std::max(lds, (size_t)(64 / Gs[s]) * (size_t)pl.group_bytes(probs[s]) + (size_t)pl.tab_lds);
+      if (lds <= (size_t)kMaxLdsBytes) return HCX_OK;
+      pl.tab_lds = 0;
     }
   }
   const int ni = round_up_idx(kNmaxList, 3, max_n);
@@ -571,6 +580,38 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
   return HCX_OK;
 }
 
+// The tables of a segment in the form that the plan's kernel reads.
+void seg_tables(Seg& S, const hcx_problem* p, const Plan& pl) {
+  S.lds_group = pl.group_bytes(p);
+  S.hxT = p->hxT;
+  S.cslot = p->d_cslot;
+  S.nslot = p->nslot;
+  if (pl.mode == 0) {
+    const auto& c = (pl.latency ? p->ltab64 : p->ctab64)[pl.tab4 ? 0 : 1];
+    S.hx = p->d_hxs;
+    S.ht = p->d_hts;
+    S.ht_ci = p->d_ht_ci;
+    S.htT = p->htT64;
+    S.htS = p->htS64;
+    S.hx_recs = p->hx_recs;
+    S.max_terms = p->max_terms;
+    std::memcpy(S.colc, p->colc64, sizeof(S.colc));
+    S.hx_cnt = p->colc64_fits ? nullptr : p->d_hxs_cnt;
+    S.ctab = c.d;
+    S.tab_words = c.words;
+    S.tab_h = c.h;
+    S.tab_slot = c.slot;
+  } else {
+    S.hx = p->d_hx;
+    S.ht = p->d_ht;
+    S.htT = p->htT;
+    std::memcpy(S.colc, p->colc, sizeof(S.colc));
+    S.hx_cnt = nullptr;
+    S.ctab = pl.tab4 ? p->d_ctab4 : p->d_ctab;
+    S.tab_words = (p->hxT * p->n + p->htT) * p->n * (pl.tab4 ? 1 : 2);
+  }
+}
+
 // Fills the segment-independent part of a Seg from a problem.
 void seg_from_problem(Seg& S, SegOut& O, const hcx_problem* p, int G, const Plan& pl) {
   std::memset(&S, 0, sizeof(S));
@@ -580,18 +621,9 @@ void seg_from_problem(Seg& S, SegOut& O, const hcx_problem* p, int G, const Plan
   S.C = p->C;
   S.M = p->M;
   S.K = p->K;
-  S.hxT = p->hxT;
-  S.htT = p->htT;
   S.G = G;
   S.R = 1;
-  S.lds_group = lds_group_bytes(pl.nmax, pl.keys(), p->C, p->M);
-  S.hx = p->d_hx;
-  S.ht = p->d_ht;
-  std::memcpy(S.hxc, p->hxc, sizeof(S.hxc));
-  S.hx_cnt = p->hxc_fits ? nullptr : p->d_hx_cnt;
-  S.cslot = p->d_cslot;
-  S.cinv = p->d_cinv;
-  S.ctab = pl.tab4 ? p->d_ctab4 : p->d_ctab;
+  seg_tables(S, p, pl);
   S.start = p->d_start;
   S.start_stride = p->n;
 }
@@ -901,6 +933,128 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   for (auto& tm : ht) tm.c = cslot[tm.c];
   for (auto& tm : hx) tm.c = cslot[tm.c];
 
+  // Term streams of the FP64 loop (layout and order: hcx_eval64.hpp).
+  int nslot = 0;  // slots that a term uses come first
+  {
+    std::vector<char> used(C + 1, 0);
+    for (const auto& tm : ht)
+      if (tm.s != 0) used[tm.c] = 1;
+    for (const auto& tm : hx)
+      if (tm.s != 0) used[tm.c] = 1;
+    for (int q = 0; q <= C; ++q)
+      if (used[q]) nslot = q + 1;
+  }
+  dev::Term zero_term;
+  zero_term.s = 1;
+  zero_term.c = 0;
+  zero_term.v03 = (uint32_t)(n + 1) | (uint32_t)n << 8 | (uint32_t)n << 16 | (uint32_t)n << 24;
+  zero_term.v47 = (uint32_t)n * 0x01010101u;
+  // appends one entry's stream [position][equation]; returns its scaled positions
+  auto add_stream = [&](std::vector<dev::Term>& out, auto&& term_at, int T) {
+    std::vector<std::vector<dev::Term>> a(n);
+    size_t cnt = 0, scaled = 0;
+    for (int i = 0; i < n; ++i) {
+      for (int tt = 0; tt < T; ++tt) {
+        const dev::Term& tm = term_at(tt, i);
+        if (tm.s == 0) continue;
+        a[i].push_back(tm);
+        if (tm.s != 1) scaled = std::max(scaled, a[i].size());
+      }
+      cnt = std::max(cnt, a[i].size());
+    }
+    for (size_t k = 0; k < cnt; ++k)
+      for (int i = 0; i < n; ++i) out.push_back(k < a[i].size() ? a[i][k] : zero_term);
+    return scaled;
+  };
+  std::vector<dev::Term> hxs, hts;
+  std::vector<int> hxs_cnt(n), ht_ci;
+  unsigned int colc64[kMaxN] = {};
+  bool colc64_fits = true;
+  int s_min = 0, s_max = 0;
+  for (int j = 0; j < n; ++j) {
+    const size_t at = hxs.size();
+    const size_t scaled = add_stream(
+        hxs, [&](int tt, int i) -> const dev::Term& { return hx[((size_t)j * d->hx_terms + tt) * n + i]; },
+        d->hx_terms);
+    const size_t cnt = (hxs.size() - at) / n;
+    colc64_fits = colc64_fits && cnt <= 0xffff;
+    colc64[j] = (unsigned int)(cnt & 0xffff) | (unsigned int)(scaled & 0xffff) << 16;
+    hxs_cnt[j] = (int)cnt;
+  }
+  const int htS = (int)add_stream(
+      hts, [&](int tt, int i) -> const dev::Term& { return ht[(size_t)tt * n + i]; }, d->ht_terms);
+  const int htT64 = (int)(hts.size() / n), hx_recs = (int)hxs.size();
+  for (const auto& tm : hts) ht_ci.push_back(cinv[tm.c]);
+  for (const auto* v : {&hxs, &hts})
+    for (const auto& tm : *v) {
+      s_min = std::min(s_min, tm.s);
+      s_max = std::max(s_max, tm.s);
+    }
+  if (hxs.empty()) hxs.push_back(zero_term);  // nothing to read, but no empty allocation
+  if (hts.empty()) {
+    hts.push_back(zero_term);
+    ht_ci.push_back(0);
+  }
+  // compact forms for the instances that hold the streams in LDS
+  struct CompactHost {
+    std::vector<uint32_t> w;
+    int h = 0, slot = 0;
+  } compact[4];  // [degree], [2 + degree]: the latency instances'
+  for (int cf = 0; cf < 4; ++cf) {
+    const int f = cf & 1;
+    const bool lat = cf >= 2;
+    // offsets of 16 bits: 4,095 slots (0xffff marks a coefficient without one);
+    // scalars of 6 or 12 bits
+    const int s_lim = f == 0 ? 32 : 2048;
+    if (!colc64_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4095 || C > 0xffff || deg > (f == 0 ? 2 : 4))
+      continue;
+    CompactHost& ch = compact[cf];
+    std::vector<uint32_t>& w = ch.w;
+    auto var = [&](const dev::Term& tm, int q) { return (uint32_t)(((tm.v03 >> (8 * q)) & 0xffu) * 16u); };
+    auto put = [&](const dev::Term& tm, bool h) {
+      const uint32_t sc = (uint32_t)tm.s;
+      w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16 | (sc & 0x3fu) << 26);
+      if (f == 0) {
+        if (h) w.push_back(var(tm, 1) | (uint32_t)cinv[tm.c] << 16);
+      } else {
+        w.push_back(var(tm, 1) | var(tm, 2) << 16 | ((sc >> 6) & 0x3fu) << 26);
+        if (h) w.push_back(var(tm, 3) | (uint32_t)cinv[tm.c] << 16);
+        if (h) w.push_back(0);
+      }
+    };
+    auto align = [&]() {
+      while (w.size() % 4) w.push_back(0);
+      return (int)(w.size() * 4);
+    };
+    auto put_lat = [&](const dev::Term& tm) {
+      const double sd = tm.s;
+      uint64_t bits;
+      std::memcpy(&bits, &sd, 8);
+      w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16);
+      if (f == 1) w.push_back(var(tm, 1) | var(tm, 2) << 16);
+      w.push_back((uint32_t)(bits >> 32));
+      if (f == 1) w.push_back(0);
+    };
+    size_t r = 0;
+    for (int j = 0; j < n; ++j) {
+      for (int k = 0; k < hxs_cnt[j] * n; ++k, ++r)
+        if (lat) put_lat(hxs[r]);
+        else put(hxs[r], false);
+      for (int i = 0; lat && i < n; ++i) put_lat(zero_term);
+    }
+    ch.h = align();
+    r = 0;
+    for (int k = 0; k < htT64 * n; ++k) put(hts[r++], true);
+    // a zero term per equation ends the H stream
+    for (int i = 0; i < n; ++i) put(zero_term, true);
+    ch.slot = align();
+    for (int c = 0; c <= C; c += 2) {
+      auto off = [&](int q) { return q > C || cslot[q] >= nslot ? 0xffffu : (uint32_t)cslot[q] * 16u; };
+      w.push_back(off(c) | off(c + 1) << 16);
+    }
+    align();
+  }
+
   // compact 8-byte terms (hx part, then ht part) for the instances that hold
   // the tables in LDS: slot and scalar in 16 bits each, <= 4 variables
   std::vector<uint2> ctab;
@@ -942,76 +1096,72 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   p->hx_vars = hxv;
   p->ht_vars = htv;
   p->deg = std::max(deg, 2);
-  p->hxc_fits = true;
-  for (int j = 0; j < n; ++j) {
-    p->hxc_fits = p->hxc_fits && hx_cnt[j] <= 0xffff;
-    p->hxc[j >> 1] |= ((unsigned int)hx_cnt[j] & 0xffffu) << (16 * (j & 1));
-  }
+  for (int j = 0; j < n; ++j) p->colc[j] = (unsigned int)hx_cnt[j];
+  std::memcpy(p->colc64, colc64, sizeof(colc64));
+  p->colc64_fits = colc64_fits;
+  p->hx_recs = hx_recs;
+  p->htT64 = htT64;
+  p->htS64 = htS;
+  p->nslot = nslot;
+  p->max_terms = *std::max_element(hxs_cnt.begin(), hxs_cnt.end());
   auto fail = [&](hipError_t e, const char* what) {
     set_error("hcx_problem_create: %s: %s", what, hipGetErrorString(e));
     hcx_problem_destroy(p);
     return HCX_ERR_HIP;
   };
   hipError_t e;
-  if ((e = hipMalloc(&p->d_hx, hx.size() * sizeof(dev::Term))) != hipSuccess) return fail(e, "hipMalloc hx");
-  if ((e = hipMalloc(&p->d_ht, ht.size() * sizeof(dev::Term))) != hipSuccess) return fail(e, "hipMalloc ht");
-  if ((e = hipMalloc(&p->d_hx_cnt, n * sizeof(int))) != hipSuccess) return fail(e, "hipMalloc hx_cnt");
-  if ((e = hipMalloc(&p->d_cslot, (C + 1) * sizeof(int))) != hipSuccess) return fail(e, "hipMalloc cslot");
-  if ((e = hipMalloc(&p->d_cinv, (C + 1) * sizeof(int))) != hipSuccess) return fail(e, "hipMalloc cinv");
-  if ((e = hipMemcpy(p->d_cslot, cslot.data(), (C + 1) * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e, "copy cslot");
-  if ((e = hipMemcpy(p->d_cinv, cinv.data(), (C + 1) * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e, "copy cinv");
+  // every table in one device allocation, filled by one copy
+  std::vector<unsigned char> blob;
+  std::vector<std::pair<void**, size_t>> parts;
+  auto add = [&](auto** dst, const void* src, size_t bytes) {
+    parts.emplace_back(reinterpret_cast<void**>(dst), blob.size());
+    const unsigned char* c = static_cast<const unsigned char*>(src);
+    blob.insert(blob.end(), c, c + bytes);
+    blob.resize((blob.size() + 255) & ~size_t(255));
+  };
+  auto add_vec = [&](auto** dst, const auto& v) { add(dst, v.data(), v.size() * sizeof(v[0])); };
+  add_vec(&p->d_hx, hx);
+  add_vec(&p->d_ht, ht);
+  add_vec(&p->d_cslot, cslot);
+  add_vec(&p->d_hxs, hxs);
+  add_vec(&p->d_hts, hts);
+  add_vec(&p->d_ht_ci, ht_ci);
+  add_vec(&p->d_hxs_cnt, hxs_cnt);
+  for (int cf = 0; cf < 4; ++cf) {
+    const CompactHost& ch = compact[cf];
+    hcx_problem::Compact& ct = cf < 2 ? p->ctab64[cf] : p->ltab64[cf - 2];
+    if (ch.w.empty()) continue;
+    add_vec(&ct.d, ch.w);
+    ct.words = (int)ch.w.size();
+    ct.h = ch.h;
+    ct.slot = ch.slot;
+  }
   if (!ctab4.empty()) {
     p->ctab4_bytes = (int)((ctab4.size() * sizeof(uint32_t) + 15) / 16 * 16);
-    if ((e = hipMalloc(&p->d_ctab4, p->ctab4_bytes)) != hipSuccess) return fail(e, "hipMalloc ctab4");
-    if ((e = hipMemcpy(p->d_ctab4, ctab4.data(), ctab4.size() * sizeof(uint32_t), hipMemcpyHostToDevice)) !=
-        hipSuccess)
-      return fail(e, "copy ctab4");
+    add_vec(&p->d_ctab4, ctab4);
   }
   if (!ctab.empty()) {
     p->ctab_bytes = (int)((ctab.size() * sizeof(uint2) + 15) / 16 * 16);
-    if ((e = hipMalloc(&p->d_ctab, p->ctab_bytes)) != hipSuccess) return fail(e, "hipMalloc ctab");
-    if ((e = hipMemcpy(p->d_ctab, ctab.data(), ctab.size() * sizeof(uint2), hipMemcpyHostToDevice)) != hipSuccess)
-      return fail(e, "copy ctab");
+    add_vec(&p->d_ctab, ctab);
   }
-  if ((e = hipMalloc(&p->d_start, (size_t)p->K * n * sizeof(double2))) != hipSuccess) return fail(e, "hipMalloc start");
-  if ((e = hipMalloc(&p->launcher_ws.base, ws_layout(sizeof(SegOut), 0, 0).bytes)) != hipSuccess)
-    return fail(e, "hipMalloc launcher workspace");
-  if ((e = hipMemcpy(p->d_hx, hx.data(), hx.size() * sizeof(dev::Term), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e, "copy hx");
-  if ((e = hipMemcpy(p->d_ht, ht.data(), ht.size() * sizeof(dev::Term), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e, "copy ht");
-  if ((e = hipMemcpy(p->d_hx_cnt, hx_cnt.data(), n * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e, "copy hx_cnt");
-  if ((e = hipMemcpy(p->d_start, d->h_start_sols, (size_t)p->K * n * sizeof(double2), hipMemcpyHostToDevice)) !=
-      hipSuccess)
-    return fail(e, "copy start");
-  if (p->k > 0 && d->h_coeff_affine) {
-    if ((e = hipMalloc(&p->d_affine, (size_t)C * (1 + p->k) * sizeof(double2))) != hipSuccess)
-      return fail(e, "hipMalloc affine");
-    if ((e = hipMemcpy(p->d_affine, d->h_coeff_affine, (size_t)C * (1 + p->k) * sizeof(double2),
-                       hipMemcpyHostToDevice)) != hipSuccess)
-      return fail(e, "copy affine");
-  }
+  add(&p->d_start, d->h_start_sols, (size_t)p->K * n * sizeof(double2));
+  if (p->k > 0 && d->h_coeff_affine) add(&p->d_affine, d->h_coeff_affine, (size_t)C * (1 + p->k) * sizeof(double2));
   if (p->k > 0 && d->h_cmap_scalar) {
     p->cmap_T = d->cmap_terms;
     p->cmap_D = d->cmap_deg;
-    const size_t ns = (size_t)C * p->cmap_T, np = ns * p->cmap_D;
-    if ((e = hipMalloc(&p->d_cmap_scalar, ns * sizeof(double2))) != hipSuccess) return fail(e, "hipMalloc cmap");
-    if ((e = hipMalloc(&p->d_cmap_params, np * sizeof(int))) != hipSuccess) return fail(e, "hipMalloc cmap");
-    if ((e = hipMemcpy(p->d_cmap_scalar, d->h_cmap_scalar, ns * sizeof(double2), hipMemcpyHostToDevice)) !=
-        hipSuccess)
-      return fail(e, "copy cmap");
-    if ((e = hipMemcpy(p->d_cmap_params, d->h_cmap_params, np * sizeof(int), hipMemcpyHostToDevice)) != hipSuccess)
-      return fail(e, "copy cmap");
+    const size_t ns = (size_t)C * p->cmap_T;
+    add(&p->d_cmap_scalar, d->h_cmap_scalar, ns * sizeof(double2));
+    add(&p->d_cmap_params, d->h_cmap_params, ns * p->cmap_D * sizeof(int));
   }
-  if (p->k > 0) {
-    if ((e = hipMalloc(&p->d_p0, (size_t)p->k * sizeof(double2))) != hipSuccess) return fail(e, "hipMalloc p0");
-    if ((e = hipMemcpy(p->d_p0, d->h_start_params, (size_t)p->k * sizeof(double2), hipMemcpyHostToDevice)) !=
-        hipSuccess)
-      return fail(e, "copy p0");
-  }
+  if (p->k > 0) add(&p->d_p0, d->h_start_params, (size_t)p->k * sizeof(double2));
+  // the launcher workspace at the end (nothing to copy)
+  const size_t ws_off = blob.size();
+  if ((e = hipMalloc(&p->d_blob, ws_off + ws_layout(sizeof(SegOut), 0, 0).bytes)) != hipSuccess)
+    return fail(e, "hipMalloc tables");
+  if ((e = hipMemcpy(p->d_blob, blob.data(), blob.size(), hipMemcpyHostToDevice)) != hipSuccess)
+    return fail(e, "copy tables");
+  for (const auto& q : parts) *q.first = p->d_blob + q.second;
+  p->launcher_ws.base = p->d_blob + ws_off;
 
   // algorithmic FLOPs of the reference algorithm (padding terms excluded)
   hcx_problem_info& in = p->info;
@@ -1055,19 +1205,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
 
 hcx_status hcx_problem_destroy(hcx_problem* p) {
   if (!p) return HCX_OK;
-  if (p->d_hx) (void)hipFree(p->d_hx);
-  if (p->d_ht) (void)hipFree(p->d_ht);
-  if (p->d_hx_cnt) (void)hipFree(p->d_hx_cnt);
-  if (p->d_cslot) (void)hipFree(p->d_cslot);
-  if (p->d_cinv) (void)hipFree(p->d_cinv);
-  if (p->d_ctab) (void)hipFree(p->d_ctab);
-  if (p->d_ctab4) (void)hipFree(p->d_ctab4);
-  if (p->d_start) (void)hipFree(p->d_start);
-  if (p->d_affine) (void)hipFree(p->d_affine);
-  if (p->d_p0) (void)hipFree(p->d_p0);
-  if (p->d_cmap_scalar) (void)hipFree(p->d_cmap_scalar);
-  if (p->d_cmap_params) (void)hipFree(p->d_cmap_params);
-  if (p->launcher_ws.base) (void)hipFree(p->launcher_ws.base);
+  if (p->d_blob) (void)hipFree(p->d_blob);
   delete p;
   return HCX_OK;
 }
@@ -1244,9 +1382,9 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   if (o->precision == HCX_PREC_FP64 && nseg == 1 && (total_groups_needed <= 4LL * g_cu || o->replicas > 1)) {
     Seg& S = LN.seg[0];
     const hcx_problem* p = probs[0];
-    const int lg = lds_group_bytes(pl.nmax, pl.keys(), p->C, p->M, true);
+    const int lg = pl.group_bytes(p, true);
     const size_t terms =
-        pl.exact ? 0 : ((size_t)p->n * p->n * p->hxT + (size_t)p->n * p->htT) * sizeof(dev::Term);
+        pl.exact ? 0 : ((size_t)p->hx_recs + (size_t)p->n * p->htT64) * sizeof(dev::Term);
     auto waves = [&](int R) {
       const long long gpw = 64 / (S.G * R);
       return (S.P + gpw - 1) / gpw;
@@ -1278,13 +1416,23 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     const KernelFn rf = pick_rep(pl.nmax, pl.deg, pl.exact);
     if (!rf) R = 1;
     const size_t regions = (size_t)(64 / (S.G * R)) * (size_t)lg;
-    if (regions + (size_t)pl.tab_lds + terms <= 65536) {
+    // the rule counts compact tables at 4 or 8 bytes a term
+    size_t tab = 0, tab_lat = 0;
+    if (pl.exact && pl.tab_lds > 0) {
+      tab = (size_t)(pl.tab4 ? p->ctab4_bytes : p->ctab_bytes);
+      tab_lat = (size_t)(rf ? p->ltab64 : p->ctab64)[pl.tab4 ? 0 : 1].words * 4;
+    }
+    if (regions + tab + terms <= 65536 && regions + tab_lat + terms <= (size_t)kMaxLdsBytes) {
       LN.dot_lds = 1;
-      S.lds_group = lg;
       S.R = R;
-      if (rf) pl.fn = rf;
-      // the generic latency instances read their term records from LDS
-      if (!pl.exact && rf) pl.tab_lds = (int)terms;
+      if (rf) {
+        pl.fn = rf;
+        pl.latency = true;
+        seg_tables(S, p, pl);
+        if (pl.exact) pl.tab_lds = (int)tab_lat;
+        else pl.tab_lds = (int)terms;  // the generic latency instances read their term records from LDS
+      }
+      S.lds_group = lg;
       seg_groups[0] = waves(R);
       total_groups_needed = seg_groups[0];
     }
@@ -1387,11 +1535,12 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     // regions stay within 64 KiB
     size_t need = 0;
     for (int s = 0; s < nseg; ++s)
-      need = std::max(need, (size_t)(64 / L2.seg[s].G) *
-                                (size_t)lds_group_bytes(p2.nmax, p2.keys(), probs[s]->C, probs[s]->M, true));
+      need = std::max(need, (size_t)(64 / L2.seg[s].G) * (size_t)p2.group_bytes(probs[s], true));
     L2.dot_lds = need + (size_t)p2.tab_lds <= 65536 ? 1 : 0;
-    for (int s = 0; s < nseg; ++s)
-      L2.seg[s].lds_group = lds_group_bytes(p2.nmax, p2.keys(), probs[s]->C, probs[s]->M, L2.dot_lds != 0);
+    for (int s = 0; s < nseg; ++s) {
+      seg_tables(L2.seg[s], probs[s], p2);
+      L2.seg[s].lds_group = p2.group_bytes(probs[s], L2.dot_lds != 0);
+    }
     st = finish_plan(L2, p2);
     if (st != HCX_OK) return st;
     // a small persistent grid: the list holds few paths; idle waves exit at once
