@@ -415,8 +415,13 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
   int label = g.gl;
   cx<T> own_rinv = cmk<T>(T(0), T(0));  // 1 / U_ii of the row this lane ends up holding
   singular = false;
+  // Every lane takes part in the LDS maximum (a mask would cost a branch): a
+  // lane that is no candidate, or belongs to a replica other than the first
+  // (whose rows are replica 0's), adds key 0, which changes no word, to a word
+  // of its own among the group's x slots.
+  constexpr int kXWords = 2 * (NMAX + 2);
+  unsigned long long* const no_key = keys - kXWords + (g.gl + g.s * g.G) % kXWords;
   if constexpr (GC == 0) {
-    // the replicas of a group hold the same rows: replica 0 searches
     if (row && g.s == 0) keys[g.gl] = 0ull;
   }
   // sp shares the group's LDS slots with x: the evaluation's reads of x come first
@@ -428,8 +433,13 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
     if constexpr (GC > 0) {
       key = group_max_key<GC>(key);
     } else {
-      if (cand && g.s == 0)
-        __hip_atomic_fetch_max(&keys[k], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+      const bool mine = cand && g.s == 0;
+      __hip_atomic_fetch_max(mine ? &keys[k] : no_key, mine ? key : 0ull, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WAVEFRONT);
+      // requested ahead of the rest of the pivot row
+      HCX_WAVE_SYNC();
+      key = keys[k];
+      HCX_WAVE_SYNC();
     }
   };
   search(0);
@@ -439,29 +449,48 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
       cx<T> rinv;
       if constexpr (SCALED) rinv = crecip_scaled(A[k]);
       else rinv = crecip_smith(A[k]);
-      if constexpr (GC == 0) {
-        HCX_WAVE_SYNC();
-        key = keys[k];
-      }
+      // keeps the reciprocal out of the pivot's branch, beside the search
+      asm volatile("" : "+v"(rinv.re), "+v"(rinv.im));
       const int blabel = 31 - (int)((unsigned int)key & 31u);
       const bool zero = key < 32ull;
       const bool piv = row && label == blabel;
       singular = singular || zero;
+      const bool more = k + 1 < NMAX && k + 1 < n;
+      // the two entries that the next search waits for go out, and are
+      // requested, before the rest of the row
+      constexpr bool kSplit = NMAX > 6;
       if (piv) {
         sp[k] = rinv;
+        if (more) sp[k + 1] = A[k + 1];
+        if constexpr (!kSplit) {
 #pragma unroll
-        for (int j = k + 1; j < NMAX; ++j)
-          if (j < n) sp[j] = A[j];
-        sp[NMAX] = b;
-        own_rinv = rinv;
+          for (int j = k + 2; j < NMAX; ++j)
+            if (j < n) sp[j] = A[j];
+          sp[NMAX] = b;
+          own_rinv = rinv;
+        }
       }
       HCX_WAVE_SYNC();
+      const cx<T> rp = sp[k];
+      cx<T> next = cmk<T>(T(0), T(0));
+      if (more) next = sp[k + 1];
+      if constexpr (kSplit) {
+        HCX_WAVE_SYNC();
+        if (piv) {
+#pragma unroll
+          for (int j = k + 2; j < NMAX; ++j)
+            if (j < n) sp[j] = A[j];
+          sp[NMAX] = b;
+          own_rinv = rinv;
+        }
+        HCX_WAVE_SYNC();
+      }
       label = piv ? k : (label == k ? blabel : label);
       const bool upd = row && !piv && !zero;
-      cx<T> l = cmul_fused(A[k], sp[k]);
+      cx<T> l = cmul_fused(A[k], rp);
       l = cmk<T>(upd ? l.re : T(0), upd ? l.im : T(0));
-      if (k + 1 < NMAX && k + 1 < n) {
-        A[k + 1] = cfnms(A[k + 1], l, sp[k + 1]);
+      if (more) {
+        A[k + 1] = cfnms(A[k + 1], l, next);
         search(k + 1);
       }
 #pragma unroll
