@@ -45,47 +45,79 @@ __device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
   return (double)((((int)r1 >> 26) << 6) | (int)(r0 >> 26));
 }
 
-// acc + one Jacobian term (xb, cb: the group's x and coefficient areas); SC: a
-// scaled position.
-template <int DEG, bool SC>
-__device__ __forceinline__ cx<double> jac_term(const unsigned char* rp, const unsigned char* xb,
-                                               const unsigned char* cb, cx<double> acc) {
-  uint32_t r0, r1 = 0;
-  if constexpr (DEG <= 2) {
-    r0 = *reinterpret_cast<const uint32_t*>(rp);
-  } else {
-    const uint2 q = *reinterpret_cast<const uint2*>(rp);
-    r0 = q.x;
-    r1 = q.y;
+// One round over NB columns of a row of dH/dx (throughput instances): term k
+// of each, the zero term past a column's last (SC: a scaled position).  All
+// records are requested together, then all gathers.  off: byte offset of the
+// first column's positions from rp; zero: that of the zero terms.
+template <int NMAX, int DEG, bool SC, int JB, int NB>
+__device__ __forceinline__ void jac_round(const unsigned char* rp, int off, int zero, const int (&cnt)[NB], int k,
+                                          const unsigned char* xb, const unsigned char* cb, cx<double> (&A)[NMAX]) {
+  constexpr int RS = StreamRec<DEG>::kJ;
+  uint32_t r0[NB], r1[NB];
+  cx<double> c[NB], p[NB];
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    if (JB + u < NMAX) {
+      const unsigned char* a = rp + (k < cnt[u] ? off + k * (NMAX * RS) : zero);
+      if constexpr (DEG <= 2) {
+        r0[u] = *reinterpret_cast<const uint32_t*>(a);
+        r1[u] = 0;
+      } else {
+        const uint2 q = *reinterpret_cast<const uint2*>(a);
+        r0[u] = q.x;
+        r1[u] = q.y;
+      }
+      off += cnt[u] * (NMAX * RS);
+    }
   }
-  cx<double> p = lds_at(xb, (r0 >> 16) & 0x3ffu);
-  const cx<double> c = lds_at(cb, r0 & 0xffffu);
-  if constexpr (SC) p = cscale(p, rec_scalar<DEG>(r0, r1));
-  if constexpr (DEG > 2) p = cmul(p, lds_at(xb, r1 & 0xffffu));
-  if constexpr (DEG > 3) p = cmul(p, lds_at(xb, (r1 >> 16) & 0x3ffu));
-  return cfma(acc, c, p);
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    if (JB + u < NMAX) {
+      c[u] = lds_at(cb, r0[u] & 0xffffu);
+      p[u] = lds_at(xb, (r0[u] >> 16) & 0x3ffu);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NB; ++u) {
+    if (JB + u < NMAX) {
+      cx<double> v = p[u];
+      if constexpr (SC) v = cscale(v, rec_scalar<DEG>(r0[u], r1[u]));
+      if constexpr (DEG > 2) v = cmul(v, lds_at(xb, r1[u] & 0xffffu));
+      if constexpr (DEG > 3) v = cmul(v, lds_at(xb, (r1[u] >> 16) & 0x3ffu));
+      A[JB + u] = cfma(A[JB + u], c[u], v);
+    }
+  }
 }
 
 // Row gl of dH/dx from the compact streams at lt
-// (dev-eval-indxing-generalized_3views_4pts.cuh:70-86).  Positions k0, k0 +
-// ks, ... of each column only (a replica's share).
-template <int NMAX, int DEG, int UNR, class SegT>
-__device__ __forceinline__ void eval_jac_stream(const SegT& S, int gle, const unsigned char* xb,
-                                                const unsigned char* cb, cx<double> (&A)[NMAX],
-                                                const unsigned char* lt, int k0, int ks) {
-  constexpr int RS = StreamRec<DEG>::kJ;
-  const unsigned char* rp = lt + gle * RS;
+// (dev-eval-indxing-generalized_3views_4pts.cuh:70-86), NB columns at a time:
+// one column after the other, each term is two exposed LDS latencies and each
+// column two loops.
+template <int NMAX, int DEG, int NB, int JB, class SegT>
+__device__ __forceinline__ void eval_jac_blocks(const SegT& S, const unsigned char* rp, int off,
+                                                const unsigned char* xb, const unsigned char* cb,
+                                                cx<double> (&A)[NMAX]) {
+  if constexpr (JB < NMAX) {
+    int cnt[NB], end = 0, scaled = 0, tot = 0;
 #pragma unroll
-  for (int j = 0; j < NMAX; ++j) {
-    const unsigned int cc = S.colc[j];
-    const int cnt = (int)(cc & 0xffffu), ns = (int)(cc >> 16);
-    cx<double> acc = cmk<double>(0, 0);
-    int k = k0;
-    for (; k < ns; k += ks) acc = jac_term<DEG, true>(rp + k * (NMAX * RS), xb, cb, acc);
-#pragma unroll UNR
-    for (; k < cnt; k += ks) acc = jac_term<DEG, false>(rp + k * (NMAX * RS), xb, cb, acc);
-    rp += cnt * (NMAX * RS);
-    A[j] = acc;
+    for (int u = 0; u < NB; ++u) {
+      cnt[u] = 0;
+      if (JB + u < NMAX) {
+        const unsigned int cc = S.colc[JB + u];
+        cnt[u] = (int)(cc & 0xffffu);
+        end = max(end, cnt[u]);
+        scaled = max(scaled, (int)(cc >> 16));
+        tot += cnt[u];
+        A[JB + u] = cmk<double>(0, 0);
+      }
+    }
+    const int zero = S.hx_recs * StreamRec<DEG>::kJ;
+    int k = 0;
+#pragma unroll 1
+    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB>(rp, off, zero, cnt, k, xb, cb, A);
+#pragma unroll 1
+    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB>(rp, off, zero, cnt, k, xb, cb, A);
+    eval_jac_blocks<NMAX, DEG, NB, JB + NB>(S, rp, off + tot * (NMAX * StreamRec<DEG>::kJ), xb, cb, A);
   }
 }
 

@@ -928,7 +928,8 @@ enum : int {
 // REP: the latency instance (launches of few paths, one wave per SIMD at
 // most): R >= 1 replicas per path (Seg::R) and chunked coefficient staging,
 // compiled apart so that the throughput loop carries none of it.
-template <int NMAX, int DEG, bool EXACT, bool REP>
+// NB: Jacobian columns evaluated together (as the register budget allows).
+template <int NMAX, int DEG, bool EXACT, bool REP, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
 __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsigned char* smem, int lane) {
   Seg S = LN.seg[si];
   constexpr int GE = exact_lanes(NMAX);
@@ -1097,7 +1098,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
           else
             r = eval_rhs_stream<NMAX, DEG, false, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
         } else {
-          eval_jac_stream<NMAX, DEG, 2>(Sk, gle, xb, cb, A, lt, k0, ks);
+          eval_jac_blocks<NMAX, DEG, NB, 0>(Sk, lt + gle * StreamRec<DEG>::kJ, 0, xb, cb, A);
           if (gdot)
             r = eval_rhs_stream<NMAX, DEG, true, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
@@ -1291,7 +1292,7 @@ void track_kernel_rep(const Launch LN) {
 template <int N, int DEG, int MODE>
 __device__ __forceinline__ void run_exact(const Launch& LN, int si, unsigned char* smem, int lane) {
   if constexpr (MODE == 0) {
-    run_segment_fp64<N, DEG, true, false>(LN, si, smem, lane);
+    run_segment_fp64<N, DEG, true, false, 2>(LN, si, smem, lane);
   } else {
     run_segment<N, DEG, MODE, true>(LN, si, smem, lane);
   }

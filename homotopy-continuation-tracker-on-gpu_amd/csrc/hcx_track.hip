@@ -1042,6 +1042,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
         else put(hxs[r], false);
       for (int i = 0; lat && i < n; ++i) put_lat(zero_term);
     }
+    for (int i = 0; !lat && i < n; ++i) put(zero_term, false);  // one row of zero terms for all columns
     ch.h = align();
     r = 0;
     for (int k = 0; k < htT64 * n; ++k) put(hts[r++], true);
