@@ -91,7 +91,7 @@ __device__ __forceinline__ double frcp(double x) {
 // of either kind, so a branch runs both of its sides).
 // Smith's scaling (as cdiv), the roles of the components selected.
 template <class T>
-__device__ __forceinline__ cx<T> crecip_smith(cx<T> b) {
+__device__ __forceinline__ cx<T> crecip(cx<T> b) {
   const bool rbig = fabs(b.re) >= fabs(b.im);
   const T big = rbig ? b.re : b.im, small = rbig ? b.im : b.re;
   const T r = small * frcp(big);
@@ -99,18 +99,8 @@ __device__ __forceinline__ cx<T> crecip_smith(cx<T> b) {
   const T ri = r * inv;
   return cmk<T>(rbig ? inv : ri, rbig ? -ri : -inv);
 }
-// FP64: conj(b) / |b|^2 with b scaled by a power of two (exact) so that
-// |b|^2 neither overflows nor underflows: one reciprocal in the dependency
-// chain instead of Smith's two.
-__device__ __forceinline__ cx<double> crecip_scaled(cx<double> b) {
-  const int e = -__builtin_amdgcn_frexp_exp(fmax(fabs(b.re), fabs(b.im)));
-  const double re = __builtin_amdgcn_ldexp(b.re, e), im = __builtin_amdgcn_ldexp(b.im, e);
-  const double r = __builtin_amdgcn_ldexp(frcp(re * re + im * im), e);
-  return cmk<double>(re * r, -im * r);
-}
 // a * b with the roundings spelled out: products of a.im rounded, those of
-// a.re fused (the mixed loop's results do not depend on what the compiler
-// fuses).
+// a.re fused (the solve's results do not depend on what the compiler fuses).
 template <class T>
 __device__ __forceinline__ cx<T> cmul_fused(cx<T> a, cx<T> b) {
   return cmk<T>(__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.re, b.im, a.im * b.re));

@@ -2,18 +2,18 @@
 //
 // A row's terms are a STREAM per lane: position p of equation i at
 // [p][i], all positions of Jacobian column 0, then of column 1, and so on
-// (dH/dx), or all terms of the row (dH/dt, H), in the order of the problem's
-// tables.  The number of positions is the maximum over the equations; an
-// equation with fewer terms holds zero terms at its end (a variable index
-// that reads the constant 0).  A column begins with the positions up to the
-// last one at which some equation has a scalar other than 1 ("scaled"), the
-// rest needs no scaling.  Every instance adds the terms of a row in stream
-// order as acc = fma(coefficient, product of the variables, acc), the scalar
-// applied to the first variable, so instances that differ only in where the
-// streams live give the same bits.
+// (dH/dx), or all terms of the row (dH/dt, H), at their places in the problem's
+// tables.  The number of positions is the maximum over the equations; where an
+// equation has no term it holds a zero term (a variable index that reads the
+// constant 0).  A column begins with the positions up to the last one at which
+// some equation has a scalar other than 1 ("scaled"), the rest needs no
+// scaling.  Every instance computes a term as ((scalar * coefficient) *
+// variable) * variable ... with the roundings of cmul_term and adds the terms
+// of a row in stream order, so instances that differ only in where the streams
+// live give the same bits.
 //
-// What bounds it: per term two or three 16-byte LDS gathers and four FP64
-// FMAs; everything else is overhead, so the records in LDS hold byte offsets
+// What bounds it: per term two or three 16-byte LDS gathers and six to ten
+// FP64 operations; everything else is overhead, so the records in LDS hold byte offsets
 // (no decoding beyond a mask and an add), unscaled positions skip the scaling,
 // and the counts come from the kernel arguments.
 #pragma once
@@ -23,6 +23,12 @@ namespace dev {
 
 __device__ __forceinline__ cx<double> lds_at(const unsigned char* base, uint32_t off) {
   return *reinterpret_cast<const cx<double>*>(base + off);
+}
+
+// a * b with the roundings spelled out (they do not depend on what the
+// compiler fuses): the products with b.im rounded, those with b.re fused.
+__device__ __forceinline__ cx<double> cmul_term(cx<double> a, cx<double> b) {
+  return cmk<double>(__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im));
 }
 
 // Compact records of the size-specialised instances, in LDS: byte offsets of
@@ -80,11 +86,12 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int off, int 
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
-      cx<double> v = p[u];
+      cx<double> v = c[u];
       if constexpr (SC) v = cscale(v, rec_scalar<DEG>(r0[u], r1[u]));
-      if constexpr (DEG > 2) v = cmul(v, lds_at(xb, r1[u] & 0xffffu));
-      if constexpr (DEG > 3) v = cmul(v, lds_at(xb, (r1[u] >> 16) & 0x3ffu));
-      A[JB + u] = cfma(A[JB + u], c[u], v);
+      v = cmul_term(v, p[u]);
+      if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, r1[u] & 0xffffu));
+      if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, (r1[u] >> 16) & 0x3ffu));
+      A[JB + u] = cadd(A[JB + u], v);
     }
   }
 }
@@ -181,10 +188,11 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
-          cx<double> v = cscale(p[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
-          if constexpr (DEG > 2) v = cmul(v, lds_at(xb, r1[u] & 0xffffu));
-          if constexpr (DEG > 3) v = cmul(v, lds_at(xb, r1[u] >> 16));
-          A[jb + u] = cfma(A[jb + u], c[u], v);
+          cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
+          v = cmul_term(v, p[u]);
+          if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, r1[u] & 0xffffu));
+          if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, r1[u] >> 16));
+          A[jb + u] = cadd(A[jb + u], v);
         }
       }
     }
@@ -230,12 +238,13 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, 
   }
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    cx<double> p = lds_at(xb, (r[q][0] >> 16) & 0x3ffu);
-    if constexpr (SC) p = cscale(p, rec_scalar<DEG>(r[q][0], r[q][1]));
-    p = cmul(p, lds_at(xb, r[q][1] & 0xffffu));
-    if constexpr (DEG > 2) p = cmul(p, lds_at(xb, (r[q][1] >> 16) & 0x3ffu));
-    if constexpr (DEG > 3) p = cmul(p, lds_at(xb, r[q][2] & 0xffffu));
-    acc = cfma(acc, c[q], p);
+    cx<double> v = c[q];
+    if constexpr (SC) v = cscale(v, rec_scalar<DEG>(r[q][0], r[q][1]));
+    v = cmul_term(v, lds_at(xb, (r[q][0] >> 16) & 0x3ffu));
+    v = cmul_term(v, lds_at(xb, r[q][1] & 0xffffu));
+    if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, (r[q][1] >> 16) & 0x3ffu));
+    if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, r[q][2] & 0xffffu));
+    acc = cadd(acc, v);
   }
   return acc;
 }
@@ -292,10 +301,10 @@ __device__ __forceinline__ cx<double> term_stream_sum(const Term* tp, int cnt, i
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q) {
       if (kb + q * ks < cnt) {
-        cx<double> p = cscale(sx[term_var(tm[q], 0)], (double)tm[q].s);
+        cx<double> v = cscale(c[q], (double)tm[q].s);
 #pragma unroll
-        for (int d = 1; d < NV; ++d) p = cmul(p, sx[term_var(tm[q], d)]);
-        acc = cfma(acc, c[q], p);
+        for (int d = 0; d < NV; ++d) v = cmul_term(v, sx[term_var(tm[q], d)]);
+        acc = cadd(acc, v);
       }
     }
   }

@@ -406,10 +406,7 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 //  * every candidate computes the reciprocal of its own entry during the
 //    search, and the pivot's goes out with its row.
 // keys: NMAX LDS slots of the group (unused with GC > 0).
-// SCALED: the FP64 reciprocal with one step less in its chain; the mixed loop
-// keeps Smith's, since the last bits of its FP64 corrector decide which FP32
-// point the next predictor starts from.
-template <int NMAX, int GC, bool SCALED, class T>
+template <int NMAX, int GC, class T>
 __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const Group& g, int n, bool row,
                                                 cx<T>* sp, unsigned long long* keys, bool& singular) {
   int label = g.gl;
@@ -446,9 +443,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
 #pragma unroll
   for (int k = 0; k < NMAX; ++k) {
     if (k < n) {
-      cx<T> rinv;
-      if constexpr (SCALED) rinv = crecip_scaled(A[k]);
-      else rinv = crecip_smith(A[k]);
+      cx<T> rinv = crecip(A[k]);
       // keeps the reciprocal out of the pivot's branch, beside the search
       asm volatile("" : "+v"(rinv.re), "+v"(rinv.im));
       const int blabel = 31 - (int)((unsigned int)key & 31u);
@@ -577,7 +572,7 @@ __device__ __forceinline__ void newton_pass(const SegT& S, int n, const OT& o, c
     eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
     const cx<T> h = eval_t_row<DEG, T, LT>(S, n, gle, sx, sc, lt);
     bool sing;
-    const cx<T> d = group_lu_solve<NMAX, GC, false, T>(A, h, g, n, row, L.template piv<T>(), L.keys(), sing);
+    const cx<T> d = group_lu_solve<NMAX, GC, T>(A, h, g, n, row, L.template piv<T>(), L.keys(), sing);
     if (run && row) x = csub(x, ccast<double>(d));
     double rs = row ? (double)cnorm2(d) : 0.0;
     double rc = row ? cnorm2(x) : 0.0;
@@ -619,7 +614,7 @@ __device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group&
     eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
     const cx<T> bt = eval_t_row<DEG, T, LT>(S, n, gle, sx, sd, lt);
     bool sing;
-    const cx<T> k = group_lu_solve<NMAX, GC, false, T>(A, cmk<T>(-bt.re, -bt.im), g, n, row, L.template piv<T>(), L.keys(), sing);
+    const cx<T> k = group_lu_solve<NMAX, GC, T>(A, cmk<T>(-bt.re, -bt.im), g, n, row, L.template piv<T>(), L.keys(), sing);
     kprev = ccast<double>(k);
     const double w = (st == 1 || st == 2) ? 2.0 : 1.0;
     acc = cmk<double>(acc.re + w * kprev.re, acc.im + w * kprev.im);
@@ -835,7 +830,7 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
           eval_jac_row<NMAX, DEG, double, LT>(Sk, n, gle, sx, sc, A, lt);
           const cx<double> hv = eval_t_row<DEG, double, LT>(Sk, n, gle, sx, sc, lt);
           bool sing;
-          const cx<double> d = group_lu_solve<NMAX, GC, false, double>(A, hv, g, n, row, L.template piv<double>(), L.keys(), sing);
+          const cx<double> d = group_lu_solve<NMAX, GC, double>(A, hv, g, n, row, L.template piv<double>(), L.keys(), sing);
           if (run && row) x = csub(x, d);
           double nd = row ? cnorm2(d) : 0.0, nx = row ? cnorm2(x) : 0.0;
           nd = group_sum(nd, g, lane);
@@ -1133,7 +1128,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       }
       bool sing;
       const cx<double> d =
-          group_lu_solve<NMAX, GC, true, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.template piv<double>(), L.keys(), sing);
+          group_lu_solve<NMAX, GC, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.template piv<double>(), L.keys(), sing);
 
       // RK4 stage: k_s = solution, accumulate k1 + 2 k2 + 2 k3 + k4
       if (stg) {

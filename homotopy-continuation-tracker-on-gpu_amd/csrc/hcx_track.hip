@@ -949,21 +949,18 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   zero_term.c = 0;
   zero_term.v03 = (uint32_t)(n + 1) | (uint32_t)n << 8 | (uint32_t)n << 16 | (uint32_t)n << 24;
   zero_term.v47 = (uint32_t)n * 0x01010101u;
-  // appends one entry's stream [position][equation]; returns its scaled positions
+  // appends one entry's stream [position][equation], up to the last position
+  // with a term; returns its scaled positions
   auto add_stream = [&](std::vector<dev::Term>& out, auto&& term_at, int T) {
-    std::vector<std::vector<dev::Term>> a(n);
-    size_t cnt = 0, scaled = 0;
-    for (int i = 0; i < n; ++i) {
-      for (int tt = 0; tt < T; ++tt) {
-        const dev::Term& tm = term_at(tt, i);
-        if (tm.s == 0) continue;
-        a[i].push_back(tm);
-        if (tm.s != 1) scaled = std::max(scaled, a[i].size());
+    int cnt = 0, scaled = 0;
+    for (int tt = 0; tt < T; ++tt)
+      for (int i = 0; i < n; ++i) {
+        const int s = term_at(tt, i).s;
+        if (s != 0) cnt = tt + 1;
+        if (s != 0 && s != 1) scaled = tt + 1;
       }
-      cnt = std::max(cnt, a[i].size());
-    }
-    for (size_t k = 0; k < cnt; ++k)
-      for (int i = 0; i < n; ++i) out.push_back(k < a[i].size() ? a[i][k] : zero_term);
+    for (int tt = 0; tt < cnt; ++tt)
+      for (int i = 0; i < n; ++i) out.push_back(term_at(tt, i).s != 0 ? term_at(tt, i) : zero_term);
     return scaled;
   };
   std::vector<dev::Term> hxs, hts;
@@ -973,15 +970,15 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   int s_min = 0, s_max = 0;
   for (int j = 0; j < n; ++j) {
     const size_t at = hxs.size();
-    const size_t scaled = add_stream(
+    const int scaled = add_stream(
         hxs, [&](int tt, int i) -> const dev::Term& { return hx[((size_t)j * d->hx_terms + tt) * n + i]; },
         d->hx_terms);
     const size_t cnt = (hxs.size() - at) / n;
     colc64_fits = colc64_fits && cnt <= 0xffff;
-    colc64[j] = (unsigned int)(cnt & 0xffff) | (unsigned int)(scaled & 0xffff) << 16;
+    colc64[j] = (unsigned int)(cnt & 0xffff) | ((unsigned int)scaled & 0xffff) << 16;
     hxs_cnt[j] = (int)cnt;
   }
-  const int htS = (int)add_stream(
+  const int htS = add_stream(
       hts, [&](int tt, int i) -> const dev::Term& { return ht[(size_t)tt * n + i]; }, d->ht_terms);
   const int htT64 = (int)(hts.size() / n), hx_recs = (int)hxs.size();
   for (const auto& tm : hts) ht_ci.push_back(cinv[tm.c]);
