@@ -148,7 +148,7 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
                                                 const unsigned char* cb, cx<double> (&A)[NMAX],
                                                 const unsigned char* lt, int k0, int ks) {
   constexpr int RS = LatencyRec<DEG>::kJ;
-  constexpr int NB = NMAX <= 8 ? NMAX : (NMAX + 1) / 2;  // columns at a time
+  constexpr int NB = NMAX <= 6 ? NMAX : (NMAX <= 10 ? (NMAX + 1) / 2 : 4);  // columns at a time
   const int rounds_end = S.max_terms;
 #pragma unroll
   for (int j = 0; j < NMAX; ++j) A[j] = cmk<double>(0, 0);
@@ -185,6 +185,7 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
           p[u] = lds_at(xb, r0[u] >> 16);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
@@ -204,7 +205,7 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
 // this lane's group sums dc/dt (an RK4 stage) instead of c(t): from its LDS
 // area at db, or (GDOT) from global memory, requested for the whole chunk
 // before the first product.
-template <int NMAX, int DEG, bool SC, bool GDOT, int Q>
+template <int NMAX, int DEG, bool SC, bool GDOT, int Q, bool PIN>
 __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, int ks, int cnt,
                                                 const unsigned char* xb, const unsigned char* cb,
                                                 const double2* dg, bool dot, cx<double> acc) {
@@ -225,8 +226,13 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, 
       r[q][2] = v.z;
     }
   }
+  cx<double> x0[Q], x1[Q];
 #pragma unroll
-  for (int q = 0; q < Q; ++q) c[q] = lds_at(cb, r[q][0] & 0xffffu);
+  for (int q = 0; q < Q; ++q) {
+    c[q] = lds_at(cb, r[q][0] & 0xffffu);
+    x0[q] = lds_at(xb, (r[q][0] >> 16) & 0x3ffu);
+    x1[q] = lds_at(xb, r[q][1] & 0xffffu);
+  }
   if constexpr (GDOT) {
     if (dot) {
 #pragma unroll
@@ -236,12 +242,15 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, 
       }
     }
   }
+  // PIN: every load of the chunk is requested before the first product, also
+  // where the compiler would rather save registers
+  if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     cx<double> v = c[q];
     if constexpr (SC) v = cscale(v, rec_scalar<DEG>(r[q][0], r[q][1]));
-    v = cmul_term(v, lds_at(xb, (r[q][0] >> 16) & 0x3ffu));
-    v = cmul_term(v, lds_at(xb, r[q][1] & 0xffffu));
+    v = cmul_term(v, x0[q]);
+    v = cmul_term(v, x1[q]);
     if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, (r[q][1] >> 16) & 0x3ffu));
     if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, r[q][2] & 0xffffu));
     acc = cadd(acc, v);
@@ -251,7 +260,7 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, 
 
 // Row gl of sum_k s * coef * prod x over the dH/dt streams (…cuh:89-120):
 // H with c(t), dH/dt with dc/dt.
-template <int NMAX, int DEG, bool GDOT, int Q, class SegT>
+template <int NMAX, int DEG, bool GDOT, int Q, bool PIN, class SegT>
 __device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int gle, const unsigned char* xb,
                                                       const unsigned char* cb, const unsigned char* db,
                                                       const double2* dg, bool dot, const unsigned char* lt, int k0,
@@ -262,9 +271,9 @@ __device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int gle, co
   cx<double> acc = cmk<double>(0, 0);
   int k = 0;
 #pragma unroll 1
-  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<NMAX, DEG, true, GDOT, Q>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<NMAX, DEG, true, GDOT, Q, PIN>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
 #pragma unroll 1
-  for (; k < cnt; k += Q * ks) acc = rhs_chunk<NMAX, DEG, false, GDOT, Q>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  for (; k < cnt; k += Q * ks) acc = rhs_chunk<NMAX, DEG, false, GDOT, Q, PIN>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
   return acc;
 }
 
@@ -349,64 +358,99 @@ __device__ __forceinline__ cx<double> eval_rhs_terms(const SegT& S, int n, int g
 }
 
 // ------------------------------------------------------------ staging
-// LDS byte offset of coefficient j's slot from the coefficient area;
-// kNoSlot: no term uses it.
-constexpr uint32_t kNoSlot = 0xffffffffu;
-// SL: the list is in LDS with the compact tables.
+// LDS byte offset of coefficient j from the group's region.  A coefficient
+// that no term uses has no slot: it goes to offset 0, x's first slot, which
+// is published after the staging (no branch per coefficient).  SL: the list is
+// in LDS with the compact tables; head: offset of the coefficient area.
 template <bool SL, class SegT>
-__device__ __forceinline__ uint32_t slot_offset(const SegT& S, const unsigned char* lt, int j) {
+__device__ __forceinline__ uint32_t slot_offset(const SegT& S, const unsigned char* lt, int j, int head) {
   if constexpr (SL) {
-    const uint32_t o = reinterpret_cast<const unsigned short*>(lt + S.tab_slot)[j];
-    return o == 0xffffu ? kNoSlot : o;
+    return reinterpret_cast<const unsigned short*>(lt + S.tab_slot)[j];
   } else {
     const int q = S.cslot[j];
-    return q < S.nslot ? (uint32_t)q * 16u : kNoSlot;
+    return q < S.nslot ? (uint32_t)(head + q * 16) : 0u;
   }
 }
 
-// c_j(t) and (with_dot) dc_j/dt(t) of order MC in t into the group's LDS
-// slots, Q of the lane's coefficients at a time: all of a chunk's loads are
-// requested before the first is used, so the staging costs one memory latency
-// per Q coefficients.  hx, ht: the instance's tables.  Surplus entries of the
-// last chunk repeat the last coefficient.
+// c_j(t) of order MC in t and (dot) dc_j/dt(t) into the group's LDS slots, Q of
+// the lane's coefficients at a time: all of a chunk's loads are requested
+// before the first is used, so the staging costs one memory latency per Q
+// coefficients; full chunks address with constant offsets, the last
+// coefficients go one by one.  hx, ht: the instance's tables; xb: the group's
+// region, db: from a slot of c to that of dc/dt.
 template <int MC, int Q, bool SL, class SegT>
 __device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, const double2* hx, const double2* ht,
-                                             double t, unsigned char* cb, unsigned char* db, bool with_dot,
+                                             double t, unsigned char* xb, int head, int db, bool dot,
                                              const unsigned char* lt) {
   const int C1 = S.C + 1, st = g.G * g.R;
+  auto put = [&](const double2* a, uint32_t o) {
+    double cr = a[MC].x, ci = a[MC].y;
+#pragma unroll
+    for (int m = MC - 1; m >= 0; --m) {
+      cr = cr * t + a[m].x;
+      ci = ci * t + a[m].y;
+    }
+    *reinterpret_cast<cx<double>*>(xb + o) = cmk<double>(cr, ci);
+  };
+  auto put_dot = [&](const double2* b, uint32_t o) {
+    double dr = b[MC - 1].x, di = b[MC - 1].y;
+#pragma unroll
+    for (int m = MC - 2; m >= 0; --m) {
+      dr = dr * t + b[m].x;
+      di = di * t + b[m].y;
+    }
+    if (o) *reinterpret_cast<cx<double>*>(xb + db + o) = cmk<double>(dr, di);
+  };
+  int j = g.gl + g.s * g.G;
+  const double2* ha = hx + (size_t)j * (MC + 1);
+  const double2* hb = ht + (size_t)j * MC;
 #pragma unroll 1
-  for (int jb = g.gl + g.s * g.G; jb < C1; jb += Q * st) {
+  for (; j + (Q - 1) * st < C1; j += Q * st) {
     double2 a[Q][MC + 1], b[Q][MC];
     uint32_t o[Q];
 #pragma unroll
     for (int u = 0; u < Q; ++u) {
-      const int j = min(jb + u * st, C1 - 1);
-      o[u] = slot_offset<SL>(S, lt, j);
 #pragma unroll
-      for (int m = 0; m <= MC; ++m) a[u][m] = hx[(size_t)((unsigned int)j * (MC + 1) + m)];
-      if (with_dot) {
+      for (int m = 0; m <= MC; ++m) a[u][m] = ha[u * st * (MC + 1) + m];
+      o[u] = slot_offset<SL>(S, lt, j + u * st, head);
+    }
+    if (dot) {
 #pragma unroll
-        for (int m = 0; m < MC; ++m) b[u][m] = ht[(size_t)((unsigned int)j * MC + m)];
+      for (int u = 0; u < Q; ++u)
+#pragma unroll
+        for (int m = 0; m < MC; ++m) b[u][m] = hb[u * st * MC + m];
+    }
+#pragma unroll
+    for (int u = 0; u < Q; ++u) put(a[u], o[u]);
+    if (dot) {
+#pragma unroll
+      for (int u = 0; u < Q; ++u) put_dot(b[u], o[u]);
+    }
+    ha += Q * st * (MC + 1);
+    hb += Q * st * MC;
+  }
+  // the rest, fewer than Q: as one chunk whose surplus repeats the last
+  // coefficient
+  if (j < C1) {
+    constexpr int Q1 = Q > 1 ? Q - 1 : 1;
+    double2 a[Q1][MC + 1], b[Q1][MC];
+    uint32_t o[Q1];
+#pragma unroll
+    for (int u = 0; u < Q1; ++u) {
+      const int d = j + u * st < C1 ? u * st : 0;
+#pragma unroll
+      for (int m = 0; m <= MC; ++m) a[u][m] = ha[d * (MC + 1) + m];
+      o[u] = slot_offset<SL>(S, lt, j + d, head);
+      if (dot) {
+#pragma unroll
+        for (int m = 0; m < MC; ++m) b[u][m] = hb[d * MC + m];
       }
     }
 #pragma unroll
-    for (int u = 0; u < Q; ++u) {
-      double cr = a[u][MC].x, ci = a[u][MC].y;
+    for (int u = 0; u < Q1; ++u) put(a[u], o[u]);
+    if (dot) {
 #pragma unroll
-      for (int m = MC - 1; m >= 0; --m) {
-        cr = cr * t + a[u][m].x;
-        ci = ci * t + a[u][m].y;
-      }
-      if (o[u] != kNoSlot) *reinterpret_cast<cx<double>*>(cb + o[u]) = cmk<double>(cr, ci);
-      if (with_dot) {
-        double dr = b[u][MC - 1].x, di = b[u][MC - 1].y;
-#pragma unroll
-        for (int m = MC - 2; m >= 0; --m) {
-          dr = dr * t + b[u][m].x;
-          di = di * t + b[u][m].y;
-        }
-        if (o[u] != kNoSlot) *reinterpret_cast<cx<double>*>(db + o[u]) = cmk<double>(dr, di);
-      }
+      for (int u = 0; u < Q1; ++u) put_dot(b[u], o[u]);
     }
   }
 }
@@ -415,52 +459,40 @@ __device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, cons
 // (eval_parameter_homotopy, …cuh:34-67).  Coefficient j goes to slot
 // cslot[j]: slots follow the order in which the rows of a group read them
 // (term by term), so the lanes of a group that read term k of their rows
-// together hit consecutive LDS words instead of words one equation apart; a
-// coefficient that no term uses has no slot.  The replicas of a group share
-// its LDS region and stage every R-th coefficient each.  Q: coefficients in
-// flight per lane at order 1 (fewer at higher orders, by their registers).
+// together hit consecutive LDS words instead of words one equation apart.  The
+// replicas of a group share its LDS region and stage every R-th coefficient
+// each.  Q: coefficients in flight per lane at order 1 (fewer at higher
+// orders, by their registers).
 template <bool SL, int Q, class SegT>
 __device__ __forceinline__ void stage_coeffs64(const SegT& S, const Group& g, const double2* hx, const double2* ht,
-                                               double t, unsigned char* cb, unsigned char* db, bool with_dot,
+                                               double t, unsigned char* xb, int head, int db, bool dot,
                                                const unsigned char* lt) {
-  if constexpr (Q >= 8) {
-    // the latency instances: a chunk that fits the lane's share
-    const int st = g.G * g.R;
-    const bool few = S.C + 1 <= 2 * st, some = S.C + 1 <= 4 * st;
-    if (S.M == 1) {
-      if (few) return stage_chunks<1, 2, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
-      if (some) return stage_chunks<1, 4, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
-    } else if (S.M == 2 && few) {
-      return stage_chunks<2, 2, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
-    }
-  }
   constexpr int Q2 = Q > 2 ? Q / 2 : 1, Q3 = Q > 3 ? Q / 3 : 1;
   switch (S.M) {
-    case 1: return stage_chunks<1, Q, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
-    case 2: return stage_chunks<2, Q2, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
-    case 3: return stage_chunks<3, Q3, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
-    case 4: return stage_chunks<4, Q3, SL>(S, g, hx, ht, t, cb, db, with_dot, lt);
+    case 1: return stage_chunks<1, Q, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 2: return stage_chunks<2, Q2, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 3: return stage_chunks<3, Q3, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 4: return stage_chunks<4, Q3, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
     default: break;
   }
   const int C1 = S.C + 1, M = S.M;
   for (int j = g.gl + g.s * g.G; j < C1; j += g.G * g.R) {
-    const uint32_t o = slot_offset<SL>(S, lt, j);
-    if (o == kNoSlot) continue;
+    const uint32_t o = slot_offset<SL>(S, lt, j, head);
     const double2* ha = hx + (size_t)j * (M + 1);
     double cr = ha[M].x, ci = ha[M].y;
     for (int m = M - 1; m >= 0; --m) {
       cr = cr * t + ha[m].x;
       ci = ci * t + ha[m].y;
     }
-    *reinterpret_cast<cx<double>*>(cb + o) = cmk<double>(cr, ci);
-    if (with_dot) {
+    *reinterpret_cast<cx<double>*>(xb + o) = cmk<double>(cr, ci);
+    if (dot && o) {
       const double2* hb = ht + (size_t)j * M;
       double dr = hb[M - 1].x, di = hb[M - 1].y;
       for (int m = M - 2; m >= 0; --m) {
         dr = dr * t + hb[m].x;
         di = di * t + hb[m].y;
       }
-      *reinterpret_cast<cx<double>*>(db + o) = cmk<double>(dr, di);
+      *reinterpret_cast<cx<double>*>(xb + db + o) = cmk<double>(dr, di);
     }
   }
 }

@@ -952,7 +952,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
     if (LN.tab_lds > 0) tl = stage_terms(S, n, smem);
   }
   // coefficients in flight per lane while staging (order 1)
-  constexpr int SQ = REP ? 8 : (EXACT && NMAX <= 16 ? 4 : 2);
+  constexpr int SQ = EXACT && NMAX <= 16 ? 4 : 2;
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
   Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
   cx<double>* sx = L.x64();
@@ -1078,7 +1078,9 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       const cx<double> xe = stg ? cmk<double>(xl.re + a * kp.re, xl.im + a * kp.im) : x;
       const bool restage = act && te != tst;
       if (restage) {
-        stage_coeffs64<LT && NMAX <= 16, SQ>(Sk, g, hxi, hti, te, cb, db, !gdot, lt);
+        // order 1: dc/dt does not depend on t, once per path is enough
+        const bool dot = !gdot && (Sk.M > 1 || tst < 0.0);
+        stage_coeffs64<LT && NMAX <= 16, SQ>(Sk, g, hxi, hti, te, xb, (int)(cb - xb), (int)(db - cb), dot, lt);
         tst = te;
       }
       publish_x64(sx, xe, g, n, act, row);
@@ -1089,15 +1091,16 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
         if constexpr (REP) {
           eval_jac_rounds<NMAX, DEG>(Sk, gle, xb, cb, A, lt, k0, ks);
           if (Sk.htT <= 2 * ks)
-            r = eval_rhs_stream<NMAX, DEG, false, 2>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<NMAX, DEG, false, 2, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<NMAX, DEG, false, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<NMAX, DEG, false, 4, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
         } else {
+          constexpr int HQ = NMAX <= 6 ? 2 : 4;  // H terms in flight
           eval_jac_blocks<NMAX, DEG, NB, 0>(Sk, lt + gle * StreamRec<DEG>::kJ, 0, xb, cb, A);
           if (gdot)
-            r = eval_rhs_stream<NMAX, DEG, true, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<NMAX, DEG, true, HQ, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<NMAX, DEG, false, 4>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<NMAX, DEG, false, HQ, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
         }
       } else {
         const cx<double>* sc = reinterpret_cast<const cx<double>*>(cb);

@@ -1000,10 +1000,10 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   for (int cf = 0; cf < 4; ++cf) {
     const int f = cf & 1;
     const bool lat = cf >= 2;
-    // offsets of 16 bits: 4,095 slots (0xffff marks a coefficient without one);
-    // scalars of 6 or 12 bits
+    // offsets of 16 bits (from the region's start in the slot list), scalars of
+    // 6 or 12 bits
     const int s_lim = f == 0 ? 32 : 2048;
-    if (!colc64_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4095 || C > 0xffff || deg > (f == 0 ? 2 : 4))
+    if (!colc64_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4000 || C > 0xffff || deg > (f == 0 ? 2 : 4))
       continue;
     CompactHost& ch = compact[cf];
     std::vector<uint32_t>& w = ch.w;
@@ -1047,7 +1047,10 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     for (int i = 0; i < n; ++i) put(zero_term, true);
     ch.slot = align();
     for (int c = 0; c <= C; c += 2) {
-      auto off = [&](int q) { return q > C || cslot[q] >= nslot ? 0xffffu : (uint32_t)cslot[q] * 16u; };
+      // offsets from the group's region, whose coefficient area follows x and
+      // the keys of the instance for n; 0: no slot
+      const int head = 16 * (n + 2) + dev::key_bytes(n, !is_pow2(exact_lanes(n)));
+      auto off = [&](int q) { return q > C || cslot[q] >= nslot ? 0u : (uint32_t)(head + cslot[q] * 16); };
       w.push_back(off(c) | off(c + 1) << 16);
     }
     align();
