@@ -56,15 +56,15 @@ __device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
 // records are requested together, then all gathers.  off: byte offset of the
 // first column's positions from rp; zero: that of the zero terms.
 template <int NMAX, int DEG, bool SC, int JB, int NB>
-__device__ __forceinline__ void jac_round(const unsigned char* rp, int off, int zero, const int (&cnt)[NB], int k,
-                                          const unsigned char* xb, const unsigned char* cb, cx<double> (&A)[NMAX]) {
+__device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int off, int zero, const int (&cnt)[NB],
+                                          int k, const unsigned char* xb, const unsigned char* cb, cx<double> (&A)[NMAX]) {
   constexpr int RS = StreamRec<DEG>::kJ;
   uint32_t r0[NB], r1[NB];
   cx<double> c[NB], p[NB];
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
-      const unsigned char* a = rp + (k < cnt[u] ? off + k * (NMAX * RS) : zero);
+      const unsigned char* a = rp + (k < cnt[u] ? off + k * (n * RS) : zero);
       if constexpr (DEG <= 2) {
         r0[u] = *reinterpret_cast<const uint32_t*>(a);
         r1[u] = 0;
@@ -73,7 +73,7 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int off, int 
         r0[u] = q.x;
         r1[u] = q.y;
       }
-      off += cnt[u] * (NMAX * RS);
+      off += cnt[u] * (n * RS);
     }
   }
 #pragma unroll
@@ -101,7 +101,7 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int off, int 
 // one column after the other, each term is two exposed LDS latencies and each
 // column two loops.
 template <int NMAX, int DEG, int NB, int JB, class SegT>
-__device__ __forceinline__ void eval_jac_blocks(const SegT& S, const unsigned char* rp, int off,
+__device__ __forceinline__ void eval_jac_blocks(const SegT& S, int n, const unsigned char* rp, int off,
                                                 const unsigned char* xb, const unsigned char* cb,
                                                 cx<double> (&A)[NMAX]) {
   if constexpr (JB < NMAX) {
@@ -121,10 +121,10 @@ __device__ __forceinline__ void eval_jac_blocks(const SegT& S, const unsigned ch
     const int zero = S.hx_recs * StreamRec<DEG>::kJ;
     int k = 0;
 #pragma unroll 1
-    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB>(rp, off, zero, cnt, k, xb, cb, A);
+    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB>(rp, n, off, zero, cnt, k, xb, cb, A);
 #pragma unroll 1
-    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB>(rp, off, zero, cnt, k, xb, cb, A);
-    eval_jac_blocks<NMAX, DEG, NB, JB + NB>(S, rp, off + tot * (NMAX * StreamRec<DEG>::kJ), xb, cb, A);
+    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB>(rp, n, off, zero, cnt, k, xb, cb, A);
+    eval_jac_blocks<NMAX, DEG, NB, JB + NB>(S, n, rp, off + tot * (n * StreamRec<DEG>::kJ), xb, cb, A);
   }
 }
 
@@ -144,7 +144,7 @@ struct LatencyRec {
 // Replica s of R takes positions s, s + R, ...; past a column's last position
 // it reads the column's zero terms.
 template <int NMAX, int DEG, class SegT>
-__device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const unsigned char* xb,
+__device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, const unsigned char* xb,
                                                 const unsigned char* cb, cx<double> (&A)[NMAX],
                                                 const unsigned char* lt, int k0, int ks) {
   constexpr int RS = LatencyRec<DEG>::kJ;
@@ -163,7 +163,7 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
           const int cnt = (int)(S.colc[jb + u] & 0xffffu);
-          const unsigned char* a = rp + min(k, cnt) * (NMAX * RS);
+          const unsigned char* a = rp + min(k, cnt) * (n * RS);
           if constexpr (DEG <= 2) {
             const uint2 q = *reinterpret_cast<const uint2*>(a);
             r0[u] = q.x;
@@ -174,7 +174,7 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
             r1[u] = q.y;
             rs[u] = q.z;
           }
-          rp += (cnt + 1) * (NMAX * RS);
+          rp += (cnt + (jb + u < n ? 1 : 0)) * (n * RS);
         }
       }
       cx<double> c[NB], p[NB];
@@ -205,8 +205,8 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int gle, const un
 // this lane's group sums dc/dt (an RK4 stage) instead of c(t): from its LDS
 // area at db, or (GDOT) from global memory, requested for the whole chunk
 // before the first product.
-template <int NMAX, int DEG, bool SC, bool GDOT, int Q, bool PIN>
-__device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, int ks, int cnt,
+template <int DEG, bool SC, bool GDOT, int Q, bool PIN>
+__device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int n, int k, int ks, int cnt,
                                                 const unsigned char* xb, const unsigned char* cb,
                                                 const double2* dg, bool dot, cx<double> acc) {
   constexpr int RS = StreamRec<DEG>::kH;
@@ -214,7 +214,7 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, 
   cx<double> c[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    const unsigned char* a = rp + min(k + q * ks, cnt) * (NMAX * RS);
+    const unsigned char* a = rp + min(k + q * ks, cnt) * (n * RS);
     if constexpr (DEG <= 2) {
       const uint2 v = *reinterpret_cast<const uint2*>(a);
       r[q][0] = v.x;
@@ -260,8 +260,8 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int k, 
 
 // Row gl of sum_k s * coef * prod x over the dH/dt streams (…cuh:89-120):
 // H with c(t), dH/dt with dc/dt.
-template <int NMAX, int DEG, bool GDOT, int Q, bool PIN, class SegT>
-__device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int gle, const unsigned char* xb,
+template <int DEG, bool GDOT, int Q, bool PIN, class SegT>
+__device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int n, int gle, const unsigned char* xb,
                                                       const unsigned char* cb, const unsigned char* db,
                                                       const double2* dg, bool dot, const unsigned char* lt, int k0,
                                                       int ks) {
@@ -271,9 +271,9 @@ __device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int gle, co
   cx<double> acc = cmk<double>(0, 0);
   int k = 0;
 #pragma unroll 1
-  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<NMAX, DEG, true, GDOT, Q, PIN>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<DEG, true, GDOT, Q, PIN>(rp, n, k + k0, ks, cnt, xb, base, dg, dot, acc);
 #pragma unroll 1
-  for (; k < cnt; k += Q * ks) acc = rhs_chunk<NMAX, DEG, false, GDOT, Q, PIN>(rp, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  for (; k < cnt; k += Q * ks) acc = rhs_chunk<DEG, false, GDOT, Q, PIN>(rp, n, k + k0, ks, cnt, xb, base, dg, dot, acc);
   return acc;
 }
 

@@ -406,6 +406,9 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 //  * every candidate computes the reciprocal of its own entry during the
 //    search, and the pivot's goes out with its row.
 // keys: NMAX LDS slots of the group (unused with GC > 0).
+// Where n is not a compile-time constant (generic instances) the columns are
+// checked against it four at a time: columns n..NMAX-1 hold values that no
+// step uses.
 template <int NMAX, int GC, class T>
 __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const Group& g, int n, bool row,
                                                 cx<T>* sp, unsigned long long* keys, bool& singular) {
@@ -460,7 +463,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
         if constexpr (!kSplit) {
 #pragma unroll
           for (int j = k + 2; j < NMAX; ++j)
-            if (j < n) sp[j] = A[j];
+            if ((j & ~3) < n) sp[j] = A[j];
           sp[NMAX] = b;
           own_rinv = rinv;
         }
@@ -474,7 +477,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
         if (piv) {
 #pragma unroll
           for (int j = k + 2; j < NMAX; ++j)
-            if (j < n) sp[j] = A[j];
+            if ((j & ~3) < n) sp[j] = A[j];
           sp[NMAX] = b;
           own_rinv = rinv;
         }
@@ -490,7 +493,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
       }
 #pragma unroll
       for (int j = k + 2; j < NMAX; ++j)
-        if (j < n) A[j] = cfnms(A[j], l, sp[j]);
+        if ((j & ~3) < n) A[j] = cfnms(A[j], l, sp[j]);
       b = cfnms(b, l, sp[NMAX]);
       HCX_WAVE_SYNC();
     }
@@ -942,14 +945,21 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   const bool row = g.in_grp && g.gl < n;
   const int gle = row ? g.gl : 0;
   constexpr bool LT = EXACT && (NMAX <= 16 || DEG <= 2);
+  // The compact streams in LDS: always (LT), or in a generic instance where
+  // the launch found room for them; else the full Term records in global
+  // memory, or (generic latency instance) in LDS.  tab_lds holds the bytes.
+  // DC: the degree of the compact records.
+  constexpr int DC = DEG <= 4 ? DEG : 4;
   const unsigned char* lt = nullptr;
-  // the generic latency instance's full Term records in LDS (tab_lds then
-  // holds their bytes)
   const Term* tl = nullptr;
   if constexpr (LT) {
     lt = static_cast<const unsigned char*>(stage_tables(S, smem));
-  } else if constexpr (!EXACT && REP) {
-    if (LN.tab_lds > 0) tl = stage_terms(S, n, smem);
+  } else if constexpr (!EXACT) {
+    if (LN.tab_lds > 0 && S.ctab) {
+      lt = static_cast<const unsigned char*>(stage_tables(S, smem));
+    } else if constexpr (REP) {
+      if (LN.tab_lds > 0) tl = stage_terms(S, n, smem);
+    }
   }
   // coefficients in flight per lane while staging (order 1)
   constexpr int SQ = EXACT && NMAX <= 16 ? 4 : 2;
@@ -1087,20 +1097,21 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       HCX_WAVE_SYNC();
       cx<double> A[NMAX];
       cx<double> r;
-      if constexpr (LT) {
+      if (LT || (!EXACT && lt)) {
+        constexpr bool kPin = REP || NMAX > 6;
         if constexpr (REP) {
-          eval_jac_rounds<NMAX, DEG>(Sk, gle, xb, cb, A, lt, k0, ks);
+          eval_jac_rounds<NMAX, DC>(Sk, n, gle, xb, cb, A, lt, k0, ks);
           if (Sk.htT <= 2 * ks)
-            r = eval_rhs_stream<NMAX, DEG, false, 2, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, false, 2, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<NMAX, DEG, false, 4, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, false, 4, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         } else {
           constexpr int HQ = NMAX <= 6 ? 2 : 4;  // H terms in flight
-          eval_jac_blocks<NMAX, DEG, NB, 0>(Sk, lt + gle * StreamRec<DEG>::kJ, 0, xb, cb, A);
+          eval_jac_blocks<NMAX, DC, NB, 0>(Sk, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
           if (gdot)
-            r = eval_rhs_stream<NMAX, DEG, true, HQ, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, true, HQ, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<NMAX, DEG, false, HQ, REP || (NMAX > 6)>(Sk, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, false, HQ, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         }
       } else {
         const cx<double>* sc = reinterpret_cast<const cx<double>*>(cb);
@@ -1252,10 +1263,11 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
 }
 
 // Register budget: the size-specialised instances up to n = 6 are compiled
-// for three waves per SIMD (at most 168 VGPRs), which their live state fits
-// without spills.
+// for three waves per SIMD (at most 168 VGPRs), the others up to 16 variables
+// for two, which their live state fits with few spills or none.
+constexpr int waves_per_simd(int nmax, bool exact) { return exact && nmax <= 6 ? 3 : (nmax <= 16 ? 2 : 1); }
 template <int NMAX, int DEG, int MODE, bool EXACT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((EXACT && NMAX <= 6) ? 3 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, EXACT))))
 void track_kernel(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = (int)threadIdx.x & 63;
@@ -1276,7 +1288,7 @@ void track_kernel(const Launch LN) {
 // per SIMD at most, so the register budget is a full SIMD's), with R >= 1
 // replicas per path.
 template <int NMAX, int DEG, bool EXACT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, false))))
 void track_kernel_rep(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
   run_segment_fp64<NMAX, DEG, EXACT, true>(LN, 0, smem, (int)threadIdx.x & 63);

@@ -573,6 +573,19 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
   pl.nmax = kNmaxList[ni];
   pl.deg = kDegList[di];
   pl.exact = false;
+  if (mode == 0 && nseg == 1 && pl.fn) {
+    // a generic FP64 instance reads the compact streams from LDS where they
+    // leave as many waves on a CU as its registers allow (one per SIMD for
+    // NMAX 32, else two) or as there were without them
+    const auto& c = probs[0]->ctab64[pl.tab4 ? 0 : 1];
+    const size_t wave = (size_t)(64 / Gs[0]) * (size_t)pl.group_bytes(probs[0]), tb = (size_t)c.words * 4;
+    const int cap = pl.nmax == 32 ? 4 : 8;
+    int with = 0;
+    for (int wpb : {1, 2, 4}) with = std::max(with, (int)(kMaxLdsBytes / (tb + wpb * wave)) * wpb);
+    if (c.d && tb <= (size_t)kMaxTabLds && std::min(with, cap) >= std::min((int)(kMaxLdsBytes / wave), cap)) {
+      pl.tab_lds = (int)tb;
+    }
+  }
   if (!pl.fn) {
     set_error("no kernel instance for n=%d degree=%d mode=%d", max_n, max_deg, mode);
     return HCX_ERR_UNSUPPORTED;
@@ -597,7 +610,7 @@ void seg_tables(Seg& S, const hcx_problem* p, const Plan& pl) {
     S.max_terms = p->max_terms;
     std::memcpy(S.colc, p->colc64, sizeof(S.colc));
     S.hx_cnt = p->colc64_fits ? nullptr : p->d_hxs_cnt;
-    S.ctab = c.d;
+    S.ctab = pl.tab_lds > 0 ? c.d : nullptr;
     S.tab_words = c.words;
     S.tab_h = c.h;
     S.tab_slot = c.slot;
@@ -1417,21 +1430,23 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     const KernelFn rf = pick_rep(pl.nmax, pl.deg, pl.exact);
     if (!rf) R = 1;
     const size_t regions = (size_t)(64 / (S.G * R)) * (size_t)lg;
-    // the rule counts compact tables at 4 or 8 bytes a term
-    size_t tab = 0, tab_lat = 0;
-    if (pl.exact && pl.tab_lds > 0) {
-      tab = (size_t)(pl.tab4 ? p->ctab4_bytes : p->ctab_bytes);
-      tab_lat = (size_t)(rf ? p->ltab64 : p->ctab64)[pl.tab4 ? 0 : 1].words * 4;
-    }
-    if (regions + tab + terms <= 65536 && regions + tab_lat + terms <= (size_t)kMaxLdsBytes) {
+    // the rule counts the compact tables of the size-specialised instances at 4
+    // or 8 bytes a term, and the full records of the generic ones, which read
+    // compact tables where they fit as well
+    const auto& lat = p->ltab64[pl.tab4 ? 0 : 1];
+    const bool compact = pl.exact ? pl.tab_lds > 0 : rf && lat.d && lat.words * 4 <= 65536;
+    size_t tab = 0, tab_new = terms;
+    if (pl.exact && pl.tab_lds > 0) tab = (size_t)(pl.tab4 ? p->ctab4_bytes : p->ctab_bytes);
+    if (compact) tab_new = (size_t)(rf ? lat.words * 4 : pl.tab_lds);
+    if (regions + tab + terms <= 65536 && regions + tab_new <= (size_t)kMaxLdsBytes) {
       LN.dot_lds = 1;
       S.R = R;
       if (rf) {
         pl.fn = rf;
         pl.latency = true;
+        pl.tab_lds = (int)tab_new;
         seg_tables(S, p, pl);
-        if (pl.exact) pl.tab_lds = (int)tab_lat;
-        else pl.tab_lds = (int)terms;  // the generic latency instances read their term records from LDS
+        if (!compact) S.ctab = nullptr;
       }
       S.lds_group = lg;
       seg_groups[0] = waves(R);
@@ -1537,6 +1552,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     size_t need = 0;
     for (int s = 0; s < nseg; ++s)
       need = std::max(need, (size_t)(64 / L2.seg[s].G) * (size_t)p2.group_bytes(probs[s], true));
+    if (!p2.exact && need + (size_t)p2.tab_lds > 65536) p2.tab_lds = 0;
     L2.dot_lds = need + (size_t)p2.tab_lds <= 65536 ? 1 : 0;
     for (int s = 0; s < nseg; ++s) {
       seg_tables(L2.seg[s], probs[s], p2);
