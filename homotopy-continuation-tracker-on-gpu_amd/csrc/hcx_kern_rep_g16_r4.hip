@@ -1,0 +1,15 @@
+// Latency tracker kernel instances (FP64, 4 replicas per path): generic, NMAX = 16.
+#include "hcx_kernel.hpp"
+
+namespace hcx {
+
+KernelFn kernel_rep_g16_r4(int deg) {
+  switch (deg) {
+    case 2: return track_kernel_rep<16, 2, false, 4>;
+    case 3: return track_kernel_rep<16, 3, false, 4>;
+    case 6: return track_kernel_rep<16, 6, false, 4>;
+    default: return nullptr;
+  }
+}
+
+}  // namespace hcx

@@ -507,6 +507,135 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
   return sol;
 }
 
+// ------------------------------------------------------------ solve of R replicas
+// One level of the reduce-scatter over the replicas: entries 2 i and 2 i + 1 of
+// V, partial sums in this replica and its partner (lane src), become the sum
+// of one of them, the odd one where `odd`.
+template <int N>
+__device__ __forceinline__ void scatter_level(const cx<double> (&V)[N], cx<double> (&W)[(N + 1) / 2], bool odd,
+                                              int src) {
+#pragma unroll
+  for (int i = 0; i < (N + 1) / 2; ++i) {
+    const cx<double> a = V[2 * i], b = 2 * i + 1 < N ? V[2 * i + 1 < N ? 2 * i + 1 : 0] : cmk<double>(0, 0);
+    const cx<double> keep = odd ? b : a, send = odd ? a : b;
+    W[i] = cmk<double>(keep.re + __shfl(send.re, src), keep.im + __shfl(send.im, src));
+  }
+}
+// Partial sums V of a row's entries in the R replicas of a group -> B[i] = the
+// sum of entry R i + s in replica s (the same additions as a butterfly that
+// leaves every sum in every replica, level by level, a half of them each).
+template <int R, int N>
+__device__ __forceinline__ void reduce_scatter(const cx<double> (&V)[N], cx<double> (&B)[(N + R - 1) / R],
+                                               const Group& g, int lane) {
+  const int w = lane - g.s * g.G;  // this row's lane in replica 0
+  cx<double> a[(N + 1) / 2];
+  scatter_level(V, a, (g.s & 1) != 0, (w + (g.s ^ 1) * g.G) & 63);
+  if constexpr (R == 2) {
+#pragma unroll
+    for (int i = 0; i < (N + 1) / 2; ++i) B[i] = a[i];
+  } else {
+    cx<double> b[(N + 3) / 4];
+    scatter_level(a, b, (g.s & 2) != 0, (w + (g.s ^ 2) * g.G) & 63);
+    if constexpr (R == 4) {
+#pragma unroll
+      for (int i = 0; i < (N + 3) / 4; ++i) B[i] = b[i];
+    } else {
+      scatter_level(b, B, (g.s & 4) != 0, (w + (g.s ^ 4) * g.G) & 63);
+    }
+  }
+}
+
+// Bytes of a group's LDS beyond the region of one replica: the column of the
+// step in every replica, and the pivot row.
+constexpr int split_bytes(int nmax, int G, int R) { return R > 1 ? 16 * (R * G + (nmax + R) / R * R) : 0; }
+
+// group_lu_solve of a group of R replicas with the columns dealt out: replica
+// s holds columns s, s + R, ... of its rows, the right-hand side as column
+// NMAX.  Every replica does only its columns' updates (1 / R of the row
+// broadcast and of the arithmetic), which the replicas would otherwise repeat;
+// the step's column, which every row's multiplier comes from, goes to the
+// other replicas through LDS while the pivot search is under way.  The same
+// operations on every entry as in group_lu_solve.  cols: R * G slots, prow:
+// the pivot row.
+// Bound by the chain of n steps (a search of two LDS round trips, the row, a
+// reciprocal), no longer by the row: one path of n = 12, R = 4: 2.82 -> 2.57 ms,
+// 8 paths of n = 3, R = 8: 282 -> 261 us, n = 16, R = 2: 5.80 -> 5.24 ms.  R is a
+// template argument, as the number of columns a lane holds has to be: with the
+// launch's R the instances spilled (n = 16: 6.99 ms).
+template <int NMAX, int R, int NC>
+__device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], const Group& g, int n, bool row,
+                                                        cx<double>* sp, unsigned long long* keys, cx<double>* cols,
+                                                        cx<double>* prow, bool& singular) {
+  static_assert(NC == (NMAX + R) / R, "columns 0..NMAX in R replicas");
+  int label = g.gl;
+  cx<double> own_rinv = cmk<double>(0, 0);
+  singular = false;
+  constexpr int kXWords = 2 * (NMAX + 2);
+  unsigned long long* const no_key = keys - kXWords + (g.gl + g.s * g.G) % kXWords;
+  cx<double>* const mine = prow + g.s;
+  if (row && g.s == 0) keys[g.gl] = 0ull;
+  HCX_WAVE_SYNC();
+  unsigned long long key = 0;
+  cx<double> ck = cmk<double>(0, 0);
+  auto search = [&](int k) {
+    const int so = k % R, io = k / R;
+    if (g.in_grp) cols[g.s * g.G + g.gl] = B[io];
+    const bool cand = row && label >= k && g.s == so;
+    key = pivot_key(cabs1(B[io]), label);
+    __hip_atomic_fetch_max(cand ? &keys[k] : no_key, cand ? key : 0ull, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+    HCX_WAVE_SYNC();
+    key = keys[k];
+    ck = cols[so * g.G + g.gl];
+    HCX_WAVE_SYNC();
+  };
+  search(0);
+#pragma unroll
+  for (int k = 0; k < NMAX; ++k) {
+    if (k < n) {
+      const int so = k % R, io = k / R;
+      cx<double> rinv = crecip(B[io]);  // the pivot's in replica so
+      asm volatile("" : "+v"(rinv.re), "+v"(rinv.im));
+      const int blabel = 31 - (int)((unsigned int)key & 31u);
+      const bool zero = key < 32ull;
+      const bool piv = row && label == blabel;
+      singular = singular || zero;
+      if (piv) {
+#pragma unroll
+        for (int i = io; i < NC; ++i) {
+          cx<double> v = B[i];
+          if (i == io) v = cmk<double>(g.s == so ? rinv.re : v.re, g.s == so ? rinv.im : v.im);
+          if (R * i < n || i == NMAX / R) mine[R * i] = v;
+        }
+      }
+      HCX_WAVE_SYNC();
+      const cx<double> rp = prow[k];
+      label = piv ? k : (label == k ? blabel : label);
+      own_rinv = cmk<double>(piv ? rp.re : own_rinv.re, piv ? rp.im : own_rinv.im);
+      const bool upd = row && !piv && !zero;
+      cx<double> l = cmul_fused(ck, rp);
+      l = cmk<double>(upd ? l.re : 0.0, upd ? l.im : 0.0);
+      const bool more = k + 1 < NMAX && k + 1 < n;
+      if (more) {
+        B[(k + 1) / R] = cfnms(B[(k + 1) / R], l, mine[R * ((k + 1) / R)]);
+        search(k + 1);
+      }
+#pragma unroll
+      for (int i = io; i < NC; ++i)
+        if (i != (k + 1) / R || !more)
+          if (R * i < n || i == NMAX / R) B[i] = cfnms(B[i], l, mine[R * i]);
+      HCX_WAVE_SYNC();
+    }
+  }
+  const cx<double> xi = cmul_fused(B[NMAX / R], own_rinv);
+  if (row && g.s == NMAX % R) sp[label] = xi;
+  HCX_WAVE_SYNC();
+  cx<double> sol = row ? sp[g.gl] : cmk<double>(0, 0);
+  HCX_WAVE_SYNC();
+  if (singular) sol = cmk<double>(NAN, NAN);
+  return sol;
+}
+
 // Copies a segment's compact term tables to the start of the dynamic LDS.
 // Every wave of the block takes part (one copy per block) and the block
 // barrier orders every wave's table reads after the copy; blocks of several
@@ -923,11 +1052,12 @@ enum : int {
 // of the groups of a wave changes.  c(t) is staged in LDS only when the
 // group's evaluation point moves (RK4 stages 0, 1 and 3; the corrector
 // reuses stage 3's c(t + dt)).
-// REP: the latency instance (launches of few paths, one wave per SIMD at
-// most): R >= 1 replicas per path (Seg::R) and chunked coefficient staging,
-// compiled apart so that the throughput loop carries none of it.
+// REP: 0: the throughput loop; else the latency instance (launches of few
+// paths, two waves per SIMD at most): 2, 4 or 8 replicas per path, which share
+// the evaluation's terms and the solve's columns, or (1) Seg::R of them, which
+// share the terms.
 // NB: Jacobian columns evaluated together (as the register budget allows).
-template <int NMAX, int DEG, bool EXACT, bool REP, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
+template <int NMAX, int DEG, bool EXACT, int REP, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
 __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsigned char* smem, int lane) {
   Seg S = LN.seg[si];
   constexpr int GE = exact_lanes(NMAX);
@@ -939,8 +1069,9 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   const KOpts* const opts_arg = launch_opts();
   const KSeg* const seg_arg = launch_seg(si);
   int iter = 0;
-  const Group g = make_group(S.G, lane, REP ? S.R : 1);
-  const int k0 = REP ? g.s : 0, ks = REP ? g.R : 1;  // the replica's terms of each sum
+  const Group g = make_group(S.G, lane, REP > 1 ? REP : (REP ? S.R : 1));
+  // the replica's terms of each sum
+  const int k0 = REP ? g.s : 0, ks = REP > 1 ? REP : (REP ? g.R : 1);
   const int n = S.n;
   const bool row = g.in_grp && g.gl < n;
   const int gle = row ? g.gl : 0;
@@ -964,11 +1095,13 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   // coefficients in flight per lane while staging (order 1)
   constexpr int SQ = EXACT && NMAX <= 16 ? 4 : 2;
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
-  Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
+  Lds<NMAX, GC == 0 || (REP > 0)> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
   cx<double>* sx = L.x64();
   unsigned char* const xb = L.base;
   unsigned char* const cb = L.coef();
   unsigned char* const db = cb + S.nslot * 16;  // dc/dt, when in LDS
+  // the split solve's columns and pivot row (latency instances: dc/dt is in LDS)
+  cx<double>* const cols = reinterpret_cast<cx<double>*>(db + S.nslot * 16);
   // the path's instance tables
   const double2 *hxi = S.chx, *hti = S.cht;
   // dc/dt of the RK4 stages: constant (M = 1) -> read from the instance's
@@ -1098,7 +1231,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       cx<double> A[NMAX];
       cx<double> r;
       if (LT || (!EXACT && lt)) {
-        constexpr bool kPin = REP || NMAX > 6;
+        constexpr bool kPin = REP > 0 || NMAX > 6;
         if constexpr (REP) {
           eval_jac_rounds<NMAX, DC>(Sk, n, gle, xb, cb, A, lt, k0, ks);
           if (Sk.htT <= 2 * ks)
@@ -1122,27 +1255,41 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
           r = eval_rhs_terms<DEG, false>(Sk, n, gle, sx, reinterpret_cast<const cx<double>*>(stg ? db : cb), hti, stg,
                                          tl, k0, ks);
       }
-      if constexpr (REP) {
-        // each replica summed every R-th term of the row's sums: a butterfly
-        // over the replicas (all sums of a level exchanged together) leaves
-        // the full sums, identical in every replica (each level adds a pair
-        // of partial sums, commutatively)
-        for (int m = 1; m < g.R; m <<= 1) {
-          const int src = (lane + ((g.s ^ m) - g.s) * g.G) & 63;
-#pragma unroll
-          for (int j = 0; j < NMAX; ++j) {
-            if (j < n) {
-              A[j].re += __shfl(A[j].re, src);
-              A[j].im += __shfl(A[j].im, src);
-            }
-          }
-          r.re += __shfl(r.re, src);
-          r.im += __shfl(r.im, src);
-        }
-      }
       bool sing;
-      const cx<double> d =
-          group_lu_solve<NMAX, GC, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.template piv<double>(), L.keys(), sing);
+      cx<double> d;
+      if constexpr (REP > 1) {
+        // each replica summed every R-th term of the row's sums
+        cx<double> V[NMAX + 1], B[(NMAX + REP) / REP];
+#pragma unroll
+        for (int j = 0; j < NMAX; ++j) V[j] = A[j];
+        V[NMAX] = r;
+        reduce_scatter<REP>(V, B, g, lane);
+        cx<double>& rb = B[NMAX / REP];
+        r = rb;  // (in replica NMAX % REP)
+        if (stg && g.s == NMAX % REP) rb = cmk<double>(-rb.re, -rb.im);
+        d = group_solve_split<NMAX, REP>(B, g, n, row, L.piv64(), L.keys(), cols, cols + REP * g.G, sing);
+      } else {
+        if constexpr (REP == 1) {
+          // more replicas than the split solve deals out: a butterfly over
+          // them (all sums of a level exchanged together) leaves the full
+          // sums, identical in every replica (each level adds a pair of
+          // partial sums, commutatively)
+          for (int m = 1; m < g.R; m <<= 1) {
+            const int src = (lane + ((g.s ^ m) - g.s) * g.G) & 63;
+#pragma unroll
+            for (int j = 0; j < NMAX; ++j) {
+              if (j < n) {
+                A[j].re += __shfl(A[j].re, src);
+                A[j].im += __shfl(A[j].im, src);
+              }
+            }
+            r.re += __shfl(r.re, src);
+            r.im += __shfl(r.im, src);
+          }
+        }
+        d = group_lu_solve<NMAX, GC, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.piv64(), L.keys(),
+                                             sing);
+      }
 
       // RK4 stage: k_s = solution, accumulate k1 + 2 k2 + 2 k3 + k4
       if (stg) {
@@ -1212,6 +1359,8 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       // residual max_i |H_i(x, 1)| of the refined root (r = H at x)
       const bool rz = pe == kPhResid;
       if (__any(rz)) {
+        // the replica that holds the right-hand side's column has the sums
+        if constexpr (REP > 1) r = lane_read(r, g.wbase + (NMAX % REP) * g.G + g.gl);
         double rr = (rz && row) ? sqrt(cnorm2(r)) : 0.0;
         if (rr != rr) rr = INFINITY;
         rr = group_max(rr, g);
@@ -1275,7 +1424,7 @@ void track_kernel(const Launch LN) {
   while (s + 1 < LN.nseg && (int)blockIdx.x >= LN.first_block[s + 1]) ++s;
   for (int tried = 0; tried < LN.nseg; ++tried) {
     if constexpr (MODE == 0) {
-      run_segment_fp64<NMAX, DEG, EXACT, false>(LN, s, smem, lane);
+      run_segment_fp64<NMAX, DEG, EXACT, 0>(LN, s, smem, lane);
     } else {
       run_segment<NMAX, DEG, MODE, EXACT>(LN, s, smem, lane);
     }
@@ -1284,14 +1433,13 @@ void track_kernel(const Launch LN) {
   }
 }
 
-// Latency instance: FP64 launches of one segment and few paths (one wave
-// per SIMD at most, so the register budget is a full SIMD's), with R >= 1
-// replicas per path.
-template <int NMAX, int DEG, bool EXACT>
+// Latency instance: FP64 launches of one segment and few paths, R replicas
+// per path (1: the launch's number).
+template <int NMAX, int DEG, bool EXACT, int R>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, false))))
 void track_kernel_rep(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
-  run_segment_fp64<NMAX, DEG, EXACT, true>(LN, 0, smem, (int)threadIdx.x & 63);
+  run_segment_fp64<NMAX, DEG, EXACT, R>(LN, 0, smem, (int)threadIdx.x & 63);
 }
 
 // One launch over segments of different sizes (uneven batches): segment s
@@ -1302,7 +1450,7 @@ void track_kernel_rep(const Launch LN) {
 template <int N, int DEG, int MODE>
 __device__ __forceinline__ void run_exact(const Launch& LN, int si, unsigned char* smem, int lane) {
   if constexpr (MODE == 0) {
-    run_segment_fp64<N, DEG, true, false, 2>(LN, si, smem, lane);
+    run_segment_fp64<N, DEG, true, 0, 2>(LN, si, smem, lane);
   } else {
     run_segment<N, DEG, MODE, true>(LN, si, smem, lane);
   }
@@ -1374,13 +1522,22 @@ KernelFn kernel_x16_m0(int deg);
 KernelFn kernel_x16_m1(int deg);
 KernelFn kernel_x30_m0(int deg);
 KernelFn kernel_x30_m1(int deg);
-// Latency instances (FP64, one segment, few paths): size-specialised for
-// n in {3, 4, 5, 6} and {8, 9, 10, 12, 16} (DEG 2 and 3), generic for NMAX 8,
-// 16 and 32 (DEG 2, 3 and 6).
-KernelFn kernel_rep_xs(int n, int deg);
-KernelFn kernel_rep_xl(int n, int deg);
-KernelFn kernel_rep_g8(int deg);
-KernelFn kernel_rep_g16(int deg);
-KernelFn kernel_rep_g32(int deg);
+// Latency instances (FP64, one segment, few paths) of R replicas per path:
+// size-specialised for n in {3, 4, 5, 6} and {8, 9, 10, 12, 16} (DEG 2 and 3,
+// n = 4, 5 also 4), generic for NMAX 8, 16 and 32 (DEG 2, 3 and 6); R = 8 up to
+// 8 lanes per replica, 4 up to 16, 2 up to 32.
+#define HCX_REP_UNITS(R) \
+  KernelFn kernel_rep_xs_r##R(int n, int deg); KernelFn kernel_rep_xl_r##R(int n, int deg); \
+  KernelFn kernel_rep_g8_r##R(int deg);
+HCX_REP_UNITS(1)
+HCX_REP_UNITS(2)
+HCX_REP_UNITS(4)
+HCX_REP_UNITS(8)
+#undef HCX_REP_UNITS
+KernelFn kernel_rep_g16_r1(int deg);
+KernelFn kernel_rep_g16_r2(int deg);
+KernelFn kernel_rep_g16_r4(int deg);
+KernelFn kernel_rep_g32_r1(int deg);
+KernelFn kernel_rep_g32_r2(int deg);
 
 }  // namespace hcx

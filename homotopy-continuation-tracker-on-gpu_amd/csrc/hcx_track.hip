@@ -314,19 +314,40 @@ static KernelFn pick_kernel(int nmax, int deg, int mode) {
   }
 }
 
-// The replica instance of a launch planned on `pl` (nullptr: none).
-static KernelFn pick_rep(int nmax, int deg, bool exact) {
+// The latency instance of R replicas (nullptr: none).  Numbers of replicas
+// that have no instance of their own run on R = 1's, which takes any.
+static KernelFn pick_rep(int nmax, int deg, bool exact, int R) {
   if (exact) {
     if (deg > 4) return nullptr;
     deg = deg < 2 ? 2 : deg;
-    if (nmax >= 3 && nmax <= 6) return kernel_rep_xs(nmax, deg);
-    if (nmax == 8 || nmax == 9 || nmax == 10 || nmax == 12 || nmax == 16) return kernel_rep_xl(nmax, deg);
+    if (nmax >= 3 && nmax <= 6) {
+      switch (R) {
+        case 2: return kernel_rep_xs_r2(nmax, deg);
+        case 4: return kernel_rep_xs_r4(nmax, deg);
+        case 8: return kernel_rep_xs_r8(nmax, deg);
+        default: return kernel_rep_xs_r1(nmax, deg);
+      }
+    }
+    if (nmax == 8 || nmax == 9 || nmax == 10 || nmax == 12 || nmax == 16) {
+      switch (R) {
+        case 2: return kernel_rep_xl_r2(nmax, deg);
+        case 4: return kernel_rep_xl_r4(nmax, deg);
+        case 8: return kernel_rep_xl_r8(nmax, deg);
+        default: return kernel_rep_xl_r1(nmax, deg);
+      }
+    }
     return nullptr;
   }
   switch (nmax) {
-    case 8: return kernel_rep_g8(deg);
-    case 16: return kernel_rep_g16(deg);
-    case 32: return kernel_rep_g32(deg);
+    case 8:
+      switch (R) {
+        case 2: return kernel_rep_g8_r2(deg);
+        case 4: return kernel_rep_g8_r4(deg);
+        case 8: return kernel_rep_g8_r8(deg);
+        default: return kernel_rep_g8_r1(deg);
+      }
+    case 16: return R == 4 ? kernel_rep_g16_r4(deg) : R == 2 ? kernel_rep_g16_r2(deg) : kernel_rep_g16_r1(deg);
+    case 32: return R == 2 ? kernel_rep_g32_r2(deg) : kernel_rep_g32_r1(deg);
     default: return nullptr;
   }
 }
@@ -498,7 +519,7 @@ struct Plan {
   int tab_lds = 0;   // LDS bytes of the compact tables (instances that hold them there)
   size_t lds = 0;
   KernelFn fn = nullptr;
-  bool keys() const { return !(exact && is_pow2(exact_lanes(nmax))); }  // pivot keys in LDS
+  bool keys() const { return latency || !(exact && is_pow2(exact_lanes(nmax))); }  // pivot keys in LDS
   int group_bytes(const hcx_problem* p, bool dot_lds = false) const {
     return lds_group_bytes(nmax, keys(), mode == 0 ? p->nslot : p->C + 1, p->M, dot_lds);
   }
@@ -1062,7 +1083,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     for (int c = 0; c <= C; c += 2) {
       // offsets from the group's region, whose coefficient area follows x and
       // the keys of the instance for n; 0: no slot
-      const int head = 16 * (n + 2) + dev::key_bytes(n, !is_pow2(exact_lanes(n)));
+      const int head = 16 * (n + 2) + dev::key_bytes(n, lat || !is_pow2(exact_lanes(n)));
       auto off = [&](int q) { return q > C || cslot[q] >= nslot ? 0u : (uint32_t)(head + cslot[q] * 16); };
       w.push_back(off(c) | off(c + 1) << 16);
     }
@@ -1425,9 +1446,8 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
              (R == 1 || heavy || waves(2 * R) <= 2LL * g_cu))
         R *= 2;
     }
-    // the latency instance (its register budget is a whole SIMD's), also
-    // for R = 1
-    const KernelFn rf = pick_rep(pl.nmax, pl.deg, pl.exact);
+    // the latency instance, also for R = 1
+    const KernelFn rf = pick_rep(pl.nmax, pl.deg, pl.exact, R);
     if (!rf) R = 1;
     const size_t regions = (size_t)(64 / (S.G * R)) * (size_t)lg;
     // the rule counts the compact tables of the size-specialised instances at 4
@@ -1438,7 +1458,10 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     size_t tab = 0, tab_new = terms;
     if (pl.exact && pl.tab_lds > 0) tab = (size_t)(pl.tab4 ? p->ctab4_bytes : p->ctab_bytes);
     if (compact) tab_new = (size_t)(rf ? lat.words * 4 : pl.tab_lds);
-    if (regions + tab + terms <= 65536 && regions + tab_new <= (size_t)kMaxLdsBytes) {
+    Plan lp = pl;
+    lp.latency = rf != nullptr;
+    const int region = ((lp.group_bytes(p, true) + dev::split_bytes(pl.nmax, S.G, R)) / 16 | 1) * 16;
+    if (regions + tab + terms <= 65536 && (size_t)(64 / (S.G * R)) * (size_t)region + tab_new <= (size_t)kMaxLdsBytes) {
       LN.dot_lds = 1;
       S.R = R;
       if (rf) {
@@ -1448,7 +1471,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
         seg_tables(S, p, pl);
         if (!compact) S.ctab = nullptr;
       }
-      S.lds_group = lg;
+      S.lds_group = rf ? region : lg;
       seg_groups[0] = waves(R);
       total_groups_needed = seg_groups[0];
     }
