@@ -38,19 +38,10 @@ template <class T>
 __device__ __forceinline__ cx<T> csub(cx<T> a, cx<T> b) {
   return cmk<T>(a.re - b.re, a.im - b.im);
 }
-template <class T>
-__device__ __forceinline__ cx<T> cmul(cx<T> a, cx<T> b) {
-  return cmk<T>(a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re);
-}
 // a - b*c
 template <class T>
 __device__ __forceinline__ cx<T> cfnms(cx<T> a, cx<T> b, cx<T> c) {
   return cmk<T>(a.re - b.re * c.re + b.im * c.im, a.im - b.re * c.im - b.im * c.re);
-}
-// a + b*c
-template <class T>
-__device__ __forceinline__ cx<T> cfma(cx<T> a, cx<T> b, cx<T> c) {
-  return cmk<T>(a.re + b.re * c.re - b.im * c.im, a.im + b.re * c.im + b.im * c.re);
 }
 template <class T>
 __device__ __forceinline__ cx<T> cscale(cx<T> a, T s) {
@@ -64,20 +55,6 @@ template <class T>
 __device__ __forceinline__ T cnorm2(cx<T> a) {
   return a.re * a.re + a.im * a.im;
 }
-// Complex division a/b by Smith's algorithm (R. L. Smith, CACM 5(8), 1962):
-// scales by the larger component of b to avoid overflow in |b|^2.
-template <class T>
-__device__ __forceinline__ cx<T> cdiv(cx<T> a, cx<T> b) {
-  if (fabs(b.re) >= fabs(b.im)) {
-    const T r = b.im / b.re;
-    const T inv = T(1) / (b.re + b.im * r);
-    return cmk<T>((a.re + a.im * r) * inv, (a.im - a.re * r) * inv);
-  } else {
-    const T r = b.re / b.im;
-    const T inv = T(1) / (b.re * r + b.im);
-    return cmk<T>((a.re * r + a.im) * inv, (a.im * r - a.re) * inv);
-  }
-}
 // Reciprocals from the hardware estimate: v_rcp_f32 (1 ulp) for FP32;
 // v_rcp_f64 refined by two Newton-Raphson steps r <- r + r (1 - x r) for FP64.
 __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -89,7 +66,9 @@ __device__ __forceinline__ double frcp(double x) {
 }
 // Complex reciprocal 1/b, without branches (the lanes of a wave hold pivots
 // of either kind, so a branch runs both of its sides).
-// Smith's scaling (as cdiv), the roles of the components selected.
+// By Smith's algorithm (R. L. Smith, CACM 5(8), 1962), which scales by the
+// larger component of b to avoid overflow in |b|^2, the roles of the components
+// selected.
 template <class T>
 __device__ __forceinline__ cx<T> crecip(cx<T> b) {
   const bool rbig = fabs(b.re) >= fabs(b.im);
@@ -221,24 +200,6 @@ struct __align__(16) Term {
 __device__ __forceinline__ int term_var(const Term& t, int q) {
   return q < 4 ? (int)((t.v03 >> (8 * q)) & 0xffu) : (int)((t.v47 >> (8 * (q - 4))) & 0xffu);
 }
-
-// Compact 8-byte form of a term for tables held in LDS: x = coefficient slot
-// (bits 0-15) | scalar (bits 16-31, two's complement); y = variable indices
-// 0..3, 8 bits each (terms of degree <= 4).
-__device__ __forceinline__ int cterm_c(uint2 t) { return (int)(t.x & 0xffffu); }
-__device__ __forceinline__ int cterm_s(uint2 t) { return (int)t.x >> 16; }
-__device__ __forceinline__ int cterm_var(uint2 t, int q) { return (int)((t.y >> (8 * q)) & 0xffu); }
-
-// Compact 4-byte form for tables of degree <= 2 (each term has at most two
-// variables): coefficient slot (bits 0-11) | scalar (bits 12-15, two's
-// complement, -8..7) | variable 0 (bits 16-23) | variable 1 (bits 24-31).
-__device__ __forceinline__ int cterm_c(uint32_t t) { return (int)(t & 0xfffu); }
-__device__ __forceinline__ int cterm_s(uint32_t t) { return (int)(t << 16) >> 28; }
-__device__ __forceinline__ int cterm_var(uint32_t t, int q) { return (int)((t >> (16 + 8 * q)) & 0xffu); }
-
-// The compact term record of a table of degree DEG.
-template <int DEG>
-using CTerm = typename std::conditional<(DEG <= 2), uint32_t, uint2>::type;
 
 }  // namespace dev
 }  // namespace hcx

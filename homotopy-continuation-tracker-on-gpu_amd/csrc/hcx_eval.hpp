@@ -1,4 +1,4 @@
-// Evaluation of the FP64 micro-step loop: term streams, coefficient staging.
+// Evaluation of the path loops: term streams, coefficient staging.
 //
 // A row's terms are a STREAM per lane: position p of equation i at
 // [p][i], all positions of Jacobian column 0, then of column 1, and so on
@@ -21,14 +21,27 @@
 namespace hcx {
 namespace dev {
 
-__device__ __forceinline__ cx<double> lds_at(const unsigned char* base, uint32_t off) {
-  return *reinterpret_cast<const cx<double>*>(base + off);
+// The records' byte offsets count 16-byte slots (FP64); FP32 data, in slots of
+// 8 bytes, lies at half of them, a shift that the field extraction includes.
+template <class T>
+constexpr int kHalf = sizeof(T) == 8 ? 0 : 1;
+// The value at the low 16 bits (lo) or at bits 16-25 (hi) of a record word.
+template <class T>
+__device__ __forceinline__ cx<T> lds_lo(const unsigned char* base, uint32_t r) {
+  return *reinterpret_cast<const cx<T>*>(base + ((r >> kHalf<T>) & (0xffffu >> kHalf<T>)));
+}
+template <class T>
+__device__ __forceinline__ cx<T> lds_hi(const unsigned char* base, uint32_t r) {
+  return *reinterpret_cast<const cx<T>*>(base + ((r >> (16 + kHalf<T>)) & (0x3ffu >> kHalf<T>)));
 }
 
 // a * b with the roundings spelled out (they do not depend on what the
 // compiler fuses): the products with b.im rounded, those with b.re fused.
 __device__ __forceinline__ cx<double> cmul_term(cx<double> a, cx<double> b) {
   return cmk<double>(__builtin_fma(a.re, b.re, -(a.im * b.im)), __builtin_fma(a.im, b.re, a.re * b.im));
+}
+__device__ __forceinline__ cx<float> cmul_term(cx<float> a, cx<float> b) {
+  return cmk<float>(__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im));
 }
 
 // Compact records of the size-specialised instances, in LDS: byte offsets of
@@ -55,12 +68,12 @@ __device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
 // of each, the zero term past a column's last (SC: a scaled position).  All
 // records are requested together, then all gathers.  off: byte offset of the
 // first column's positions from rp; zero: that of the zero terms.
-template <int NMAX, int DEG, bool SC, int JB, int NB>
+template <int NMAX, int DEG, bool SC, int JB, int NB, class T>
 __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int off, int zero, const int (&cnt)[NB],
-                                          int k, const unsigned char* xb, const unsigned char* cb, cx<double> (&A)[NMAX]) {
+                                          int k, const unsigned char* xb, const unsigned char* cb, cx<T> (&A)[NMAX]) {
   constexpr int RS = StreamRec<DEG>::kJ;
   uint32_t r0[NB], r1[NB];
-  cx<double> c[NB], p[NB];
+  cx<T> c[NB], p[NB];
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
@@ -79,18 +92,18 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int of
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
-      c[u] = lds_at(cb, r0[u] & 0xffffu);
-      p[u] = lds_at(xb, (r0[u] >> 16) & 0x3ffu);
+      c[u] = lds_lo<T>(cb, r0[u]);
+      p[u] = lds_hi<T>(xb, r0[u]);
     }
   }
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
-      cx<double> v = c[u];
-      if constexpr (SC) v = cscale(v, rec_scalar<DEG>(r0[u], r1[u]));
+      cx<T> v = c[u];
+      if constexpr (SC) v = cscale(v, (T)rec_scalar<DEG>(r0[u], r1[u]));
       v = cmul_term(v, p[u]);
-      if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, r1[u] & 0xffffu));
-      if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, (r1[u] >> 16) & 0x3ffu));
+      if constexpr (DEG > 2) v = cmul_term(v, lds_lo<T>(xb, r1[u]));
+      if constexpr (DEG > 3) v = cmul_term(v, lds_hi<T>(xb, r1[u]));
       A[JB + u] = cadd(A[JB + u], v);
     }
   }
@@ -100,10 +113,10 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int of
 // (dev-eval-indxing-generalized_3views_4pts.cuh:70-86), NB columns at a time:
 // one column after the other, each term is two exposed LDS latencies and each
 // column two loops.
-template <int NMAX, int DEG, int NB, int JB, class SegT>
+template <int NMAX, int DEG, int NB, int JB, class T, class SegT>
 __device__ __forceinline__ void eval_jac_blocks(const SegT& S, int n, const unsigned char* rp, int off,
                                                 const unsigned char* xb, const unsigned char* cb,
-                                                cx<double> (&A)[NMAX]) {
+                                                cx<T> (&A)[NMAX]) {
   if constexpr (JB < NMAX) {
     int cnt[NB], end = 0, scaled = 0, tot = 0;
 #pragma unroll
@@ -115,16 +128,16 @@ __device__ __forceinline__ void eval_jac_blocks(const SegT& S, int n, const unsi
         end = max(end, cnt[u]);
         scaled = max(scaled, (int)(cc >> 16));
         tot += cnt[u];
-        A[JB + u] = cmk<double>(0, 0);
+        A[JB + u] = cmk<T>(0, 0);
       }
     }
     const int zero = S.hx_recs * StreamRec<DEG>::kJ;
     int k = 0;
 #pragma unroll 1
-    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB>(rp, n, off, zero, cnt, k, xb, cb, A);
+    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB, T>(rp, n, off, zero, cnt, k, xb, cb, A);
 #pragma unroll 1
-    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB>(rp, n, off, zero, cnt, k, xb, cb, A);
-    eval_jac_blocks<NMAX, DEG, NB, JB + NB>(S, n, rp, off + tot * (n * StreamRec<DEG>::kJ), xb, cb, A);
+    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB, T>(rp, n, off, zero, cnt, k, xb, cb, A);
+    eval_jac_blocks<NMAX, DEG, NB, JB + NB, T>(S, n, rp, off + tot * (n * StreamRec<DEG>::kJ), xb, cb, A);
   }
 }
 
@@ -181,8 +194,8 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
-          c[u] = lds_at(cb, r0[u] & 0xffffu);
-          p[u] = lds_at(xb, r0[u] >> 16);
+          c[u] = lds_lo<double>(cb, r0[u]);
+          p[u] = lds_hi<double>(xb, r0[u]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
@@ -191,8 +204,8 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
         if (jb + u < NMAX) {
           cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
           v = cmul_term(v, p[u]);
-          if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, r1[u] & 0xffffu));
-          if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, r1[u] >> 16));
+          if constexpr (DEG > 2) v = cmul_term(v, lds_lo<double>(xb, r1[u]));
+          if constexpr (DEG > 3) v = cmul_term(v, lds_hi<double>(xb, r1[u]));
           A[jb + u] = cadd(A[jb + u], v);
         }
       }
@@ -205,13 +218,13 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
 // this lane's group sums dc/dt (an RK4 stage) instead of c(t): from its LDS
 // area at db, or (GDOT) from global memory, requested for the whole chunk
 // before the first product.
-template <int DEG, bool SC, bool GDOT, int Q, bool PIN>
-__device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int n, int k, int ks, int cnt,
+template <int DEG, bool SC, bool GDOT, int Q, bool PIN, class T>
+__device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k, int ks, int cnt,
                                                 const unsigned char* xb, const unsigned char* cb,
-                                                const double2* dg, bool dot, cx<double> acc) {
+                                                const double2* dg, bool dot, cx<T> acc) {
   constexpr int RS = StreamRec<DEG>::kH;
   uint32_t r[Q][3];
-  cx<double> c[Q];
+  cx<T> c[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     const unsigned char* a = rp + min(k + q * ks, cnt) * (n * RS);
@@ -226,19 +239,19 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int n, 
       r[q][2] = v.z;
     }
   }
-  cx<double> x0[Q], x1[Q];
+  cx<T> x0[Q], x1[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    c[q] = lds_at(cb, r[q][0] & 0xffffu);
-    x0[q] = lds_at(xb, (r[q][0] >> 16) & 0x3ffu);
-    x1[q] = lds_at(xb, r[q][1] & 0xffffu);
+    c[q] = lds_lo<T>(cb, r[q][0]);
+    x0[q] = lds_hi<T>(xb, r[q][0]);
+    x1[q] = lds_lo<T>(xb, r[q][1]);
   }
   if constexpr (GDOT) {
     if (dot) {
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
         const double2 d = dg[r[q][DEG <= 2 ? 1 : 2] >> 16];
-        c[q] = cmk<double>(d.x, d.y);
+        c[q] = cmk<T>((T)d.x, (T)d.y);
       }
     }
   }
@@ -247,12 +260,12 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int n, 
   if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    cx<double> v = c[q];
-    if constexpr (SC) v = cscale(v, rec_scalar<DEG>(r[q][0], r[q][1]));
+    cx<T> v = c[q];
+    if constexpr (SC) v = cscale(v, (T)rec_scalar<DEG>(r[q][0], r[q][1]));
     v = cmul_term(v, x0[q]);
     v = cmul_term(v, x1[q]);
-    if constexpr (DEG > 2) v = cmul_term(v, lds_at(xb, (r[q][1] >> 16) & 0x3ffu));
-    if constexpr (DEG > 3) v = cmul_term(v, lds_at(xb, r[q][2] & 0xffffu));
+    if constexpr (DEG > 2) v = cmul_term(v, lds_hi<T>(xb, r[q][1]));
+    if constexpr (DEG > 3) v = cmul_term(v, lds_lo<T>(xb, r[q][2]));
     acc = cadd(acc, v);
   }
   return acc;
@@ -260,20 +273,20 @@ __device__ __forceinline__ cx<double> rhs_chunk(const unsigned char* rp, int n, 
 
 // Row gl of sum_k s * coef * prod x over the dH/dt streams (…cuh:89-120):
 // H with c(t), dH/dt with dc/dt.
-template <int DEG, bool GDOT, int Q, bool PIN, class SegT>
-__device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int n, int gle, const unsigned char* xb,
+template <int DEG, bool GDOT, int Q, bool PIN, class T, class SegT>
+__device__ __forceinline__ cx<T> eval_rhs_stream(const SegT& S, int n, int gle, const unsigned char* xb,
                                                       const unsigned char* cb, const unsigned char* db,
                                                       const double2* dg, bool dot, const unsigned char* lt, int k0,
                                                       int ks) {
   const unsigned char* base = (!GDOT && dot) ? db : cb;
   const unsigned char* rp = lt + S.tab_h + gle * StreamRec<DEG>::kH;
   const int cnt = S.htT;
-  cx<double> acc = cmk<double>(0, 0);
+  cx<T> acc = cmk<T>(0, 0);
   int k = 0;
 #pragma unroll 1
-  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<DEG, true, GDOT, Q, PIN>(rp, n, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  for (; k < S.htS; k += Q * ks) acc = rhs_chunk<DEG, true, GDOT, Q, PIN, T>(rp, n, k + k0, ks, cnt, xb, base, dg, dot, acc);
 #pragma unroll 1
-  for (; k < cnt; k += Q * ks) acc = rhs_chunk<DEG, false, GDOT, Q, PIN>(rp, n, k + k0, ks, cnt, xb, base, dg, dot, acc);
+  for (; k < cnt; k += Q * ks) acc = rhs_chunk<DEG, false, GDOT, Q, PIN, T>(rp, n, k + k0, ks, cnt, xb, base, dg, dot, acc);
   return acc;
 }
 
@@ -281,15 +294,15 @@ __device__ __forceinline__ cx<double> eval_rhs_stream(const SegT& S, int n, int 
 // (n apart from tp; global memory or an LDS copy).  The records of a chunk
 // are requested before the first is used.  GDOT: lanes with dot take dc/dt
 // from global memory (dg, indexed by the coefficient numbers ci).
-template <int NV, bool GDOT>
-__device__ __forceinline__ cx<double> term_stream_sum(const Term* tp, int cnt, int n, const cx<double>* sx,
-                                                      const cx<double>* coef, const double2* dg, const int* ci,
+template <int NV, bool GDOT, class T>
+__device__ __forceinline__ cx<T> term_stream_sum(const Term* tp, int cnt, int n, const cx<T>* sx,
+                                                      const cx<T>* coef, const double2* dg, const int* ci,
                                                       bool dot, int k0, int ks) {
-  cx<double> acc = cmk<double>(0, 0);
+  cx<T> acc = cmk<T>(0, 0);
   for (int kb = k0; kb < cnt; kb += kTermChunk * ks) {
     Term tm[kTermChunk];
     int cj[kTermChunk];
-    cx<double> c[kTermChunk];
+    cx<T> c[kTermChunk];
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q)
       if (kb + q * ks < cnt) {
@@ -303,14 +316,14 @@ __device__ __forceinline__ cx<double> term_stream_sum(const Term* tp, int cnt, i
         if constexpr (GDOT) {
           if (dot) {
             const double2 d = dg[cj[q]];
-            c[q] = cmk<double>(d.x, d.y);
+            c[q] = cmk<T>((T)d.x, (T)d.y);
           }
         }
       }
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q) {
       if (kb + q * ks < cnt) {
-        cx<double> v = cscale(c[q], (double)tm[q].s);
+        cx<T> v = cscale(c[q], (T)tm[q].s);
 #pragma unroll
         for (int d = 0; d < NV; ++d) v = cmul_term(v, sx[term_var(tm[q], d)]);
         acc = cadd(acc, v);
@@ -322,14 +335,14 @@ __device__ __forceinline__ cx<double> term_stream_sum(const Term* tp, int cnt, i
 
 // Row gl of dH/dx from the full records: those of the LDS copy at tl, or in
 // global memory (tl null).
-template <int NMAX, int DEG, class SegT>
-__device__ __forceinline__ void eval_jac_terms(const SegT& S, int n, int gle, const cx<double>* sx,
-                                               const cx<double>* sc, cx<double> (&A)[NMAX], const Term* tl, int k0,
+template <int NMAX, int DEG, class T, class SegT>
+__device__ __forceinline__ void eval_jac_terms(const SegT& S, int n, int gle, const cx<T>* sx,
+                                               const cx<T>* sc, cx<T> (&A)[NMAX], const Term* tl, int k0,
                                                int ks) {
   size_t off = gle;
 #pragma unroll
   for (int j = 0; j < NMAX; ++j) {
-    cx<double> acc = cmk<double>(0, 0);
+    cx<T> acc = cmk<T>(0, 0);
     if (j < n) {
       int cnt;
       if (S.hx_cnt) {
@@ -338,9 +351,9 @@ __device__ __forceinline__ void eval_jac_terms(const SegT& S, int n, int gle, co
         cnt = (int)(S.colc[j] & 0xffffu);
       }
       if (tl)
-        acc = term_stream_sum<DEG - 1, false>(tl + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
+        acc = term_stream_sum<DEG - 1, false, T>(tl + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
       else
-        acc = term_stream_sum<DEG - 1, false>(S.hx + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
+        acc = term_stream_sum<DEG - 1, false, T>(S.hx + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
       off += (size_t)cnt * n;
     }
     A[j] = acc;
@@ -348,13 +361,13 @@ __device__ __forceinline__ void eval_jac_terms(const SegT& S, int n, int gle, co
 }
 
 // Row gl of dH/dt or H from the full records (base: c(t) or dc/dt in LDS).
-template <int DEG, bool GDOT, class SegT>
-__device__ __forceinline__ cx<double> eval_rhs_terms(const SegT& S, int n, int gle, const cx<double>* sx,
-                                                     const cx<double>* base, const double2* dg, bool dot,
+template <int DEG, bool GDOT, class T, class SegT>
+__device__ __forceinline__ cx<T> eval_rhs_terms(const SegT& S, int n, int gle, const cx<T>* sx,
+                                                     const cx<T>* base, const double2* dg, bool dot,
                                                      const Term* tl, int k0, int ks) {
   const int* ci = S.ht_ci + gle;
-  if (tl) return term_stream_sum<DEG, GDOT>(tl + (size_t)S.hx_recs + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
-  return term_stream_sum<DEG, GDOT>(S.ht + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
+  if (tl) return term_stream_sum<DEG, GDOT, T>(tl + (size_t)S.hx_recs + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
+  return term_stream_sum<DEG, GDOT, T>(S.ht + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
 }
 
 // ------------------------------------------------------------ staging
@@ -376,9 +389,9 @@ __device__ __forceinline__ uint32_t slot_offset(const SegT& S, const unsigned ch
 // the lane's coefficients at a time: all of a chunk's loads are requested
 // before the first is used, so the staging costs one memory latency per Q
 // coefficients; full chunks address with constant offsets, the last
-// coefficients go one by one.  hx, ht: the instance's tables; xb: the group's
-// region, db: from a slot of c to that of dc/dt.
-template <int MC, int Q, bool SL, class SegT>
+// coefficients go as one chunk.  hx, ht: the instance's tables; xb: where the
+// offsets of T's slots count from, db: from a slot of c to that of dc/dt.
+template <int MC, int Q, bool SL, class T, class SegT>
 __device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, const double2* hx, const double2* ht,
                                              double t, unsigned char* xb, int head, int db, bool dot,
                                              const unsigned char* lt) {
@@ -390,7 +403,7 @@ __device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, cons
       cr = cr * t + a[m].x;
       ci = ci * t + a[m].y;
     }
-    *reinterpret_cast<cx<double>*>(xb + o) = cmk<double>(cr, ci);
+    *reinterpret_cast<cx<T>*>(xb + (o >> kHalf<T>)) = cmk<T>((T)cr, (T)ci);
   };
   auto put_dot = [&](const double2* b, uint32_t o) {
     double dr = b[MC - 1].x, di = b[MC - 1].y;
@@ -399,7 +412,7 @@ __device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, cons
       dr = dr * t + b[m].x;
       di = di * t + b[m].y;
     }
-    if (o) *reinterpret_cast<cx<double>*>(xb + db + o) = cmk<double>(dr, di);
+    if (o) *reinterpret_cast<cx<T>*>(xb + db + (o >> kHalf<T>)) = cmk<T>((T)dr, (T)di);
   };
   int j = g.gl + g.s * g.G;
   const double2* ha = hx + (size_t)j * (MC + 1);
@@ -462,17 +475,20 @@ __device__ __forceinline__ void stage_chunks(const SegT& S, const Group& g, cons
 // together hit consecutive LDS words instead of words one equation apart.  The
 // replicas of a group share its LDS region and stage every R-th coefficient
 // each.  Q: coefficients in flight per lane at order 1 (fewer at higher
-// orders, by their registers).
-template <bool SL, int Q, class SegT>
-__device__ __forceinline__ void stage_coeffs64(const SegT& S, const Group& g, const double2* hx, const double2* ht,
+// orders, by their registers).  Computed in FP64 and stored as T: at FP64 the
+// offsets count from the group's region, at FP32 (half of them) from the middle of
+// what precedes the coefficient area, so that the area begins at the same place
+// and an unused coefficient goes to x's slots past those that FP32 uses.
+template <bool SL, int Q, class T, class SegT>
+__device__ __forceinline__ void stage_coeffs(const SegT& S, const Group& g, const double2* hx, const double2* ht,
                                                double t, unsigned char* xb, int head, int db, bool dot,
                                                const unsigned char* lt) {
   constexpr int Q2 = Q > 2 ? Q / 2 : 1, Q3 = Q > 3 ? Q / 3 : 1;
   switch (S.M) {
-    case 1: return stage_chunks<1, Q, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
-    case 2: return stage_chunks<2, Q2, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
-    case 3: return stage_chunks<3, Q3, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
-    case 4: return stage_chunks<4, Q3, SL>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 1: return stage_chunks<1, Q, SL, T>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 2: return stage_chunks<2, Q2, SL, T>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 3: return stage_chunks<3, Q3, SL, T>(S, g, hx, ht, t, xb, head, db, dot, lt);
+    case 4: return stage_chunks<4, Q3, SL, T>(S, g, hx, ht, t, xb, head, db, dot, lt);
     default: break;
   }
   const int C1 = S.C + 1, M = S.M;
@@ -484,7 +500,7 @@ __device__ __forceinline__ void stage_coeffs64(const SegT& S, const Group& g, co
       cr = cr * t + ha[m].x;
       ci = ci * t + ha[m].y;
     }
-    *reinterpret_cast<cx<double>*>(xb + o) = cmk<double>(cr, ci);
+    *reinterpret_cast<cx<T>*>(xb + (o >> kHalf<T>)) = cmk<T>((T)cr, (T)ci);
     if (dot && o) {
       const double2* hb = ht + (size_t)j * M;
       double dr = hb[M - 1].x, di = hb[M - 1].y;
@@ -492,17 +508,18 @@ __device__ __forceinline__ void stage_coeffs64(const SegT& S, const Group& g, co
         dr = dr * t + hb[m].x;
         di = di * t + hb[m].y;
       }
-      *reinterpret_cast<cx<double>*>(xb + db + o) = cmk<double>(dr, di);
+      *reinterpret_cast<cx<T>*>(xb + db + (o >> kHalf<T>)) = cmk<T>((T)dr, (T)di);
     }
   }
 }
 
 // x and the constants 1 and 0 (variable indices n and n + 1).
-__device__ __forceinline__ void publish_x64(cx<double>* sx, cx<double> x, const Group& g, int n, bool act, bool row) {
-  if (act && row) sx[g.gl] = x;
+template <class T>
+__device__ __forceinline__ void publish_x(cx<T>* sx, cx<double> x, const Group& g, int n, bool act, bool row) {
+  if (act && row) sx[g.gl] = ccast<T>(x);
   if (act && g.gl == 0) {
-    sx[n] = cmk<double>(1.0, 0.0);
-    sx[n + 1] = cmk<double>(0.0, 0.0);
+    sx[n] = cmk<T>(T(1), T(0));
+    sx[n + 1] = cmk<T>(T(0), T(0));
   }
 }
 

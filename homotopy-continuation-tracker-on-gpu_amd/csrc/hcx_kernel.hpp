@@ -21,12 +21,6 @@ constexpr int kMaxN = 32;
 #define HCX_TERM_CHUNK 4
 #endif
 constexpr int kTermChunk = HCX_TERM_CHUNK;
-// terms of an LDS-table row per unrolled loop iteration: two in FP64 (the
-// loads in flight then fit a budget of 168 VGPRs, three waves per SIMD),
-// four in FP32
-template <class T>
-constexpr int kTermUnroll = sizeof(T) == 8 ? 2 : 4;
-
 // Lanes per path of the size-specialised instance for n: n, except n = 30,
 // which runs on aligned 32-lane groups (still two paths per wave) so that
 // its group reductions can use DPP row permutations.
@@ -67,23 +61,23 @@ struct LaunchWork {
 // Hot, wave-uniform description of one segment (kernel arguments).
 struct Seg {
   int n, C, M, K;
-  int hxT, htT;
+  int htT;
   int G;
   int R;                       // replicas per path (lanes per path = G * R; FP64 loop)
   int lds_group;               // bytes of one group's LDS region
   int start_stride;
   int I;
   long long P;
-  const dev::Term* hx;         // mixed: [n var][hxT][n eq]; FP64: streams (hcx_eval64.hpp)
-  const dev::Term* ht;         // [htT][n eq]
-  // terms per Jacobian column (max over equations); FP64 loop: positions of the
-  // column's stream | scaled ones << 16, and where a number does not fit,
-  // hx_cnt (device memory) holds the positions instead (else nullptr)
+  const dev::Term* hx;         // term streams (hcx_eval.hpp), full records
+  const dev::Term* ht;
+  // per Jacobian column: positions of its stream | scaled ones << 16; where a
+  // number does not fit, hx_cnt (device memory) holds the positions instead
+  // (else nullptr)
   unsigned int colc[kMaxN];
   const int* hx_cnt;
-  const int* ht_ci;            // FP64 loop: coefficient numbers of the ht records
-  // FP64 loop: scaled positions of ht (htT: all); Term
-  // records of hx; coefficients with an LDS slot
+  const int* ht_ci;            // coefficient numbers of the ht records
+  // scaled positions of ht (htT: all); records of hx; coefficients with an
+  // LDS slot
   int htS, hx_recs, nslot;
   int max_terms;               // positions of the longest column
   int tab_words;               // 4-byte words of the compact tables
@@ -92,8 +86,7 @@ struct Seg {
   const double2* chx;          // [I][C+1][M+1]
   const double2* cht;          // [I][C+1][M]
   const int* cslot;            // [C+1] LDS slot of coefficient j (the tables hold slots)
-  const uint32_t* ctab;        // compact tables (LDS-table instances): mixed: hx then ht, 4-byte
-                               // terms for DEG <= 2, else 8-byte; FP64: streams
+  const uint32_t* ctab;        // compact tables (instances that hold the streams in LDS)
   unsigned int* counter;
   const SegOut* out;           // device copy written by init_kernel
   const int* plist;            // optional: track only these paths (count in *plist_count)
@@ -128,7 +121,7 @@ typedef const __attribute__((address_space(4))) Seg KSeg;
 
 }  // namespace hcx
 
-#include "hcx_eval64.hpp"
+#include "hcx_eval.hpp"
 
 namespace hcx {
 namespace dev {
@@ -155,144 +148,6 @@ template <class T>
 __device__ __forceinline__ T* iteration_view(T* p, int iter) {
   asm("" : "+s"(p) : "s"(iter));
   return p;
-}
-
-// ------------------------------------------------------------ evaluation
-// sum_k s_k * coef[c_k] * prod_{d < NV} x[var_kd] over the cnt terms of one
-// table row (full Term records n apart from tp in global memory).  The
-// records of a chunk of terms are all requested before the first is used, so
-// their latencies overlap.
-template <int NV, class T>
-__device__ __forceinline__ cx<T> term_row_sum(const Term* tp, int cnt, int n, const cx<T>* sx, const cx<T>* coef) {
-  cx<T> acc = cmk<T>(0, 0);
-  for (int kb = 0; kb < cnt; kb += kTermChunk) {
-    Term tm[kTermChunk];
-#pragma unroll
-    for (int q = 0; q < kTermChunk; ++q)
-      if (kb + q < cnt) tm[q] = tp[(size_t)(kb + q) * n];
-#pragma unroll
-    for (int q = 0; q < kTermChunk; ++q) {
-      if (kb + q < cnt) {
-        cx<T> v = cscale(coef[tm[q].c], (T)tm[q].s);
-#pragma unroll
-        for (int d = 0; d < NV; ++d) v = cmul(v, sx[term_var(tm[q], d)]);
-        acc = cadd(acc, v);
-      }
-    }
-  }
-  return acc;
-}
-
-// Evaluation of the mixed loop: row gl of dH/dx
-// (dev-eval-indxing-generalized_3views_4pts.cuh:70-86).
-// LT: the tables are the compact copy in LDS at lt (hx part first); else
-// full Term records in global memory.
-template <int NMAX, int DEG, class T, bool LT, class SegT>
-__device__ __forceinline__ void eval_jac_row(const SegT& S, int n, int gle, const cx<T>* sx, const cx<T>* sc,
-                                             cx<T> (&A)[NMAX], const void* lt) {
-#pragma unroll
-  for (int j = 0; j < NMAX; ++j) {
-    cx<T> acc = cmk<T>(0, 0);
-    if (j < n) {
-      // the counts travel in the kernel arguments: read from device memory,
-      // each was a vector load and a full memory latency at the head of its
-      // column's loop
-      const int cnt = (int)S.colc[j];
-      if constexpr (LT) {
-        const CTerm<DEG>* tp = static_cast<const CTerm<DEG>*>(lt) + (size_t)j * S.hxT * n + gle;
-#pragma unroll kTermUnroll<T>
-        for (int k = 0; k < cnt; ++k) {
-          const CTerm<DEG> tm = tp[(size_t)k * n];
-          cx<T> v = cscale(sc[cterm_c(tm)], (T)cterm_s(tm));
-#pragma unroll
-          for (int q = 0; q < DEG - 1; ++q) v = cmul(v, sx[cterm_var(tm, q)]);
-          acc = cadd(acc, v);
-        }
-      } else {
-        acc = term_row_sum<DEG - 1, T>(S.hx + (size_t)j * S.hxT * n + gle, cnt, n, sx, sc);
-      }
-    }
-    A[j] = acc;
-  }
-}
-
-// Row gl of sum_k s * coef[c] * prod x over the dHdt table: H when coef = c(t),
-// dH/dt when coef = dc/dt (…cuh:89-120).
-template <int DEG, class T, bool LT, class SegT>
-__device__ __forceinline__ cx<T> eval_t_row(const SegT& S, int n, int gle, const cx<T>* sx, const cx<T>* coef,
-                                            const void* lt) {
-  if constexpr (LT) {
-    cx<T> acc = cmk<T>(0, 0);
-    const CTerm<DEG>* tp = static_cast<const CTerm<DEG>*>(lt) + (size_t)n * S.hxT * n + gle;
-#pragma unroll kTermUnroll<T>
-    for (int k = 0; k < S.htT; ++k) {
-      const CTerm<DEG> tm = tp[(size_t)k * n];
-      cx<T> v = cscale(coef[cterm_c(tm)], (T)cterm_s(tm));
-#pragma unroll
-      for (int q = 0; q < DEG; ++q) v = cmul(v, sx[cterm_var(tm, q)]);
-      acc = cadd(acc, v);
-    }
-    return acc;
-  } else {
-    return term_row_sum<DEG, T>(S.ht + gle, S.htT, n, sx, coef);
-  }
-}
-
-// Staging of the mixed loop: coefficient polynomials in t of the group's
-// instance into LDS (eval_parameter_homotopy, …cuh:34-67), computed in FP64
-// and stored as T, coefficient j in slot cslot[j].
-template <class T, class SegT>
-__device__ __forceinline__ void stage_coeffs(const SegT& S, const Group& g, bool act, int inst, double t,
-                                             unsigned char* scb, bool with_dot) {
-  if (!act) return;
-  cx<T>* sc = reinterpret_cast<cx<T>*>(scb);
-  cx<T>* sd = sc + (S.C + 1);
-  const int C1 = S.C + 1, M = S.M;
-  const double2* hx = S.chx + (size_t)inst * C1 * (M + 1);
-  const double2* ht = S.cht + (size_t)inst * C1 * M;
-  if (M == 1) {
-    // c(t) = c0 + t c1, dc/dt = Ht[j][0]
-#pragma unroll kTermUnroll<T>
-    for (int j = g.gl; j < C1; j += g.G) {
-      const int q = S.cslot[j];
-      const double2 a = hx[2 * (size_t)j], b = hx[2 * (size_t)j + 1];
-      sc[q] = cmk<T>((T)(a.x + t * b.x), (T)(a.y + t * b.y));
-      if (with_dot) {
-        const double2 d = ht[j];
-        sd[q] = cmk<T>((T)d.x, (T)d.y);
-      }
-    }
-    return;
-  }
-  for (int j = g.gl; j < C1; j += g.G) {
-    double2 a = hx[(size_t)j * (M + 1) + M];
-    double cr = a.x, ci = a.y;
-    for (int m = M - 1; m >= 0; --m) {
-      const double2 b = hx[(size_t)j * (M + 1) + m];
-      const double nr = cr * t + b.x, ni = ci * t + b.y;
-      cr = nr;
-      ci = ni;
-    }
-    const int q = S.cslot[j];
-    sc[q] = cmk<T>((T)cr, (T)ci);
-    if (with_dot) {
-      double2 d = ht[(size_t)j * M + M - 1];
-      double dr = d.x, di = d.y;
-      for (int m = M - 2; m >= 0; --m) {
-        const double2 b = ht[(size_t)j * M + m];
-        const double nr = dr * t + b.x, ni = di * t + b.y;
-        dr = nr;
-        di = ni;
-      }
-      sd[q] = cmk<T>((T)dr, (T)di);
-    }
-  }
-}
-
-template <class T>
-__device__ __forceinline__ void publish_x(cx<T>* sx, cx<double> x, const Group& g, int n, bool act, bool row) {
-  if (act && row) sx[g.gl] = ccast<T>(x);
-  if (act && g.gl == 0) sx[n] = cmk<T>(T(1), T(0));
 }
 
 template <class T>
@@ -349,29 +204,43 @@ __device__ __forceinline__ unsigned long long group_max_key(unsigned long long k
 // Sums over the group's rows of two per-row values (the corrector's and the
 // refinement's |d|^2 and |x|^2), returned to every lane of the group.  Aligned
 // power-of-two groups use lane exchanges; other group sizes publish the
-// pairs in the group's LDS slots `q` and every lane adds them in row order
-// (one LDS round trip).
-template <int NMAX, int GC>
+// pairs in the group's LDS slots `q` and every lane adds them, in row order
+// (TREE: in pairs, pairs of pairs, ..., the order of the lane exchanges), for
+// one LDS round trip where the exchanges are ten.
+template <int NMAX, int GC, bool TREE>
 __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g, int n, bool row, int lane,
                                            cx<double>* q) {
-  if constexpr (GC > 0) {
+  if constexpr (GC > 0 || (TREE && NMAX > 16)) {
     a = group_sum(a, g, lane);
     b = group_sum(b, g, lane);
   } else {
     if (row) q[g.gl] = cmk<double>(a, b);
     HCX_WAVE_SYNC();
-    double sa = 0.0, sb = 0.0;
+    if constexpr (TREE) {
+      cx<double> v[NMAX];
 #pragma unroll
-    for (int j = 0; j < NMAX; ++j) {
-      if (j < n) {
-        const cx<double> v = q[j];
-        sa += v.re;
-        sb += v.im;
+      for (int j = 0; j < NMAX; ++j) v[j] = j < n ? q[j] : cmk<double>(0, 0);
+#pragma unroll
+      for (int w = 1; w < NMAX; w <<= 1)
+#pragma unroll
+        for (int j = 0; j + w < NMAX; j += 2 * w) v[j] = cadd(v[j], v[j + w]);
+      HCX_WAVE_SYNC();
+      a = v[0].re;
+      b = v[0].im;
+    } else {
+      double sa = 0.0, sb = 0.0;
+#pragma unroll
+      for (int j = 0; j < NMAX; ++j) {
+        if (j < n) {
+          const cx<double> v = q[j];
+          sa += v.re;
+          sb += v.im;
+        }
       }
+      HCX_WAVE_SYNC();
+      a = sa;
+      b = sb;
     }
-    HCX_WAVE_SYNC();
-    a = sa;
-    b = sb;
   }
 }
 
@@ -683,38 +552,32 @@ struct Lds {
   __device__ cx<T>* piv() const { return reinterpret_cast<cx<T>*>(piv64()); }
 };
 
-// Newton corrector at fixed t in precision T (…4pts.cu:189-223).  The
-// coefficients c(t) must already be in the group's LDS.  `run` enters as the
-// set of groups to correct; ok / inf return the reference's r_isSuccessful /
-// r_isInfFail.
-template <int NMAX, int GC, int DEG, class T, bool LT, class OT, class SegT>
-__device__ __forceinline__ void newton_pass(const SegT& S, int n, const OT& o, const Group& g, const Lds<NMAX, GC == 0>& L,
-                                            const void* lt, bool run, bool row, cx<double>& x, int& nnewt, bool& ok,
-                                            bool& inf) {
-  ok = false;
-  inf = false;
-  const int gle = row ? g.gl : 0;
-  cx<T>* sx = L.template x<T>();
-  const cx<T>* sc = reinterpret_cast<const cx<T>*>(L.coef());
-  for (int it = 0; it < o.max_corr; ++it) {
-    if (!__any(run)) break;
-    publish_x<T>(sx, x, g, n, run, row);
-    HCX_WAVE_SYNC();
-    cx<T> A[NMAX];
-    eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
-    const cx<T> h = eval_t_row<DEG, T, LT>(S, n, gle, sx, sc, lt);
-    bool sing;
-    const cx<T> d = group_lu_solve<NMAX, GC, T>(A, h, g, n, row, L.template piv<T>(), L.keys(), sing);
-    if (run && row) x = csub(x, ccast<double>(d));
-    double rs = row ? (double)cnorm2(d) : 0.0;
-    double rc = row ? cnorm2(x) : 0.0;
-    rs = group_sum(rs, g, g.gbase + g.gl);
-    rc = group_sum(rc, g, g.gbase + g.gl);
-    if (run) {
-      ++nnewt;
-      ok = rs < o.corr_tol * rc;
-      inf = rc > o.inf_tol;
-      if (ok || inf) run = false;
+// Outputs of a finished path.
+template <class SegT>
+__device__ __forceinline__ void store_path(const SegT& S, long long path, int inst, int n, bool row, const Group& g,
+                                           cx<double> x, uint32_t fl, int nsteps, int nnewt, int nref, double t,
+                                           double dt, double resid) {
+  const SegOut* O = S.out;
+  double2* roots = O->roots;
+  const int rstride = O->roots_stride;
+  if (row && g.s == 0) roots[(size_t)path * rstride + g.gl] = make_double2(x.re, x.im);
+  if (g.gl == 0 && g.s == 0) {
+    if (rstride > n) roots[(size_t)path * rstride + n] = make_double2(1.0, 0.0);
+    if (O->flags) O->flags[path] = fl;
+    if (O->steps) O->steps[path] = nsteps;
+    if (O->newton) O->newton[path] = nnewt;
+    if (O->refine) O->refine[path] = nref;
+    if (O->tfin) O->tfin[path] = t;
+    if (O->dtfin) O->dtfin[path] = dt;
+    if (O->resid) O->resid[path] = resid;
+    if (O->conv8) O->conv8[path] = (fl & HCX_FLAG_TRACKED) ? 1 : 0;
+    if (O->inf8) O->inf8[path] = (fl & HCX_FLAG_INFINITY) ? 1 : 0;
+    if (O->debug) O->debug[path] = (fl & HCX_FLAG_TRACKED) ? make_double2(1.0, 0.0) : make_double2(t, dt);
+    if (O->inst_left) {
+      const int left = atomicSub(&O->inst_left[inst], 1);
+      if (left == 1 && O->inst_done) O->inst_done[inst] = wall_clock64();
+    } else if (O->inst_done && S.plist) {
+      atomicMax(&O->inst_done[inst], (unsigned long long)wall_clock64());
     }
   }
 }
@@ -723,58 +586,66 @@ __device__ __forceinline__ void newton_pass(const SegT& S, int n, const OT& o, c
 
 using namespace dev;
 
-// One RK4 predictor step in precision T for the groups in `act`
-// (…4pts.cu:139-183): stages at (x0, t), (x0 + h k1, t + h), (x0 + h k2, t + h),
-// (x0 + dt k3, t + dt); returns k1 + 2 k2 + 2 k3 + k4 (component gl).
-template <int NMAX, int GC, int DEG, class T, bool LT, class SegT>
-__device__ __forceinline__ cx<double> predict(const SegT& S, int n, const Group& g, const Lds<NMAX, GC == 0>& L, const void* lt,
-                                              bool act, bool row, int gle, int inst, double ts, double dt,
-                                              cx<double> xl) {
-  const double h = 0.5 * dt;
-  cx<double> acc = cmk<double>(0, 0), kprev = cmk<double>(0, 0);
-  cx<T>* sx = L.template x<T>();
-  const cx<T>* sc = reinterpret_cast<const cx<T>*>(L.coef());
-  const cx<T>* sd = sc + (S.C + 1);
-#pragma unroll 1
-  for (int st = 0; st < 4; ++st) {
-    const double a = st == 0 ? 0.0 : (st == 3 ? dt : h);
-    if (st != 2) stage_coeffs<T>(S, g, act, inst, ts + a, L.coef(), true);
-    const cx<double> xs = cmk<double>(xl.re + a * kprev.re, xl.im + a * kprev.im);
-    publish_x<T>(sx, xs, g, n, act, row);
-    HCX_WAVE_SYNC();
-    cx<T> A[NMAX];
-    eval_jac_row<NMAX, DEG, T, LT>(S, n, gle, sx, sc, A, lt);
-    const cx<T> bt = eval_t_row<DEG, T, LT>(S, n, gle, sx, sd, lt);
-    bool sing;
-    const cx<T> k = group_lu_solve<NMAX, GC, T>(A, cmk<T>(-bt.re, -bt.im), g, n, row, L.template piv<T>(), L.keys(), sing);
-    kprev = ccast<double>(k);
-    const double w = (st == 1 || st == 2) ? 2.0 : 1.0;
-    acc = cmk<double>(acc.re + w * kprev.re, acc.im + w * kprev.im);
+// Phases of a lane group in the path loops.
+enum : int {
+  kPhIdle = 0,
+  kPhLoop,     // at the loop top of the step loop (…4pts.cu:116)
+  kPhStage0,   // RK4 stages 0..3 (…4pts.cu:139-183)
+  kPhStage1,
+  kPhStage2,
+  kPhStage3,
+  kPhNewton,   // corrector iteration at the new t (…4pts.cu:189-223)
+  kPhRefine,   // refinement iteration on H(x, 1)
+  kPhResid,    // residual H(x, 1) of the refined root
+  kPhOut,      // outputs pending
+};
+
+
+// Mixed-precision lane-group path loop: FP32 RK4 predictor (Jacobian, dH/dt
+// and solve of the four stages), FP64 Newton corrector (FP32 before the end
+// zone when o.newton32), FP64 refinement; a path that ends without a refined
+// root is re-tracked from t = 0 entirely in FP64 (escalation) by the FP64 pass
+// after the launch, which keeps the FP64 predictor out of the kernel and with
+// it the registers of a second predictor.
+// The wave alternates between the predictor of every group that steps and
+// FP64 iterations.  An FP64 iteration serves every group that has one to do: the
+// corrector, the refinement and the final residual.  The FP64 turn ends when no
+// group corrects any more; a group that refines goes on in the next turn, beside
+// the others' correctors, so that no group waits for another's refinement.
+// Streams, staging and rounds are those of the FP64 loop, at FP32 on half the
+// bytes (hcx_eval.hpp); the FP32 c(t) and dc/dt of the predictor and the FP64 c(t)
+// share the coefficient area.
+// NB: Jacobian columns evaluated together (twice as many in FP32 were no
+// faster: the rounds of a block are its longest column's).
+// Measured (n = 12, 240 coefficients, degrees 2 and 3, 512 x 1024 paths): 159.5 ->
+// 150.3 ms.
+template <class T, int NMAX, int DEG, bool LT, int NB, class SegT>
+__device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, const unsigned char* xb,
+                                             const unsigned char* cb, const unsigned char* rhs,
+                                             const unsigned char* lt, cx<T> (&A)[NMAX]) {
+  constexpr int DC = DEG <= 4 ? DEG : 4;
+  if (LT || lt) {
+    constexpr int HQ = NMAX <= 6 && sizeof(T) == 8 ? 2 : 4;
+    eval_jac_blocks<NMAX, DC, NB, 0, T>(S, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
+    return eval_rhs_stream<DC, false, HQ, (NMAX > 6), T>(S, n, gle, xb, rhs, rhs, nullptr, false, lt, 0, 1);
   }
-  return acc;
+  if constexpr (!LT) {
+    const cx<T>* const sx = reinterpret_cast<const cx<T>*>(xb);
+    eval_jac_terms<NMAX, DEG, T>(S, n, gle, sx, reinterpret_cast<const cx<T>*>(cb), A, nullptr, 0, 1);
+    return eval_rhs_terms<DEG, false, T>(S, n, gle, sx, reinterpret_cast<const cx<T>*>(rhs), nullptr, false, nullptr, 0,
+                                         1);
+  }
+  return cmk<T>(0, 0);
 }
 
-// Mixed-precision lane-group path loop (MODE 1; the FP64 mode runs
-// run_segment_fp64), phase-synchronous: FP32 RK4
-// predictor (Jacobian, dH/dt and LU of the four stages), FP64 Newton
-// corrector (FP32 before the end zone when o.newton32), FP64 refinement; a
-// path that ends without a refined root is re-tracked from t = 0 entirely in
-// FP64 (escalation) by the FP64 pass after the launch, which keeps the FP64
-// predictor out of the kernel and with it the registers of a second predictor.
-template <int NMAX, int DEG, int MODE, bool EXACT>
-__device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned char* smem, int lane) {
-  static_assert(MODE == 1, "the FP64 mode runs run_segment_fp64");
-  // local copies: the fields are wave-uniform and live in SGPRs (scalar
-  // kernarg loads) instead of being re-read through a generic pointer
+template <int NMAX, int DEG, bool EXACT, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
+__device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsigned char* smem, int lane) {
   Seg S = LN.seg[si];
   constexpr int GE = exact_lanes(NMAX);
   if (EXACT) {
-    // size-specialised instance: n = NMAX and G are compile-time constants,
-    // so every loop bound and the lane-group geometry fold away
     S.n = NMAX;
     S.G = GE;
   }
-  // compile-time power-of-two lanes per path: DPP group reductions
   constexpr int GC = (EXACT && is_pow2(GE)) ? GE : 0;
   const KOpts* const opts_arg = launch_opts();
   const KSeg* const seg_arg = launch_seg(si);
@@ -783,61 +654,48 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
   const int n = S.n;
   const bool row = g.in_grp && g.gl < n;
   const int gle = row ? g.gl : 0;
-  // Size-specialised instances up to n = 16, and n = 30 with quadratic
-  // terms, read the segment's tables from a compact copy in LDS (at the start
-  // of the dynamic LDS, LN.tab_lds bytes) instead of global memory: the term
-  // loads head every evaluation's dependency chain, and LDS returns them
-  // several times sooner.
   constexpr bool LT = EXACT && (NMAX <= 16 || DEG <= 2);
-  const void* lt = nullptr;
-  if constexpr (LT) lt = stage_tables(S, smem);
-  // lanes outside the full groups (64 % G of them) alias region 0: they
-  // track nothing and store nothing to LDS
+  const unsigned char* lt = nullptr;
+  if constexpr (LT) {
+    lt = static_cast<const unsigned char*>(stage_tables(S, smem));
+  } else if constexpr (!EXACT) {
+    if (LN.tab_lds > 0) lt = static_cast<const unsigned char*>(stage_tables(S, smem));
+  }
+  constexpr int SQ = EXACT && NMAX <= 16 ? 4 : 2;  // coefficients in flight per lane while staging
+  constexpr bool SL = LT && NMAX <= 16;
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
   Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
+  unsigned char* const xb = L.base;
+  unsigned char* const cb = L.coef();
+  const int head = (int)(cb - xb);
+  const unsigned char* const db = cb + S.nslot * 8;  // dc/dt (FP32)
+  const double2 *hxi = S.chx, *hti = S.cht;
 
-  // per-group path state, replicated over the group's lanes
   long long path = -1;
   int inst = 0, root = 0;
-  double t = 0.0, dt = 0.0;
-  int cnt = 0, nsteps = 0, asteps = 0, nnewt = 0, nref = 0;
-  bool ez = false;
-  int status = 0;  // 0 idle, 1 tracking, 2 finishing
+  double t = 0.0, dt = 0.0, tst = -1.0, resid = 0.0;  // tst: t of the FP64 c(t) in LDS
+  int cnt = 0, nsteps = 0, asteps = 0, nnewt = 0, nref = 0, nit = 0;
+  bool ez = false, conv = false, sing_any = false;
+  int ph = kPhIdle;
   uint32_t fl = 0;
   bool exhausted = !g.in_grp;
   long long static_path = ((long long)((int)blockIdx.x - LN.first_block[si]) * LN.wpb + wv) * g.gpw + g.grp;
-  // lane-distributed state: component gl of x and of the last accepted x
+  double ts = 0.0;
   cx<double> x = cmk<double>(0, 0), xl = x;
-
-  auto start_path = [&](const KSeg& Sv) {
-    t = 0.0;
-    dt = opts_arg->dt0;
-    cnt = 0;
-    asteps = 0;
-    ez = false;
-    status = 1;
-    if (row) {
-      const double2 v = Sv.start[(size_t)root * Sv.start_stride + g.gl];
-      x = cmk<double>(v.x, v.y);
-    } else {
-      x = cmk<double>(0, 0);
-    }
-    xl = x;
-  };
 
   for (;;) {
     const KOpts& o = *iteration_view(opts_arg, iter);
     const KSeg& Sk = *iteration_view(seg_arg, iter);
     ++iter;
     // ------------------------------------------------ refill idle groups
-    const bool want = status == 0 && !exhausted;
+    const bool want = ph == kPhIdle && !exhausted;
     if (__any(want)) {
       long long p;
       if (LN.persistent) {
         unsigned int q = 0;
         if (want && g.gl == 0) {
           q = atomicAdd(Sk.counter, 1u);
-          // path-list launch (FP64 re-track of selected paths)
+          // path-list launch
           if (Sk.plist) q = q < *Sk.plist_count ? (unsigned int)Sk.plist[q] : 0xffffffffu;
         }
         p = (long long)(unsigned int)lane_read((int)q, g.gbase);
@@ -852,193 +710,229 @@ __device__ __forceinline__ void run_segment(const Launch& LN, int si, unsigned c
           path = p;
           inst = (int)(p / Sk.K);
           root = (int)(p - (long long)inst * Sk.K);
-          nsteps = 0;
-          nnewt = 0;
-          nref = 0;
+          hxi = Sk.chx + (size_t)inst * (Sk.C + 1) * (Sk.M + 1);
+          hti = Sk.cht + (size_t)inst * (Sk.C + 1) * Sk.M;
+          nsteps = asteps = nnewt = nref = cnt = 0;
           fl = Sk.plist ? HCX_FLAG_ESCALATED : 0u;
-          start_path(Sk);
+          t = 0.0;
+          dt = o.dt0;
+          ez = false;
+          tst = -1.0;
+          resid = 0.0;
+          if (row) {
+            const double2 v = Sk.start[(size_t)root * Sk.start_stride + g.gl];
+            x = cmk<double>(v.x, v.y);
+          } else {
+            x = cmk<double>(0, 0);
+          }
+          xl = x;
+          ph = kPhLoop;
           if (!LN.persistent) exhausted = true;
         }
       }
     }
-    if (!__any(status != 0)) break;
+    if (!__any(ph != kPhIdle)) break;
 
-    // ------------------------------------------------ loop-top tests (:116)
-    bool stepping = false;
-    if (status == 1) {
+    // ------------------------------------------------ loop top (:116-131)
+    bool fin = false, stepping = false;
+    if (ph == kPhLoop) {
       if (!(t < 1.0 && 1.0 - t > o.t_tol)) {
-        status = 2;
         fl |= HCX_FLAG_TRACKED;
+        fin = true;
       } else if (asteps > o.max_steps) {
-        status = 2;
         fl |= HCX_FLAG_BUDGET;
+        fin = true;
       } else {
-        stepping = true;
-      }
-    }
-
-    if (__any(stepping)) {
-      // end zone and step clamp (:121-131)
-      if (stepping) {
+        // end zone and step clamp
         if (!ez && fabs(1.0 - t) <= o.ez_enter) ez = true;
         if (ez) {
           if (dt > fabs(1.0 - t)) dt = fabs(1.0 - t);
         } else if (dt > fabs(o.ez_land - t)) {
           dt = fabs(o.ez_land - t);
         }
+        ts = t;
+        stepping = true;
       }
-      const double ts = t;
-      const cx<double> acc = predict<NMAX, GC, DEG, float, LT>(Sk, n, g, L, lt, stepping, row, gle, inst, ts, dt, xl);
+    }
+    if (__any(fin)) {
+      // the reference's real test on the tracked root, before refinement
+      // (Evaluations.cpp:96-104: converged and every |Im x_i| <= 1e-4)
+      double imt = (fin && row) ? fabs(x.im) : 0.0;
+      if (imt != imt) imt = INFINITY;
+      imt = group_max(imt, g);
+      if (fin) {
+        if ((fl & HCX_FLAG_TRACKED) && imt <= o.real_ref_tol) fl |= HCX_FLAG_REAL_REF;
+        if ((fl & HCX_FLAG_TRACKED) && o.refine_iters > 0) {
+          ph = kPhRefine;
+          nit = 0;
+          conv = false;
+          sing_any = false;
+        } else {
+          ph = kPhOut;
+        }
+      }
+    }
+
+    // step control (:225-249) of a corrected step
+    auto control = [&](bool ok, bool inf) {
+      ++nsteps;
+      ++asteps;
+      ph = kPhLoop;
+      if (inf) {
+        fl |= HCX_FLAG_INFINITY;
+        ph = kPhOut;
+      } else if (!ok) {
+        dt *= 0.5;
+        x = xl;
+        t = ts;
+        cnt = 0;
+        if (dt < o.dt_min) {
+          fl |= HCX_FLAG_MINSTEP;
+          ph = kPhOut;
+        }
+      } else {
+        ++cnt;
+        xl = x;
+        if (cnt >= o.incr) {
+          cnt = 0;
+          dt *= 2.0;
+        }
+      }
+    };
+
+    // ------------------------------------------------ FP32 predictor
+    if (__any(stepping)) {
+      // RK4 (:139-183): stages at (x0, t), (x0 + h k1, t + h),
+      // (x0 + h k2, t + h), (x0 + dt k3, t + dt)
+      const double h = 0.5 * dt;
+      cx<double> acc = cmk<double>(0, 0), kp = acc;
+      cx<float>* const sx = L.template x<float>();
+#pragma unroll 1
+      for (int st = 0; st < 4; ++st) {
+        const double a = st == 0 ? 0.0 : (st == 3 ? dt : h);
+        // order 1: dc/dt does not depend on t, but the FP64 c(t) of the last
+        // corrector lies over it
+        if (stepping && st != 2)
+          stage_coeffs<SL, SQ, float>(Sk, g, hxi, hti, ts + a, xb + head / 2, head, Sk.nslot * 8, st == 0 || Sk.M > 1,
+                                      lt);
+        const cx<double> xs = cmk<double>(xl.re + a * kp.re, xl.im + a * kp.im);
+        publish_x<float>(sx, xs, g, n, stepping, row);
+        HCX_WAVE_SYNC();
+        cx<float> A[NMAX];
+        const cx<float> bt = eval_system<float, NMAX, DEG, LT, NB>(Sk, n, gle, xb, cb, db, lt, A);
+        bool sing;
+        const cx<float> k = group_lu_solve<NMAX, GC, float>(A, cmk<float>(-bt.re, -bt.im), g, n, row,
+                                                            L.template piv<float>(), L.keys(), sing);
+        kp = ccast<double>(k);
+        const double w = (st == 1 || st == 2) ? 2.0 : 1.0;
+        acc = cmk<double>(acc.re + w * kp.re, acc.im + w * kp.im);
+      }
       if (stepping) {
         const double f = dt * (1.0 / 6.0);
         x = cmk<double>(xl.re + f * acc.re, xl.im + f * acc.im);
         t = ts + dt;
+        ph = kPhNewton;
+        nit = 0;
+        tst = -1.0;
       }
-      // Newton corrector at the new t (:189-223)
-      bool ok = false, inf = false;
-      {
-        const bool run32 = stepping && !ez && o.newton32, run64 = stepping && !run32;
-        bool ok32 = false, inf32 = false, ok64 = false, inf64 = false;
-        if (__any(run32)) newton_pass<NMAX, GC, DEG, float, LT>(Sk, n, o, g, L, lt, run32, row, x, nnewt, ok32, inf32);
-        if (__any(run64)) {
+      // FP32 corrector before the end zone (o.newton32), on stage 3's c(t + dt)
+      bool run = stepping && !ez && o.newton32;
+      if (__any(run)) {
+        const bool run32 = run;
+        bool ok = false, inf = false;
+        for (int it = 0; it < o.max_corr; ++it) {
+          if (!__any(run)) break;
+          publish_x<float>(sx, x, g, n, run, row);
           HCX_WAVE_SYNC();
-          stage_coeffs<double>(Sk, g, run64, inst, t, L.coef(), false);
-          newton_pass<NMAX, GC, DEG, double, LT>(Sk, n, o, g, L, lt, run64, row, x, nnewt, ok64, inf64);
-        }
-        ok = run64 ? ok64 : ok32;
-        inf = run64 ? inf64 : inf32;
-      }
-      // step control (:225-249)
-      if (stepping) {
-        ++nsteps;
-        ++asteps;
-        if (inf) {
-          status = 2;
-          fl |= HCX_FLAG_INFINITY;
-        } else if (!ok) {
-          dt *= 0.5;
-          x = xl;
-          t = ts;
-          cnt = 0;
-          if (dt < o.dt_min) {
-            status = 2;
-            fl |= HCX_FLAG_MINSTEP;
-          }
-        } else {
-          ++cnt;
-          xl = x;
-          if (cnt >= o.incr) {
-            cnt = 0;
-            dt *= 2.0;
+          cx<float> A[NMAX];
+          const cx<float> hv = eval_system<float, NMAX, DEG, LT, NB>(Sk, n, gle, xb, cb, cb, lt, A);
+          bool sing;
+          const cx<float> d =
+              group_lu_solve<NMAX, GC, float>(A, hv, g, n, row, L.template piv<float>(), L.keys(), sing);
+          if (run && row) x = csub(x, ccast<double>(d));
+          double s1 = row ? (double)cnorm2(d) : 0.0, s2 = row ? cnorm2(x) : 0.0;
+          group_sum2<NMAX, GC, true>(s1, s2, g, n, row, lane, L.piv64());
+          if (run) {
+            ++nnewt;
+            ok = s1 < o.corr_tol * s2;
+            inf = s2 > o.inf_tol;
+            if (ok || inf) run = false;
           }
         }
+        if (run32) control(ok, inf);
+        HCX_WAVE_SYNC();
       }
-      HCX_WAVE_SYNC();
     }
 
-    // ------------------------------------------------ finish: refine + outputs
-    const bool fin = status == 2;
-    if (__any(fin)) {
-      // the reference's real test on the tracked root, before refinement
-      // (Evaluations.cpp:96-104: converged and every |Im x_i| <= 1e-4)
-      {
-        double imt = (fin && row) ? fabs(x.im) : 0.0;
-        if (imt != imt) imt = INFINITY;
-        imt = group_max(imt, g);
-        if (fin && (fl & HCX_FLAG_TRACKED) && imt <= o.real_ref_tol) fl |= HCX_FLAG_REAL_REF;
+    // ------------------------------------------------ FP64 iterations
+    for (;;) {
+      const int pe = ph;
+      const bool act = pe == kPhNewton || pe == kPhRefine || pe == kPhResid;
+      if (!__any(act)) break;
+      const double te = pe == kPhNewton ? t : 1.0;
+      if (act && te != tst) {
+        stage_coeffs<SL, SQ, double>(Sk, g, hxi, hti, te, xb, head, 0, false, lt);
+        tst = te;
       }
-      const bool ref = fin && (fl & HCX_FLAG_TRACKED) && o.refine_iters > 0;
-      double resid = 0.0;
-      if (__any(ref)) {
-        stage_coeffs<double>(Sk, g, ref, inst, 1.0, L.coef(), false);
-        cx<double>* sx = L.template x<double>();
-        const cx<double>* sc = reinterpret_cast<const cx<double>*>(L.coef());
-        bool run = ref, conv = false, sing_any = false;
-        for (int it = 0; it < o.refine_iters; ++it) {
-          if (!__any(run)) break;
-          publish_x<double>(sx, x, g, n, run, row);
-          HCX_WAVE_SYNC();
-          cx<double> A[NMAX];
-          eval_jac_row<NMAX, DEG, double, LT>(Sk, n, gle, sx, sc, A, lt);
-          const cx<double> hv = eval_t_row<DEG, double, LT>(Sk, n, gle, sx, sc, lt);
-          bool sing;
-          const cx<double> d = group_lu_solve<NMAX, GC, double>(A, hv, g, n, row, L.template piv<double>(), L.keys(), sing);
-          if (run && row) x = csub(x, d);
-          double nd = row ? cnorm2(d) : 0.0, nx = row ? cnorm2(x) : 0.0;
-          nd = group_sum(nd, g, lane);
-          nx = group_sum(nx, g, lane);
-          if (run) {
-            ++nref;
-            sing_any = sing;
-            if (!(nx < o.inf_tol)) {
-              run = false;
-            } else if (sqrt(nd) <= o.refine_tol * fmax(1.0, sqrt(nx))) {
-              conv = true;
-              run = false;
-            }
-          }
+      cx<double>* const sx = L.x64();
+      publish_x<double>(sx, x, g, n, act, row);
+      HCX_WAVE_SYNC();
+      cx<double> A[NMAX];
+      const cx<double> r = eval_system<double, NMAX, DEG, LT, NB>(Sk, n, gle, xb, cb, cb, lt, A);
+      bool sing;
+      const cx<double> d = group_lu_solve<NMAX, GC, double>(A, r, g, n, row, L.piv64(), L.keys(), sing);
+      const bool nr = pe == kPhNewton || pe == kPhRefine;
+      if (nr && row) x = csub(x, d);
+      double s1 = (nr && row) ? cnorm2(d) : 0.0, s2 = (nr && row) ? cnorm2(x) : 0.0;
+      group_sum2<NMAX, GC, true>(s1, s2, g, n, row, lane, L.piv64());
+      if (pe == kPhNewton) {
+        ++nnewt;
+        ++nit;
+        const bool ok = s1 < o.corr_tol * s2, inf = s2 > o.inf_tol;
+        if (ok || inf || nit >= o.max_corr) control(ok, inf);
+      } else if (pe == kPhRefine) {
+        ++nref;
+        ++nit;
+        sing_any = sing;
+        bool stop = false;
+        if (!(s2 < o.inf_tol)) {
+          stop = true;
+        } else if (sqrt(s1) <= o.refine_tol * fmax(1.0, sqrt(s2))) {
+          conv = true;
+          stop = true;
         }
-        // residual max_i |H_i(x, 1)|
-        publish_x<double>(sx, x, g, n, ref, row);
-        HCX_WAVE_SYNC();
-        const cx<double> hv = eval_t_row<DEG, double, LT>(Sk, n, gle, sx, sc, lt);
-        double r = row ? sqrt(cnorm2(hv)) : 0.0;
-        if (r != r) r = INFINITY;
-        resid = group_max(r, g);
-        double im = row ? fabs(x.im) : 0.0;
+        if (stop || nit >= o.refine_iters) ph = kPhResid;
+      }
+      // residual max_i |H_i(x, 1)| of the refined root (r = H at x)
+      const bool rz = pe == kPhResid;
+      if (__any(rz)) {
+        double rr = (rz && row) ? sqrt(cnorm2(r)) : 0.0;
+        if (rr != rr) rr = INFINITY;
+        rr = group_max(rr, g);
+        double im = (rz && row) ? fabs(x.im) : 0.0;
         if (im != im) im = INFINITY;
         im = group_max(im, g);
-        if (ref) {
+        if (rz) {
+          resid = rr;
           if (conv) fl |= HCX_FLAG_REFINED;
           if (conv && im <= o.real_tol) fl |= HCX_FLAG_REAL;
           if (sing_any) fl |= HCX_FLAG_SINGULAR;
+          ph = kPhOut;
         }
-        HCX_WAVE_SYNC();
       }
-      if (fin) {
-        const SegOut* O = Sk.out;
-        double2* roots = O->roots;
-        const int rstride = O->roots_stride;
-        if (row) roots[(size_t)path * rstride + g.gl] = make_double2(x.re, x.im);
-        if (g.gl == 0) {
-          if (rstride > n) roots[(size_t)path * rstride + n] = make_double2(1.0, 0.0);
-          if (O->flags) O->flags[path] = fl;
-          if (O->steps) O->steps[path] = nsteps;
-          if (O->newton) O->newton[path] = nnewt;
-          if (O->refine) O->refine[path] = nref;
-          if (O->tfin) O->tfin[path] = t;
-          if (O->dtfin) O->dtfin[path] = dt;
-          if (O->resid) O->resid[path] = resid;
-          if (O->conv8) O->conv8[path] = (fl & HCX_FLAG_TRACKED) ? 1 : 0;
-          if (O->inf8) O->inf8[path] = (fl & HCX_FLAG_INFINITY) ? 1 : 0;
-          if (O->debug) O->debug[path] = (fl & HCX_FLAG_TRACKED) ? make_double2(1.0, 0.0) : make_double2(t, dt);
-          if (O->inst_left) {
-            const int left = atomicSub(&O->inst_left[inst], 1);
-            if (left == 1 && O->inst_done) O->inst_done[inst] = wall_clock64();
-          } else if (O->inst_done && Sk.plist) {
-            atomicMax(&O->inst_done[inst], (unsigned long long)wall_clock64());
-          }
-        }
-        status = 0;
-        path = -1;
-      }
+      HCX_WAVE_SYNC();
+      if (!__any(ph == kPhNewton)) break;
+    }
+
+    // ------------------------------------------------ outputs
+    const bool out = ph == kPhOut;
+    if (__any(out) && out) {
+      store_path(Sk, path, inst, n, row, g, x, fl, nsteps, nnewt, nref, t, dt, resid);
+      ph = kPhIdle;
+      path = -1;
     }
   }
 }
-
-// Phases of a lane group in the FP64 micro-step loop.
-enum : int {
-  kPhIdle = 0,
-  kPhLoop,     // at the loop top of the step loop (…4pts.cu:116)
-  kPhStage0,   // RK4 stages 0..3 (…4pts.cu:139-183)
-  kPhStage1,
-  kPhStage2,
-  kPhStage3,
-  kPhNewton,   // corrector iteration at the new t (…4pts.cu:189-223)
-  kPhRefine,   // refinement iteration on H(x, 1)
-  kPhResid,    // residual H(x, 1) of the refined root
-  kPhOut,      // outputs pending
-};
 
 // FP64 lane-group path loop in uniform micro-steps.  Every iteration of the
 // wave performs ONE evaluation (Jacobian rows and a right-hand side) and ONE
@@ -1223,10 +1117,10 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       if (restage) {
         // order 1: dc/dt does not depend on t, once per path is enough
         const bool dot = !gdot && (Sk.M > 1 || tst < 0.0);
-        stage_coeffs64<LT && NMAX <= 16, SQ>(Sk, g, hxi, hti, te, xb, (int)(cb - xb), (int)(db - cb), dot, lt);
+        stage_coeffs<LT && NMAX <= 16, SQ, double>(Sk, g, hxi, hti, te, xb, (int)(cb - xb), (int)(db - cb), dot, lt);
         tst = te;
       }
-      publish_x64(sx, xe, g, n, act, row);
+      publish_x<double>(sx, xe, g, n, act, row);
       HCX_WAVE_SYNC();
       cx<double> A[NMAX];
       cx<double> r;
@@ -1235,24 +1129,24 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
         if constexpr (REP) {
           eval_jac_rounds<NMAX, DC>(Sk, n, gle, xb, cb, A, lt, k0, ks);
           if (Sk.htT <= 2 * ks)
-            r = eval_rhs_stream<DC, false, 2, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, false, 2, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<DC, false, 4, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, false, 4, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         } else {
           constexpr int HQ = NMAX <= 6 ? 2 : 4;  // H terms in flight
-          eval_jac_blocks<NMAX, DC, NB, 0>(Sk, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
+          eval_jac_blocks<NMAX, DC, NB, 0, double>(Sk, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
           if (gdot)
-            r = eval_rhs_stream<DC, true, HQ, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, true, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<DC, false, HQ, kPin>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DC, false, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         }
       } else {
         const cx<double>* sc = reinterpret_cast<const cx<double>*>(cb);
-        eval_jac_terms<NMAX, DEG>(Sk, n, gle, sx, sc, A, tl, k0, ks);
+        eval_jac_terms<NMAX, DEG, double>(Sk, n, gle, sx, sc, A, tl, k0, ks);
         if (gdot)
-          r = eval_rhs_terms<DEG, true>(Sk, n, gle, sx, sc, hti, stg, tl, k0, ks);
+          r = eval_rhs_terms<DEG, true, double>(Sk, n, gle, sx, sc, hti, stg, tl, k0, ks);
         else
-          r = eval_rhs_terms<DEG, false>(Sk, n, gle, sx, reinterpret_cast<const cx<double>*>(stg ? db : cb), hti, stg,
+          r = eval_rhs_terms<DEG, false, double>(Sk, n, gle, sx, reinterpret_cast<const cx<double>*>(stg ? db : cb), hti, stg,
                                          tl, k0, ks);
       }
       bool sing;
@@ -1310,7 +1204,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       const bool nr = pe == kPhNewton || pe == kPhRefine;
       if (nr && row) x = csub(x, d);
       double s1 = (nr && row) ? cnorm2(d) : 0.0, s2 = (nr && row) ? cnorm2(x) : 0.0;
-      if (__any(nr)) group_sum2<NMAX, GC>(s1, s2, g, n, row, lane, L.template piv<double>());
+      if (__any(nr)) group_sum2<NMAX, GC, false>(s1, s2, g, n, row, lane, L.template piv<double>());
       if (pe == kPhNewton) {
         ++nnewt;
         ++nit;
@@ -1381,30 +1275,8 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
     // ------------------------------------------------ outputs
     const bool out = ph == kPhOut;
     if (__any(out) && out) {
-      const SegOut* O = Sk.out;
-      double2* roots = O->roots;
-      const int rstride = O->roots_stride;
       // replica 0 stores (the other replicas hold the same values)
-      if (row && g.s == 0) roots[(size_t)path * rstride + g.gl] = make_double2(x.re, x.im);
-      if (g.gl == 0 && g.s == 0) {
-        if (rstride > n) roots[(size_t)path * rstride + n] = make_double2(1.0, 0.0);
-        if (O->flags) O->flags[path] = fl;
-        if (O->steps) O->steps[path] = nsteps;
-        if (O->newton) O->newton[path] = nnewt;
-        if (O->refine) O->refine[path] = nref;
-        if (O->tfin) O->tfin[path] = t;
-        if (O->dtfin) O->dtfin[path] = dt;
-        if (O->resid) O->resid[path] = resid;
-        if (O->conv8) O->conv8[path] = (fl & HCX_FLAG_TRACKED) ? 1 : 0;
-        if (O->inf8) O->inf8[path] = (fl & HCX_FLAG_INFINITY) ? 1 : 0;
-        if (O->debug) O->debug[path] = (fl & HCX_FLAG_TRACKED) ? make_double2(1.0, 0.0) : make_double2(t, dt);
-        if (O->inst_left) {
-          const int left = atomicSub(&O->inst_left[inst], 1);
-          if (left == 1 && O->inst_done) O->inst_done[inst] = wall_clock64();
-        } else if (O->inst_done && Sk.plist) {
-          atomicMax(&O->inst_done[inst], (unsigned long long)wall_clock64());
-        }
-      }
+      store_path(Sk, path, inst, n, row, g, x, fl, nsteps, nnewt, nref, t, dt, resid);
       ph = kPhIdle;
       path = -1;
     }
@@ -1426,7 +1298,7 @@ void track_kernel(const Launch LN) {
     if constexpr (MODE == 0) {
       run_segment_fp64<NMAX, DEG, EXACT, 0>(LN, s, smem, lane);
     } else {
-      run_segment<NMAX, DEG, MODE, EXACT>(LN, s, smem, lane);
+      run_segment_mixed<NMAX, DEG, EXACT>(LN, s, smem, lane);
     }
     if (!LN.persistent) break;
     s = s + 1 == LN.nseg ? 0 : s + 1;
@@ -1452,7 +1324,7 @@ __device__ __forceinline__ void run_exact(const Launch& LN, int si, unsigned cha
   if constexpr (MODE == 0) {
     run_segment_fp64<N, DEG, true, 0, 2>(LN, si, smem, lane);
   } else {
-    run_segment<N, DEG, MODE, true>(LN, si, smem, lane);
+    run_segment_mixed<N, DEG, true, 2>(LN, si, smem, lane);
   }
 }
 

@@ -17,32 +17,25 @@
 struct hcx_problem {
   int device = 0;
   int n = 0, C = 0, M = 1, K = 0, k = 0;
-  int hxT = 0, htT = 0, hx_vars = 0, ht_vars = 0, deg = 2;
+  int hxT = 0, htT_padded = 0, hx_vars = 0, ht_vars = 0, deg = 2;
   unsigned char* d_blob = nullptr;     // the allocation that holds every table below
-  hcx::dev::Term* d_hx = nullptr;
-  hcx::dev::Term* d_ht = nullptr;
-  unsigned int colc[hcx::kMaxN] = {};  // terms per Jacobian column (max over equations)
   int* d_cslot = nullptr;              // [C+1] LDS slot of each coefficient
-  uint32_t* d_ctab = nullptr;          // compact hx + ht tables (8-byte terms), or null
-  int ctab_bytes = 0;                  // their size rounded up to 16 bytes
-  uint32_t* d_ctab4 = nullptr;         // the same with 4-byte terms (degree <= 2), or null
-  int ctab4_bytes = 0;
-  // Term streams of the FP64 loop (hcx_eval64.hpp): full records in global
-  // memory, and the compact tables of the size-specialised instances for
-  // terms of degree <= 2 ([0], when the problem has no higher ones) and <= 4.
+  // Term streams (hcx_eval.hpp): full records in global memory, and the
+  // compact tables of the instances that hold them in LDS for terms of degree
+  // <= 2 ([0], when the problem has no higher ones) and <= 4.
   struct Compact {
     uint32_t* d = nullptr;
     int words = 0, h = 0, slot = 0;    // size; byte offsets of the H streams and the slot list
   };
-  hcx::dev::Term* d_hxs = nullptr;
-  hcx::dev::Term* d_hts = nullptr;
-  int* d_ht_ci = nullptr;              // coefficient number of each d_hts record
-  int* d_hxs_cnt = nullptr;            // [n] positions per column
-  unsigned int colc64[hcx::kMaxN] = {};  // per column: positions | scaled ones << 16
-  bool colc64_fits = false;
-  int hx_recs = 0, htT64 = 0, htS64 = 0, nslot = 0;
+  hcx::dev::Term* d_hx = nullptr;
+  hcx::dev::Term* d_ht = nullptr;
+  int* d_ht_ci = nullptr;              // coefficient number of each d_ht record
+  int* d_hx_cnt = nullptr;             // [n] positions per column
+  unsigned int colc[hcx::kMaxN] = {};  // per column: positions | scaled ones << 16
+  bool colc_fits = false;
+  int hx_recs = 0, htT = 0, htS = 0, nslot = 0;
   int max_terms = 0;                   // positions of the longest column
-  Compact ctab64[2], ltab64[2];        // throughput and latency instances
+  Compact ctab[2], ltab[2];            // throughput and latency instances
   double2* d_start = nullptr;
   double2* d_affine = nullptr;
   double2* d_p0 = nullptr;

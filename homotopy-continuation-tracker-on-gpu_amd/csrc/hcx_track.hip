@@ -7,9 +7,8 @@
 // corrector with |dx|^2 < tol |x|^2 success and |x|^2 > 1e14 infinity tests
 // (:189-225), halving / doubling step control (:230-249), outputs (:256-264).
 // Table semantics follow dev-eval-indxing-generalized_3views_4pts.cuh:34-120,
-// the LU follows dev-cgesv-batched-small.cuh:38-107 (cabs1 partial pivoting,
-// first maximum in current row order, multiply-by-reciprocal elimination,
-// division in back substitution).
+// the solve follows dev-cgesv-batched-small.cuh:38-107 (cabs1 partial pivoting,
+// first maximum in current row order, elimination with the pivot's reciprocal).
 //
 // Work decomposition (MI355X-first): a wave64 holds floor(64/G) lane groups;
 // each group tracks one path at a time, lane gl < n owns equation gl.  Groups
@@ -521,7 +520,7 @@ struct Plan {
   KernelFn fn = nullptr;
   bool keys() const { return latency || !(exact && is_pow2(exact_lanes(nmax))); }  // pivot keys in LDS
   int group_bytes(const hcx_problem* p, bool dot_lds = false) const {
-    return lds_group_bytes(nmax, keys(), mode == 0 ? p->nslot : p->C + 1, p->M, dot_lds);
+    return lds_group_bytes(nmax, keys(), p->nslot, mode == 0 ? p->M : 1, dot_lds);
   }
 };
 
@@ -529,6 +528,12 @@ struct Plan {
 // with quadratic terms) stage in
 // LDS; a problem with larger tables runs on the generic instance.
 constexpr int kMaxTabLds = 32 * 1024;
+// The measure of that limit: the tables at their full width (every equation's
+// and column's padded number of terms), 4 or 8 bytes a term; the compact
+// streams drop the padding and take up to twice that for the terms of H.
+long long table_bytes(const hcx_problem* p, bool t4) {
+  return (((long long)p->hxT * p->n + p->htT_padded) * p->n * (t4 ? 4 : 8) + 15) / 16 * 16;
+}
 // LDS per workgroup on gfx950
 constexpr int kMaxLdsBytes = 160 * 1024;
 
@@ -553,11 +558,9 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
     max_n = std::max(max_n, n);
     same = same && n == probs[0]->n && Gs[s] == exact_lanes(n);
     in_set = in_set && (n == 3 || n == 5 || n == 6 || n == 9 || n == 12) && Gs[s] == n;
-    const void* ct = t4 ? (const void*)probs[s]->d_ctab4 : (const void*)probs[s]->d_ctab;
-    const int cb = t4 ? probs[s]->ctab4_bytes : probs[s]->ctab_bytes;
-    const auto& c64 = probs[s]->ctab64[t4 ? 0 : 1];
-    tab_ok = tab_ok && ct && cb <= kMaxTabLds && (mode != 0 || c64.d);
-    tab = std::max(tab, mode == 0 ? c64.words * 4 : cb);
+    const auto& c = probs[s]->ctab[t4 ? 0 : 1];
+    tab_ok = tab_ok && c.d && table_bytes(probs[s], t4) <= kMaxTabLds;
+    tab = std::max(tab, c.words * 4);
   }
   if (specialize && !same && in_set && tab_ok && max_deg <= 2) {
     pl.fn = mode == 0 ? kernel_set_m0() : kernel_set_m1();
@@ -594,11 +597,11 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
   pl.nmax = kNmaxList[ni];
   pl.deg = kDegList[di];
   pl.exact = false;
-  if (mode == 0 && nseg == 1 && pl.fn) {
-    // a generic FP64 instance reads the compact streams from LDS where they
+  if (nseg == 1 && pl.fn) {
+    // a generic instance reads the compact streams from LDS where they
     // leave as many waves on a CU as its registers allow (one per SIMD for
     // NMAX 32, else two) or as there were without them
-    const auto& c = probs[0]->ctab64[pl.tab4 ? 0 : 1];
+    const auto& c = probs[0]->ctab[pl.tab4 ? 0 : 1];
     const size_t wave = (size_t)(64 / Gs[0]) * (size_t)pl.group_bytes(probs[0]), tb = (size_t)c.words * 4;
     const int cap = pl.nmax == 32 ? 4 : 8;
     int with = 0;
@@ -617,33 +620,22 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
 // The tables of a segment in the form that the plan's kernel reads.
 void seg_tables(Seg& S, const hcx_problem* p, const Plan& pl) {
   S.lds_group = pl.group_bytes(p);
-  S.hxT = p->hxT;
   S.cslot = p->d_cslot;
   S.nslot = p->nslot;
-  if (pl.mode == 0) {
-    const auto& c = (pl.latency ? p->ltab64 : p->ctab64)[pl.tab4 ? 0 : 1];
-    S.hx = p->d_hxs;
-    S.ht = p->d_hts;
-    S.ht_ci = p->d_ht_ci;
-    S.htT = p->htT64;
-    S.htS = p->htS64;
-    S.hx_recs = p->hx_recs;
-    S.max_terms = p->max_terms;
-    std::memcpy(S.colc, p->colc64, sizeof(S.colc));
-    S.hx_cnt = p->colc64_fits ? nullptr : p->d_hxs_cnt;
-    S.ctab = pl.tab_lds > 0 ? c.d : nullptr;
-    S.tab_words = c.words;
-    S.tab_h = c.h;
-    S.tab_slot = c.slot;
-  } else {
-    S.hx = p->d_hx;
-    S.ht = p->d_ht;
-    S.htT = p->htT;
-    std::memcpy(S.colc, p->colc, sizeof(S.colc));
-    S.hx_cnt = nullptr;
-    S.ctab = pl.tab4 ? p->d_ctab4 : p->d_ctab;
-    S.tab_words = (p->hxT * p->n + p->htT) * p->n * (pl.tab4 ? 1 : 2);
-  }
+  const auto& c = (pl.latency ? p->ltab : p->ctab)[pl.tab4 ? 0 : 1];
+  S.hx = p->d_hx;
+  S.ht = p->d_ht;
+  S.ht_ci = p->d_ht_ci;
+  S.htT = p->htT;
+  S.htS = p->htS;
+  S.hx_recs = p->hx_recs;
+  S.max_terms = p->max_terms;
+  std::memcpy(S.colc, p->colc, sizeof(S.colc));
+  S.hx_cnt = p->colc_fits ? nullptr : p->d_hx_cnt;
+  S.ctab = pl.tab_lds > 0 ? c.d : nullptr;
+  S.tab_words = c.words;
+  S.tab_h = c.h;
+  S.tab_slot = c.slot;
 }
 
 // Fills the segment-independent part of a Seg from a problem.
@@ -886,7 +878,6 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   const int hxv = d->hx_parts - 2, htv = d->ht_parts - 2;
   // repack + validate tables: hx [var j][term][eq i], ht [term][eq i]
   std::vector<dev::Term> hx((size_t)n * d->hx_terms * n), ht((size_t)d->ht_terms * n);
-  std::vector<int> hx_cnt(n, 0);
   auto pack = [&](const int* rec, int nv, dev::Term& tm) -> bool {
     tm.s = rec[0];
     tm.c = rec[1];
@@ -917,7 +908,6 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
       }
     }
     for (int j = 0; j < n; ++j) {
-      int real = 0;
       for (int tt = 0; tt < d->hx_terms; ++tt) {
         const int* rec = d->h_hx_idx + (((size_t)i * n + j) * d->hx_terms + tt) * d->hx_parts;
         if (!pack(rec, hxv, hx[((size_t)j * d->hx_terms + tt) * n + i])) {
@@ -925,13 +915,11 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
           return HCX_ERR_INVALID_ARG;
         }
         if (rec[0] != 0) {
-          real = tt + 1;
           int dg = 1;
           for (int q = 0; q < hxv; ++q) dg += rec[2 + q] != n;
           max_deg = std::max(max_deg, dg);
         }
       }
-      hx_cnt[j] = std::max(hx_cnt[j], real);
     }
   }
   // a padded H term still multiplies ht_vars factors; the kernel reads DEG slots
@@ -967,7 +955,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   for (auto& tm : ht) tm.c = cslot[tm.c];
   for (auto& tm : hx) tm.c = cslot[tm.c];
 
-  // Term streams of the FP64 loop (layout and order: hcx_eval64.hpp).
+  // Term streams (layout and order: hcx_eval.hpp).
   int nslot = 0;  // slots that a term uses come first
   {
     std::vector<char> used(C + 1, 0);
@@ -999,8 +987,8 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   };
   std::vector<dev::Term> hxs, hts;
   std::vector<int> hxs_cnt(n), ht_ci;
-  unsigned int colc64[kMaxN] = {};
-  bool colc64_fits = true;
+  unsigned int colc[kMaxN] = {};
+  bool colc_fits = true;
   int s_min = 0, s_max = 0;
   for (int j = 0; j < n; ++j) {
     const size_t at = hxs.size();
@@ -1008,13 +996,13 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
         hxs, [&](int tt, int i) -> const dev::Term& { return hx[((size_t)j * d->hx_terms + tt) * n + i]; },
         d->hx_terms);
     const size_t cnt = (hxs.size() - at) / n;
-    colc64_fits = colc64_fits && cnt <= 0xffff;
-    colc64[j] = (unsigned int)(cnt & 0xffff) | ((unsigned int)scaled & 0xffff) << 16;
+    colc_fits = colc_fits && cnt <= 0xffff;
+    colc[j] = (unsigned int)(cnt & 0xffff) | ((unsigned int)scaled & 0xffff) << 16;
     hxs_cnt[j] = (int)cnt;
   }
   const int htS = add_stream(
       hts, [&](int tt, int i) -> const dev::Term& { return ht[(size_t)tt * n + i]; }, d->ht_terms);
-  const int htT64 = (int)(hts.size() / n), hx_recs = (int)hxs.size();
+  const int htT = (int)(hts.size() / n), hx_recs = (int)hxs.size();
   for (const auto& tm : hts) ht_ci.push_back(cinv[tm.c]);
   for (const auto* v : {&hxs, &hts})
     for (const auto& tm : *v) {
@@ -1037,7 +1025,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     // offsets of 16 bits (from the region's start in the slot list), scalars of
     // 6 or 12 bits
     const int s_lim = f == 0 ? 32 : 2048;
-    if (!colc64_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4000 || C > 0xffff || deg > (f == 0 ? 2 : 4))
+    if (!colc_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4000 || C > 0xffff || deg > (f == 0 ? 2 : 4))
       continue;
     CompactHost& ch = compact[cf];
     std::vector<uint32_t>& w = ch.w;
@@ -1076,7 +1064,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     for (int i = 0; !lat && i < n; ++i) put(zero_term, false);  // one row of zero terms for all columns
     ch.h = align();
     r = 0;
-    for (int k = 0; k < htT64 * n; ++k) put(hts[r++], true);
+    for (int k = 0; k < htT * n; ++k) put(hts[r++], true);
     // a zero term per equation ends the H stream
     for (int i = 0; i < n; ++i) put(zero_term, true);
     ch.slot = align();
@@ -1090,35 +1078,6 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     align();
   }
 
-  // compact 8-byte terms (hx part, then ht part) for the instances that hold
-  // the tables in LDS: slot and scalar in 16 bits each, <= 4 variables
-  std::vector<uint2> ctab;
-  {
-    bool fits = C <= 0xffff && std::max(deg, 2) <= 4;
-    auto pack = [&](const dev::Term& tm) {
-      if (tm.s < -32768 || tm.s > 32767) fits = false;
-      return make_uint2(((uint32_t)tm.c & 0xffffu) | ((uint32_t)tm.s << 16), tm.v03);
-    };
-    ctab.reserve(hx.size() + ht.size());
-    for (const auto& tm : hx) ctab.push_back(pack(tm));
-    for (const auto& tm : ht) ctab.push_back(pack(tm));
-    if (!fits) ctab.clear();
-  }
-  // compact 4-byte terms for degree <= 2: slot in 12 bits, scalar in 4 bits
-  // signed, two variables of 8 bits
-  std::vector<uint32_t> ctab4;
-  if (std::max(deg, 2) <= 2 && C <= 0xfff) {
-    bool fits = true;
-    auto pack4 = [&](const dev::Term& tm) {
-      if (tm.s < -8 || tm.s > 7) fits = false;
-      return ((uint32_t)tm.c & 0xfffu) | (((uint32_t)tm.s & 0xfu) << 12) | ((tm.v03 & 0xffffu) << 16);
-    };
-    ctab4.reserve(hx.size() + ht.size());
-    for (const auto& tm : hx) ctab4.push_back(pack4(tm));
-    for (const auto& tm : ht) ctab4.push_back(pack4(tm));
-    if (!fits) ctab4.clear();
-  }
-
   auto* p = new hcx_problem();
   (void)hipGetDevice(&p->device);
   p->n = n;
@@ -1127,16 +1086,15 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   p->K = d->num_tracks;
   p->k = d->num_params;
   p->hxT = d->hx_terms;
-  p->htT = d->ht_terms;
+  p->htT_padded = d->ht_terms;
   p->hx_vars = hxv;
   p->ht_vars = htv;
   p->deg = std::max(deg, 2);
-  for (int j = 0; j < n; ++j) p->colc[j] = (unsigned int)hx_cnt[j];
-  std::memcpy(p->colc64, colc64, sizeof(colc64));
-  p->colc64_fits = colc64_fits;
+  std::memcpy(p->colc, colc, sizeof(colc));
+  p->colc_fits = colc_fits;
   p->hx_recs = hx_recs;
-  p->htT64 = htT64;
-  p->htS64 = htS;
+  p->htT = htT;
+  p->htS = htS;
   p->nslot = nslot;
   p->max_terms = *std::max_element(hxs_cnt.begin(), hxs_cnt.end());
   auto fail = [&](hipError_t e, const char* what) {
@@ -1155,29 +1113,19 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     blob.resize((blob.size() + 255) & ~size_t(255));
   };
   auto add_vec = [&](auto** dst, const auto& v) { add(dst, v.data(), v.size() * sizeof(v[0])); };
-  add_vec(&p->d_hx, hx);
-  add_vec(&p->d_ht, ht);
   add_vec(&p->d_cslot, cslot);
-  add_vec(&p->d_hxs, hxs);
-  add_vec(&p->d_hts, hts);
+  add_vec(&p->d_hx, hxs);
+  add_vec(&p->d_ht, hts);
   add_vec(&p->d_ht_ci, ht_ci);
-  add_vec(&p->d_hxs_cnt, hxs_cnt);
+  add_vec(&p->d_hx_cnt, hxs_cnt);
   for (int cf = 0; cf < 4; ++cf) {
     const CompactHost& ch = compact[cf];
-    hcx_problem::Compact& ct = cf < 2 ? p->ctab64[cf] : p->ltab64[cf - 2];
+    hcx_problem::Compact& ct = cf < 2 ? p->ctab[cf] : p->ltab[cf - 2];
     if (ch.w.empty()) continue;
     add_vec(&ct.d, ch.w);
     ct.words = (int)ch.w.size();
     ct.h = ch.h;
     ct.slot = ch.slot;
-  }
-  if (!ctab4.empty()) {
-    p->ctab4_bytes = (int)((ctab4.size() * sizeof(uint32_t) + 15) / 16 * 16);
-    add_vec(&p->d_ctab4, ctab4);
-  }
-  if (!ctab.empty()) {
-    p->ctab_bytes = (int)((ctab.size() * sizeof(uint2) + 15) / 16 * 16);
-    add_vec(&p->d_ctab, ctab);
   }
   add(&p->d_start, d->h_start_sols, (size_t)p->K * n * sizeof(double2));
   if (p->k > 0 && d->h_coeff_affine) add(&p->d_affine, d->h_coeff_affine, (size_t)C * (1 + p->k) * sizeof(double2));
@@ -1206,7 +1154,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   in.num_tracks = p->K;
   in.num_params = p->k;
   in.hx_terms = p->hxT;
-  in.ht_terms = p->htT;
+  in.ht_terms = p->htT_padded;
   in.hx_vars = hxv;
   in.ht_vars = htv;
   double fh = 0, fhx = 0;
@@ -1419,7 +1367,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     const hcx_problem* p = probs[0];
     const int lg = pl.group_bytes(p, true);
     const size_t terms =
-        pl.exact ? 0 : ((size_t)p->hx_recs + (size_t)p->n * p->htT64) * sizeof(dev::Term);
+        pl.exact ? 0 : ((size_t)p->hx_recs + (size_t)p->n * p->htT) * sizeof(dev::Term);
     auto waves = [&](int R) {
       const long long gpw = 64 / (S.G * R);
       return (S.P + gpw - 1) / gpw;
@@ -1440,7 +1388,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
       // waves) than at R = 1, and 2,560 paths at n = 16 faster at R = 2
       // (1,280 waves) than at R = 1
       const int dg = std::max(p->deg, 1);
-      const double row_products = (double)p->n * p->hxT * (dg - 1) + (double)p->htT * dg;
+      const double row_products = (double)p->n * p->hxT * (dg - 1) + (double)p->htT_padded * dg;
       const bool heavy = row_products >= 8.0 * (p->n + 1);
       while (R < 8 && 2 * R * S.G <= 64 && waves(2 * R) <= 8LL * g_cu &&
              (R == 1 || heavy || waves(2 * R) <= 2LL * g_cu))
@@ -1453,10 +1401,10 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     // the rule counts the compact tables of the size-specialised instances at 4
     // or 8 bytes a term, and the full records of the generic ones, which read
     // compact tables where they fit as well
-    const auto& lat = p->ltab64[pl.tab4 ? 0 : 1];
+    const auto& lat = p->ltab[pl.tab4 ? 0 : 1];
     const bool compact = pl.exact ? pl.tab_lds > 0 : rf && lat.d && lat.words * 4 <= 65536;
     size_t tab = 0, tab_new = terms;
-    if (pl.exact && pl.tab_lds > 0) tab = (size_t)(pl.tab4 ? p->ctab4_bytes : p->ctab_bytes);
+    if (pl.exact && pl.tab_lds > 0) tab = (size_t)table_bytes(p, pl.tab4);
     if (compact) tab_new = (size_t)(rf ? lat.words * 4 : pl.tab_lds);
     Plan lp = pl;
     lp.latency = rf != nullptr;
