@@ -617,8 +617,9 @@ enum : int {
 // share the coefficient area.
 // NB: Jacobian columns evaluated together (twice as many in FP32 were no
 // faster: the rounds of a block are its longest column's).
-// Measured (n = 12, 240 coefficients, degrees 2 and 3, 512 x 1024 paths): 159.5 ->
-// 150.3 ms.
+// Bound by latency at the 7 waves per CU that its LDS allows (VALU 52% and LDS
+// 53% busy at 6 waves).  n = 12, 240 coefficients, degrees 2 and 3, 512 x 1024
+// paths: 159.5 -> 150.3 ms over the padded tables, 137.4 ms with 7 waves for 6.
 template <class T, int NMAX, int DEG, bool LT, int NB, class SegT>
 __device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, const unsigned char* xb,
                                              const unsigned char* cb, const unsigned char* rhs,
@@ -1287,8 +1288,10 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
 // for three waves per SIMD (at most 168 VGPRs), the others up to 16 variables
 // for two, which their live state fits with few spills or none.
 constexpr int waves_per_simd(int nmax, bool exact) { return exact && nmax <= 6 ? 3 : (nmax <= 16 ? 2 : 1); }
+// Blocks of up to 8 waves, as many as fit the CU's four SIMDs.
+constexpr int block_threads(int nmax, bool exact) { return waves_per_simd(nmax, exact) > 1 ? 512 : 256; }
 template <int NMAX, int DEG, int MODE, bool EXACT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, EXACT))))
+__global__ __launch_bounds__(block_threads(NMAX, EXACT)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, EXACT))))
 void track_kernel(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int lane = (int)threadIdx.x & 63;
@@ -1308,7 +1311,7 @@ void track_kernel(const Launch LN) {
 // Latency instance: FP64 launches of one segment and few paths, R replicas
 // per path (1: the launch's number).
 template <int NMAX, int DEG, bool EXACT, int R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, false))))
+__global__ __launch_bounds__(block_threads(NMAX, false)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, false))))
 void track_kernel_rep(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
   run_segment_fp64<NMAX, DEG, EXACT, R>(LN, 0, smem, (int)threadIdx.x & 63);
