@@ -213,6 +213,75 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
   }
 }
 
+// The same with the columns dealt out: replica s of R sums columns s, s + R, ...
+// whole (B[i]: column R i + s; past the last column, 0), each in the order of
+// its stream, so the sums are those of one replica.  p, end: the lane's place
+// in each of its columns and their zero terms.
+template <int NMAX, int DEG, int R, int NC, class SegT>
+__device__ __forceinline__ void eval_jac_dealt(const SegT& S, int n, int gle, int s, const unsigned char* xb,
+                                               const unsigned char* cb, cx<double> (&B)[NC],
+                                               const unsigned char* lt) {
+  constexpr int RS = LatencyRec<DEG>::kJ;
+  constexpr int NB = NC <= 5 ? NC : (NC + 1) / 2;  // columns at a time
+  const int rounds_end = S.max_terms, row = n * RS;
+  int p[NC], end[NC], off = gle * RS;
+  const int none = off + (int)(S.colc[0] & 0xffffu) * row;  // zero terms of column 0
+#pragma unroll
+  for (int j = 0; j < R * NC; ++j) {
+    const int cnt = j < NMAX ? (int)(S.colc[j < NMAX ? j : 0] & 0xffffu) : 0;
+    const bool in = j < NMAX && j < n;
+    const int b = in ? off : none, z = in ? off + cnt * row : none;
+    p[j / R] = (j % R == 0 || s == j % R) ? b : p[j / R];
+    end[j / R] = (j % R == 0 || s == j % R) ? z : end[j / R];
+    off += in ? (cnt + 1) * row : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i) B[i] = cmk<double>(0, 0);
+#pragma unroll 1
+  for (int k = 0; k < rounds_end; ++k) {
+#pragma unroll
+    for (int ib = 0; ib < NC; ib += NB) {
+      uint32_t r0[NB], r1[NB], rs[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (ib + u < NC) {
+          const unsigned char* a = lt + p[ib + u];
+          if constexpr (DEG <= 2) {
+            const uint2 q = *reinterpret_cast<const uint2*>(a);
+            r0[u] = q.x;
+            rs[u] = q.y;
+          } else {
+            const uint4 q = *reinterpret_cast<const uint4*>(a);
+            r0[u] = q.x;
+            r1[u] = q.y;
+            rs[u] = q.z;
+          }
+          p[ib + u] = min(p[ib + u] + row, end[ib + u]);
+        }
+      }
+      cx<double> c[NB], x[NB];
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (ib + u < NC) {
+          c[u] = lds_lo<double>(cb, r0[u]);
+          x[u] = lds_hi<double>(xb, r0[u]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
+#pragma unroll
+      for (int u = 0; u < NB; ++u) {
+        if (ib + u < NC) {
+          cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
+          v = cmul_term(v, x[u]);
+          if constexpr (DEG > 2) v = cmul_term(v, lds_lo<double>(xb, r1[u]));
+          if constexpr (DEG > 3) v = cmul_term(v, lds_hi<double>(xb, r1[u]));
+          B[ib + u] = cadd(B[ib + u], v);
+        }
+      }
+    }
+  }
+}
+
 // One chunk of Q terms of a row of dH/dt or H, positions k, k + ks, ...
 // (positions past the last read the zero terms that end the stream).  dot:
 // this lane's group sums dc/dt (an RK4 stage) instead of c(t): from its LDS

@@ -951,8 +951,11 @@ __device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsi
 // paths, two waves per SIMD at most): 2, 4 or 8 replicas per path, which share
 // the evaluation's terms and the solve's columns, or (1) Seg::R of them, which
 // share the terms.
+// DEAL: the replicas share the columns in the evaluation as well: each sums its
+// own whole, in the order of one replica, and all of them the right-hand side.
+// 142 paths of each of 64 instances of n = 9, R = 2: 3.46 -> 3.03 ms.
 // NB: Jacobian columns evaluated together (as the register budget allows).
-template <int NMAX, int DEG, bool EXACT, int REP, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
+template <int NMAX, int DEG, bool EXACT, int REP, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6)), bool DEAL = false>
 __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsigned char* smem, int lane) {
   Seg S = LN.seg[si];
   constexpr int GE = exact_lanes(NMAX);
@@ -966,7 +969,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   int iter = 0;
   const Group g = make_group(S.G, lane, REP > 1 ? REP : (REP ? S.R : 1));
   // the replica's terms of each sum
-  const int k0 = REP ? g.s : 0, ks = REP > 1 ? REP : (REP ? g.R : 1);
+  const int k0 = REP && !DEAL ? g.s : 0, ks = DEAL ? 1 : (REP > 1 ? REP : (REP ? g.R : 1));
   const int n = S.n;
   const bool row = g.in_grp && g.gl < n;
   const int gle = row ? g.gl : 0;
@@ -1123,12 +1126,16 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       }
       publish_x<double>(sx, xe, g, n, act, row);
       HCX_WAVE_SYNC();
-      cx<double> A[NMAX];
+      constexpr int NC = REP > 1 ? (NMAX + REP) / REP : 1;  // columns of a replica (the right-hand side's included)
+      cx<double> A[NMAX], B[NC];
       cx<double> r;
-      if (LT || (!EXACT && lt)) {
+      if (DEAL || LT || (!EXACT && lt)) {
         constexpr bool kPin = REP > 0 || NMAX > 6;
         if constexpr (REP) {
-          eval_jac_rounds<NMAX, DC>(Sk, n, gle, xb, cb, A, lt, k0, ks);
+          if constexpr (DEAL)
+            eval_jac_dealt<NMAX, DC, REP, NC>(Sk, n, gle, g.s, xb, cb, B, lt);
+          else
+            eval_jac_rounds<NMAX, DC>(Sk, n, gle, xb, cb, A, lt, k0, ks);
           if (Sk.htT <= 2 * ks)
             r = eval_rhs_stream<DC, false, 2, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
@@ -1153,15 +1160,19 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       bool sing;
       cx<double> d;
       if constexpr (REP > 1) {
-        // each replica summed every R-th term of the row's sums
-        cx<double> V[NMAX + 1], B[(NMAX + REP) / REP];
+        cx<double>& rb = B[NMAX / REP];  // (the right-hand side: in replica NMAX % REP)
+        if constexpr (DEAL) {
+          if (g.s == NMAX % REP) rb = stg ? cmk<double>(-r.re, -r.im) : r;
+        } else {
+          // each replica summed every R-th term of the row's sums
+          cx<double> V[NMAX + 1];
 #pragma unroll
-        for (int j = 0; j < NMAX; ++j) V[j] = A[j];
-        V[NMAX] = r;
-        reduce_scatter<REP>(V, B, g, lane);
-        cx<double>& rb = B[NMAX / REP];
-        r = rb;  // (in replica NMAX % REP)
-        if (stg && g.s == NMAX % REP) rb = cmk<double>(-rb.re, -rb.im);
+          for (int j = 0; j < NMAX; ++j) V[j] = A[j];
+          V[NMAX] = r;
+          reduce_scatter<REP>(V, B, g, lane);
+          r = rb;
+          if (stg && g.s == NMAX % REP) rb = cmk<double>(-rb.re, -rb.im);
+        }
         d = group_solve_split<NMAX, REP>(B, g, n, row, L.piv64(), L.keys(), cols, cols + REP * g.G, sing);
       } else {
         if constexpr (REP == 1) {
@@ -1255,7 +1266,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
       const bool rz = pe == kPhResid;
       if (__any(rz)) {
         // the replica that holds the right-hand side's column has the sums
-        if constexpr (REP > 1) r = lane_read(r, g.wbase + (NMAX % REP) * g.G + g.gl);
+        if constexpr (REP > 1 && !DEAL) r = lane_read(r, g.wbase + (NMAX % REP) * g.G + g.gl);
         double rr = (rz && row) ? sqrt(cnorm2(r)) : 0.0;
         if (rr != rr) rr = INFINITY;
         rr = group_max(rr, g);
@@ -1310,11 +1321,11 @@ void track_kernel(const Launch LN) {
 
 // Latency instance: FP64 launches of one segment and few paths, R replicas
 // per path (1: the launch's number).
-template <int NMAX, int DEG, bool EXACT, int R>
+template <int NMAX, int DEG, bool EXACT, int R, bool DEAL = false>
 __global__ __launch_bounds__(block_threads(NMAX, false)) __attribute__((amdgpu_waves_per_eu(waves_per_simd(NMAX, false))))
 void track_kernel_rep(const Launch LN) {
   extern __shared__ __align__(16) unsigned char smem[];
-  run_segment_fp64<NMAX, DEG, EXACT, R>(LN, 0, smem, (int)threadIdx.x & 63);
+  run_segment_fp64<NMAX, DEG, EXACT, R, 4, DEAL>(LN, 0, smem, (int)threadIdx.x & 63);
 }
 
 // One launch over segments of different sizes (uneven batches): segment s
@@ -1409,6 +1420,10 @@ HCX_REP_UNITS(2)
 HCX_REP_UNITS(4)
 HCX_REP_UNITS(8)
 #undef HCX_REP_UNITS
+// The same with the evaluation dealt out by columns (DEAL), R = 2 and 4, for
+// terms of degree <= 3.
+KernelFn kernel_deal_x(int n, int deg, int R);
+KernelFn kernel_deal_g(int nmax, int deg, int R);
 KernelFn kernel_rep_g16_r1(int deg);
 KernelFn kernel_rep_g16_r2(int deg);
 KernelFn kernel_rep_g16_r4(int deg);

@@ -313,6 +313,11 @@ static KernelFn pick_kernel(int nmax, int deg, int mode) {
   }
 }
 
+// The latency instance of R replicas with the columns dealt out (nullptr: none).
+static KernelFn pick_deal(int nmax, int deg, bool exact, int R) {
+  return exact ? kernel_deal_x(nmax, deg, R) : kernel_deal_g(nmax, deg, R);
+}
+
 // The latency instance of R replicas (nullptr: none).  Numbers of replicas
 // that have no instance of their own run on R = 1's, which takes any.
 static KernelFn pick_rep(int nmax, int deg, bool exact, int R) {
@@ -537,6 +542,58 @@ long long table_bytes(const hcx_problem* p, bool t4) {
 // LDS per workgroup on gfx950
 constexpr int kMaxLdsBytes = 160 * 1024;
 
+// Waves of `wave` bytes of LDS that fit a CU at once, blocks of any number of
+// waves (at most cap) sharing `tab` bytes.
+int resident_waves(size_t tab, size_t wave, int cap) {
+  int w = 0;
+  for (int wpb = 1; wpb <= cap; ++wpb) w = std::max(w, (int)(kMaxLdsBytes / (tab + wpb * wave)) * wpb);
+  return std::min(w, cap);
+}
+
+// Replicas of a launch beyond those that split the term sums: the columns are
+// dealt out instead, each summed whole, so the additions are those of one
+// replica.
+//
+// Two replicas halve a path's step (0.45), and a launch of up to about two
+// rounds of resident waves is as long as its longest paths, so they pay past
+// the 8 waves that a CU holds: up to 16 per CU at up to 8 variables, 12 beyond
+// or where pairs leave more lanes of the wave empty than single groups do.  Throughput instance -> R = 2, us,
+// by waves at R = 1:
+//   n = 3  1300: 1615 1576  2048: 1808 1662  3000: 1432 1611
+//   n = 6  1300: 2055 2014  2048: 3272 3115  3000: 3253 3360
+//   n = 8  1296: 2673 2398  2048: 3340 3016  4096: 4211 4346
+//   n = 10 1302: 3432 3137  2048: 3833 4165
+//   n = 9   609: 2779 2275  1300: 3000 2810  2049: 3324 3615
+//   n = 12  589: 3415 3011  1306: 4165 4073  2048: 5053 5023  2996: 5620 6584
+//
+// Where LDS holds fewer waves of a CU than the registers (wide coefficient
+// tables), R with the best rate of a full chip is taken at any number of
+// waves: resident paths times the speed of their steps.  n = 16, 352
+// coefficients: 24 paths in 6 waves -> 12 in 6 at R = 2, 4100 waves 14.3 -> 13.1 ms,
+// 2050 10.4 -> 8.9; n = 10, 660 coefficients: 12 paths in 2 waves -> 7 in 7 at R = 4,
+// 4096 waves 35.1 -> 30.5 ms, 598 11.6 -> 8.6.
+template <class Region, class Waves>
+int dealt_replicas(const Seg& S, const Plan& pl, int tab, const Region& region, const Waves& waves) {
+  auto groups = [&](int R) { return 64 / (S.G * R); };
+  int R = 1;
+  if (2 * S.G <= 64 && waves(2) <= (groups(1) <= 2 * groups(2) && S.n <= 8 ? 16LL : 12LL) * g_cu) R = 2;
+  const int cap = 4 * waves_per_simd(pl.nmax, pl.exact), capr = 4 * waves_per_simd(pl.nmax, false);
+  const int w1 = resident_waves((size_t)pl.tab_lds, (size_t)groups(1) * S.lds_group, cap);
+  if (w1 < cap) {
+    const double speed[] = {1.0, 2.2, 2.9};
+    double best = groups(1) * w1;
+    for (int i = 1; i < 3 && (S.G << i) <= 64; ++i) {
+      const double rate = speed[i] * groups(1 << i) *
+                          resident_waves((size_t)tab, (size_t)groups(1 << i) * region(1 << i), capr);
+      if (rate > best) {
+        best = rate;
+        R = std::max(R, 1 << i);
+      }
+    }
+  }
+  return R;
+}
+
 // Kernel instance for a launch: the size-specialised one when every segment
 // has the same n, runs its lanes per path (G = exact_lanes(n)) and fits
 // DEG <= 3 (and, for
@@ -604,9 +661,7 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
     const auto& c = probs[0]->ctab[pl.tab4 ? 0 : 1];
     const size_t wave = (size_t)(64 / Gs[0]) * (size_t)pl.group_bytes(probs[0]), tb = (size_t)c.words * 4;
     const int cap = pl.nmax == 32 ? 4 : 8;
-    int with = 0;
-    for (int wpb = 1; wpb <= cap; ++wpb) with = std::max(with, (int)(kMaxLdsBytes / (tb + wpb * wave)) * wpb);
-    if (c.d && tb <= (size_t)kMaxTabLds && std::min(with, cap) >= std::min((int)(kMaxLdsBytes / wave), cap)) {
+    if (c.d && tb <= (size_t)kMaxTabLds && resident_waves(tb, wave, cap) >= std::min((int)(kMaxLdsBytes / wave), cap)) {
       pl.tab_lds = (int)tb;
     }
   }
@@ -1358,25 +1413,29 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     seg_groups[s] = (S.P + gpw - 1) / gpw;
     total_groups_needed += seg_groups[s];
   }
-  // A one-segment FP64 launch of at most one wave per SIMD is latency bound:
-  // no other waves hide the latency of its evaluations.  It runs the latency
-  // instance of its size when one exists; dc/dt goes to LDS next to c(t),
-  // the generic instances read their Term records from an LDS copy, and
-  // each path gets R replicas of its lane group, which split the
-  // evaluation's term sums (the most, a power of two up to 8 with R * G <=
-  // 64, that keep the launch within two waves per SIMD, or half of one above
-  // R = 2 for light rows; or o->replicas).  All of it only when the group
-  // regions and the records fit in 64 KiB.
-  if (o->precision == HCX_PREC_FP64 && nseg == 1 && (total_groups_needed <= 4LL * g_cu || o->replicas > 1)) {
+  // One-segment FP64 launches of few waves are latency bound: no other waves
+  // hide the latency of their evaluations and solves.  They run the latency
+  // instance of their size: dc/dt in LDS next to c(t), tables laid out for it,
+  // and R replicas of each path's lane group.  In launches of at most one
+  // wave per SIMD (or with o->replicas) the replicas split the evaluation's term
+  // sums and the solve's columns (the most, a power of two up to 8 with R * G
+  // <= 64, that keep the launch within two waves per SIMD, or half of one above
+  // R = 2 for light rows), when the group regions and the records fit in 64 KiB.
+  // R = 1 takes up to one and a half waves per SIMD (1300 waves: n = 6 2274 -> 2053
+  // us, n = 12 4371 -> 4039; at 2048 waves n = 9 loses, 3356 -> 3801).
+  if (o->precision == HCX_PREC_FP64 && nseg == 1) {
     Seg& S = LN.seg[0];
     const hcx_problem* p = probs[0];
+    const auto& lat = p->ltab[pl.tab4 ? 0 : 1];
     const int lg = pl.group_bytes(p, true);
     const size_t terms =
         pl.exact ? 0 : ((size_t)p->hx_recs + (size_t)p->n * p->htT) * sizeof(dev::Term);
-    auto waves = [&](int R) {
-      const long long gpw = 64 / (S.G * R);
-      return (S.P + gpw - 1) / gpw;
-    };
+    Plan lp = pl;
+    lp.latency = true;
+    auto region = [&](int R) { return ((lp.group_bytes(p, true) + dev::split_bytes(pl.nmax, S.G, R)) / 16 | 1) * 16; };
+    auto groups = [&](int R) { return 64 / (S.G * R); };
+    auto waves = [&](int R) { return (S.P + groups(R) - 1) / groups(R); };
+    const long long w1 = total_groups_needed;
     int R = 1;
     if (o->replicas > 0) {
       R = o->replicas;
@@ -1384,14 +1443,11 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
         set_error("track: %d replicas of %d lanes exceed a wave", R, S.G);
         return HCX_ERR_INVALID_ARG;
       }
-    } else {
+    } else if (w1 <= 4LL * g_cu) {
       // at most 8 replicas; beyond 2 and half a wave per SIMD only for rows
-      // whose evaluation outweighs the butterfly (complex products per row
-      // >= 8 per exchanged sum).  Measured: 583 paths of 46 quadratic terms
-      // per row ran slower at R = 4 than at R = 2, 668 paths of 84 cubic
-      // terms faster, 4,096 paths of a light n = 6 type faster at R = 2 (820
-      // waves) than at R = 1, and 2,560 paths at n = 16 faster at R = 2
-      // (1,280 waves) than at R = 1
+      // whose evaluation outweighs the exchange (complex products per row
+      // >= 8 per exchanged sum).  The number of replicas is part of the order
+      // in which a row's terms are added.
       const int dg = std::max(p->deg, 1);
       const double row_products = (double)p->n * p->hxT * (dg - 1) + (double)p->htT_padded * dg;
       const bool heavy = row_products >= 8.0 * (p->n + 1);
@@ -1400,21 +1456,34 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
         R *= 2;
     }
     // the latency instance, also for R = 1
-    const KernelFn rf = pick_rep(pl.nmax, pl.deg, pl.exact, R);
+    const bool one = w1 <= 6LL * g_cu;
+    const KernelFn rf = one || R > 1 ? pick_rep(pl.nmax, pl.deg, pl.exact, R) : nullptr;
     if (!rf) R = 1;
-    const size_t regions = (size_t)(64 / (S.G * R)) * (size_t)lg;
+    const size_t regions = (size_t)groups(R) * (size_t)lg;
     // the rule counts the compact tables of the size-specialised instances at 4
     // or 8 bytes a term, and the full records of the generic ones, which read
     // compact tables where they fit as well
-    const auto& lat = p->ltab[pl.tab4 ? 0 : 1];
     const bool compact = pl.exact ? pl.tab_lds > 0 : rf && lat.d && lat.words * 4 <= 65536;
     size_t tab = 0, tab_new = terms;
     if (pl.exact && pl.tab_lds > 0) tab = (size_t)table_bytes(p, pl.tab4);
     if (compact) tab_new = (size_t)(rf ? lat.words * 4 : pl.tab_lds);
-    Plan lp = pl;
-    lp.latency = rf != nullptr;
-    const int region = ((lp.group_bytes(p, true) + dev::split_bytes(pl.nmax, S.G, R)) / 16 | 1) * 16;
-    if (regions + tab + terms <= 65536 && (size_t)(64 / (S.G * R)) * (size_t)region + tab_new <= (size_t)kMaxLdsBytes) {
+    const size_t used = (size_t)groups(R) * (size_t)(rf ? region(R) : lg) + tab_new;
+    const bool fits = (rf || one) && regions + tab + terms <= 65536 && used <= (size_t)kMaxLdsBytes;
+    int deal = 1;
+    if ((!fits || R == 1) && o->replicas == 0 && pl.nmax <= 16 && (pl.exact ? pl.tab_lds > 0 : lat.d != nullptr))
+      deal = dealt_replicas(S, pl, lat.words * 4, region, waves);
+    const KernelFn df = deal > 1 ? pick_deal(pl.nmax, pl.deg, pl.exact, deal) : nullptr;
+    if (df && (size_t)groups(deal) * (size_t)region(deal) + (size_t)lat.words * 4 <= (size_t)kMaxLdsBytes) {
+      LN.dot_lds = 1;
+      S.R = deal;
+      pl.fn = df;
+      pl.latency = true;
+      pl.tab_lds = lat.words * 4;
+      seg_tables(S, p, pl);
+      S.lds_group = region(deal);
+      seg_groups[0] = waves(deal);
+      total_groups_needed = seg_groups[0];
+    } else if (fits) {
       LN.dot_lds = 1;
       S.R = R;
       if (rf) {
@@ -1424,7 +1493,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
         seg_tables(S, p, pl);
         if (!compact) S.ctab = nullptr;
       }
-      S.lds_group = rf ? region : lg;
+      S.lds_group = rf ? region(R) : lg;
       seg_groups[0] = waves(R);
       total_groups_needed = seg_groups[0];
     }
