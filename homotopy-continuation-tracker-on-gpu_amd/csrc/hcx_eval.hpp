@@ -68,12 +68,12 @@ __device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
 // of each, the zero term past a column's last (SC: a scaled position).  All
 // records are requested together, then all gathers.  off: byte offset of the
 // first column's positions from rp; zero: that of the zero terms.
-template <int NMAX, int DEG, bool SC, int JB, int NB, class T>
+template <int NMAX, int DEG, bool SC, int JB, int NB, bool PIN, class T>
 __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int off, int zero, const int (&cnt)[NB],
                                           int k, const unsigned char* xb, const unsigned char* cb, cx<T> (&A)[NMAX]) {
   constexpr int RS = StreamRec<DEG>::kJ;
   uint32_t r0[NB], r1[NB];
-  cx<T> c[NB], p[NB];
+  cx<T> c[NB], p[NB], p1[NB], p2[NB];
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
@@ -94,16 +94,20 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int of
     if (JB + u < NMAX) {
       c[u] = lds_lo<T>(cb, r0[u]);
       p[u] = lds_hi<T>(xb, r0[u]);
+      if constexpr (DEG > 2) p1[u] = lds_lo<T>(xb, r1[u]);
+      if constexpr (DEG > 3) p2[u] = lds_hi<T>(xb, r1[u]);
     }
   }
+  // PIN: all gathers before the first product
+  if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
       cx<T> v = c[u];
       if constexpr (SC) v = cscale(v, (T)rec_scalar<DEG>(r0[u], r1[u]));
       v = cmul_term(v, p[u]);
-      if constexpr (DEG > 2) v = cmul_term(v, lds_lo<T>(xb, r1[u]));
-      if constexpr (DEG > 3) v = cmul_term(v, lds_hi<T>(xb, r1[u]));
+      if constexpr (DEG > 2) v = cmul_term(v, p1[u]);
+      if constexpr (DEG > 3) v = cmul_term(v, p2[u]);
       A[JB + u] = cadd(A[JB + u], v);
     }
   }
@@ -113,7 +117,7 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int of
 // (dev-eval-indxing-generalized_3views_4pts.cuh:70-86), NB columns at a time:
 // one column after the other, each term is two exposed LDS latencies and each
 // column two loops.
-template <int NMAX, int DEG, int NB, int JB, class T, class SegT>
+template <int NMAX, int DEG, int NB, int JB, bool PIN, class T, class SegT>
 __device__ __forceinline__ void eval_jac_blocks(const SegT& S, int n, const unsigned char* rp, int off,
                                                 const unsigned char* xb, const unsigned char* cb,
                                                 cx<T> (&A)[NMAX]) {
@@ -134,10 +138,10 @@ __device__ __forceinline__ void eval_jac_blocks(const SegT& S, int n, const unsi
     const int zero = S.hx_recs * StreamRec<DEG>::kJ;
     int k = 0;
 #pragma unroll 1
-    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB, T>(rp, n, off, zero, cnt, k, xb, cb, A);
+    for (; k < scaled; ++k) jac_round<NMAX, DEG, true, JB, NB, PIN, T>(rp, n, off, zero, cnt, k, xb, cb, A);
 #pragma unroll 1
-    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB, T>(rp, n, off, zero, cnt, k, xb, cb, A);
-    eval_jac_blocks<NMAX, DEG, NB, JB + NB, T>(S, n, rp, off + tot * (n * StreamRec<DEG>::kJ), xb, cb, A);
+    for (; k < end; ++k) jac_round<NMAX, DEG, false, JB, NB, PIN, T>(rp, n, off, zero, cnt, k, xb, cb, A);
+    eval_jac_blocks<NMAX, DEG, NB, JB + NB, PIN, T>(S, n, rp, off + tot * (n * StreamRec<DEG>::kJ), xb, cb, A);
   }
 }
 
@@ -190,12 +194,14 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
           rp += (cnt + (jb + u < n ? 1 : 0)) * (n * RS);
         }
       }
-      cx<double> c[NB], p[NB];
+      cx<double> c[NB], p[NB], p1[NB], p2[NB];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
           c[u] = lds_lo<double>(cb, r0[u]);
           p[u] = lds_hi<double>(xb, r0[u]);
+          if constexpr (DEG > 2) p1[u] = lds_lo<double>(xb, r1[u]);
+          if constexpr (DEG > 3) p2[u] = lds_hi<double>(xb, r1[u]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
@@ -204,8 +210,8 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
         if (jb + u < NMAX) {
           cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
           v = cmul_term(v, p[u]);
-          if constexpr (DEG > 2) v = cmul_term(v, lds_lo<double>(xb, r1[u]));
-          if constexpr (DEG > 3) v = cmul_term(v, lds_hi<double>(xb, r1[u]));
+          if constexpr (DEG > 2) v = cmul_term(v, p1[u]);
+          if constexpr (DEG > 3) v = cmul_term(v, p2[u]);
           A[jb + u] = cadd(A[jb + u], v);
         }
       }
@@ -259,12 +265,14 @@ __device__ __forceinline__ void eval_jac_dealt(const SegT& S, int n, int gle, in
           p[ib + u] = min(p[ib + u] + row, end[ib + u]);
         }
       }
-      cx<double> c[NB], x[NB];
+      cx<double> c[NB], x[NB], x1[NB], x2[NB];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (ib + u < NC) {
           c[u] = lds_lo<double>(cb, r0[u]);
           x[u] = lds_hi<double>(xb, r0[u]);
+          if constexpr (DEG > 2) x1[u] = lds_lo<double>(xb, r1[u]);
+          if constexpr (DEG > 3) x2[u] = lds_hi<double>(xb, r1[u]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
@@ -273,8 +281,8 @@ __device__ __forceinline__ void eval_jac_dealt(const SegT& S, int n, int gle, in
         if (ib + u < NC) {
           cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
           v = cmul_term(v, x[u]);
-          if constexpr (DEG > 2) v = cmul_term(v, lds_lo<double>(xb, r1[u]));
-          if constexpr (DEG > 3) v = cmul_term(v, lds_hi<double>(xb, r1[u]));
+          if constexpr (DEG > 2) v = cmul_term(v, x1[u]);
+          if constexpr (DEG > 3) v = cmul_term(v, x2[u]);
           B[ib + u] = cadd(B[ib + u], v);
         }
       }
@@ -308,12 +316,14 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
       r[q][2] = v.z;
     }
   }
-  cx<T> x0[Q], x1[Q];
+  cx<T> x0[Q], x1[Q], x2[Q], x3[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     c[q] = lds_lo<T>(cb, r[q][0]);
     x0[q] = lds_hi<T>(xb, r[q][0]);
     x1[q] = lds_lo<T>(xb, r[q][1]);
+    if constexpr (DEG > 2) x2[q] = lds_hi<T>(xb, r[q][1]);
+    if constexpr (DEG > 3) x3[q] = lds_lo<T>(xb, r[q][2]);
   }
   if constexpr (GDOT) {
     if (dot) {
@@ -333,8 +343,8 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
     if constexpr (SC) v = cscale(v, (T)rec_scalar<DEG>(r[q][0], r[q][1]));
     v = cmul_term(v, x0[q]);
     v = cmul_term(v, x1[q]);
-    if constexpr (DEG > 2) v = cmul_term(v, lds_hi<T>(xb, r[q][1]));
-    if constexpr (DEG > 3) v = cmul_term(v, lds_lo<T>(xb, r[q][2]));
+    if constexpr (DEG > 2) v = cmul_term(v, x2[q]);
+    if constexpr (DEG > 3) v = cmul_term(v, x3[q]);
     acc = cadd(acc, v);
   }
   return acc;
@@ -361,9 +371,12 @@ __device__ __forceinline__ cx<T> eval_rhs_stream(const SegT& S, int n, int gle, 
 
 // sum over positions k0, k0 + ks, ... < cnt of a stream of full Term records
 // (n apart from tp; global memory or an LDS copy).  The records of a chunk
-// are requested before the first is used.  GDOT: lanes with dot take dc/dt
+// are requested before the first is used.  CLAMP (records in global memory):
+// past the last position that position again, not added, so a chunk has no
+// branches; from LDS, where a record costs little, the branches are cheaper than
+// the products.  GDOT: lanes with dot take dc/dt
 // from global memory (dg, indexed by the coefficient numbers ci).
-template <int NV, bool GDOT, class T>
+template <int NV, bool GDOT, bool CLAMP, class T>
 __device__ __forceinline__ cx<T> term_stream_sum(const Term* tp, int cnt, int n, const cx<T>* sx,
                                                       const cx<T>* coef, const double2* dg, const int* ci,
                                                       bool dot, int k0, int ks) {
@@ -373,30 +386,35 @@ __device__ __forceinline__ cx<T> term_stream_sum(const Term* tp, int cnt, int n,
     int cj[kTermChunk];
     cx<T> c[kTermChunk];
 #pragma unroll
-    for (int q = 0; q < kTermChunk; ++q)
-      if (kb + q * ks < cnt) {
-        tm[q] = tp[(size_t)(kb + q * ks) * n];
-        if constexpr (GDOT) cj[q] = ci[(size_t)(kb + q * ks) * n];
+    for (int q = 0; q < kTermChunk; ++q) {
+      const int k = kb + q * ks;
+      const size_t at = (size_t)(CLAMP ? min(k, cnt - 1) : k) * n;
+      if (CLAMP || k < cnt) {
+        tm[q] = tp[at];
+        if constexpr (GDOT) cj[q] = ci[at];
       }
+    }
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q)
-      if (kb + q * ks < cnt) {
-        c[q] = coef[tm[q].c];
-        if constexpr (GDOT) {
-          if (dot) {
+      if (CLAMP || kb + q * ks < cnt) c[q] = coef[tm[q].c];
+    if constexpr (GDOT) {
+      if (dot) {
+#pragma unroll
+        for (int q = 0; q < kTermChunk; ++q)
+          if (CLAMP || kb + q * ks < cnt) {
             const double2 d = dg[cj[q]];
             c[q] = cmk<T>((T)d.x, (T)d.y);
           }
-        }
       }
+    }
 #pragma unroll
     for (int q = 0; q < kTermChunk; ++q) {
-      if (kb + q * ks < cnt) {
-        cx<T> v = cscale(c[q], (T)tm[q].s);
+      if (!CLAMP && kb + q * ks >= cnt) continue;
+      cx<T> v = cscale(c[q], (T)tm[q].s);
 #pragma unroll
-        for (int d = 0; d < NV; ++d) v = cmul_term(v, sx[term_var(tm[q], d)]);
-        acc = cadd(acc, v);
-      }
+      for (int d = 0; d < NV; ++d) v = cmul_term(v, sx[term_var(tm[q], d)]);
+      const cx<T> sum = cadd(acc, v);
+      if (kb + q * ks < cnt) acc = sum;
     }
   }
   return acc;
@@ -420,9 +438,9 @@ __device__ __forceinline__ void eval_jac_terms(const SegT& S, int n, int gle, co
         cnt = (int)(S.colc[j] & 0xffffu);
       }
       if (tl)
-        acc = term_stream_sum<DEG - 1, false, T>(tl + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
+        acc = term_stream_sum<DEG - 1, false, false, T>(tl + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
       else
-        acc = term_stream_sum<DEG - 1, false, T>(S.hx + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
+        acc = term_stream_sum<DEG - 1, false, true, T>(S.hx + off, cnt, n, sx, sc, nullptr, nullptr, false, k0, ks);
       off += (size_t)cnt * n;
     }
     A[j] = acc;
@@ -435,8 +453,8 @@ __device__ __forceinline__ cx<T> eval_rhs_terms(const SegT& S, int n, int gle, c
                                                      const cx<T>* base, const double2* dg, bool dot,
                                                      const Term* tl, int k0, int ks) {
   const int* ci = S.ht_ci + gle;
-  if (tl) return term_stream_sum<DEG, GDOT, T>(tl + (size_t)S.hx_recs + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
-  return term_stream_sum<DEG, GDOT, T>(S.ht + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
+  if (tl) return term_stream_sum<DEG, GDOT, false, T>(tl + (size_t)S.hx_recs + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
+  return term_stream_sum<DEG, GDOT, true, T>(S.ht + gle, S.htT, n, sx, base, dg, ci, dot, k0, ks);
 }
 
 // ------------------------------------------------------------ staging

@@ -627,7 +627,7 @@ __device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, cons
   constexpr int DC = DEG <= 4 ? DEG : 4;
   if (LT || lt) {
     constexpr int HQ = NMAX <= 6 && sizeof(T) == 8 ? 2 : 4;
-    eval_jac_blocks<NMAX, DC, NB, 0, T>(S, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
+    eval_jac_blocks<NMAX, DC, NB, 0, !LT && sizeof(T) == 4, T>(S, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
     return eval_rhs_stream<DC, false, HQ, (NMAX > 6), T>(S, n, gle, xb, rhs, rhs, nullptr, false, lt, 0, 1);
   }
   if constexpr (!LT) {
@@ -662,7 +662,7 @@ __device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsi
   } else if constexpr (!EXACT) {
     if (LN.tab_lds > 0) lt = static_cast<const unsigned char*>(stage_tables(S, smem));
   }
-  constexpr int SQ = EXACT && NMAX <= 16 ? 4 : 2;  // coefficients in flight per lane while staging
+  constexpr int SQ = NMAX <= 16 ? 4 : 2;  // coefficients in flight per lane while staging
   constexpr bool SL = LT && NMAX <= 16;
   const int wv = (int)threadIdx.x >> 6;  // wave of the block
   Lds<NMAX, GC == 0> L{smem + LN.tab_lds + ((size_t)wv * g.gpw + (g.in_grp ? g.grp : 0)) * S.lds_group};
@@ -1142,7 +1142,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
             r = eval_rhs_stream<DC, false, 4, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         } else {
           constexpr int HQ = NMAX <= 6 ? 2 : 4;  // H terms in flight
-          eval_jac_blocks<NMAX, DC, NB, 0, double>(Sk, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
+          eval_jac_blocks<NMAX, DC, NB, 0, false, double>(Sk, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
           if (gdot)
             r = eval_rhs_stream<DC, true, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else

@@ -655,13 +655,16 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
   pl.deg = kDegList[di];
   pl.exact = false;
   if (nseg == 1 && pl.fn) {
-    // a generic instance reads the compact streams from LDS where they
-    // leave as many waves on a CU as its registers allow (one per SIMD for
-    // NMAX 32, else two) or as there were without them
+    // a generic instance reads the compact streams from LDS where they take at
+    // most 64 KiB and leave half the waves that a CU holds without them (its
+    // registers allow one per SIMD for NMAX 32, else two): the records in
+    // global memory cost more than half the waves.  1024 waves, ms, global -> LDS:
+    // n = 7, degree 4, mixed (7 -> 6 waves) 19.3 -> 9.0; n = 18, 1080 coefficients (3 -> 2)
+    // 37.8 -> 20.4; n = 28, 1680 coefficients (3 -> 2) 49.4 -> 29.1.
     const auto& c = probs[0]->ctab[pl.tab4 ? 0 : 1];
     const size_t wave = (size_t)(64 / Gs[0]) * (size_t)pl.group_bytes(probs[0]), tb = (size_t)c.words * 4;
     const int cap = pl.nmax == 32 ? 4 : 8;
-    if (c.d && tb <= (size_t)kMaxTabLds && resident_waves(tb, wave, cap) >= std::min((int)(kMaxLdsBytes / wave), cap)) {
+    if (c.d && tb <= 65536 && 2 * resident_waves(tb, wave, cap) >= resident_waves(0, wave, cap)) {
       pl.tab_lds = (int)tb;
     }
   }
