@@ -87,8 +87,8 @@ typedef struct {
                              ZERO_IMAG_PART_TOL_FOR_SP = 1e-4 (definitions.hpp:25, Evaluations.cpp:96-104) */
   int replicas;           /* FP64, one-segment launches on sizes with a latency instance: R copies of each
                              path's lane group, each summing every R-th term of the evaluation (a power of
-                             two, R * lanes <= 64); 0 = automatic (launches of at most one wave per SIMD),
-                             1 = off */
+                             two, R * lanes <= 64); 0 = automatic (launches of at most one wave per SIMD;
+                             larger ones may share columns, which changes no bit), 1 = off */
 } hcx_track_opts;
 
 void hcx_track_opts_default(hcx_track_opts* o);
