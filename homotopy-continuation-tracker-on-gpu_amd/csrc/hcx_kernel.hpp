@@ -53,7 +53,7 @@ struct LaunchWork {
   SegOut* out;
   int* inst_left;              // capacity inst_cap
   int* plist;                  // re-track path list (capacity plist_cap)
-  unsigned int* plist_count;   // [1]
+  unsigned int* plist_count;   // [2], one per round of the re-track pass
   long long inst_cap;
   long long plist_cap;
 };
@@ -89,8 +89,8 @@ struct Seg {
   const uint32_t* ctab;        // compact tables (instances that hold the streams in LDS)
   unsigned int* counter;
   const SegOut* out;           // device copy written by init_kernel
-  const int* plist;            // optional: track only these paths (count in *plist_count)
-  const unsigned int* plist_count;
+  int* plist;                  // optional: track only these paths (count in *plist_count)
+  unsigned int* plist_count;   // mixed: set in the first launch too, whose set-up clears the counts
 };
 
 struct Opts {

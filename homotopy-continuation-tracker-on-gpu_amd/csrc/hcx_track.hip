@@ -38,8 +38,9 @@ struct OutPack {
   SegOut out[kMaxSeg];
 };
 
-// Launch set-up on the device (graph-safe, no memset): path queues,
-// per-instance remaining-path counters, output descriptors, start stamp.
+// Launch set-up on the device (graph-safe, no memset): path queues, lengths of
+// the re-track lists, per-instance remaining-path counters, output
+// descriptors, start stamp.
 __global__ void init_kernel(const Launch LN, const OutPack OP, unsigned long long* batch_start) {
   const int s = blockIdx.y;
   if (s >= LN.nseg) return;
@@ -48,6 +49,7 @@ __global__ void init_kernel(const Launch LN, const OutPack OP, unsigned long lon
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) {
     *S.counter = 0u;
+    if (S.plist_count) S.plist_count[0] = S.plist_count[1] = 0u;
     *const_cast<SegOut*>(S.out) = O;
   }
   if (O.inst_left && i < S.I) O.inst_left[i] = S.K;
@@ -252,47 +254,45 @@ __global__ void collect_kernel(int n, int K, const double2* __restrict__ roots, 
   atomicAdd(&counts[6], c_rref);
 }
 
-// Lists the paths of a mixed-precision launch that the FP64 pass re-tracks
-// from t = 0: every path without a refined root that the launch did not
-// already re-track in FP64 (precision escalation) and, when mark_dups is set,
-// every refined path whose root equals another refined root of the same
-// instance (|dRe|, |dIm| < tol in every coordinate): a path that jumped onto
-// another path's root shares that root.  The listed paths are appended to
-// plist.  One block per instance.
-__global__ void dup_mark_kernel(int n, int K, const double2* __restrict__ roots, const uint32_t* __restrict__ flags,
-                                double tol, int mark_dups, int* __restrict__ plist,
-                                unsigned int* __restrict__ count) {
-  const int inst = blockIdx.x;
-  const size_t base = (size_t)inst * K;
-  for (int j = threadIdx.x; j < K; j += blockDim.x) {
-    const uint32_t fj = flags[base + j];
-    if (!(fj & HCX_FLAG_REFINED)) {
-      if (!(fj & HCX_FLAG_ESCALATED)) {
-        const unsigned int q = atomicAdd(count, 1u);
-        plist[q] = (int)(base + j);
-      }
-      continue;
-    }
-    if (!mark_dups) continue;
-    const double2* xj = roots + (base + j) * n;
-    bool dup = false;
-    for (int i = 0; i < K && !dup; ++i) {
-      if (i == j || !(flags[base + i] & HCX_FLAG_REFINED)) continue;
-      const double2* xi = roots + (base + i) * n;
-      bool same = true;
-      for (int v = 0; v < n && same; ++v) same = fabs(xi[v].x - xj[v].x) < tol && fabs(xi[v].y - xj[v].y) < tol;
-      dup = same;
-    }
-    if (dup) {
-      const unsigned int q = atomicAdd(count, 1u);
-      plist[q] = (int)(base + j);
-    }
-  }
+// The FP64 pass of a mixed-precision launch re-tracks paths from t = 0 in two
+// rounds, whose lists these kernels write (grid.y: the segments).  First every
+// path without a refined root (precision escalation).  Then, with the roots of
+// those in place, every refined path of mixed precision whose root equals
+// another refined root of its instance (|dRe|, |dIm| < tol in every
+// coordinate): a path that jumped onto another path's root shares that root,
+// also where the other path is one that the first round tracked.  Both kernels
+// prepare the segment's path queue and output descriptor for the launch that
+// follows (a re-tracked path does not count its instance's paths down again).
+__device__ __forceinline__ void start_retrack(const Seg& S) {
+  *S.counter = 0u;
+  const_cast<SegOut*>(S.out)->inst_left = nullptr;
 }
 
-__global__ void zero_u32_kernel(unsigned int* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0u;
+__global__ void list_unrefined_kernel(const Launch LN) {
+  const Seg& S = LN.seg[blockIdx.y];
+  const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j == 0) start_retrack(S);
+  if (j < S.P && !(S.out->flags[j] & HCX_FLAG_REFINED)) S.plist[atomicAdd(S.plist_count, 1u)] = (int)j;
+}
+
+// One block per instance.
+__global__ void list_duplicates_kernel(const Launch LN, double tol) {
+  const Seg& S = LN.seg[blockIdx.y];
+  const int inst = blockIdx.x, n = S.n, K = S.K;
+  if (inst == 0 && threadIdx.x == 0) start_retrack(S);
+  if (inst >= S.I) return;
+  const size_t base = (size_t)inst * K;
+  const uint32_t* const flags = S.out->flags + base;
+  const double2* const roots = S.out->roots + base * n;
+  for (int j = threadIdx.x; j < K; j += blockDim.x) {
+    const uint32_t fj = flags[j];
+    if (!(fj & HCX_FLAG_REFINED) || (fj & HCX_FLAG_ESCALATED)) continue;
+    const double2* xj = roots + (size_t)j * n;
+    bool dup = false;
+    for (int i = 0; i < K && !dup; ++i)
+      dup = i != j && (flags[i] & HCX_FLAG_REFINED) && same_root(roots + (size_t)i * n, xj, n, tol);
+    if (dup) S.plist[atomicAdd(S.plist_count, 1u)] = (int)(base + j);
+  }
 }
 
 __global__ void zero_u64_kernel(unsigned long long* p, int n) {
@@ -1412,6 +1412,13 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
       }
       O.inst_left = work[s].inst_left;
     }
+    if (o->precision == HCX_PREC_MIXED) {
+      if (work[s].plist_cap < S.P || !work[s].plist || !work[s].plist_count) {
+        set_error("track: launch workspace path list too small (%lld < %lld)", work[s].plist_cap, S.P);
+        return HCX_ERR_INVALID_ARG;
+      }
+      S.plist_count = work[s].plist_count;
+    }
     const int gpw = 64 / G;
     seg_groups[s] = (S.P + gpw - 1) / gpw;
     total_groups_needed += seg_groups[s];
@@ -1564,34 +1571,18 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   HIP_TRY(hipGetLastError());
 
   // Mixed precision: re-track in FP64 from t = 0 every path that ended
-  // without a refined root (precision escalation) and every path whose root
+  // without a refined root (precision escalation), then every path whose root
   // duplicates another root of its instance (a jump onto another path), so
   // the refined roots and counts are those of the FP64 tracker.
   if (o->precision == HCX_PREC_MIXED) {
     Launch L2 = LN;
     L2.persistent = 1;
     L2.wpb = 1;
-    OutPack OP2 = OP;
+    long long max_paths = 1;
     for (int s = 0; s < nseg; ++s) {
-      hcx_problem* p = probs[s];
-      Seg& S = L2.seg[s];
-      (void)p;
-      if (work[s].plist_cap < S.P || !work[s].plist || !work[s].plist_count) {
-        set_error("track: launch workspace path list too small (%lld < %lld)", work[s].plist_cap, S.P);
-        return HCX_ERR_INVALID_ARG;
-      }
-      int* plist = work[s].plist;
-      unsigned int* pcount = work[s].plist_count;
-      hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, stream, pcount, 1);
-      if (S.I > 0)
-        hipLaunchKernelGGL(dup_mark_kernel, dim3(S.I), dim3(256), 0, stream, S.n, S.K,
-                           reinterpret_cast<const double2*>(results[s].d_roots), results[s].d_flags, o->unique_tol,
-                           o->retrack_duplicates, plist, pcount);
-      S.plist = plist;
-      S.plist_count = pcount;
-      OP2.out[s].inst_left = nullptr;
+      L2.seg[s].plist = work[s].plist;
+      max_paths = std::max(max_paths, L2.seg[s].P);
     }
-    HIP_TRY(hipGetLastError());
     Plan p2;
     st = choose_kernel(nseg, probs, Gs, max_deg, HCX_PREC_FP64, specialize, p2);
     if (st != HCX_OK) return st;
@@ -1616,8 +1607,14 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
       b2 += std::max<long long>(1, std::min<long long>((L2.seg[s].P + gpw - 1) / gpw, g_cu / nseg + 1));
     }
     L2.first_block[nseg] = (int)b2;
-    hipLaunchKernelGGL(init_kernel, dim3(1, nseg), dim3(64), 0, stream, L2, OP2, (unsigned long long*)nullptr);
+    hipLaunchKernelGGL(list_unrefined_kernel, dim3((unsigned)((max_paths + 255) / 256), nseg), dim3(256), 0, stream,
+                       L2);
     hipLaunchKernelGGL(p2.fn, dim3((unsigned)b2), dim3(64), p2.lds, stream, L2);
+    if (o->retrack_duplicates) {
+      for (int s = 0; s < nseg; ++s) ++L2.seg[s].plist_count;
+      hipLaunchKernelGGL(list_duplicates_kernel, dim3(max_inst, nseg), dim3(256), 0, stream, L2, o->unique_tol);
+      hipLaunchKernelGGL(p2.fn, dim3((unsigned)b2), dim3(64), p2.lds, stream, L2);
+    }
     HIP_TRY(hipGetLastError());
   }
   return HCX_OK;

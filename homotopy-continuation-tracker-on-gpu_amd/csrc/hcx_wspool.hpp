@@ -41,7 +41,7 @@
 namespace hcx {
 
 // Fixed part of every workspace block: kSegSlots segments x 64 counter words
-// (word 0 the path queue, word 32 the re-track list length), then the
+// (word 0 the path queue, words 32 and 33 the re-track list lengths), then the
 // device copies of the segment output descriptors.
 constexpr int kSegSlots = 8;
 constexpr size_t kCounterBytes = (size_t)kSegSlots * 64 * sizeof(uint32_t);
