@@ -16,6 +16,13 @@ using cd = std::complex<double>;
 void set_error(const char* fmt, ...);
 void clear_error();
 
+// Shape of the calling thread's latest tracking launch: replicas per path (and
+// whether they hold whole columns), waves per block, blocks, blocks of the FP64
+// pass of mixed precision.  Read by the tests through hcx_internal_launch_shape.
+struct LaunchShape {
+  int replicas, dealt, waves_per_block, blocks, pass_blocks;
+};
+
 inline cd to_cd(hcx_complex z) { return cd(z.re, z.im); }
 inline hcx_complex to_hc(cd z) { return hcx_complex{z.real(), z.imag()}; }
 

@@ -969,6 +969,14 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   const KSeg* const seg_arg = launch_seg(si);
   int iter = 0;
   const Group g = make_group(S.G, lane, REP > 1 ? REP : (REP ? S.R : 1));
+  if constexpr (REP == 0) {
+    // a list with too few paths for this wave (persistent launches of one-wave
+    // blocks; each segment's first waves cover its list)
+    if (S.plist) {
+      const int rel = (int)blockIdx.x - LN.first_block[si], paths = (int)*S.plist_count;
+      if (rel >= (paths + g.gpw - 1) / g.gpw) return;
+    }
+  }
   // the replica's terms of each sum
   const int k0 = REP && !DEAL ? g.s : 0, ks = DEAL ? 1 : (REP > 1 ? REP : (REP ? g.R : 1));
   const int n = S.n;

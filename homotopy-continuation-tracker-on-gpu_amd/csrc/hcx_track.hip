@@ -1287,6 +1287,8 @@ hcx_status hcx_stream_release(void* stream) {
 }  // extern "C"
 
 namespace hcx {
+static thread_local LaunchShape g_shape;
+
 // Shared implementation of hcx_track / hcx_track_multi / graphs / the server.
 // `work` (one per segment) is the launch workspace: the stream's pooled
 // block, a graph's own block, a server slot's block or the static scratch.
@@ -1433,6 +1435,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   // R = 2 for light rows), when the group regions and the records fit in 64 KiB.
   // R = 1 takes up to one and a half waves per SIMD (1300 waves: n = 6 2274 -> 2053
   // us, n = 12 4371 -> 4039; at 2048 waves n = 9 loses, 3356 -> 3801).
+  bool dealt = false;
   if (o->precision == HCX_PREC_FP64 && nseg == 1) {
     Seg& S = LN.seg[0];
     const hcx_problem* p = probs[0];
@@ -1485,6 +1488,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     const KernelFn df = deal > 1 ? pick_deal(pl.nmax, pl.deg, pl.exact, deal) : nullptr;
     if (df && (size_t)groups(deal) * (size_t)region(deal) + (size_t)lat.words * 4 <= (size_t)kMaxLdsBytes) {
       LN.dot_lds = 1;
+      dealt = true;
       S.R = deal;
       pl.fn = df;
       pl.latency = true;
@@ -1569,6 +1573,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(pl.fn, dim3((unsigned)blocks), dim3(64 * wpb), pl.lds, stream, LN);
   HIP_TRY(hipGetLastError());
+  g_shape = {LN.seg[0].R, dealt ? 1 : 0, wpb, (int)blocks, 0};
 
   // Mixed precision: re-track in FP64 from t = 0 every path that ended
   // without a refined root (precision escalation), then every path whose root
@@ -1599,14 +1604,22 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     }
     st = finish_plan(L2, p2);
     if (st != HCX_OK) return st;
-    // a small persistent grid: the list holds few paths; idle waves exit at once
-    long long b2 = 0;
+    // as many waves as the GPU holds, shared out by the segments' paths: of a
+    // batch of diverging paths most are re-tracked (about one wave per CU took
+    // 40.8 ms of 10,200 of n = 12, all that fit 24.1 ms).  The waves that a list
+    // has no paths for end at once (run_segment_fp64), so the usual list, of few
+    // paths, costs what it did.
+    int occ = 0;
+    HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(p2.fn), 64, p2.lds));
+    long long all = 0, b2 = 0;
+    for (int s = 0; s < nseg; ++s) all += seg_groups[s];
+    const double share = std::min(1.0, (double)std::max(occ, 1) * g_cu / (double)std::max(all, 1LL));
     for (int s = 0; s < nseg; ++s) {
       L2.first_block[s] = (int)b2;
-      const int gpw = 64 / L2.seg[s].G;
-      b2 += std::max<long long>(1, std::min<long long>((L2.seg[s].P + gpw - 1) / gpw, g_cu / nseg + 1));
+      b2 += std::max<long long>(1, std::llround(share * (double)seg_groups[s]));
     }
     L2.first_block[nseg] = (int)b2;
+    g_shape.pass_blocks = (int)b2;
     hipLaunchKernelGGL(list_unrefined_kernel, dim3((unsigned)((max_paths + 255) / 256), nseg), dim3(256), 0, stream,
                        L2);
     hipLaunchKernelGGL(p2.fn, dim3((unsigned)b2), dim3(64), p2.lds, stream, L2);
@@ -1623,6 +1636,9 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
 }  // namespace hcx
 
 extern "C" {
+
+// {replicas, dealt, waves per block, blocks, blocks of the FP64 pass}
+void hcx_internal_launch_shape(int* out) { std::memcpy(out, &g_shape, sizeof(g_shape)); }
 
 hcx_status hcx_track(hcx_problem* p, const hcx_batch_desc* b, const hcx_track_opts* o, const hcx_result_desc* r,
                      void* stream) {

@@ -58,3 +58,41 @@ def test_jump_onto_root_of_escalated_path(hcx_mod, gpu, n):
     assert (m["flags"] & hcx.FLAG_ESCALATED).all()
     assert hcx.collect(r[1], hcx.default_opts())["unique"] == 2
     prob.close()
+
+
+@pytest.mark.parametrize("n,waves", [(7, 1100), (12, 1100), (18, 700)])
+def test_batch_without_a_path_for_fp32(hcx_mod, gpu, n, waves):
+    """Coefficients beyond FP32: the FP64 pass tracks the whole batch, on as
+    many waves as the batch has (its LDS lets a CU hold at least four, n = 18
+    three), with the results of an FP64 launch bit for bit."""
+    import ctypes
+    import torch
+    from hcx import workloads
+    hcx = hcx_mod
+    k, K = 2 * n, 32
+    sysf = hcx.System.synthetic(n, k, num_quadratic=n, monomials=n + 6, seed=3 + n)
+    p0 = workloads.random_cn(5 + n, k)
+    start = workloads.seed_start_roots(sysf, p0, K, 7)
+    count = waves * (64 // n) // K
+    hx, ht = zip(*(sysf.param_homotopy_coeffs(p0, p) for p in workloads.targets(k, count, seed=11)))
+    hx, ht = np.array(hx), np.array(ht)
+    hx[:, :-1] *= 1e39
+    ht[:, :-1] *= 1e39
+    prob = hcx.Problem.from_system(sysf, start, with_affine=False)
+    b = hcx.Batch(prob, count, coeffs_hx=hx, coeffs_ht=ht)
+    f = hcx.track(prob, b, hcx.default_opts(precision=0, replicas=1))
+    m = hcx.track(prob, b, hcx.default_opts(precision=1))
+    shape = (ctypes.c_int * 5)()
+    hcx.lib().hcx_internal_launch_shape(shape)
+    torch.cuda.synchronize()
+    f, m = f.to_host(), m.to_host()
+    ok = (f["flags"] & hcx.FLAG_REFINED) != 0
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    needed = -(-len(ok) // (64 // n))
+    print(f"[n={n}] {len(ok)} paths, {int(ok.sum())} refined, pass on {shape[4]} blocks of {needed}", flush=True)
+    assert ok.mean() > 0.9
+    assert shape[4] >= min(needed, (3 if n > 16 else 4) * cus)
+    assert (m["flags"] == (f["flags"] | hcx.FLAG_ESCALATED)).all()
+    for key in ("steps", "newton", "refine", "t_final", "roots"):
+        assert np.array_equal(m[key], f[key], equal_nan=True), key
+    prob.close()
