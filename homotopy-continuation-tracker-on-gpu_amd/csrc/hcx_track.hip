@@ -254,44 +254,48 @@ __global__ void collect_kernel(int n, int K, const double2* __restrict__ roots, 
   atomicAdd(&counts[6], c_rref);
 }
 
-// The FP64 pass of a mixed-precision launch re-tracks paths from t = 0 in two
-// rounds, whose lists these kernels write (grid.y: the segments).  First every
-// path without a refined root (precision escalation).  Then, with the roots of
-// those in place, every refined path of mixed precision whose root equals
-// another refined root of its instance (|dRe|, |dIm| < tol in every
-// coordinate): a path that jumped onto another path's root shares that root,
-// also where the other path is one that the first round tracked.  Both kernels
-// prepare the segment's path queue and output descriptor for the launch that
-// follows (a re-tracked path does not count its instance's paths down again).
-__device__ __forceinline__ void start_retrack(const Seg& S) {
-  *S.counter = 0u;
-  const_cast<SegOut*>(S.out)->inst_left = nullptr;
-}
-
-__global__ void list_unrefined_kernel(const Launch LN) {
-  const Seg& S = LN.seg[blockIdx.y];
-  const long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j == 0) start_retrack(S);
-  if (j < S.P && !(S.out->flags[j] & HCX_FLAG_REFINED)) S.plist[atomicAdd(S.plist_count, 1u)] = (int)j;
-}
-
-// One block per instance.
-__global__ void list_duplicates_kernel(const Launch LN, double tol) {
+// Lists the paths that the FP64 pass of a mixed-precision launch re-tracks from
+// t = 0 (grid.x: instances, grid.y: segments).  Round 0: every path without a
+// refined root (precision escalation) and, with dups, every refined path whose
+// root equals another refined root of its instance (|dRe|, |dIm| < tol in every
+// coordinate): a path that jumped onto another path's root shares that root.
+// Round 1, when the paths of round 0 have their FP64 roots: every path still of
+// mixed precision whose root equals one of those.  Also prepares the segment's
+// path queue and output descriptor for the launch that follows (a re-tracked path
+// does not count its instance's paths down again).
+// Round 1 reads the flags only where no path of the instance was re-tracked.
+__global__ void list_retrack_kernel(const Launch LN, double tol, int round, int dups) {
   const Seg& S = LN.seg[blockIdx.y];
   const int inst = blockIdx.x, n = S.n, K = S.K;
-  if (inst == 0 && threadIdx.x == 0) start_retrack(S);
+  if (inst == 0 && threadIdx.x == 0) {
+    *S.counter = 0u;
+    const_cast<SegOut*>(S.out)->inst_left = nullptr;
+  }
   if (inst >= S.I) return;
   const size_t base = (size_t)inst * K;
   const uint32_t* const flags = S.out->flags + base;
   const double2* const roots = S.out->roots + base * n;
+  // the roots compared with
+  const uint32_t with = round == 0 ? HCX_FLAG_REFINED : HCX_FLAG_REFINED | HCX_FLAG_ESCALATED;
+  if (round > 0) {
+    __shared__ int any;
+    if (threadIdx.x == 0) any = 0;
+    __syncthreads();
+    for (int i = threadIdx.x; i < K; i += blockDim.x)
+      if ((flags[i] & with) == with) any = 1;
+    __syncthreads();
+    if (!any) return;
+  }
   for (int j = threadIdx.x; j < K; j += blockDim.x) {
     const uint32_t fj = flags[j];
-    if (!(fj & HCX_FLAG_REFINED) || (fj & HCX_FLAG_ESCALATED)) continue;
-    const double2* xj = roots + (size_t)j * n;
-    bool dup = false;
-    for (int i = 0; i < K && !dup; ++i)
-      dup = i != j && (flags[i] & HCX_FLAG_REFINED) && same_root(roots + (size_t)i * n, xj, n, tol);
-    if (dup) S.plist[atomicAdd(S.plist_count, 1u)] = (int)(base + j);
+    if (fj & HCX_FLAG_ESCALATED) continue;
+    bool list = !(fj & HCX_FLAG_REFINED);
+    if (!list && dups) {
+      const double2* xj = roots + (size_t)j * n;
+      for (int i = 0; i < K && !list; ++i)
+        list = i != j && (flags[i] & with) == with && same_root(roots + (size_t)i * n, xj, n, tol);
+    }
+    if (list) S.plist[atomicAdd(S.plist_count, 1u)] = (int)(base + j);
   }
 }
 
@@ -1576,18 +1580,15 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   g_shape = {LN.seg[0].R, dealt ? 1 : 0, wpb, (int)blocks, 0};
 
   // Mixed precision: re-track in FP64 from t = 0 every path that ended
-  // without a refined root (precision escalation), then every path whose root
-  // duplicates another root of its instance (a jump onto another path), so
-  // the refined roots and counts are those of the FP64 tracker.
+  // without a refined root (precision escalation) and every path whose root
+  // duplicates another root of its instance (a jump onto another path), then
+  // those whose root duplicates a root found by that, so the refined roots and
+  // counts are those of the FP64 tracker.
   if (o->precision == HCX_PREC_MIXED) {
     Launch L2 = LN;
     L2.persistent = 1;
     L2.wpb = 1;
-    long long max_paths = 1;
-    for (int s = 0; s < nseg; ++s) {
-      L2.seg[s].plist = work[s].plist;
-      max_paths = std::max(max_paths, L2.seg[s].P);
-    }
+    for (int s = 0; s < nseg; ++s) L2.seg[s].plist = work[s].plist;
     Plan p2;
     st = choose_kernel(nseg, probs, Gs, max_deg, HCX_PREC_FP64, specialize, p2);
     if (st != HCX_OK) return st;
@@ -1620,12 +1621,10 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     }
     L2.first_block[nseg] = (int)b2;
     g_shape.pass_blocks = (int)b2;
-    hipLaunchKernelGGL(list_unrefined_kernel, dim3((unsigned)((max_paths + 255) / 256), nseg), dim3(256), 0, stream,
-                       L2);
-    hipLaunchKernelGGL(p2.fn, dim3((unsigned)b2), dim3(64), p2.lds, stream, L2);
-    if (o->retrack_duplicates) {
-      for (int s = 0; s < nseg; ++s) ++L2.seg[s].plist_count;
-      hipLaunchKernelGGL(list_duplicates_kernel, dim3(max_inst, nseg), dim3(256), 0, stream, L2, o->unique_tol);
+    for (int round = 0; round < (o->retrack_duplicates ? 2 : 1); ++round) {
+      for (int s = 0; s < nseg; ++s) L2.seg[s].plist_count = work[s].plist_count + round;
+      hipLaunchKernelGGL(list_retrack_kernel, dim3(max_inst, nseg), dim3(256), 0, stream, L2, o->unique_tol, round,
+                         o->retrack_duplicates);
       hipLaunchKernelGGL(p2.fn, dim3((unsigned)b2), dim3(64), p2.lds, stream, L2);
     }
     HIP_TRY(hipGetLastError());
