@@ -163,41 +163,66 @@ __device__ __forceinline__ T group_max(T v, const Group& g) {
 
 // Pivot key of a candidate row: its magnitude's bits above 31 - label, so the
 // largest key is the largest magnitude and, among equal ones, the first row in
-// current row order.  A row that is no candidate holds key 0; a key below 32
-// is a zero magnitude.  FP64 gives up the 5 lowest of its 52 mantissa bits to
-// the label (candidates within 2^-47 of each other count as equal); FP32
-// magnitudes stay whole.  NaN orders above every number.
-__device__ __forceinline__ unsigned long long pivot_key(double mag, int label) {
-  return ((unsigned long long)__double_as_longlong(mag) & ~31ull) | (unsigned int)(31 - label);
-}
+// current row order.  A row that is no candidate holds key 0; NaN orders above
+// every number.  An FP32 key is two words and holds the whole magnitude (0: a key below 32).
+// An FP64 key is one word, the upper 27 bits without the sign: candidates that
+// share these (one pair in 2^16 of unrelated ones, and exact ties) are compared
+// by the other bits and the label in a second search (pivot_rest), so the pivot
+// is that of the whole magnitudes.
 __device__ __forceinline__ unsigned long long pivot_key(float mag, int label) {
   return ((unsigned long long)(__float_as_uint(mag) & 0x7fffffffu) << 32) | (unsigned int)(31 - label);
 }
+__device__ __forceinline__ unsigned int pivot_key(double mag, int label) {
+  return ((unsigned int)((unsigned long long)__double_as_longlong(mag) >> 31) & ~31u) | (unsigned int)(31 - label);
+}
+// The bits that the FP64 key leaves out, above 31 - label; bit 63 is set.  A
+// magnitude is 0 where its key is below 32 and this below 32 without bit 63.
+__device__ __forceinline__ unsigned long long pivot_rest(double mag, int label) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(mag) & ((1ull << 36) - 1);
+  return 1ull << 63 | b << 5 | (unsigned int)(31 - label);
+}
+// A group's key words hold one kind or the other.
+typedef unsigned int __attribute__((may_alias)) key32;
+typedef unsigned long long __attribute__((may_alias)) key64;
+__device__ __forceinline__ bool same_upper(unsigned int a, unsigned int b) { return (a ^ b) < 32u; }
+// Whether a search of the wave is still open: more than one candidate shares a
+// key's upper bits, or these are 0 (the group's other lanes hold key 0).  One
+// scalar branch.  part: the lanes of the paths that take part, searches: their
+// number (-1 where a path has one lane).
+__device__ __forceinline__ bool pivot_open(unsigned int own, unsigned int key, unsigned long long part, int searches) {
+  return (int)__builtin_popcountll(__ballot(same_upper(own, key)) & part) != searches;
+}
 
-// Largest key over an aligned group of GC lanes (a power of two), to every
+// Largest value over an aligned group of GC lanes (a power of two), to every
 // lane: DPP inside 16-lane rows, a row swap between the two rows of 32.
 template <int CTRL>
-__device__ __forceinline__ unsigned long long key_max_dpp(unsigned long long k) {
+__device__ __forceinline__ unsigned int max_dpp(unsigned int k) {
+  return max(k, (unsigned int)dpp_read<CTRL>((int)k));
+}
+template <int CTRL>
+__device__ __forceinline__ unsigned long long max_dpp(unsigned long long k) {
   const unsigned int lo = (unsigned int)dpp_read<CTRL>((int)(unsigned int)k);
   const unsigned int hi = (unsigned int)dpp_read<CTRL>((int)(unsigned int)(k >> 32));
-  const unsigned long long o = ((unsigned long long)hi << 32) | lo;
-  return o > k ? o : k;
+  return max(k, ((unsigned long long)hi << 32) | lo);
 }
-template <int GC>
-__device__ __forceinline__ unsigned long long group_max_key(unsigned long long k) {
+// rows (0, 0, 2, 2) and (1, 1, 3, 3) of the wave
+__device__ __forceinline__ unsigned int max_rows(unsigned int k) {
+  const auto r = __builtin_amdgcn_permlane16_swap(k, k, false, false);
+  return max((unsigned int)r[0], (unsigned int)r[1]);
+}
+__device__ __forceinline__ unsigned long long max_rows(unsigned long long k) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned int)k, (unsigned int)k, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned int)(k >> 32), (unsigned int)(k >> 32), false, false);
+  return max(((unsigned long long)hi[0] << 32) | lo[0], ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+template <int GC, class K>
+__device__ __forceinline__ K group_max_key(K k) {
   static_assert(is_pow2(GC) && GC <= 32, "aligned power-of-two groups");
-  if constexpr (GC >= 2) k = key_max_dpp<kDppQuadXor1>(k);
-  if constexpr (GC >= 4) k = key_max_dpp<kDppQuadXor2>(k);
-  if constexpr (GC >= 8) k = key_max_dpp<kDppHalfMirror>(k);
-  if constexpr (GC >= 16) k = key_max_dpp<kDppRowMirror>(k);
-  if constexpr (GC >= 32) {
-    // rows (0, 0, 2, 2) and (1, 1, 3, 3) of the wave
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned int)k, (unsigned int)k, false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned int)(k >> 32), (unsigned int)(k >> 32), false, false);
-    const unsigned long long u = ((unsigned long long)hi[0] << 32) | lo[0];
-    const unsigned long long v = ((unsigned long long)hi[1] << 32) | lo[1];
-    k = u > v ? u : v;
-  }
+  if constexpr (GC >= 2) k = max_dpp<kDppQuadXor1>(k);
+  if constexpr (GC >= 4) k = max_dpp<kDppQuadXor2>(k);
+  if constexpr (GC >= 8) k = max_dpp<kDppHalfMirror>(k);
+  if constexpr (GC >= 16) k = max_dpp<kDppRowMirror>(k);
+  if constexpr (GC >= 32) k = max_rows(k);
   return k;
 }
 
@@ -250,7 +275,7 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 // pivoting (dev-cgesv-batched-small.cuh:51-95): cabs1, the first maximum in
 // current row order (rows carry a position label swapped like a physical
 // row interchange), multipliers by the pivot reciprocal, a zero pivot column
-// skipped and reported through `singular`.  Every step eliminates the pivot
+// reported through `singular`.  Every step eliminates the pivot
 // column from the rows ABOVE the pivot as well (Gauss-Jordan), in place of the
 // reference's back substitution (:97-106): on a lane group the lanes of those
 // rows would only wait during the step, so the extra row updates cost no
@@ -266,10 +291,14 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 //
 // The solve is a chain of n steps, each bound by its latencies: find the
 // pivot, broadcast its row, update.  So
-//  * a candidate packs its magnitude and position into one 64-bit key; the
-//    largest comes from DPP row permutations (aligned power-of-two groups) or
-//    from an LDS maximum per group and step (one instruction and one read in
-//    place of a scan of every candidate's magnitude);
+//  * a candidate packs its magnitude and position into one key; the largest
+//    comes from DPP row permutations (aligned power-of-two groups) or from an
+//    LDS maximum per group and step (one instruction and one read in place of
+//    a scan of every candidate's magnitude);
+//  * whether an FP64 key left candidates to compare further (pivot_open) is
+//    looked at while the pivot's row is on its way; then the row goes out again.
+//    Against keys of 59 bits that called the rest equal: n = 3 and 5 in lone
+//    launches +1.6%, n = 9 +0.8%, n = 30 -2.9% (DPP steps on one word);
 //  * the next step's candidates enter their search as soon as their column is
 //    updated, and the remaining columns are updated while it is under way;
 //  * every candidate computes the reciprocal of its own entry during the
@@ -278,9 +307,12 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 // Where n is not a compile-time constant (generic instances) the columns are
 // checked against it four at a time: columns n..NMAX-1 hold values that no
 // step uses.
+// act: the group's path takes part (the others' results are not used).
 template <int NMAX, int GC, class T>
-__device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const Group& g, int n, bool row,
+__device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const Group& g, int n, bool row, bool act,
                                                 cx<T>* sp, unsigned long long* keys, bool& singular) {
+  const unsigned long long part = __ballot(act);
+  const int searches = g.G == 1 ? -1 : __popcll(__ballot(act && g.gl == 0));  // one per path and replica
   int label = g.gl;
   cx<T> own_rinv = cmk<T>(T(0), T(0));  // 1 / U_ii of the row this lane ends up holding
   singular = false;
@@ -295,21 +327,26 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
   }
   // sp shares the group's LDS slots with x: the evaluation's reads of x come first
   HCX_WAVE_SYNC();
-  unsigned long long key = 0;
+  // the group's largest key for step k, and this lane's
+  decltype(pivot_key(T(0), 0)) key = 0, own = 0;
+  bool cand = false;
+  auto largest = [&](int k, bool in, auto v) {
+    using V = decltype(v);
+    using W = std::conditional_t<sizeof(V) == 4, key32, key64>;
+    if constexpr (GC > 0) return group_max_key<GC>(in ? v : V(0));
+    const bool mine = in && g.s == 0;
+    __hip_atomic_fetch_max(reinterpret_cast<W*>(mine ? &keys[k] : no_key), mine ? v : V(0), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+    // requested ahead of the rest of the pivot row
+    HCX_WAVE_SYNC();
+    const V m = *reinterpret_cast<W*>(&keys[k]);
+    HCX_WAVE_SYNC();
+    return m;
+  };
   auto search = [&](int k) {
-    const bool cand = row && label >= k;
-    key = cand ? pivot_key(cabs1(A[k]), label) : 0ull;
-    if constexpr (GC > 0) {
-      key = group_max_key<GC>(key);
-    } else {
-      const bool mine = cand && g.s == 0;
-      __hip_atomic_fetch_max(mine ? &keys[k] : no_key, mine ? key : 0ull, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_WAVEFRONT);
-      // requested ahead of the rest of the pivot row
-      HCX_WAVE_SYNC();
-      key = keys[k];
-      HCX_WAVE_SYNC();
-    }
+    cand = row && label >= k;
+    own = cand ? pivot_key(cabs1(A[k]), label) : 0;
+    key = largest(k, cand, own);
   };
   search(0);
 #pragma unroll
@@ -318,29 +355,43 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
       cx<T> rinv = crecip(A[k]);
       // keeps the reciprocal out of the pivot's branch, beside the search
       asm volatile("" : "+v"(rinv.re), "+v"(rinv.im));
-      const int blabel = 31 - (int)((unsigned int)key & 31u);
-      const bool zero = key < 32ull;
-      const bool piv = row && label == blabel;
-      singular = singular || zero;
+      int blabel = 31 - (int)((unsigned int)key & 31u);
+      if constexpr (sizeof(T) == 4) singular = singular || key < 32;
+      bool piv = row && label == blabel;
       const bool more = k + 1 < NMAX && k + 1 < n;
       // the two entries that the next search waits for go out, and are
       // requested, before the rest of the row
       constexpr bool kSplit = NMAX > 6;
-      if (piv) {
-        sp[k] = rinv;
-        if (more) sp[k + 1] = A[k + 1];
-        if constexpr (!kSplit) {
+      cx<T> rp, next = cmk<T>(T(0), T(0));
+      auto publish = [&]() {
+        if (piv) {
+          sp[k] = rinv;
+          if (more) sp[k + 1] = A[k + 1];
+          if constexpr (!kSplit) {
 #pragma unroll
-          for (int j = k + 2; j < NMAX; ++j)
-            if ((j & ~3) < n) sp[j] = A[j];
-          sp[NMAX] = b;
-          own_rinv = rinv;
+            for (int j = k + 2; j < NMAX; ++j)
+              if ((j & ~3) < n) sp[j] = A[j];
+            sp[NMAX] = b;
+          }
+        }
+        HCX_WAVE_SYNC();
+        rp = sp[k];
+        if (more) next = sp[k + 1];
+        HCX_WAVE_SYNC();
+      };
+      publish();
+      // while the row is on its way: is the pivot the only one of its key?
+      if constexpr (sizeof(T) == 8) {
+        if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
+          const unsigned long long rest =
+              largest(k, cand && same_upper(own, key), pivot_rest(cabs1(A[k]), label));
+          blabel = 31 - (int)((unsigned int)rest & 31u);
+          singular = singular || (key < 32u && rest << 1 < 64u);
+          piv = row && label == blabel;
+          publish();
         }
       }
-      HCX_WAVE_SYNC();
-      const cx<T> rp = sp[k];
-      cx<T> next = cmk<T>(T(0), T(0));
-      if (more) next = sp[k + 1];
+      if (piv) own_rinv = rinv;
       if constexpr (kSplit) {
         HCX_WAVE_SYNC();
         if (piv) {
@@ -348,12 +399,11 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
           for (int j = k + 2; j < NMAX; ++j)
             if ((j & ~3) < n) sp[j] = A[j];
           sp[NMAX] = b;
-          own_rinv = rinv;
         }
         HCX_WAVE_SYNC();
       }
       label = piv ? k : (label == k ? blabel : label);
-      const bool upd = row && !piv && !zero;
+      const bool upd = row && !piv;
       cx<T> l = cmul_fused(A[k], rp);
       l = cmk<T>(upd ? l.re : T(0), upd ? l.im : T(0));
       if (more) {
@@ -434,8 +484,10 @@ constexpr int split_bytes(int nmax, int G, int R) { return R > 1 ? 16 * (R * G +
 template <int NMAX, int R, int NC>
 __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], const Group& g, int n, bool row,
                                                         cx<double>* sp, unsigned long long* keys, cx<double>* cols,
-                                                        cx<double>* prow, bool& singular) {
+                                                        cx<double>* prow, bool act, bool& singular) {
   static_assert(NC == (NMAX + R) / R, "columns 0..NMAX in R replicas");
+  const unsigned long long part = __ballot(act);
+  const int searches = g.G == 1 ? -1 : __popcll(__ballot(act && g.gl == 0 && g.s == 0));
   int label = g.gl;
   cx<double> own_rinv = cmk<double>(0, 0);
   singular = false;
@@ -444,17 +496,18 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
   cx<double>* const mine = prow + g.s;
   if (row && g.s == 0) keys[g.gl] = 0ull;
   HCX_WAVE_SYNC();
-  unsigned long long key = 0;
+  unsigned int key = 0, own = 0;
+  bool cand = false;
   cx<double> ck = cmk<double>(0, 0);
   auto search = [&](int k) {
     const int so = k % R, io = k / R;
     if (g.in_grp) cols[g.s * g.G + g.gl] = B[io];
-    const bool cand = row && label >= k && g.s == so;
-    key = pivot_key(cabs1(B[io]), label);
-    __hip_atomic_fetch_max(cand ? &keys[k] : no_key, cand ? key : 0ull, __ATOMIC_RELAXED,
+    cand = row && label >= k && g.s == so;
+    own = cand ? pivot_key(cabs1(B[io]), label) : 0u;
+    __hip_atomic_fetch_max(reinterpret_cast<key32*>(cand ? &keys[k] : no_key), own, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WAVEFRONT);
     HCX_WAVE_SYNC();
-    key = keys[k];
+    key = *reinterpret_cast<key32*>(&keys[k]);
     ck = cols[so * g.G + g.gl];
     HCX_WAVE_SYNC();
   };
@@ -465,28 +518,45 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
       const int so = k % R, io = k / R;
       cx<double> rinv = crecip(B[io]);  // the pivot's in replica so
       asm volatile("" : "+v"(rinv.re), "+v"(rinv.im));
-      const int blabel = 31 - (int)((unsigned int)key & 31u);
-      const bool zero = key < 32ull;
-      const bool piv = row && label == blabel;
-      singular = singular || zero;
-      if (piv) {
+      int blabel = 31 - (int)(key & 31u);
+      bool piv = row && label == blabel;
+      const bool more = k + 1 < NMAX && k + 1 < n;
+      cx<double> rp, next = cmk<double>(0, 0);
+      auto publish = [&]() {
+        if (piv) {
 #pragma unroll
-        for (int i = io; i < NC; ++i) {
-          cx<double> v = B[i];
-          if (i == io) v = cmk<double>(g.s == so ? rinv.re : v.re, g.s == so ? rinv.im : v.im);
-          if (R * i < n || i == NMAX / R) mine[R * i] = v;
+          for (int i = io; i < NC; ++i) {
+            cx<double> v = B[i];
+            if (i == io) v = cmk<double>(g.s == so ? rinv.re : v.re, g.s == so ? rinv.im : v.im);
+            if (R * i < n || i == NMAX / R) mine[R * i] = v;
+          }
         }
+        HCX_WAVE_SYNC();
+        rp = prow[k];
+        if (more) next = mine[R * ((k + 1) / R)];
+        HCX_WAVE_SYNC();
+      };
+      publish();
+      if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
+        const bool c = cand && same_upper(own, key);
+        __hip_atomic_fetch_max(reinterpret_cast<key64*>(c ? &keys[k] : no_key),
+                               c ? pivot_rest(cabs1(B[io]), label) : 0ull, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WAVEFRONT);
+        HCX_WAVE_SYNC();
+        const unsigned long long rest = *reinterpret_cast<key64*>(&keys[k]);
+        blabel = 31 - (int)((unsigned int)rest & 31u);
+        singular = singular || (key < 32u && rest << 1 < 64u);
+        piv = row && label == blabel;
+        HCX_WAVE_SYNC();
+        publish();
       }
-      HCX_WAVE_SYNC();
-      const cx<double> rp = prow[k];
       label = piv ? k : (label == k ? blabel : label);
       own_rinv = cmk<double>(piv ? rp.re : own_rinv.re, piv ? rp.im : own_rinv.im);
-      const bool upd = row && !piv && !zero;
+      const bool upd = row && !piv;
       cx<double> l = cmul_fused(ck, rp);
       l = cmk<double>(upd ? l.re : 0.0, upd ? l.im : 0.0);
-      const bool more = k + 1 < NMAX && k + 1 < n;
       if (more) {
-        B[(k + 1) / R] = cfnms(B[(k + 1) / R], l, mine[R * ((k + 1) / R)]);
+        B[(k + 1) / R] = cfnms(B[(k + 1) / R], l, next);
         search(k + 1);
       }
 #pragma unroll
@@ -823,7 +893,7 @@ __device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsi
         cx<float> A[NMAX];
         const cx<float> bt = eval_system<float, NMAX, DEG, LT, NB>(Sk, n, gle, xb, cb, db, lt, A);
         bool sing;
-        const cx<float> k = group_lu_solve<NMAX, GC, float>(A, cmk<float>(-bt.re, -bt.im), g, n, row,
+        const cx<float> k = group_lu_solve<NMAX, GC, float>(A, cmk<float>(-bt.re, -bt.im), g, n, row, stepping,
                                                             L.template piv<float>(), L.keys(), sing);
         kp = ccast<double>(k);
         const double w = (st == 1 || st == 2) ? 2.0 : 1.0;
@@ -850,7 +920,7 @@ __device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsi
           const cx<float> hv = eval_system<float, NMAX, DEG, LT, NB>(Sk, n, gle, xb, cb, cb, lt, A);
           bool sing;
           const cx<float> d =
-              group_lu_solve<NMAX, GC, float>(A, hv, g, n, row, L.template piv<float>(), L.keys(), sing);
+              group_lu_solve<NMAX, GC, float>(A, hv, g, n, row, run, L.template piv<float>(), L.keys(), sing);
           if (run && row) x = csub(x, ccast<double>(d));
           double s1 = row ? (double)cnorm2(d) : 0.0, s2 = row ? cnorm2(x) : 0.0;
           group_sum2<NMAX, GC, true>(s1, s2, g, n, row, lane, L.piv64());
@@ -882,7 +952,7 @@ __device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsi
       cx<double> A[NMAX];
       const cx<double> r = eval_system<double, NMAX, DEG, LT, NB>(Sk, n, gle, xb, cb, cb, lt, A);
       bool sing;
-      const cx<double> d = group_lu_solve<NMAX, GC, double>(A, r, g, n, row, L.piv64(), L.keys(), sing);
+      const cx<double> d = group_lu_solve<NMAX, GC, double>(A, r, g, n, row, act, L.piv64(), L.keys(), sing);
       const bool nr = pe == kPhNewton || pe == kPhRefine;
       if (nr && row) x = csub(x, d);
       double s1 = (nr && row) ? cnorm2(d) : 0.0, s2 = (nr && row) ? cnorm2(x) : 0.0;
@@ -1182,7 +1252,7 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
           r = rb;
           if (stg && g.s == NMAX % REP) rb = cmk<double>(-rb.re, -rb.im);
         }
-        d = group_solve_split<NMAX, REP>(B, g, n, row, L.piv64(), L.keys(), cols, cols + REP * g.G, sing);
+        d = group_solve_split<NMAX, REP>(B, g, n, row, L.piv64(), L.keys(), cols, cols + REP * g.G, act, sing);
       } else {
         if constexpr (REP == 1) {
           // more replicas than the split solve deals out: a butterfly over
@@ -1202,8 +1272,8 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
             r.im += __shfl(r.im, src);
           }
         }
-        d = group_lu_solve<NMAX, GC, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, L.piv64(), L.keys(),
-                                             sing);
+        d = group_lu_solve<NMAX, GC, double>(A, stg ? cmk<double>(-r.re, -r.im) : r, g, n, row, act, L.piv64(),
+                                             L.keys(), sing);
       }
 
       // RK4 stage: k_s = solution, accumulate k1 + 2 k2 + 2 k3 + k4
