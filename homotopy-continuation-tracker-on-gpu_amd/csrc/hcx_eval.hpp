@@ -44,24 +44,34 @@ __device__ __forceinline__ cx<float> cmul_term(cx<float> a, cx<float> b) {
   return cmk<float>(__builtin_fmaf(a.re, b.re, -(a.im * b.im)), __builtin_fmaf(a.im, b.re, a.re * b.im));
 }
 
-// Compact records of the size-specialised instances, in LDS: byte offsets of
-// the coefficient slot (16 bits, from the group's coefficient area) and of
-// the variables (10 bits, from its x area), the scalar in the spare bits.
-//   word 0: c | v0 << 16 | low 6 bits of s << 26
-//   word 1: degree <= 2 (H only): v1 | j << 16
-//           degree 3, 4:          v1 | v2 << 16 | high 6 bits of s << 26
-//   word 2: degree 3, 4 (H only): v3 | j << 16   (word 3 unused)
-// with j the coefficient's number (index of dc/dt in global memory) and s 6
-// bits (degree <= 2) or 12, two's complement.
+// Compact records of the throughput instances, in LDS: byte offsets of the
+// coefficient slot (16 bits, from the group's coefficient area) and of the
+// variables (10 bits, multiples of 16, from its x area), and the scalar s.
+//   degree <= 2:  dH/dx  c | v0 << 16 | s << 26
+//                 H      c | v0 << 16 | s << 26,  v1 | j << 16
+//   degree 3, 4:  dH/dx  c | v0 << 16,  v1 | v2 << 6 | s << 16
+//                 H      c | v0 << 16,  v1 | v2 << 16,  v3 | j << 16,  s
+// with j the coefficient's number (index of dc/dt in global memory); s is of 6
+// bits in 26.., of 16 in 16.. and whole in a word of its own.
 template <int DEG>
 struct StreamRec {
   static constexpr int kJ = DEG <= 2 ? 4 : 8;
   static constexpr int kH = DEG <= 2 ? 8 : 16;
 };
+// The values of v1 and v2 of a dH/dx record of degree 3 or 4.
+template <class T>
+__device__ __forceinline__ cx<T> lds_v1(const unsigned char* base, uint32_t r) {
+  return *reinterpret_cast<const cx<T>*>(base + ((r >> kHalf<T>) & (0x3ffu >> kHalf<T>)));
+}
+template <class T>
+__device__ __forceinline__ cx<T> lds_v2(const unsigned char* base, uint32_t r) {
+  return *reinterpret_cast<const cx<T>*>(base + (((r >> 10) & 0x3fu) << (4 - kHalf<T>)));
+}
+// s of a dH/dx record
 template <int DEG>
 __device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
   if constexpr (DEG <= 2) return (double)((int)r0 >> 26);
-  return (double)((((int)r1 >> 26) << 6) | (int)(r0 >> 26));
+  return (double)((int)r1 >> 16);
 }
 
 // One round over NB columns of a row of dH/dx (throughput instances): term k
@@ -94,8 +104,8 @@ __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int of
     if (JB + u < NMAX) {
       c[u] = lds_lo<T>(cb, r0[u]);
       p[u] = lds_hi<T>(xb, r0[u]);
-      if constexpr (DEG > 2) p1[u] = lds_lo<T>(xb, r1[u]);
-      if constexpr (DEG > 3) p2[u] = lds_hi<T>(xb, r1[u]);
+      if constexpr (DEG > 2) p1[u] = lds_v1<T>(xb, r1[u]);
+      if constexpr (DEG > 3) p2[u] = lds_v2<T>(xb, r1[u]);
     }
   }
   // PIN: all gathers before the first product
@@ -300,7 +310,7 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
                                                 const unsigned char* xb, const unsigned char* cb,
                                                 const double2* dg, bool dot, cx<T> acc) {
   constexpr int RS = StreamRec<DEG>::kH;
-  uint32_t r[Q][3];
+  uint32_t r[Q][4];
   cx<T> c[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
@@ -314,6 +324,7 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
       r[q][0] = v.x;
       r[q][1] = v.y;
       r[q][2] = v.z;
+      r[q][3] = v.w;
     }
   }
   cx<T> x0[Q], x1[Q], x2[Q], x3[Q];
@@ -340,7 +351,7 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     cx<T> v = c[q];
-    if constexpr (SC) v = cscale(v, (T)rec_scalar<DEG>(r[q][0], r[q][1]));
+    if constexpr (SC) v = cscale(v, (T)(DEG <= 2 ? (int)r[q][0] >> 26 : (int)r[q][3]));
     v = cmul_term(v, x0[q]);
     v = cmul_term(v, x1[q]);
     if constexpr (DEG > 2) v = cmul_term(v, x2[q]);

@@ -18,9 +18,11 @@ void clear_error();
 
 // Shape of the calling thread's latest tracking launch: replicas per path (and
 // whether they hold whole columns), waves per block, blocks, blocks of the FP64
-// pass of mixed precision.  Read by the tests through hcx_internal_launch_shape.
+// pass of mixed precision; whether the instance is one of the size, and the
+// bytes of term records in a block's LDS.  Read by the tests through
+// hcx_internal_launch_shape.
 struct LaunchShape {
-  int replicas, dealt, waves_per_block, blocks, pass_blocks;
+  int replicas, dealt, waves_per_block, blocks, pass_blocks, specialized, record_bytes;
 };
 
 inline cd to_cd(hcx_complex z) { return cd(z.re, z.im); }

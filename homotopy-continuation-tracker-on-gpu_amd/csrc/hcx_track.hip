@@ -1090,22 +1090,25 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     const int f = cf & 1;
     const bool lat = cf >= 2;
     // offsets of 16 bits (from the region's start in the slot list), scalars of
-    // 6 or 12 bits
-    const int s_lim = f == 0 ? 32 : 2048;
+    // 6 or 16 bits
+    const int s_lim = f == 0 ? 32 : 32768;
     if (!colc_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4000 || C > 0xffff || deg > (f == 0 ? 2 : 4))
       continue;
     CompactHost& ch = compact[cf];
     std::vector<uint32_t>& w = ch.w;
     auto var = [&](const dev::Term& tm, int q) { return (uint32_t)(((tm.v03 >> (8 * q)) & 0xffu) * 16u); };
     auto put = [&](const dev::Term& tm, bool h) {
-      const uint32_t sc = (uint32_t)tm.s;
-      w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16 | (sc & 0x3fu) << 26);
+      const uint32_t sc = (uint32_t)tm.s, j = (uint32_t)cinv[tm.c];
       if (f == 0) {
-        if (h) w.push_back(var(tm, 1) | (uint32_t)cinv[tm.c] << 16);
+        w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16 | sc << 26);
+        if (h) w.push_back(var(tm, 1) | j << 16);
+        return;
+      }
+      w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16);
+      if (h) {
+        w.insert(w.end(), {var(tm, 1) | var(tm, 2) << 16, var(tm, 3) | j << 16, sc});
       } else {
-        w.push_back(var(tm, 1) | var(tm, 2) << 16 | ((sc >> 6) & 0x3fu) << 26);
-        if (h) w.push_back(var(tm, 3) | (uint32_t)cinv[tm.c] << 16);
-        if (h) w.push_back(0);
+        w.push_back(var(tm, 1) | var(tm, 2) << 6 | sc << 16);
       }
     };
     auto align = [&]() {
@@ -1577,7 +1580,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL(pl.fn, dim3((unsigned)blocks), dim3(64 * wpb), pl.lds, stream, LN);
   HIP_TRY(hipGetLastError());
-  g_shape = {LN.seg[0].R, dealt ? 1 : 0, wpb, (int)blocks, 0};
+  g_shape = {LN.seg[0].R, dealt ? 1 : 0, wpb, (int)blocks, 0, pl.exact ? 1 : 0, pl.tab_lds};
 
   // Mixed precision: re-track in FP64 from t = 0 every path that ended
   // without a refined root (precision escalation) and every path whose root
@@ -1636,7 +1639,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
 
 extern "C" {
 
-// {replicas, dealt, waves per block, blocks, blocks of the FP64 pass}
+// The fields of LaunchShape.
 void hcx_internal_launch_shape(int* out) { std::memcpy(out, &g_shape, sizeof(g_shape)); }
 
 hcx_status hcx_track(hcx_problem* p, const hcx_batch_desc* b, const hcx_track_opts* o, const hcx_result_desc* r,

@@ -82,7 +82,7 @@ def test_batch_without_a_path_for_fp32(hcx_mod, gpu, n, waves):
     b = hcx.Batch(prob, count, coeffs_hx=hx, coeffs_ht=ht)
     f = hcx.track(prob, b, hcx.default_opts(precision=0, replicas=1))
     m = hcx.track(prob, b, hcx.default_opts(precision=1))
-    shape = (ctypes.c_int * 5)()
+    shape = (ctypes.c_int * 7)()
     hcx.lib().hcx_internal_launch_shape(shape)
     torch.cuda.synchronize()
     f, m = f.to_host(), m.to_host()
