@@ -51,27 +51,70 @@ __device__ __forceinline__ cx<float> cmul_term(cx<float> a, cx<float> b) {
 //                 H      c | v0 << 16 | s << 26,  v1 | j << 16
 //   degree 3, 4:  dH/dx  c | v0 << 16,  v1 | v2 << 6 | s << 16
 //                 H      c | v0 << 16,  v1 | v2 << 16,  v3 | j << 16,  s
+//   degree 5, 6:  dH/dx  c | v0 << 16,  v1 | v2 << 16,  v3 | v4 << 16,  s
+//                 H      c | v0 << 16 | s << 26,  v1 | v2 << 16 | s' << 26,
+//                        v3 | v4 << 16 | s'' << 26,  v5 | j << 16
 // with j the coefficient's number (index of dc/dt in global memory); s is of 6
-// bits in 26.., of 16 in 16.. and whole in a word of its own.
+// bits in 26.., of 16 in 16.. and whole in a word of its own; in three parts
+// s, s', s'' of 6 bits, the lowest first.
 template <int DEG>
 struct StreamRec {
-  static constexpr int kJ = DEG <= 2 ? 4 : 8;
+  static constexpr int kJ = DEG <= 2 ? 4 : (DEG <= 4 ? 8 : 16);
   static constexpr int kH = DEG <= 2 ? 8 : 16;
+  static constexpr int kJWord = DEG <= 2 ? 1 : (DEG <= 4 ? 2 : 3);  // word of j
 };
-// The values of v1 and v2 of a dH/dx record of degree 3 or 4.
-template <class T>
-__device__ __forceinline__ cx<T> lds_v1(const unsigned char* base, uint32_t r) {
-  return *reinterpret_cast<const cx<T>*>(base + ((r >> kHalf<T>) & (0x3ffu >> kHalf<T>)));
+// A record of N bytes.
+template <int N>
+__device__ __forceinline__ void load_rec(const unsigned char* a, uint32_t (&r)[4]) {
+  if constexpr (N == 4) {
+    r[0] = *reinterpret_cast<const uint32_t*>(a);
+  } else if constexpr (N == 8) {
+    const uint2 q = *reinterpret_cast<const uint2*>(a);
+    r[0] = q.x;
+    r[1] = q.y;
+  } else {
+    const uint4 q = *reinterpret_cast<const uint4*>(a);
+    r[0] = q.x;
+    r[1] = q.y;
+    r[2] = q.z;
+    r[3] = q.w;
+  }
 }
-template <class T>
-__device__ __forceinline__ cx<T> lds_v2(const unsigned char* base, uint32_t r) {
-  return *reinterpret_cast<const cx<T>*>(base + (((r >> 10) & 0x3fu) << (4 - kHalf<T>)));
+// The values of a term's NV variables (v0 in the first word's upper half, then
+// two per word).
+template <int NV, class T>
+__device__ __forceinline__ void rec_vars(const unsigned char* xb, const uint32_t (&r)[4], cx<T> (&x)[NV]) {
+#pragma unroll
+  for (int q = 0; q < NV; ++q) x[q] = q % 2 == 0 ? lds_hi<T>(xb, r[q / 2]) : lds_lo<T>(xb, r[(q + 1) / 2]);
 }
-// s of a dH/dx record
+// Those of a dH/dx record of the throughput instances.
+template <int DEG, class T>
+__device__ __forceinline__ void jac_vars(const unsigned char* xb, const uint32_t (&r)[4], cx<T> (&x)[DEG - 1]) {
+  if constexpr (DEG <= 2 || DEG > 4) {
+    rec_vars<DEG - 1, T>(xb, r, x);
+  } else {
+    x[0] = lds_hi<T>(xb, r[0]);
+    x[1] = *reinterpret_cast<const cx<T>*>(xb + ((r[1] >> kHalf<T>) & (0x3ffu >> kHalf<T>)));
+    if constexpr (DEG > 3) x[2] = *reinterpret_cast<const cx<T>*>(xb + (((r[1] >> 10) & 0x3fu) << (4 - kHalf<T>)));
+  }
+}
 template <int DEG>
-__device__ __forceinline__ double rec_scalar(uint32_t r0, uint32_t r1) {
-  if constexpr (DEG <= 2) return (double)((int)r0 >> 26);
-  return (double)((int)r1 >> 16);
+__device__ __forceinline__ int jac_scalar(const uint32_t (&r)[4]) {
+  return DEG <= 2 ? (int)r[0] >> 26 : (DEG <= 4 ? (int)r[1] >> 16 : (int)r[3]);
+}
+template <int DEG>
+__device__ __forceinline__ int h_scalar(const uint32_t (&r)[4]) {
+  if constexpr (DEG <= 2) return (int)r[0] >> 26;
+  if constexpr (DEG <= 4) return (int)r[3];
+  return ((int)r[2] >> 26 << 12) | (int)(r[1] >> 26 << 6) | (int)(r[0] >> 26);
+}
+// (scalar * coefficient) * variable ..., SC: with a scalar other than 1
+template <int NV, bool SC, class T, class S>
+__device__ __forceinline__ cx<T> term_value(cx<T> c, S s, const cx<T> (&x)[NV]) {
+  if constexpr (SC) c = cscale(c, (T)s);
+#pragma unroll
+  for (int q = 0; q < NV; ++q) c = cmul_term(c, x[q]);
+  return c;
 }
 
 // One round over NB columns of a row of dH/dx (throughput instances): term k
@@ -82,45 +125,27 @@ template <int NMAX, int DEG, bool SC, int JB, int NB, bool PIN, class T>
 __device__ __forceinline__ void jac_round(const unsigned char* rp, int n, int off, int zero, const int (&cnt)[NB],
                                           int k, const unsigned char* xb, const unsigned char* cb, cx<T> (&A)[NMAX]) {
   constexpr int RS = StreamRec<DEG>::kJ;
-  uint32_t r0[NB], r1[NB];
-  cx<T> c[NB], p[NB], p1[NB], p2[NB];
+  uint32_t r[NB][4];
+  cx<T> c[NB], x[NB][DEG - 1];
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
-      const unsigned char* a = rp + (k < cnt[u] ? off + k * (n * RS) : zero);
-      if constexpr (DEG <= 2) {
-        r0[u] = *reinterpret_cast<const uint32_t*>(a);
-        r1[u] = 0;
-      } else {
-        const uint2 q = *reinterpret_cast<const uint2*>(a);
-        r0[u] = q.x;
-        r1[u] = q.y;
-      }
+      load_rec<RS>(rp + (k < cnt[u] ? off + k * (n * RS) : zero), r[u]);
       off += cnt[u] * (n * RS);
     }
   }
 #pragma unroll
   for (int u = 0; u < NB; ++u) {
     if (JB + u < NMAX) {
-      c[u] = lds_lo<T>(cb, r0[u]);
-      p[u] = lds_hi<T>(xb, r0[u]);
-      if constexpr (DEG > 2) p1[u] = lds_v1<T>(xb, r1[u]);
-      if constexpr (DEG > 3) p2[u] = lds_v2<T>(xb, r1[u]);
+      c[u] = lds_lo<T>(cb, r[u][0]);
+      jac_vars<DEG, T>(xb, r[u], x[u]);
     }
   }
   // PIN: all gathers before the first product
   if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int u = 0; u < NB; ++u) {
-    if (JB + u < NMAX) {
-      cx<T> v = c[u];
-      if constexpr (SC) v = cscale(v, (T)rec_scalar<DEG>(r0[u], r1[u]));
-      v = cmul_term(v, p[u]);
-      if constexpr (DEG > 2) v = cmul_term(v, p1[u]);
-      if constexpr (DEG > 3) v = cmul_term(v, p2[u]);
-      A[JB + u] = cadd(A[JB + u], v);
-    }
-  }
+  for (int u = 0; u < NB; ++u)
+    if (JB + u < NMAX) A[JB + u] = cadd(A[JB + u], term_value<DEG - 1, SC, T>(c[u], jac_scalar<DEG>(r[u]), x[u]));
 }
 
 // Row gl of dH/dx from the compact streams at lt
@@ -159,10 +184,16 @@ __device__ __forceinline__ void eval_jac_blocks(const SegT& S, int n, const unsi
 // its double (the low word is 0), and one row of zero terms after each
 // column's positions.
 //   degree <= 2:  {c | v0 << 16, s}     degree 3, 4:  {c | v0 << 16, v1 | v2 << 16, s, 0}
+//   degree 5, 6:  {c | v0 << 16, v1 | v2 << 16, v3 | v4 << 16, s}
 template <int DEG>
 struct LatencyRec {
   static constexpr int kJ = DEG <= 2 ? 8 : 16;
+  static constexpr int kS = DEG <= 2 ? 1 : (DEG <= 4 ? 2 : 3);  // word of the scalar
 };
+template <int DEG>
+__device__ __forceinline__ double latency_scalar(const uint32_t (&r)[4]) {
+  return __longlong_as_double((long long)((unsigned long long)r[LatencyRec<DEG>::kS] << 32));
+}
 
 // Row gl of dH/dx on the latency instances (one wave per SIMD: every LDS
 // round trip is exposed).  Round by round, one term of every column at once:
@@ -175,56 +206,42 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
                                                 const unsigned char* cb, cx<double> (&A)[NMAX],
                                                 const unsigned char* lt, int k0, int ks) {
   constexpr int RS = LatencyRec<DEG>::kJ;
-  constexpr int NB = NMAX <= 6 ? NMAX : (NMAX <= 10 ? (NMAX + 1) / 2 : 4);  // columns at a time
+  // columns at a time; degree 5 and 6: 5 variables of two columns fill the registers
+  constexpr int NB = DEG > 4 ? 2 : (NMAX <= 6 ? NMAX : (NMAX <= 10 ? (NMAX + 1) / 2 : 4));
   const int rounds_end = S.max_terms;
 #pragma unroll
   for (int j = 0; j < NMAX; ++j) A[j] = cmk<double>(0, 0);
 #pragma unroll 1
-  for (int r = 0; r < rounds_end; r += ks) {
-    const int k = r + k0;
+  for (int rd = 0; rd < rounds_end; rd += ks) {
+    const int k = rd + k0;
     const unsigned char* rp = lt + gle * RS;
 #pragma unroll
     for (int jb = 0; jb < NMAX; jb += NB) {
-      uint32_t r0[NB], r1[NB], rs[NB];
+      // generic instances skip blocks of no column, where there are many (n = 3,
+      // degree 5, 1024 waves 6.31 -> 4.59 ms; in larger blocks the branches cost more)
+      if (DEG > 4 && jb >= n) continue;
+      uint32_t r[NB][4];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
           const int cnt = (int)(S.colc[jb + u] & 0xffffu);
-          const unsigned char* a = rp + min(k, cnt) * (n * RS);
-          if constexpr (DEG <= 2) {
-            const uint2 q = *reinterpret_cast<const uint2*>(a);
-            r0[u] = q.x;
-            rs[u] = q.y;
-          } else {
-            const uint4 q = *reinterpret_cast<const uint4*>(a);
-            r0[u] = q.x;
-            r1[u] = q.y;
-            rs[u] = q.z;
-          }
+          load_rec<RS>(rp + min(k, cnt) * (n * RS), r[u]);
           rp += (cnt + (jb + u < n ? 1 : 0)) * (n * RS);
         }
       }
-      cx<double> c[NB], p[NB], p1[NB], p2[NB];
+      cx<double> c[NB], x[NB][DEG - 1];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (jb + u < NMAX) {
-          c[u] = lds_lo<double>(cb, r0[u]);
-          p[u] = lds_hi<double>(xb, r0[u]);
-          if constexpr (DEG > 2) p1[u] = lds_lo<double>(xb, r1[u]);
-          if constexpr (DEG > 3) p2[u] = lds_hi<double>(xb, r1[u]);
+          c[u] = lds_lo<double>(cb, r[u][0]);
+          rec_vars<DEG - 1, double>(xb, r[u], x[u]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
 #pragma unroll
-      for (int u = 0; u < NB; ++u) {
-        if (jb + u < NMAX) {
-          cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
-          v = cmul_term(v, p[u]);
-          if constexpr (DEG > 2) v = cmul_term(v, p1[u]);
-          if constexpr (DEG > 3) v = cmul_term(v, p2[u]);
-          A[jb + u] = cadd(A[jb + u], v);
-        }
-      }
+      for (int u = 0; u < NB; ++u)
+        if (jb + u < NMAX)
+          A[jb + u] = cadd(A[jb + u], term_value<DEG - 1, true, double>(c[u], latency_scalar<DEG>(r[u]), x[u]));
     }
   }
 }
@@ -257,45 +274,27 @@ __device__ __forceinline__ void eval_jac_dealt(const SegT& S, int n, int gle, in
   for (int k = 0; k < rounds_end; ++k) {
 #pragma unroll
     for (int ib = 0; ib < NC; ib += NB) {
-      uint32_t r0[NB], r1[NB], rs[NB];
+      uint32_t r[NB][4];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (ib + u < NC) {
-          const unsigned char* a = lt + p[ib + u];
-          if constexpr (DEG <= 2) {
-            const uint2 q = *reinterpret_cast<const uint2*>(a);
-            r0[u] = q.x;
-            rs[u] = q.y;
-          } else {
-            const uint4 q = *reinterpret_cast<const uint4*>(a);
-            r0[u] = q.x;
-            r1[u] = q.y;
-            rs[u] = q.z;
-          }
+          load_rec<RS>(lt + p[ib + u], r[u]);
           p[ib + u] = min(p[ib + u] + row, end[ib + u]);
         }
       }
-      cx<double> c[NB], x[NB], x1[NB], x2[NB];
+      cx<double> c[NB], x[NB][DEG - 1];
 #pragma unroll
       for (int u = 0; u < NB; ++u) {
         if (ib + u < NC) {
-          c[u] = lds_lo<double>(cb, r0[u]);
-          x[u] = lds_hi<double>(xb, r0[u]);
-          if constexpr (DEG > 2) x1[u] = lds_lo<double>(xb, r1[u]);
-          if constexpr (DEG > 3) x2[u] = lds_hi<double>(xb, r1[u]);
+          c[u] = lds_lo<double>(cb, r[u][0]);
+          rec_vars<DEG - 1, double>(xb, r[u], x[u]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);  // all gathers before the first product
 #pragma unroll
-      for (int u = 0; u < NB; ++u) {
-        if (ib + u < NC) {
-          cx<double> v = cscale(c[u], __longlong_as_double((long long)((unsigned long long)rs[u] << 32)));
-          v = cmul_term(v, x[u]);
-          if constexpr (DEG > 2) v = cmul_term(v, x1[u]);
-          if constexpr (DEG > 3) v = cmul_term(v, x2[u]);
-          B[ib + u] = cadd(B[ib + u], v);
-        }
-      }
+      for (int u = 0; u < NB; ++u)
+        if (ib + u < NC)
+          B[ib + u] = cadd(B[ib + u], term_value<DEG - 1, true, double>(c[u], latency_scalar<DEG>(r[u]), x[u]));
     }
   }
 }
@@ -311,36 +310,19 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
                                                 const double2* dg, bool dot, cx<T> acc) {
   constexpr int RS = StreamRec<DEG>::kH;
   uint32_t r[Q][4];
-  cx<T> c[Q];
+  cx<T> c[Q], x[Q][DEG];
 #pragma unroll
-  for (int q = 0; q < Q; ++q) {
-    const unsigned char* a = rp + min(k + q * ks, cnt) * (n * RS);
-    if constexpr (DEG <= 2) {
-      const uint2 v = *reinterpret_cast<const uint2*>(a);
-      r[q][0] = v.x;
-      r[q][1] = v.y;
-    } else {
-      const uint4 v = *reinterpret_cast<const uint4*>(a);
-      r[q][0] = v.x;
-      r[q][1] = v.y;
-      r[q][2] = v.z;
-      r[q][3] = v.w;
-    }
-  }
-  cx<T> x0[Q], x1[Q], x2[Q], x3[Q];
+  for (int q = 0; q < Q; ++q) load_rec<RS>(rp + min(k + q * ks, cnt) * (n * RS), r[q]);
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
     c[q] = lds_lo<T>(cb, r[q][0]);
-    x0[q] = lds_hi<T>(xb, r[q][0]);
-    x1[q] = lds_lo<T>(xb, r[q][1]);
-    if constexpr (DEG > 2) x2[q] = lds_hi<T>(xb, r[q][1]);
-    if constexpr (DEG > 3) x3[q] = lds_lo<T>(xb, r[q][2]);
+    rec_vars<DEG, T>(xb, r[q], x[q]);
   }
   if constexpr (GDOT) {
     if (dot) {
 #pragma unroll
       for (int q = 0; q < Q; ++q) {
-        const double2 d = dg[r[q][DEG <= 2 ? 1 : 2] >> 16];
+        const double2 d = dg[r[q][StreamRec<DEG>::kJWord] >> 16];
         c[q] = cmk<T>((T)d.x, (T)d.y);
       }
     }
@@ -349,15 +331,7 @@ __device__ __forceinline__ cx<T> rhs_chunk(const unsigned char* rp, int n, int k
   // where the compiler would rather save registers
   if constexpr (PIN) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int q = 0; q < Q; ++q) {
-    cx<T> v = c[q];
-    if constexpr (SC) v = cscale(v, (T)(DEG <= 2 ? (int)r[q][0] >> 26 : (int)r[q][3]));
-    v = cmul_term(v, x0[q]);
-    v = cmul_term(v, x1[q]);
-    if constexpr (DEG > 2) v = cmul_term(v, x2[q]);
-    if constexpr (DEG > 3) v = cmul_term(v, x3[q]);
-    acc = cadd(acc, v);
-  }
+  for (int q = 0; q < Q; ++q) acc = cadd(acc, term_value<DEG, SC, T>(c[q], h_scalar<DEG>(r[q]), x[q]));
   return acc;
 }
 

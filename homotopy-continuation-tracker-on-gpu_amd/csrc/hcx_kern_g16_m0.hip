@@ -9,6 +9,7 @@ KernelFn kernel_g16_m0(int deg) {
   switch (deg) {
     case 2: return kernel_g16_m0_d2();
     case 3: return kernel_g16_m0_d3();
+    case 4: return kernel_g16_m0_d4();
     case 6: return kernel_g16_m0_d6();
     default: return nullptr;
   }

@@ -7,6 +7,7 @@ KernelFn kernel_rep_g32_r1(int deg) {
   switch (deg) {
     case 2: return track_kernel_rep<32, 2, false, 1>;
     case 3: return track_kernel_rep<32, 3, false, 1>;
+    case 4: return track_kernel_rep<32, 4, false, 1>;
     case 6: return track_kernel_rep<32, 6, false, 1>;
     default: return nullptr;
   }

@@ -7,6 +7,7 @@ KernelFn kernel_rep_g8_r2(int deg) {
   switch (deg) {
     case 2: return track_kernel_rep<8, 2, false, 2>;
     case 3: return track_kernel_rep<8, 3, false, 2>;
+    case 4: return track_kernel_rep<8, 4, false, 2>;
     case 6: return track_kernel_rep<8, 6, false, 2>;
     default: return nullptr;
   }

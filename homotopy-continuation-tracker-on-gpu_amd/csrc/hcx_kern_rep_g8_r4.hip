@@ -7,6 +7,7 @@ KernelFn kernel_rep_g8_r4(int deg) {
   switch (deg) {
     case 2: return track_kernel_rep<8, 2, false, 4>;
     case 3: return track_kernel_rep<8, 3, false, 4>;
+    case 4: return track_kernel_rep<8, 4, false, 4>;
     case 6: return track_kernel_rep<8, 6, false, 4>;
     default: return nullptr;
   }

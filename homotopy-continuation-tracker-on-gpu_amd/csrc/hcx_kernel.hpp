@@ -695,11 +695,11 @@ template <class T, int NMAX, int DEG, bool LT, int NB, class SegT>
 __device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, const unsigned char* xb,
                                              const unsigned char* cb, const unsigned char* rhs,
                                              const unsigned char* lt, cx<T> (&A)[NMAX]) {
-  constexpr int DC = DEG <= 4 ? DEG : 4;
   if (LT || lt) {
-    constexpr int HQ = NMAX <= 6 && sizeof(T) == 8 ? 2 : 4;
-    eval_jac_blocks<NMAX, DC, NB, 0, !LT && sizeof(T) == 4, T>(S, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
-    return eval_rhs_stream<DC, false, HQ, (NMAX > 6), T>(S, n, gle, xb, rhs, rhs, nullptr, false, lt, 0, 1);
+    constexpr int HQ = (NMAX <= 6 && sizeof(T) == 8) || DEG > 4 ? 2 : 4;
+    eval_jac_blocks<NMAX, DEG, (DEG > 4 ? 2 : NB), 0, !LT && sizeof(T) == 4, T>(S, n, lt + gle * StreamRec<DEG>::kJ, 0,
+                                                                              xb, cb, A);
+    return eval_rhs_stream<DEG, false, HQ, (NMAX > 6), T>(S, n, gle, xb, rhs, rhs, nullptr, false, lt, 0, 1);
   }
   if constexpr (!LT) {
     const cx<T>* const sx = reinterpret_cast<const cx<T>*>(xb);
@@ -1056,8 +1056,6 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   // The compact streams in LDS: always (LT), or in a generic instance where
   // the launch found room for them; else the full Term records in global
   // memory, or (generic latency instance) in LDS.  tab_lds holds the bytes.
-  // DC: the degree of the compact records.
-  constexpr int DC = DEG <= 4 ? DEG : 4;
   const unsigned char* lt = nullptr;
   const Term* tl = nullptr;
   if constexpr (LT) {
@@ -1212,20 +1210,21 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
         constexpr bool kPin = REP > 0 || NMAX > 6;
         if constexpr (REP) {
           if constexpr (DEAL)
-            eval_jac_dealt<NMAX, DC, REP, NC>(Sk, n, gle, g.s, xb, cb, B, lt);
+            eval_jac_dealt<NMAX, DEG, REP, NC>(Sk, n, gle, g.s, xb, cb, B, lt);
           else
-            eval_jac_rounds<NMAX, DC>(Sk, n, gle, xb, cb, A, lt, k0, ks);
-          if (Sk.htT <= 2 * ks)
-            r = eval_rhs_stream<DC, false, 2, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            eval_jac_rounds<NMAX, DEG>(Sk, n, gle, xb, cb, A, lt, k0, ks);
+          if (DEG > 4 || Sk.htT <= 2 * ks)
+            r = eval_rhs_stream<DEG, false, 2, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<DC, false, 4, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DEG, false, 4, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         } else {
-          constexpr int HQ = NMAX <= 6 ? 2 : 4;  // H terms in flight
-          eval_jac_blocks<NMAX, DC, NB, 0, false, double>(Sk, n, lt + gle * StreamRec<DC>::kJ, 0, xb, cb, A);
+          constexpr int HQ = NMAX <= 6 || DEG > 4 ? 2 : 4;  // H terms in flight
+          eval_jac_blocks<NMAX, DEG, (DEG > 4 ? 2 : NB), 0, false, double>(Sk, n, lt + gle * StreamRec<DEG>::kJ, 0, xb,
+                                                                           cb, A);
           if (gdot)
-            r = eval_rhs_stream<DC, true, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DEG, true, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
           else
-            r = eval_rhs_stream<DC, false, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
+            r = eval_rhs_stream<DEG, false, HQ, kPin, double>(Sk, n, gle, xb, cb, db, hti, stg, lt, k0, ks);
         }
       } else {
         const cx<double>* sc = reinterpret_cast<const cx<double>*>(cb);
@@ -1453,7 +1452,8 @@ KernelFn kernel_g16_m1(int deg);
 KernelFn kernel_g32_m0(int deg);
 KernelFn kernel_g32_m1(int deg);
 #define HCX_GENERIC_UNITS(G, M) \
-  KernelFn kernel_g##G##_m##M##_d2(); KernelFn kernel_g##G##_m##M##_d3(); KernelFn kernel_g##G##_m##M##_d6();
+  KernelFn kernel_g##G##_m##M##_d2(); KernelFn kernel_g##G##_m##M##_d3(); \
+  KernelFn kernel_g##G##_m##M##_d4(); KernelFn kernel_g##G##_m##M##_d6();
 HCX_GENERIC_UNITS(8, 0)
 HCX_GENERIC_UNITS(8, 1)
 HCX_GENERIC_UNITS(16, 0)
@@ -1489,7 +1489,7 @@ KernelFn kernel_x30_m0(int deg);
 KernelFn kernel_x30_m1(int deg);
 // Latency instances (FP64, one segment, few paths) of R replicas per path:
 // size-specialised for n in {3, 4, 5, 6} and {8, 9, 10, 12, 16} (DEG 2 and 3,
-// n = 4, 5 also 4), generic for NMAX 8, 16 and 32 (DEG 2, 3 and 6); R = 8 up to
+// n = 4, 5 also 4), generic for NMAX 8, 16 and 32 (DEG 2, 3, 4 and 6); R = 8 up to
 // 8 lanes per replica, 4 up to 16, 2 up to 32.
 #define HCX_REP_UNITS(R) \
   KernelFn kernel_rep_xs_r##R(int n, int deg); KernelFn kernel_rep_xl_r##R(int n, int deg); \

@@ -21,8 +21,9 @@ struct hcx_problem {
   unsigned char* d_blob = nullptr;     // the allocation that holds every table below
   int* d_cslot = nullptr;              // [C+1] LDS slot of each coefficient
   // Term streams (hcx_eval.hpp): full records in global memory, and the
-  // compact tables of the instances that hold them in LDS for terms of degree
-  // <= 2 ([0], when the problem has no higher ones) and <= 4.
+  // compact tables of the instances that hold them in LDS: for terms of degree
+  // <= 2 ([0], when the problem has no higher ones), <= 4 and <= 6 (when the
+  // second form does not hold the problem).
   struct Compact {
     uint32_t* d = nullptr;
     int words = 0, h = 0, slot = 0;    // size; byte offsets of the H streams and the slot list
@@ -35,7 +36,7 @@ struct hcx_problem {
   bool colc_fits = false;
   int hx_recs = 0, htT = 0, htS = 0, nslot = 0;
   int max_terms = 0;                   // positions of the longest column
-  Compact ctab[2], ltab[2];            // throughput and latency instances
+  Compact ctab[3], ltab[3];            // throughput and latency instances
   double2* d_start = nullptr;
   double2* d_affine = nullptr;
   double2* d_p0 = nullptr;

@@ -306,7 +306,7 @@ __global__ void zero_u64_kernel(unsigned long long* p, int n) {
 
 // ------------------------------------------------------------ dispatch table
 static const int kNmaxList[] = {8, 16, 32};
-static const int kDegList[] = {2, 3, 6};
+static const int kDegList[] = {2, 3, 4, 6};
 
 static KernelFn pick_kernel(int nmax, int deg, int mode) {
   switch (nmax) {
@@ -518,12 +518,15 @@ int lds_group_bytes(int nmax, bool keys, int slots, int M, bool dot_lds = false)
   return (((b + 15) / 16) | 1) * 16;
 }
 
+// Form of the compact tables for terms of up to `deg` variables.
+int compact_format(int deg) { return deg <= 2 ? 0 : (deg <= 4 ? 1 : 2); }
+
 struct Plan {
   int nmax = 0, mode = 0;
   int deg = 2;       // term degree of the instance (generic: rounded up to its instance's)
   bool exact = false;
   bool latency = false;  // the latency instance, with its own compact tables
-  bool tab4 = false; // the compact tables are those of DEG <= 2
+  int fmt = 0;       // the compact tables are those of degree <= 2 (0), 4 (1) or 6 (2)
   int tab_lds = 0;   // LDS bytes of the compact tables (instances that hold them there)
   size_t lds = 0;
   KernelFn fn = nullptr;
@@ -611,15 +614,14 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
   pl.tab_lds = 0;
   int max_n = 1, tab = 0;
   bool same = true, tab_ok = true, in_set = true;
-  // the compact term format of the kernel's degree: 4 bytes up to degree 2
   const bool t4 = max_deg <= 2;
-  pl.tab4 = t4;
+  pl.fmt = compact_format(max_deg);
   for (int s = 0; s < nseg; ++s) {
     const int n = probs[s]->n;
     max_n = std::max(max_n, n);
     same = same && n == probs[0]->n && Gs[s] == exact_lanes(n);
     in_set = in_set && (n == 3 || n == 5 || n == 6 || n == 9 || n == 12) && Gs[s] == n;
-    const auto& c = probs[s]->ctab[t4 ? 0 : 1];
+    const auto& c = probs[s]->ctab[pl.fmt];
     tab_ok = tab_ok && c.d && table_bytes(probs[s], t4) <= kMaxTabLds;
     tab = std::max(tab, c.words * 4);
   }
@@ -649,10 +651,15 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
     }
   }
   const int ni = round_up_idx(kNmaxList, 3, max_n);
-  const int di = round_up_idx(kDegList, 3, max_deg);
+  int di = round_up_idx(kDegList, 4, max_deg);
   if (ni < 0 || di < 0) {
     set_error("unsupported sizes: n=%d (max %d), degree=%d (max 6)", max_n, kMaxN, max_deg);
     return HCX_ERR_UNSUPPORTED;
+  }
+  // terms of degree 3 or 4 with scalars beyond their compact form
+  if (di >= 0 && nseg == 1 && pl.fmt == 1 && !probs[0]->ctab[1].d && probs[0]->ctab[2].d) {
+    pl.fmt = 2;
+    di = 3;
   }
   pl.fn = pick_kernel(kNmaxList[ni], kDegList[di], mode);
   pl.nmax = kNmaxList[ni];
@@ -665,7 +672,7 @@ hcx_status choose_kernel(int nseg, const hcx_problem* const* probs, const int* G
     // global memory cost more than half the waves.  1024 waves, ms, global -> LDS:
     // n = 7, degree 4, mixed (7 -> 6 waves) 19.3 -> 9.0; n = 18, 1080 coefficients (3 -> 2)
     // 37.8 -> 20.4; n = 28, 1680 coefficients (3 -> 2) 49.4 -> 29.1.
-    const auto& c = probs[0]->ctab[pl.tab4 ? 0 : 1];
+    const auto& c = probs[0]->ctab[pl.fmt];
     const size_t wave = (size_t)(64 / Gs[0]) * (size_t)pl.group_bytes(probs[0]), tb = (size_t)c.words * 4;
     const int cap = pl.nmax == 32 ? 4 : 8;
     if (c.d && tb <= 65536 && 2 * resident_waves(tb, wave, cap) >= resident_waves(0, wave, cap)) {
@@ -684,7 +691,7 @@ void seg_tables(Seg& S, const hcx_problem* p, const Plan& pl) {
   S.lds_group = pl.group_bytes(p);
   S.cslot = p->d_cslot;
   S.nslot = p->nslot;
-  const auto& c = (pl.latency ? p->ltab : p->ctab)[pl.tab4 ? 0 : 1];
+  const auto& c = (pl.latency ? p->ltab : p->ctab)[pl.fmt];
   S.hx = p->d_hx;
   S.ht = p->d_ht;
   S.ht_ci = p->d_ht_ci;
@@ -1085,18 +1092,21 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   struct CompactHost {
     std::vector<uint32_t> w;
     int h = 0, slot = 0;
-  } compact[4];  // [degree], [2 + degree]: the latency instances'
-  for (int cf = 0; cf < 4; ++cf) {
-    const int f = cf & 1;
-    const bool lat = cf >= 2;
+  } compact[6];  // [format], [3 + format]: the latency instances'
+  for (int cf = 0; cf < 6; ++cf) {
+    const int f = cf % 3;
+    const bool lat = cf >= 3;
     // offsets of 16 bits (from the region's start in the slot list), scalars of
-    // 6 or 16 bits
-    const int s_lim = f == 0 ? 32 : 32768;
-    if (!colc_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4000 || C > 0xffff || deg > (f == 0 ? 2 : 4))
+    // 6, 16 or 18 bits; the last form where the others do not hold the problem
+    const int s_lim = f == 0 ? 32 : (f == 1 ? 32768 : 1 << 17);
+    if (!colc_fits || s_min < -s_lim || s_max >= s_lim || nslot > 4000 || C > 0xffff || deg > 2 * f + 2 ||
+        (f == 2 && (deg <= 2 || !compact[1].w.empty())))
       continue;
     CompactHost& ch = compact[cf];
     std::vector<uint32_t>& w = ch.w;
-    auto var = [&](const dev::Term& tm, int q) { return (uint32_t)(((tm.v03 >> (8 * q)) & 0xffu) * 16u); };
+    auto var = [&](const dev::Term& tm, int q) {
+      return (uint32_t)((((q < 4 ? tm.v03 : tm.v47) >> (8 * (q & 3))) & 0xffu) * 16u);
+    };
     auto put = [&](const dev::Term& tm, bool h) {
       const uint32_t sc = (uint32_t)tm.s, j = (uint32_t)cinv[tm.c];
       if (f == 0) {
@@ -1104,9 +1114,18 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
         if (h) w.push_back(var(tm, 1) | j << 16);
         return;
       }
-      w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16);
+      const uint32_t w0 = (uint32_t)(tm.c * 16) | var(tm, 0) << 16, w1 = var(tm, 1) | var(tm, 2) << 16;
+      if (f == 2) {
+        const uint32_t w2 = var(tm, 3) | var(tm, 4) << 16;
+        if (h)
+          w.insert(w.end(), {w0 | sc << 26, w1 | sc >> 6 << 26, w2 | sc >> 12 << 26, var(tm, 5) | j << 16});
+        else
+          w.insert(w.end(), {w0, w1, w2, sc});
+        return;
+      }
+      w.push_back(w0);
       if (h) {
-        w.insert(w.end(), {var(tm, 1) | var(tm, 2) << 16, var(tm, 3) | j << 16, sc});
+        w.insert(w.end(), {w1, var(tm, 3) | j << 16, sc});
       } else {
         w.push_back(var(tm, 1) | var(tm, 2) << 6 | sc << 16);
       }
@@ -1120,7 +1139,8 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
       uint64_t bits;
       std::memcpy(&bits, &sd, 8);
       w.push_back((uint32_t)(tm.c * 16) | var(tm, 0) << 16);
-      if (f == 1) w.push_back(var(tm, 1) | var(tm, 2) << 16);
+      if (f >= 1) w.push_back(var(tm, 1) | var(tm, 2) << 16);
+      if (f == 2) w.push_back(var(tm, 3) | var(tm, 4) << 16);
       w.push_back((uint32_t)(bits >> 32));
       if (f == 1) w.push_back(0);
     };
@@ -1188,9 +1208,9 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
   add_vec(&p->d_ht, hts);
   add_vec(&p->d_ht_ci, ht_ci);
   add_vec(&p->d_hx_cnt, hxs_cnt);
-  for (int cf = 0; cf < 4; ++cf) {
+  for (int cf = 0; cf < 6; ++cf) {
     const CompactHost& ch = compact[cf];
-    hcx_problem::Compact& ct = cf < 2 ? p->ctab[cf] : p->ltab[cf - 2];
+    hcx_problem::Compact& ct = cf < 3 ? p->ctab[cf] : p->ltab[cf - 3];
     if (ch.w.empty()) continue;
     add_vec(&ct.d, ch.w);
     ct.words = (int)ch.w.size();
@@ -1446,7 +1466,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
   if (o->precision == HCX_PREC_FP64 && nseg == 1) {
     Seg& S = LN.seg[0];
     const hcx_problem* p = probs[0];
-    const auto& lat = p->ltab[pl.tab4 ? 0 : 1];
+    const auto& lat = p->ltab[pl.fmt];
     const int lg = pl.group_bytes(p, true);
     const size_t terms =
         pl.exact ? 0 : ((size_t)p->hx_recs + (size_t)p->n * p->htT) * sizeof(dev::Term);
@@ -1485,7 +1505,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     // compact tables where they fit as well
     const bool compact = pl.exact ? pl.tab_lds > 0 : rf && lat.d && lat.words * 4 <= 65536;
     size_t tab = 0, tab_new = terms;
-    if (pl.exact && pl.tab_lds > 0) tab = (size_t)table_bytes(p, pl.tab4);
+    if (pl.exact && pl.tab_lds > 0) tab = (size_t)table_bytes(p, pl.fmt == 0);
     if (compact) tab_new = (size_t)(rf ? lat.words * 4 : pl.tab_lds);
     const size_t used = (size_t)groups(R) * (size_t)(rf ? region(R) : lg) + tab_new;
     const bool fits = (rf || one) && regions + tab + terms <= 65536 && used <= (size_t)kMaxLdsBytes;
