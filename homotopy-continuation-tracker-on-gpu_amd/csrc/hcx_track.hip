@@ -752,20 +752,22 @@ hcx_status finish_plan(Launch& LN, Plan& pl) {
   return HCX_OK;
 }
 
-// Waves per block of a persistent one-segment launch whose instance holds
+// Waves per block and blocks per CU of a persistent launch of `waves` waves.
+// request: waves per CU; 0: as many as fit; negative: that many fewer (room for
+// other solves in flight).  A request is never exceeded.
+// Blocks of several waves only in one-segment launches whose instance holds
 // the compact tables in LDS: the waves of a block share one copy of the
-// tables, so blocks of several waves can leave room for more waves per CU.
-// The candidate with the most resident waves per CU wins, the smaller block
-// on ties; a launch of `waves` waves takes no block that would leave a CU
-// without one (blocks of 4 waves put 640 waves on 160 CUs).
+// tables, so they can leave room for more waves per CU.  The candidate with
+// the most resident waves per CU within the request wins, the smaller block
+// on ties; a launch takes no block that would leave a CU without one (blocks of
+// 4 waves put 640 waves on 160 CUs).
 // Against 1, 2 or 4 waves for any launch: n = 12, mixed, 21 KB per wave: 7 waves
 // in place of 6, 150.3 -> 137.4 ms; 64 instances of n = 16 on 1280 waves: 5
 // waves per CU in one block, 5.26 -> 4.84 ms.
-hcx_status choose_waves_per_block(Launch& LN, Plan& pl, long long waves, int& best_wpb, int& best_nb) {
-  best_wpb = 1;
-  best_nb = 0;
-  int best_waves = -1;
-  const int most = std::min(8, 4 * waves_per_simd(pl.nmax, pl.exact));
+hcx_status launch_density(Launch& LN, Plan& pl, long long waves, int request, int& blocks_per_cu) {
+  const bool wide = LN.nseg == 1 && pl.tab_lds > 0;
+  const int most = wide ? std::min(8, 4 * waves_per_simd(pl.nmax, pl.exact)) : 1;
+  int resident[9] = {}, full = 1;
   for (int wpb = 1; wpb <= most && (wpb == 1 || waves >= (long long)wpb * g_cu); ++wpb) {
     LN.wpb = wpb;
     Plan q = pl;
@@ -775,13 +777,19 @@ hcx_status choose_waves_per_block(Launch& LN, Plan& pl, long long waves, int& be
     int nb = 0;
     HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(pl.fn), 64 * wpb,
                                                          q.lds));
-    if (nb * wpb > best_waves) {
-      best_waves = nb * wpb;
-      best_wpb = wpb;
-      best_nb = nb;
+    resident[wpb] = nb * wpb;
+    full = std::max(full, resident[wpb]);
+  }
+  const int limit = request > 0 ? request : std::max(full + request, 1);
+  int best = -1;
+  for (int wpb = 1; wpb <= std::min(most, limit); ++wpb) {
+    const int w = std::min(resident[wpb], limit / wpb * wpb);
+    if (w > best) {
+      best = w;
+      LN.wpb = wpb;
     }
   }
-  LN.wpb = best_wpb;
+  blocks_per_cu = limit / LN.wpb;
   return finish_plan(LN, pl);
 }
 
@@ -1539,34 +1547,17 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
       total_groups_needed = seg_groups[0];
     }
   }
+  // grid: persistent -> limited by occupancy or the requested waves per CU,
+  // split over segments by work
   LN.wpb = 1;
-  int occ_blocks = -1;  // blocks per CU at full occupancy, when already known
-  if (persistent && nseg == 1 && pl.tab_lds > 0) {
-    int wpb = 1;
-    st = choose_waves_per_block(LN, pl, total_groups_needed, wpb, occ_blocks);
-  } else {
-    st = finish_plan(LN, pl);
-  }
-  if (st != HCX_OK) return st;
-  const int wpb = LN.wpb;
-
-  // grid: persistent -> occupancy-limited, split over segments by work
   long long blocks;
   if (persistent) {
-    int per_cu = o->waves_per_cu;  // waves per CU
-    if (per_cu == 0 && all_tuned && nseg == 1) per_cu = probs[0]->tuned_wpc;
-    if (per_cu <= 0) {
-      // occupancy, less -waves_per_cu waves when that is negative (room for
-      // the work of other solves in flight on other streams)
-      int nb = occ_blocks;
-      if (nb < 0)
-        HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(pl.fn), 64 * wpb,
-                                                             pl.lds));
-      per_cu = std::max(nb * wpb + std::min(per_cu, 0), 1);
-    }
-    // blocks of wpb waves: waves per CU rounded up to whole blocks
+    int request = o->waves_per_cu, per_cu = 1;
+    if (request == 0 && all_tuned && nseg == 1) request = probs[0]->tuned_wpc;
     const long long waves_needed = std::max<long long>(total_groups_needed, 1);
-    blocks = std::min<long long>((long long)((per_cu + wpb - 1) / wpb) * g_cu, (waves_needed + wpb - 1) / wpb);
+    st = launch_density(LN, pl, waves_needed, request, per_cu);
+    if (st != HCX_OK) return st;
+    blocks = std::min<long long>((long long)per_cu * g_cu, (waves_needed + LN.wpb - 1) / LN.wpb);
     // proportional split by estimated work (paths * n^2 as a cost proxy)
     std::vector<double> w(nseg);
     double wsum = 0;
@@ -1585,6 +1576,8 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     if (acc < blocks) blocks = std::max<long long>(acc, 1);
     if (acc == 0) blocks = 1;
   } else {
+    st = finish_plan(LN, pl);
+    if (st != HCX_OK) return st;
     long long acc = 0;
     for (int s = 0; s < nseg; ++s) {
       LN.first_block[s] = (int)acc;
@@ -1593,6 +1586,7 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     LN.first_block[nseg] = (int)acc;
     blocks = std::max<long long>(acc, 1);
   }
+  const int wpb = LN.wpb;
   int max_inst = 1;
   for (int s = 0; s < nseg; ++s) max_inst = std::max(max_inst, LN.seg[s].I);
   dim3 ig((max_inst + 255) / 256, nseg);
@@ -1877,7 +1871,7 @@ hcx_status hcx_autotune(hcx_problem* p, const hcx_batch_desc* sample, const hcx_
   std::vector<Cand> cands;
   int occ = 0;
   {
-    // occupancy of the default shape, to derive the half-density candidate
+    // waves per CU of the default shape, to derive the half-density candidate
     Plan pl;
     int G = G0;
     if (choose_kernel(1, &p, &G, p->deg, o->precision, 1, pl) == HCX_OK) {
@@ -1886,8 +1880,10 @@ hcx_status hcx_autotune(hcx_problem* p, const hcx_batch_desc* sample, const hcx_
       SegOut O;
       LN.nseg = 1;
       seg_from_problem(LN.seg[0], O, p, G, pl);
-      if (finish_plan(LN, pl) == HCX_OK)
-        (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, reinterpret_cast<const void*>(pl.fn), 64, pl.lds);
+      int nb = 0;
+      if (ensure_device_info() == HCX_OK &&
+          launch_density(LN, pl, (P + 64 / G - 1) / (64 / G), 0, nb) == HCX_OK)
+        occ = nb * LN.wpb;
     }
   }
   for (int spec = 1; spec >= (G0 == p->n ? 0 : 1); --spec) {
