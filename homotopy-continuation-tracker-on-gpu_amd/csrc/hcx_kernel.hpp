@@ -329,7 +329,6 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
   HCX_WAVE_SYNC();
   // the group's largest key for step k, and this lane's
   decltype(pivot_key(T(0), 0)) key = 0, own = 0;
-  bool cand = false;
   auto largest = [&](int k, bool in, auto v) {
     using V = decltype(v);
     using W = std::conditional_t<sizeof(V) == 4, key32, key64>;
@@ -344,7 +343,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
     return m;
   };
   auto search = [&](int k) {
-    cand = row && label >= k;
+    const bool cand = row && label >= k;
     own = cand ? pivot_key(cabs1(A[k]), label) : 0;
     key = largest(k, cand, own);
   };
@@ -384,7 +383,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
       if constexpr (sizeof(T) == 8) {
         if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
           const unsigned long long rest =
-              largest(k, cand && same_upper(own, key), pivot_rest(cabs1(A[k]), label));
+              largest(k, row && label >= k && same_upper(own, key), pivot_rest(cabs1(A[k]), label));
           blabel = 31 - (int)((unsigned int)rest & 31u);
           singular = singular || (key < 32u && rest << 1 < 64u);
           piv = row && label == blabel;
@@ -497,12 +496,11 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
   if (row && g.s == 0) keys[g.gl] = 0ull;
   HCX_WAVE_SYNC();
   unsigned int key = 0, own = 0;
-  bool cand = false;
   cx<double> ck = cmk<double>(0, 0);
   auto search = [&](int k) {
     const int so = k % R, io = k / R;
     if (g.in_grp) cols[g.s * g.G + g.gl] = B[io];
-    cand = row && label >= k && g.s == so;
+    const bool cand = row && label >= k && g.s == so;
     own = cand ? pivot_key(cabs1(B[io]), label) : 0u;
     __hip_atomic_fetch_max(reinterpret_cast<key32*>(cand ? &keys[k] : no_key), own, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WAVEFRONT);
@@ -538,7 +536,7 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
       };
       publish();
       if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
-        const bool c = cand && same_upper(own, key);
+        const bool c = row && label >= k && g.s == so && same_upper(own, key);
         __hip_atomic_fetch_max(reinterpret_cast<key64*>(c ? &keys[k] : no_key),
                                c ? pivot_rest(cabs1(B[io]), label) : 0ull, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WAVEFRONT);
