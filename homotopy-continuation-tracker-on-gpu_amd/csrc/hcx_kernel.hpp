@@ -184,6 +184,14 @@ __device__ __forceinline__ unsigned long long pivot_rest(double mag, int label) 
 // A group's key words hold one kind or the other.
 typedef unsigned int __attribute__((may_alias)) key32;
 typedef unsigned long long __attribute__((may_alias)) key64;
+// A group has few of them, used in turn and cleared together when the steps
+// come round (every step's result has been read by then): a word per step took
+// up to 256 bytes of a region, which refused problems of the widest tables.
+constexpr int kKeyWords = 4;
+__device__ __forceinline__ void clear_keys(unsigned long long* keys, const Group& g, bool row) {
+  if (row && g.s == 0 && g.gl < kKeyWords) keys[g.gl] = 0ull;
+  HCX_WAVE_SYNC();
+}
 __device__ __forceinline__ bool same_upper(unsigned int a, unsigned int b) { return (a ^ b) < 32u; }
 // Whether a search of the wave is still open: more than one candidate shares a
 // key's upper bits, or these are 0 (the group's other lanes hold key 0).  One
@@ -303,7 +311,7 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 //    updated, and the remaining columns are updated while it is under way;
 //  * every candidate computes the reciprocal of its own entry during the
 //    search, and the pivot's goes out with its row.
-// keys: NMAX LDS slots of the group (unused with GC > 0).
+// keys: kKeyWords LDS words of the group (unused with GC > 0).
 // Where n is not a compile-time constant (generic instances) the columns are
 // checked against it four at a time: columns n..NMAX-1 hold values that no
 // step uses.
@@ -322,9 +330,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
   // of its own among the group's x slots.
   constexpr int kXWords = 2 * (NMAX + 2);
   unsigned long long* const no_key = keys - kXWords + (g.gl + g.s * g.G) % kXWords;
-  if constexpr (GC == 0) {
-    if (row && g.s == 0) keys[g.gl] = 0ull;
-  }
+  if constexpr (GC == 0) clear_keys(keys, g, row);
   // sp shares the group's LDS slots with x: the evaluation's reads of x come first
   HCX_WAVE_SYNC();
   // the group's largest key for step k, and this lane's
@@ -334,11 +340,11 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
     using W = std::conditional_t<sizeof(V) == 4, key32, key64>;
     if constexpr (GC > 0) return group_max_key<GC>(in ? v : V(0));
     const bool mine = in && g.s == 0;
-    __hip_atomic_fetch_max(reinterpret_cast<W*>(mine ? &keys[k] : no_key), mine ? v : V(0), __ATOMIC_RELAXED,
+    __hip_atomic_fetch_max(reinterpret_cast<W*>(mine ? &keys[k % kKeyWords] : no_key), mine ? v : V(0), __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WAVEFRONT);
     // requested ahead of the rest of the pivot row
     HCX_WAVE_SYNC();
-    const V m = *reinterpret_cast<W*>(&keys[k]);
+    const V m = *reinterpret_cast<W*>(&keys[k % kKeyWords]);
     HCX_WAVE_SYNC();
     return m;
   };
@@ -406,6 +412,7 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
       cx<T> l = cmul_fused(A[k], rp);
       l = cmk<T>(upd ? l.re : T(0), upd ? l.im : T(0));
       if (more) {
+        if (GC == 0 && (k + 1) % kKeyWords == 0) clear_keys(keys, g, row);
         A[k + 1] = cfnms(A[k + 1], l, next);
         search(k + 1);
       }
@@ -493,7 +500,7 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
   constexpr int kXWords = 2 * (NMAX + 2);
   unsigned long long* const no_key = keys - kXWords + (g.gl + g.s * g.G) % kXWords;
   cx<double>* const mine = prow + g.s;
-  if (row && g.s == 0) keys[g.gl] = 0ull;
+  clear_keys(keys, g, row);
   HCX_WAVE_SYNC();
   unsigned int key = 0, own = 0;
   cx<double> ck = cmk<double>(0, 0);
@@ -502,10 +509,10 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
     if (g.in_grp) cols[g.s * g.G + g.gl] = B[io];
     const bool cand = row && label >= k && g.s == so;
     own = cand ? pivot_key(cabs1(B[io]), label) : 0u;
-    __hip_atomic_fetch_max(reinterpret_cast<key32*>(cand ? &keys[k] : no_key), own, __ATOMIC_RELAXED,
+    __hip_atomic_fetch_max(reinterpret_cast<key32*>(cand ? &keys[k % kKeyWords] : no_key), own, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WAVEFRONT);
     HCX_WAVE_SYNC();
-    key = *reinterpret_cast<key32*>(&keys[k]);
+    key = *reinterpret_cast<key32*>(&keys[k % kKeyWords]);
     ck = cols[so * g.G + g.gl];
     HCX_WAVE_SYNC();
   };
@@ -537,11 +544,11 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
       publish();
       if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
         const bool c = row && label >= k && g.s == so && same_upper(own, key);
-        __hip_atomic_fetch_max(reinterpret_cast<key64*>(c ? &keys[k] : no_key),
+        __hip_atomic_fetch_max(reinterpret_cast<key64*>(c ? &keys[k % kKeyWords] : no_key),
                                c ? pivot_rest(cabs1(B[io]), label) : 0ull, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WAVEFRONT);
         HCX_WAVE_SYNC();
-        const unsigned long long rest = *reinterpret_cast<key64*>(&keys[k]);
+        const unsigned long long rest = *reinterpret_cast<key64*>(&keys[k % kKeyWords]);
         blabel = 31 - (int)((unsigned int)rest & 31u);
         singular = singular || (key < 32u && rest << 1 < 64u);
         piv = row && label == blabel;
@@ -554,6 +561,7 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
       cx<double> l = cmul_fused(ck, rp);
       l = cmk<double>(upd ? l.re : 0.0, upd ? l.im : 0.0);
       if (more) {
+        if ((k + 1) % kKeyWords == 0) clear_keys(keys, g, row);
         B[(k + 1) / R] = cfnms(B[(k + 1) / R], l, next);
         search(k + 1);
       }
@@ -606,14 +614,14 @@ __device__ __forceinline__ const Term* stage_terms(const Seg& S, int n, unsigned
 // starts with a wave-scope fence that keeps the evaluation's reads before its
 // writes.  KEYS: the instance searches
 // pivots through LDS (no DPP groups).
-constexpr int key_bytes(int nmax, bool keys) { return keys ? (8 * nmax + 15) & ~15 : 0; }
+constexpr int key_bytes(bool keys) { return keys ? 8 * kKeyWords : 0; }
 template <int NMAX, bool KEYS>
 struct Lds {
   unsigned char* base;
   __device__ cx<double>* x64() const { return reinterpret_cast<cx<double>*>(base); }
   __device__ cx<double>* piv64() const { return x64(); }
   __device__ unsigned long long* keys() const { return reinterpret_cast<unsigned long long*>(x64() + (NMAX + 2)); }
-  __device__ unsigned char* coef() const { return base + 16 * (NMAX + 2) + key_bytes(NMAX, KEYS); }
+  __device__ unsigned char* coef() const { return base + 16 * (NMAX + 2) + key_bytes(KEYS); }
   template <class T>
   __device__ cx<T>* x() const { return reinterpret_cast<cx<T>*>(base); }
   template <class T>

@@ -514,7 +514,7 @@ Opts to_opts(const hcx_track_opts* o) {
 // (64 banks x 4 bytes) for 8- and 16-byte accesses.
 int lds_group_bytes(int nmax, bool keys, int slots, int M, bool dot_lds = false) {
   const int per = (M > 1 || dot_lds) ? 32 : 16;
-  const int b = 16 * (nmax + 2) + dev::key_bytes(nmax, keys) + slots * per;
+  const int b = 16 * (nmax + 2) + dev::key_bytes(keys) + slots * per;
   return (((b + 15) / 16) | 1) * 16;
 }
 
@@ -1169,7 +1169,7 @@ hcx_status hcx_problem_create(const hcx_problem_desc* d, hcx_problem** out) {
     for (int c = 0; c <= C; c += 2) {
       // offsets from the group's region, whose coefficient area follows x and
       // the keys of the instance for n; 0: no slot
-      const int head = 16 * (n + 2) + dev::key_bytes(n, lat || !is_pow2(exact_lanes(n)));
+      const int head = 16 * (n + 2) + dev::key_bytes(lat || !is_pow2(exact_lanes(n)));
       auto off = [&](int q) { return q > C || cslot[q] >= nslot ? 0u : (uint32_t)(head + cslot[q] * 16); };
       w.push_back(off(c) | off(c + 1) << 16);
     }
