@@ -134,18 +134,19 @@ __device__ __forceinline__ double dpp_read(double v) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// Orders LDS traffic between the phases of a wave.  Kernels run with
-// 64-thread workgroups (one wave); a wave's LDS instructions execute in issue
+// Orders LDS traffic between the phases of a wave.  The waves of a block (up to
+// eight) share only the term records, complete before the path loop; the rest of
+// the LDS belongs to one wave each.  A wave's LDS instructions execute in issue
 // order, so a wave-scope fence (no memory-counter drain) is enough to keep the
 // compiler from moving LDS reads above the writes they depend on.
 #define HCX_WAVE_SYNC() __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront")
 
 // Group geometry of one lane.
-// A path's lanes: R replicas of G lanes each (R = 1 but in launches of few
-// paths).  The replicas hold identical path state and perform identical
-// operations, except that each sums every R-th term of the evaluation's
-// table rows; a butterfly over the replicas then gives all of them the same
-// full sums.
+// A path's lanes: R replicas of G lanes each (R = 1 but in FP64 launches of
+// few paths).  The replicas hold identical path state.  They share the evaluation
+// (each sums every R-th term of a row, or every R-th column whole) and the
+// solve (each holds every R-th column; the one-replica instance run with R > 1
+// solves in every replica, from sums that a butterfly makes equal).
 struct Group {
   int G;      // lanes per replica (rows / equations)
   int R;      // replicas per path

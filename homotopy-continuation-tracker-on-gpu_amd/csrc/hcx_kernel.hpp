@@ -677,6 +677,27 @@ enum : int {
 };
 
 
+// One evaluation of the mixed loop, at FP32 or FP64: the Jacobian's row into A,
+// the row of H or dH/dt (its coefficients at rhs) returned.
+template <class T, int NMAX, int DEG, bool LT, int NB, class SegT>
+__device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, const unsigned char* xb,
+                                             const unsigned char* cb, const unsigned char* rhs,
+                                             const unsigned char* lt, cx<T> (&A)[NMAX]) {
+  if (LT || lt) {
+    constexpr int HQ = (NMAX <= 6 && sizeof(T) == 8) || DEG > 4 ? 2 : 4;
+    eval_jac_blocks<NMAX, DEG, (DEG > 4 ? 2 : NB), 0, !LT && sizeof(T) == 4, T>(S, n, lt + gle * StreamRec<DEG>::kJ, 0,
+                                                                              xb, cb, A);
+    return eval_rhs_stream<DEG, false, HQ, (NMAX > 6), T>(S, n, gle, xb, rhs, rhs, nullptr, false, lt, 0, 1);
+  }
+  if constexpr (!LT) {
+    const cx<T>* const sx = reinterpret_cast<const cx<T>*>(xb);
+    eval_jac_terms<NMAX, DEG, T>(S, n, gle, sx, reinterpret_cast<const cx<T>*>(cb), A, nullptr, 0, 1);
+    return eval_rhs_terms<DEG, false, T>(S, n, gle, sx, reinterpret_cast<const cx<T>*>(rhs), nullptr, false, nullptr, 0,
+                                         1);
+  }
+  return cmk<T>(0, 0);
+}
+
 // Mixed-precision lane-group path loop: FP32 RK4 predictor (Jacobian, dH/dt
 // and solve of the four stages), FP64 Newton corrector (FP32 before the end
 // zone when o.newton32), FP64 refinement; a path that ends without a refined
@@ -697,25 +718,6 @@ enum : int {
 // 53% busy at 6 waves).  n = 12, 240 coefficients, degrees 2 and 3, 512 x 1024
 // paths: 159.5 -> 150.3 ms over the padded tables, 137.4 ms with 7 waves for 6,
 // 135.1 with every gather of a round requested up front.
-template <class T, int NMAX, int DEG, bool LT, int NB, class SegT>
-__device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, const unsigned char* xb,
-                                             const unsigned char* cb, const unsigned char* rhs,
-                                             const unsigned char* lt, cx<T> (&A)[NMAX]) {
-  if (LT || lt) {
-    constexpr int HQ = (NMAX <= 6 && sizeof(T) == 8) || DEG > 4 ? 2 : 4;
-    eval_jac_blocks<NMAX, DEG, (DEG > 4 ? 2 : NB), 0, !LT && sizeof(T) == 4, T>(S, n, lt + gle * StreamRec<DEG>::kJ, 0,
-                                                                              xb, cb, A);
-    return eval_rhs_stream<DEG, false, HQ, (NMAX > 6), T>(S, n, gle, xb, rhs, rhs, nullptr, false, lt, 0, 1);
-  }
-  if constexpr (!LT) {
-    const cx<T>* const sx = reinterpret_cast<const cx<T>*>(xb);
-    eval_jac_terms<NMAX, DEG, T>(S, n, gle, sx, reinterpret_cast<const cx<T>*>(cb), A, nullptr, 0, 1);
-    return eval_rhs_terms<DEG, false, T>(S, n, gle, sx, reinterpret_cast<const cx<T>*>(rhs), nullptr, false, nullptr, 0,
-                                         1);
-  }
-  return cmk<T>(0, 0);
-}
-
 template <int NMAX, int DEG, bool EXACT, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
 __device__ __forceinline__ void run_segment_mixed(const Launch& LN, int si, unsigned char* smem, int lane) {
   Seg S = LN.seg[si];
@@ -1087,8 +1089,9 @@ __device__ __forceinline__ void run_segment_fp64(const Launch& LN, int si, unsig
   const double2 *hxi = S.chx, *hti = S.cht;
   // dc/dt of the RK4 stages: constant (M = 1) -> read from the instance's
   // table in global memory (half the group's LDS), unless the launch stages
-  // it in LDS (dot_lds: launches of few paths, latency bound); M > 1 -> LDS
-  const bool gdot = S.M == 1 && !LN.dot_lds;
+  // it in LDS (dot_lds: launches of few paths, and every latency instance);
+  // M > 1 -> LDS
+  const bool gdot = REP == 0 && S.M == 1 && !LN.dot_lds;
 
   long long path = -1;
   int inst = 0, root = 0;

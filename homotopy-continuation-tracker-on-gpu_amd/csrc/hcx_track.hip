@@ -1623,8 +1623,8 @@ hcx_status track_impl(int nseg, hcx_problem* const* probs, const hcx_batch_desc*
     st = finish_plan(L2, p2);
     if (st != HCX_OK) return st;
     // as many waves as the GPU holds, shared out by the segments' paths: of a
-    // batch of diverging paths most are re-tracked (about one wave per CU took
-    // 40.8 ms of 10,200 of n = 12, all that fit 24.1 ms).  The waves that a list
+    // batch of diverging paths most are re-tracked (12,288 of n = 12: 40.8 ms on
+    // about one wave per CU, 24.1 on all that fit).  The waves that a list
     // has no paths for end at once (run_segment_fp64), so the usual list, of few
     // paths, costs what it did.
     int occ = 0;

@@ -96,3 +96,29 @@ def test_batch_without_a_path_for_fp32(hcx_mod, gpu, n, waves):
     for key in ("steps", "newton", "refine", "t_final", "roots"):
         assert np.array_equal(m[key], f[key], equal_nan=True), key
     prob.close()
+
+
+def test_captured_retrack(hcx_mod, gpu):
+    """Both rounds of the pass in a captured launch of two types: every replay
+    gives the eager launch's results."""
+    import torch
+    hcx = hcx_mod
+    problems, batches = zip(*(jump_and_escalate(hcx, n) for n in (5, 7)))
+    opts = hcx.default_opts(precision=1, **OPTS)
+    eager = [r.to_host() for r in hcx.track_multi(problems, batches, opts)]
+    assert all((e["flags"] & hcx.FLAG_ESCALATED).all() for e in eager)
+    graph = hcx.Graph(problems, batches, opts)
+    for _ in range(4):
+        for r in graph.results:
+            r.flags.zero_()
+            r.roots.zero_()
+        hcx.track_multi(problems, batches, opts)
+        replay = graph.launch()
+        torch.cuda.synchronize()
+        for r, e in zip(replay, eager):
+            g = r.to_host()
+            for key in ("flags", "steps", "newton", "refine", "roots"):
+                assert np.array_equal(g[key], e[key], equal_nan=True), key
+    graph.close()
+    for p in problems:
+        p.close()
