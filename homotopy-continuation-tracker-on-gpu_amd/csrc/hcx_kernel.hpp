@@ -165,18 +165,18 @@ __device__ __forceinline__ T group_max(T v, const Group& g) {
 // largest key is the largest magnitude and, among equal ones, the first row in
 // current row order.  A row that is no candidate holds key 0; NaN orders above
 // every number.  An FP32 key is two words and holds the whole magnitude (0: a key below 32).
-// An FP64 key is one word, the upper 27 bits without the sign: candidates that
-// share these (one pair in 2^16 of unrelated ones, and exact ties) are compared
-// by the other bits and the label in a second search (pivot_rest), so the pivot
-// is that of the whole magnitudes.
+// An FP64 key is one word, the upper 27 bits without the sign.  Where candidates
+// share these (one pair in 2^16 of unrelated ones, and exact ties), the key's
+// pivot is compared with them, and a larger one is found in a second search over
+// the other bits and the label (pivot_rest), so the pivot is that of the whole
+// magnitudes.
 __device__ __forceinline__ unsigned long long pivot_key(float mag, int label) {
   return ((unsigned long long)(__float_as_uint(mag) & 0x7fffffffu) << 32) | (unsigned int)(31 - label);
 }
 __device__ __forceinline__ unsigned int pivot_key(double mag, int label) {
   return ((unsigned int)((unsigned long long)__double_as_longlong(mag) >> 31) & ~31u) | (unsigned int)(31 - label);
 }
-// The bits that the FP64 key leaves out, above 31 - label; bit 63 is set.  A
-// magnitude is 0 where its key is below 32 and this below 32 without bit 63.
+// The bits that the FP64 key leaves out, above 31 - label; bit 63 is set.
 __device__ __forceinline__ unsigned long long pivot_rest(double mag, int label) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(mag) & ((1ull << 36) - 1);
   return 1ull << 63 | b << 5 | (unsigned int)(31 - label);
@@ -304,9 +304,12 @@ __device__ __forceinline__ void group_sum2(double& a, double& b, const Group& g,
 //    LDS maximum per group and step (one instruction and one read in place of
 //    a scan of every candidate's magnitude);
 //  * whether an FP64 key left candidates to compare further (pivot_open) is
-//    looked at while the pivot's row is on its way; then the row goes out again.
-//    Against keys of 59 bits that called the rest equal: n = 3 and 5 in lone
-//    launches +1.6%, n = 9 +0.8%, n = 30 -2.9% (DPP steps on one word);
+//    looked at while the pivot's row is on its way; if a larger one is found the
+//    row goes out again.  Against keys of 59 bits that called the rest equal:
+//    lone launches of n = 3 and 5 +0.2 and +1.1%, n = 12 -0.8%, n = 30 -3.1%
+//    (DPP steps on one word); generalized_3views_4pts, whose columns hold equal
+//    magnitudes at most steps, 1.31 -> 1.39 ms (1.47 with a second search for
+//    every tie);
 //  * the next step's candidates enter their search as soon as their column is
 //    updated, and the remaining columns are updated while it is under way;
 //  * every candidate computes the reciprocal of its own entry during the
@@ -388,12 +391,29 @@ __device__ __forceinline__ cx<T> group_lu_solve(cx<T> (&A)[NMAX], cx<T> b, const
       // while the row is on its way: is the pivot the only one of its key?
       if constexpr (sizeof(T) == 8) {
         if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
-          const unsigned long long rest =
-              largest(k, row && label >= k && same_upper(own, key), pivot_rest(cabs1(A[k]), label));
-          blabel = 31 - (int)((unsigned int)rest & 31u);
-          singular = singular || (key < 32u && rest << 1 < 64u);
-          piv = row && label == blabel;
-          publish();
+          // the key's pivot against the others that share its bits: nothing
+          // changes where they are equal (ties go to the first row)
+          const double mag = cabs1(A[k]);
+          const bool near = row && label >= k && same_upper(own, key);
+          double top;
+          if constexpr (GC > 0) {
+            top = lane_read(mag, g.gbase + __builtin_ctzll(__ballot(piv) >> g.gbase));
+          } else {
+            double* const w = reinterpret_cast<double*>(&keys[k % kKeyWords]);
+            if (piv && g.s == 0) *w = mag;
+            HCX_WAVE_SYNC();
+            top = *w;
+            HCX_WAVE_SYNC();
+          }
+          bool zero = top == 0.0;
+          if (__ballot(near && mag > top) & part) {
+            const unsigned long long rest = largest(k, near, pivot_rest(mag, label));
+            blabel = 31 - (int)((unsigned int)rest & 31u);
+            zero = key < 32u && rest << 1 < 64u;
+            piv = row && label == blabel;
+            publish();
+          }
+          singular = singular || zero;
         }
       }
       if (piv) own_rinv = rinv;
@@ -543,17 +563,27 @@ __device__ __forceinline__ cx<double> group_solve_split(cx<double> (&B)[NC], con
       };
       publish();
       if (__builtin_expect(pivot_open(own, key, part, searches), 0)) {
-        const bool c = row && label >= k && g.s == so && same_upper(own, key);
-        __hip_atomic_fetch_max(reinterpret_cast<key64*>(c ? &keys[k % kKeyWords] : no_key),
-                               c ? pivot_rest(cabs1(B[io]), label) : 0ull, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_WAVEFRONT);
+        const double mag = cabs1(B[io]);
+        const bool near = row && label >= k && g.s == so && same_upper(own, key);
+        double* const w = reinterpret_cast<double*>(&keys[k % kKeyWords]);
+        if (piv && g.s == so) *w = mag;
         HCX_WAVE_SYNC();
-        const unsigned long long rest = *reinterpret_cast<key64*>(&keys[k % kKeyWords]);
-        blabel = 31 - (int)((unsigned int)rest & 31u);
-        singular = singular || (key < 32u && rest << 1 < 64u);
-        piv = row && label == blabel;
+        const double top = *w;
         HCX_WAVE_SYNC();
-        publish();
+        bool zero = top == 0.0;
+        if (__ballot(near && mag > top) & part) {
+          __hip_atomic_fetch_max(reinterpret_cast<key64*>(near ? &keys[k % kKeyWords] : no_key),
+                                 near ? pivot_rest(mag, label) : 0ull, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_WAVEFRONT);
+          HCX_WAVE_SYNC();
+          const unsigned long long rest = *reinterpret_cast<key64*>(&keys[k % kKeyWords]);
+          blabel = 31 - (int)((unsigned int)rest & 31u);
+          zero = key < 32u && rest << 1 < 64u;
+          piv = row && label == blabel;
+          HCX_WAVE_SYNC();
+          publish();
+        }
+        singular = singular || zero;
       }
       label = piv ? k : (label == k ? blabel : label);
       own_rinv = cmk<double>(piv ? rp.re : own_rinv.re, piv ? rp.im : own_rinv.im);
