@@ -217,8 +217,8 @@ __device__ __forceinline__ void eval_jac_rounds(const SegT& S, int n, int gle, c
     const unsigned char* rp = lt + gle * RS;
 #pragma unroll
     for (int jb = 0; jb < NMAX; jb += NB) {
-      // generic instances skip blocks of no column, where there are many (n = 3,
-      // degree 5, 1024 waves 6.31 -> 4.59 ms; in larger blocks the branches cost more)
+      // generic instances skip the blocks of absent columns (n = 3, degree 5, 1024
+      // waves: 6.31 -> 4.59 ms)
       if (DEG > 4 && jb >= n) continue;
       uint32_t r[NB][4];
 #pragma unroll

@@ -744,8 +744,8 @@ __device__ __forceinline__ cx<T> eval_system(const SegT& S, int n, int gle, cons
 // share the coefficient area.
 // NB: Jacobian columns evaluated together (twice as many in FP32 were no
 // faster: the rounds of a block are its longest column's).
-// Bound by latency at the 7 waves per CU that its LDS allows (VALU 52% and LDS
-// 53% busy at 6 waves).  n = 12, 240 coefficients, degrees 2 and 3, 512 x 1024
+// Bound by latency at the 7 waves per CU that its LDS allows (VALU 57% and LDS
+// 61% busy).  n = 12, 240 coefficients, degrees 2 and 3, 512 x 1024
 // paths: 159.5 -> 150.3 ms over the padded tables, 137.4 ms with 7 waves for 6,
 // 135.1 with every gather of a round requested up front.
 template <int NMAX, int DEG, bool EXACT, int NB = (NMAX <= 6 ? 3 : (NMAX <= 16 ? 4 : 6))>
